@@ -45,6 +45,8 @@ struct rp3dg_batch {
     int* jt_ranges = nullptr;          // [2*slot] colour ranges of the joint rows, slots in solve order
     int2* jt_wr = nullptr;             // fused solver: [w * jt_slots + slot] joint rows of world w
     int jt_slots = 0;
+    std::vector<int> jt_kind;          // [slot] joint kind (JT_*) of the slot
+    int* d_jt_kind = nullptr;
     std::vector<int> joint_order;      // global joint index of each joint row
     bool cur_is_a = true;
     int pair_cap = 0;
@@ -58,10 +60,14 @@ struct rp3dg_batch {
     int fused_block = 64;              // threads per world of the position kernel (and of the single-class solve)
     int color_block = 256;             // per-colour layout: threads per block of the colour kernels
     // fused layout: worlds grouped into size classes (bodies in (L/2, L], L = 64, 128, ... 4096), largest
-    // first; each class is one launch with its own workgroup size and LDS, the classes run concurrently
-    struct WorldClass { int first, count, max_bodies, block, lds_bodies; };
+    // first, `largest` bodies the largest); each class is one launch with its own workgroup size and LDS, the
+    // classes run concurrently
+    struct WorldClass { int first, count, max_bodies, largest, block; };
+    // LDS layout of a class's workgroups (STATE_* of solver_quad.h, bodies and manifolds held)
+    struct ClassLds { int state, bodies, rows; };
+    ClassLds class_lds(const WorldClass& c) const;
     std::vector<WorldClass> wclasses;
-    int block_div = 2;                 // class workgroup = clamp(L / block_div, 64, 256) (autotuned)
+    int block_div = 2;                 // class workgroup = clamp(2 L / block_div, 64, 1024) (autotuned)
     std::vector<hipStream_t> side_streams;
     std::vector<hipEvent_t> fork_events;
     std::vector<std::pair<int, double>> tune_table;   // autotuner trials: (shape, ms per step)
@@ -201,7 +207,7 @@ struct rp3dg_batch {
     ~rp3dg_batch();
     int upload(rp3dg_world* const* worlds, int n, const rp3dg_batch_options* opt);
     void set_class_blocks();
-    int launch_world_classes(const char* name, const rp3dg::FusedArgs& F, bool lds);
+    int launch_world_classes(const char* name, const rp3dg::FusedArgs& F);
     int upload_joints(rp3dg_world* const* worlds, int n);
     void enqueue_sleep(float dt, const rp3dg::DevPairs& N, int pair_grid);
     int enqueue_step(float dt, bool capturing);

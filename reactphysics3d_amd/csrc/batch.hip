@@ -20,6 +20,7 @@
 #include "kcommon.h"
 #include "narrowphase.h"
 #include "solver.h"
+#include "solver_quad.h"
 #include "world.h"
 
 namespace rp3dg {
@@ -426,6 +427,9 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     jt_slots = 0;
     for (int k = 0; k < JT_KINDS * 64; k++)
         if (slot_of[k] >= 0) slot_of[k] = jt_slots++;
+    jt_kind.clear();
+    for (int k = 0; k < JT_KINDS * 64; k++)
+        if (slot_of[k] >= 0) jt_kind.push_back(k / 64);
     for (Row& r : rows) r.slot = slot_of[r.kind * 64 + r.color];
     const bool wmajor = fused;
     std::stable_sort(rows.begin(), rows.end(), [wmajor](const Row& a, const Row& b) {
@@ -454,9 +458,8 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     J.n = n;
     const size_t m = std::max(1, n);
     J.type = dalloc<int>(this, m); J.bodies = dalloc<int2>(this, m); J.flags = dalloc<int>(this, m);
-    for (float4** a : {&J.la1, &J.la2, &J.ax1, &J.ax2, &J.qinit, &J.lim, &J.impT, &J.impR, &J.impL, &J.i1r0, &J.i1r1,
-                       &J.i1r2, &J.i2r0, &J.i2r1, &J.i2r2, &J.r1, &J.r2, &J.kt0, &J.kt1, &J.kt2, &J.kr0, &J.kr1,
-                       &J.kr2, &J.a1, &J.b2xa1, &J.c2xa1, &J.un1, &J.un2, &J.ua, &J.rn1, &J.rn2, &J.ra})
+    for (float4** a : {&J.la1, &J.la2, &J.ax1, &J.ax2, &J.qinit, &J.lim, &J.impT, &J.impR, &J.impL, &J.r1, &J.r2,
+                       &J.kt0, &J.kt1, &J.kt2, &J.kr0, &J.kr1, &J.kr2, &J.a1, &J.b2xa1, &J.c2xa1, &J.un1, &J.un2, &J.ua, &J.rn1, &J.rn2, &J.ra})
         *a = dalloc<float4>(this, m);
     J.bias0 = dalloc<float4>(this, m);
     J.bias1 = dalloc<float4>(this, m);
@@ -479,7 +482,8 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     J.imm = dalloc<float>(this, m);
     jt_ranges = dalloc<int>(this, std::max<size_t>(2, ranges.size()));
     jt_wr = dalloc<int2>(this, wr.size());
-    if (!J.imlm || !J.imm || !jt_ranges || !jt_wr) { set_error("device allocation failed (joints)"); return RP3DG_EHIP; }
+    d_jt_kind = dalloc<int>(this, jt_kind.size());
+    if (!J.imlm || !J.imm || !jt_ranges || !jt_wr || !d_jt_kind) { set_error("device allocation failed (joints)"); return RP3DG_EHIP; }
     if (n == 0) return RP3DG_OK;
     std::vector<int> type(n), flags(n);
     std::vector<int2> bodies(n);
@@ -507,6 +511,7 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     HIPCHECK(hipMemset(J.imm, 0, sizeof(float) * n));
     if (!ranges.empty()) HIPCHECK(hipMemcpy(jt_ranges, ranges.data(), sizeof(int) * ranges.size(), hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(jt_wr, wr.data(), sizeof(int2) * wr.size(), hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(d_jt_kind, jt_kind.data(), sizeof(int) * jt_kind.size(), hipMemcpyHostToDevice));
     return RP3DG_OK;
 }
 
@@ -515,7 +520,7 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     rp3dg_batch_options o{};
     if (opt) o = *opt;
     if (o.solver < RP3DG_SOLVER_AUTO || o.solver > RP3DG_SOLVER_FUSED) { set_error("invalid solver layout"); return RP3DG_EINVAL; }
-    if (o.fused_block && (o.fused_block < 64 || o.fused_block > kFusedMaxBlock || o.fused_block % 64)) {
+    if (o.fused_block && (o.fused_block < 64 || o.fused_block > kPositionMaxBlock || o.fused_block % 64)) {
         set_error("fused_block must be a multiple of 64 in [64, 256]");
         return RP3DG_EINVAL;
     }
@@ -711,8 +716,6 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
         set_error("the fused solver layout takes worlds of up to 4096 bodies (use the per-colour layout)");
         return RP3DG_EINVAL;
     }
-    // (solver velocities and inverse inertia of worlds up to 512 bodies live in LDS during the sweeps,
-    // 112 B per body: see the world classes below)
     // world groups: consecutive worlds share a workgroup up to group_bodies bodies (64 worlds), so the
     // colour phases of small worlds fill the wavefronts; a larger world is a group of its own
     group_bodies = std::min(o.group_bodies ? o.group_bodies : 256, 512);
@@ -982,7 +985,7 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
                 int j = i;
                 while (j < ng && gsize(order[j]) > L / 2) j++;
                 if (L == 64) j = ng;   // everything up to 64 bodies is one class
-                wclasses.push_back({i, j - i, L, 64, L <= kFusedMaxLds ? L : 0});   // LDS: 64, 128, 256 or 512
+                wclasses.push_back({i, j - i, L, sz, 64});
                 i = j;
             }
             set_class_blocks();
@@ -1010,7 +1013,8 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     S.pair = dalloc<int>(this, man_cap); S.bodies = dalloc<int2>(this, man_cap); S.npts = dalloc<int>(this, man_cap);
     for (float4** a : {&S.n, &S.r1f, &S.r2f, &S.t1, &S.t2, &S.imp, &S.oldt1, &S.oldt2})
         *a = dalloc<float4>(this, man_cap);
-    for (float4** a : {&S.pn, &S.r1, &S.r2, &S.lam, &S.pred}) *a = dalloc<float4>(this, 4 * (size_t)man_cap);
+    for (float4** a : {&S.pn, &S.r1, &S.r2, &S.i1, &S.i2, &S.lam, &S.pred}) *a = dalloc<float4>(this, 4 * (size_t)man_cap);
+    S.lq = dalloc<float4>(this, 2 * (size_t)man_cap);
     scan_sums_cap = 1 << 16;
     scan_sums_buf = dalloc<int>(this, scan_sums_cap);
     sort_hist_cap = 256 * (std::max(man_cap, nc) / 4096 + 2);
@@ -1025,7 +1029,7 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     alloc_bytes.push_back(sizeof(DevCounters));
     HIPCHECK(hipHostMalloc(&hcounters, sizeof(DevCounters), hipHostMallocDefault));
     HIPCHECK(hipMemsetAsync(counters, 0, sizeof(DevCounters), stream));
-    if (!sort_offs || !S.lam) { set_error("device allocation failed (pair arenas)"); return RP3DG_EHIP; }
+    if (!sort_offs || !S.lam || !S.lq) { set_error("device allocation failed (pair arenas)"); return RP3DG_EHIP; }
     // collider creation: world transforms, initial fat AABBs, all colliders in the moved set
     bp_refit<<<grid_for(nc), 256, 0, stream>>>(B, C, d_hbounds, 1);
     HIPCHECK(hipGetLastError());
@@ -1336,7 +1340,6 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     SA.restitution_threshold = settings.restitution_threshold;
     SA.learned = learned ? 1 : 0;
     SA.adj_offs = adj_offs;
-    SA.split = settings.split_impulse;
     const float beta_dt = 0.2f / dt;
 
     if (fused) {
@@ -1347,6 +1350,7 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         F.settings = settings;
         F.seg_start = seg_start;
         F.jt_wr = jt_wr;
+        F.jt_kind = d_jt_kind;
         F.jt_slots = jt_slots;
         F.wbody = d_wbody;
         F.wcoll = d_wcoll;
@@ -1364,35 +1368,28 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         F.nrows = &counters->nb_new_points;
         F.feat_cap = feat_cap;
         F.row_slot = row_slot;
-        F.lds_bodies = 0;
-        F.lds_residual = 0;
-        F.feats = nullptr;
-        F.phase = 2;
+        F.lds_bodies = F.lds_rows = 0;
+        F.feats = features ? feat_buf : nullptr;
+        if (J.bfirst) LAUNCH_T("fill_int", grid_for(nworlds), 256, fill_int, J.bfirst, nworlds, INT_MAX);
+        LAUNCH_T("sv_setup", grid_for(nb + hm + J.n + 128), 256, sv_setup, SA, J, settings, dt);
         if (res_thr > 0.0f && order_by_sweeps && !wclasses.empty())   // residual mode: groups differ in length
             LAUNCH_TS("sv_order_groups", (int)wclasses.size(), 256, 0, sv_order_groups, d_block_static, d_gworld,
                       world_iters, d_block_world, d_class_ranges, (int)wclasses.size());
-        if (!features) {
-            r = launch_world_classes("sv_world_solve", F, true);
-            if (r) return r;
-        } else {
-            F.feats = feat_buf;
-            F.phase = 0;
-            if (settings.split_impulse) LAUNCH_TS("sv_world_prepare", ngroups, fused_block, 0, sv_world_solve<true>, F);
-            else LAUNCH_TS("sv_world_prepare", ngroups, fused_block, 0, sv_world_solve<false>, F);
+        if (features) {
+            LAUNCH_T("sv_features", mg, 256, sv_features, F);
             if (SA.learned) {
                 const int rows = capturing ? feat_cap : std::min(feat_cap, last.nb_new_points + last.nb_new_points / 4 + 1024);
                 const int grid = std::max(1, std::min(2048, (rows + 63) / 64));
                 LAUNCH_T("mlp_infer", grid, 256, mlp_infer, mlp_view(mlp), feat_buf, &counters->nb_new_points, feat_cap,
                          nullptr, row_slot, S.pred);
             }
-            F.phase = 1;
-            r = launch_world_classes("sv_world_solve", F, true);
-            if (r) return r;
-            if (log_cap > 0) {
-                LAUNCH_T("sv_log_samples", grid_for(feat_cap), 256, sv_log_samples, F, log_feats, log_targets, log_count,
-                         log_cap);
-                sv_log_advance<<<1, 1, 0, stream>>>(&counters->nb_new_points, feat_cap, log_count, log_cap);
-            }
+        }
+        r = launch_world_classes("sv_world_solve", F);
+        if (r) return r;
+        if (log_cap > 0) {
+            LAUNCH_T("sv_log_samples", grid_for(feat_cap), 256, sv_log_samples, F, log_feats, log_targets, log_count,
+                     log_cap);
+            sv_log_advance<<<1, 1, 0, stream>>>(&counters->nb_new_points, feat_cap, log_count, log_cap);
         }
         LAUNCH_T("world_position", ngroups, fused_block, world_position, F);
         enqueue_sleep(dt, N, pg);
@@ -1405,23 +1402,23 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     HIPCHECK(hipStreamSynchronize(stream));
     const int ncol = hcounters->nb_colors;
     const int bg = grid_for(nb);
-    // inverse world inertia + velocity integration (PhysicsWorld.cpp:266-272)
-    LAUNCH_T("dyn_integrate_velocities", bg, 256, dyn_integrate_velocities, B, settings, dt);
+    // inverse world inertia + velocity integration (PhysicsWorld.cpp:266-272), contact and joint rows
+    if (J.bfirst) LAUNCH_T("fill_int", grid_for(nworlds), 256, fill_int, J.bfirst, nworlds, INT_MAX);
+    LAUNCH_T("sv_setup", grid_for(nb + hm + J.n + 128), 256, sv_setup, SA, J, settings, dt);
     // contact solver (PhysicsWorld.cpp:321-345)
-    const int jg = grid_for(std::max(J.n, 1));
-    LAUNCH_T("sv_prepare", mg, 256, sv_prepare, SA);
+    const int jg = grid_for(std::max(J.n, 1)), jg2 = grid_for(std::max(2 * J.n, 1));
     const int cg = grid_for(hm / std::max(1, ncol) + 1, color_block);
+    const int qg = grid_for(4 * (hm / std::max(1, ncol) + 1), color_block);
     for (int c = 0; c < ncol; c++) LAUNCH_T("sv_warmstart", cg, color_block, sv_warmstart, SA, c);
-    // ConstraintSolverSystem::initialize: initBeforeSolve + warm start of every joint kind
-    if (J.n > 0) {
-        if (J.bfirst) LAUNCH_T("fill_int", grid_for(nworlds), 256, fill_int, J.bfirst, nworlds, INT_MAX);
-        LAUNCH_T("jt_init", jg, 256, jt_init, B, J, dt);
-        for (int s = 0; s < jt_slots; s++) LAUNCH_T("jt_warmstart", jg, 256, jt_warmstart, B, J, jt_ranges, s);
-    }
+    // ConstraintSolverSystem::initialize: warm start of every joint kind
+    for (int s = 0; s < jt_slots; s++) LAUNCH_T("jt_warmstart", jg, 256, jt_warmstart, B, J, jt_ranges, s);
     for (int it = 0; it < settings.vel_iters; it++) {
         for (int s = 0; s < jt_slots; s++)
-            LAUNCH_T("jt_solve_velocity", jg, 256, jt_solve_velocity, B, J, jt_ranges, s, dt);
-        for (int c = 0; c < ncol; c++) LAUNCH_T("sv_solve_color", cg, color_block, sv_solve_color, SA, c, beta_dt);
+            LAUNCH_T("jt_solve_velocity", jg2, 256, jt_solve_velocity, B, J, jt_ranges, s, jt_kind[s], dt);
+        for (int c = 0; c < ncol; c++) {
+            if (settings.split_impulse) LAUNCH_T("sv_solve_color", qg, color_block, sv_solve_color<true>, SA, c, beta_dt);
+            else LAUNCH_T("sv_solve_color", qg, color_block, sv_solve_color<false>, SA, c, beta_dt);
+        }
     }
     LAUNCH_T("sv_store", mg, 256, sv_store, SA);
     // position integration, joint position correction, state update, refit (PhysicsWorld.cpp:275-288, :348-360)
@@ -1443,15 +1440,45 @@ void rp3dg_batch::enqueue_sleep(float dt, const DevPairs& N, int pair_grid) {
     LAUNCH_T("isl_sleep", pair_grid, 256, isl_reset_disabled_pairs, B, C, N, &counters->nb_pairs);
 }
 
-// Workgroup size of every world class: clamp(L / block_div, 64, 256).
+using SolveKernel = void (*)(FusedArgs);
+static const SolveKernel kSolveKernels[2][3] = {   // [split impulses][STATE_*]
+    {sv_world_solve<false, STATE_LDS>, sv_world_solve<false, STATE_VEL>, sv_world_solve<false, STATE_HBM>},
+    {sv_world_solve<true, STATE_LDS>, sv_world_solve<true, STATE_VEL>, sv_world_solve<true, STATE_HBM>}};
+
+// Workgroup size of every world class: clamp(2 L / block_div, 64, 1024).  Four lanes solve a manifold and
+// a world of n bodies has about n / 6 to n / 4 manifolds a colour, so L threads fill the colour phases.
 void rp3dg_batch::set_class_blocks() {
     for (WorldClass& c : wclasses)
-        c.block = user_block ? user_block : std::max(64, std::min(kFusedMaxBlock, c.max_bodies / block_div));
+        c.block = user_block ? user_block : std::max(64, std::min(kFusedMaxBlock, 2 * c.max_bodies / block_div));
+}
+
+// LDS of a class's workgroups.  The body state is staged whole when it fits (100 B a body, up to about
+// 1600 bodies), else the velocities alone (48 B, up to about 3300), else it stays in HBM; the rest of the
+// workgroup's share of the CU takes the impulses of its manifolds (48 B each; rows beyond it use HBM).
+// The share is what the number of workgroups in flight leaves: a launch with few groups gives each one the
+// whole CU, a full one as many as the registers admit (16 wavefronts a CU at 128 registers).
+rp3dg_batch::ClassLds rp3dg_batch::class_lds(const WorldClass& c) const {
+    constexpr size_t kStatic = 1024, kRow = 3 * sizeof(float4);   // the kernel's static LDS; bytes a manifold
+    const size_t cu = (size_t)max_lds_per_cu, block_max = (size_t)std::min(max_lds_per_block, max_lds_per_cu) - kStatic;
+    ClassLds l{STATE_LDS, (c.largest + 3) & ~3, 0};
+    if (fused_lds_bytes(STATE_LDS, l.bodies, 0) > block_max) l.state = STATE_VEL;
+    if (l.state == STATE_VEL && fused_lds_bytes(STATE_VEL, l.bodies, 0) > block_max) {
+        l.state = STATE_HBM;
+        l.bodies = 0;
+    }
+    const size_t base = fused_lds_bytes(l.state, l.bodies, 0);
+    int k = std::max(1, std::min(16 * kWave / c.block, (ngroups + 255) / 256));
+    const size_t rows_min = (size_t)(c.largest + c.largest / 8) * kRow;   // 1.1 manifolds a body
+    while (k > 1 && base + rows_min + kStatic > cu / k) k--;
+    const size_t share = std::min(cu / k, block_max + kStatic) - kStatic;
+    const size_t left = share > base ? share - base : 0;
+    l.rows = (int)std::min<size_t>(left / kRow, (size_t)4 * c.largest + 64);
+    return l;
 }
 
 // One launch per world class of the fused solver, each on its own stream between a fork and a join
 // event (captured as parallel graph branches), so small and large worlds share the CUs.
-int rp3dg_batch::launch_world_classes(const char* name, const FusedArgs& F0, bool lds) {
+int rp3dg_batch::launch_world_classes(const char* name, const FusedArgs& F0) {
     timer_begin(name);
     const int nclass = (int)wclasses.size();
     if (nclass > 1) {
@@ -1461,22 +1488,14 @@ int rp3dg_batch::launch_world_classes(const char* name, const FusedArgs& F0, boo
     for (int c = 0; c < nclass; c++) {
         const WorldClass& wc = wclasses[c];
         if (wc.count == 0) continue;
+        const ClassLds l = class_lds(wc);
         FusedArgs F = F0;
         F.block_world = d_block_world + wc.first;
-        F.lds_bodies = lds ? wc.lds_bodies : 0;
-        // the residual's previous velocities join the staged state when that costs no resident workgroup
-        // per CU: LDS bounds how many groups a CU holds, and fewer groups in flight cost more than the HBM
-        // round trips saved (measured: 9.0 -> 9.6 ms per launch on the 4096-world batch when the
-        // 256-body class dropped from five to four groups per CU)
-        {
-            const size_t base = fused_lds_bytes(F.lds_bodies, false) + 1024, with = fused_lds_bytes(F.lds_bodies, true) + 1024;
-            F.lds_residual = F.lds_bodies > 0 && F.res_thr > 0.0f && with <= (size_t)max_lds_per_block &&
-                             (size_t)max_lds_per_cu / with == (size_t)max_lds_per_cu / base;
-        }
-        const size_t shmem = fused_lds_bytes(F.lds_bodies, F.lds_residual != 0);
+        F.lds_bodies = l.bodies;
+        F.lds_rows = l.rows;
+        const size_t shmem = fused_lds_bytes(l.state, l.bodies, l.rows);
         hipStream_t s = c == 0 ? stream : side_streams[c - 1];
-        if (settings.split_impulse) sv_world_solve<true><<<wc.count, wc.block, shmem, s>>>(F);
-        else sv_world_solve<false><<<wc.count, wc.block, shmem, s>>>(F);
+        kSolveKernels[settings.split_impulse ? 1 : 0][l.state]<<<wc.count, wc.block, shmem, s>>>(F);
     }
     if (nclass > 1) {
         for (int c = 1; c < nclass; c++) {

@@ -1,9 +1,9 @@
 // Fused per-world solver for batches of many small worlds.
 //
-// One workgroup owns one group of consecutive worlds for the whole solver phase
-// of a step: velocity integration of its bodies, contact rows, joint rows, warm
-// start, every velocity iteration (colours and joint slots separated by
-// workgroup barriers), impulse store; a second kernel does position
+// sv_setup integrates the velocities and writes the contact and joint rows of the
+// whole batch.  Then one workgroup owns one group of consecutive worlds for the
+// sweeps: warm start, every velocity iteration (colours and joint slots separated
+// by workgroup barriers), impulse store; a third kernel does position
 // integration, the joint position iterations, the state update and the
 // fat-AABB refit.  Groups share nothing, so no grid-wide synchronisation and no
 // per-colour launches are needed.  Colour c of a group is colour c of each of
@@ -20,11 +20,14 @@
 // (PhysicsWorld.cpp:334).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "fused.h"
 #include "joints_dev.h"
 #include "kcommon.h"
 #include "refit_dev.h"
 #include "solver_dev.h"
+#include "solver_quad.h"
 
 namespace rp3dg {
 
@@ -40,43 +43,218 @@ __device__ __forceinline__ float block_maxf(float v, float* red) {
     return r;
 }
 
-// Warm start, velocity iterations and impulse store of one group.  Instantiated twice: with the body
-// state in LDS (A.B's velocity, inertia and flag arrays point into the workgroup's LDS, so every access
-// compiles to an LDS instruction) and with it in HBM (groups larger than the LDS budget).
-// PV / PW: the velocities after the previous sweep (residual mode), indexed by body - b0, in LDS or HBM.
-template <bool SPLIT>
-__device__ __forceinline__ void group_sweeps(const FusedArgs& F, const SvArgs& A, const DevBodies& B, bool staged,
-                                             int w0, int ngw, int b0, int b1, int m1, const int* seg, const int2* jr,
-                                             float* red, unsigned int* s_wres, unsigned long long* s_done,
-                                             float4* PV, float4* PW) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int nbw = b1 - b0;
-    const DevBodies& BS = A.B;
-    // contact warm start, colour by colour (CS.cpp:326-476)
-    for (int c = 0; c < kMaxColors; c++) {
-        const int lo = seg[c], hi = seg[c + 1];
-        if (lo == m1) break;
-        for (int i = lo + tid; i < hi; i += nt) sv_warmstart_one(A, i);
-        __syncthreads();
+// Start of the solver phase, over the whole batch at once: inverse world inertia tensors and velocity
+// integration of every body (PhysicsWorld.cpp:266-272), contact rows (ContactSolverSystem::init), joint
+// rows (ConstraintSolverSystem::initialize).  The three parts share no data: the rows recompute the inertia
+// of their bodies instead of waiting for the integration to store it, which saves a launch or a barrier
+// and lets a single large world use the whole chip here.
+__global__ __launch_bounds__(256) void sv_setup(SvArgs A, DevJoints J, Settings settings, float dt) {
+    const DevBodies& B = A.B;
+    const int nm = *A.nm;
+    const int jw = (J.n + kWave - 1) & ~(kWave - 1), mw = (nm + kWave - 1) & ~(kWave - 1);   // whole wavefronts each
+    const int total = jw + mw + B.n;
+    RP3DG_GRID_STRIDE(t, total) {
+        if (t < jw) {
+            if (t < J.n) jt_init_one(B, J, t, dt);
+        } else if (t < jw + mw) {
+            if (t - jw < nm) sv_prepare_one(A, t - jw);
+        } else {
+            dyn_integrate_velocities_one(B, settings, dt, t - jw - mw);
+        }
     }
-    // joint warm start, slot by slot
-    for (int s = 0; s < F.jt_slots; s++) {
+}
+
+// Feature rows of the points without a cached impulse (learned warm start, sample log), after sv_setup.
+__global__ __launch_bounds__(256) void sv_features(FusedArgs F) {
+    const SvArgs& A = F.A;
+    const int nm = *A.nm;
+    const int lane = lane_id();
+    for (int base = (blockIdx.x * blockDim.x + threadIdx.x) & ~(kWave - 1); base < nm; base += gridDim.x * blockDim.x) {
+        const int i = base + lane;
+        int k = 0;
+        if (i < nm) {
+            const int np = A.S.npts[i];
+            for (int p = 0; p < np; p++) k += A.S.lam[4 * i + p].z == 0.0f ? 1 : 0;
+        }
+        const int incl = wave_incl_scan(k);
+        int start = 0;
+        if (lane == kWave - 1 && incl > 0) start = atomicAdd(F.nrows, incl);
+        start = __shfl(start, kWave - 1, kWave) + incl - k;
+        if (i < nm) {
+            const int np = A.S.npts[i];
+            for (int p = 0; p < np; p++) {
+                const int q = 4 * i + p;
+                if (A.S.lam[q].z != 0.0f) continue;
+                A.S.pred[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (start < F.feat_cap) {
+                    float f[kFeatures];
+                    sv_point_features(A, i, p, f);
+                    for (int e = 0; e < kFeatures; e++) F.feats[(size_t)start * kFeatures + e] = f[e];
+                    F.row_slot[start] = q;
+                }
+                start++;
+            }
+        }
+    }
+}
+
+// Barrier between two phases of a group.  With the body state in LDS only LDS is shared between threads
+// (a row is always solved by the same quad, a joint by the same thread), so loads and stores to HBM stay
+// in flight across it.
+template <int STATE>
+__device__ __forceinline__ void phase_barrier() {
+    if constexpr (STATE == STATE_HBM) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+}
+
+// The kernel's arguments, read again from the kernel argument segment.  The sweeps name some sixty arrays;
+// kept in registers over the whole iteration they exceed the scalar registers and spill, so each phase
+// reads the pointers it needs (scalar loads that hit the constant cache).
+__device__ __forceinline__ const FusedArgs& phase_args() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const FusedArgs*)p;
+}
+
+// Thread index of a phase from the wavefront's number, computed anew (two instructions) so that it is not
+// kept in a register, or spilled, across the other phases.
+__device__ __forceinline__ int phase_thread(int wave) {
+    int zero = 0;
+    asm volatile("" : "+v"(zero));
+    return wave * kWave + (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, (unsigned)zero));
+}
+
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ unsigned long long uniform(unsigned long long x) {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(x >> 32)) << 32 |
+           (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)x);
+}
+
+// Header of a row: bodies relative to the group's first (14 bits each), points (3 bits).
+__device__ __forceinline__ unsigned int row_header(int u1, int u2, int np) {
+    return (unsigned)u1 | (unsigned)u2 << 14 | (unsigned)np << 28;
+}
+__device__ __forceinline__ int header_points(unsigned int h) { return (int)(h >> 28); }
+
+// Warm start, velocity iterations and impulse store of one group of worlds.  The body state is in LDS or
+// HBM as STATE says (solver_quad.h).  When the group has at most F.lds_rows manifolds and only unit lock
+// factors (`fast`), the accumulated impulses and the headers of its rows are in LDS too: the sweeps then
+// read the constant part of a row (up to 352 B) from HBM and write nothing there, and the next row is
+// loaded while the current one is solved.  (The two cases are separate code: a pointer that may be either
+// becomes a flat access, which waits for every load in flight.)
+template <bool SPLIT, int STATE>
+__global__ __launch_bounds__(kFusedMaxBlock) void sv_world_solve(FusedArgs F) {
+    __shared__ float red[16];
+    __shared__ unsigned int s_wres[kGroupMaxWorlds];   // residual of each world of the group (float bits)
+    __shared__ unsigned long long s_done;               // converged worlds of the group
+    __shared__ int s_seg[kMaxColors + 1];               // first row of each colour
+    extern __shared__ float4 s_dyn[];   // STATE_LDS: [lds_bodies] cv, cw, sv, sw, iw0, iw1, flags; STATE_VEL: cv,
+                                        // cw, sv; then [lds_rows] impulses (velocity half, split half: two each)
+                                        // and (friction impulses, header)
+    const DevBodies& B = F.A.B;
+    const int g = F.block_world[blockIdx.x];
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int w0 = F.gworld[g], ngw = F.gworld[g + 1] - w0;
+    const int b0 = F.wbody[w0], b1 = F.wbody[w0 + ngw], nbw = b1 - b0;
+    const int* seg = F.seg_start + (size_t)g * kMaxColors;
+    const int m0 = seg[0], m1 = seg[kMaxColors];
+    const int2* jr = F.jt_wr + (size_t)g * F.jt_slots;
+    const int nslots = F.jt_slots && jr[0].x < jr[F.jt_slots - 1].y ? F.jt_slots : 0;
+    const int mcap = F.lds_rows;
+
+    // ---------------- staging
+    const int L = F.lds_bodies;
+    constexpr int kArrays = STATE == STATE_LDS ? 6 : (STATE == STATE_VEL ? 3 : 0);
+    float4* s_rows = s_dyn + (size_t)kArrays * L + (STATE == STATE_LDS ? (L + 3) / 4 : 0);
+    float4* s_lq = s_rows;              // [2 * row + half]
+    float4* s_ih = s_rows + 2 * mcap;   // friction 1, friction 2, twist, header
+    for (int k = tid; k <= kMaxColors; k += nt) s_seg[k] = seg[k];
+    SvArgs A = F.A;
+    DevBodies& BS = A.B;
+    if constexpr (STATE == STATE_LDS) {
+        float4 *lcv = s_dyn, *lcw = s_dyn + L, *lsv = s_dyn + 2 * L, *lsw = s_dyn + 3 * L;
+        float4 *li0 = s_dyn + 4 * L, *li1 = s_dyn + 5 * L;
+        int* lfl = reinterpret_cast<int*>(s_dyn + 6 * L);
+        for (int i = tid; i < nbw; i += nt) {
+            lfl[i] = B.flags[b0 + i] | ((B.world[b0 + i] - w0) << kGroupShift);
+            const float4 r2 = B.iw2[b0 + i];
+            lcv[i] = B.cv[b0 + i];
+            lcw[i] = f4(ld3(B.cw, b0 + i), r2.x);
+            lsv[i] = f4(ld3(B.sv, b0 + i), r2.y);
+            lsw[i] = f4(ld3(B.sw, b0 + i), r2.z);
+            li0[i] = B.iw0[b0 + i];
+            li1[i] = B.iw1[b0 + i];
+        }
+        BS.cv = lcv; BS.cw = lcw; BS.sv = lsv; BS.sw = lsw;
+        BS.iw0 = li0; BS.iw1 = li1; BS.iw2 = nullptr;
+        BS.flags = lfl;
+        BS.vbase = b0;
+    } else if constexpr (STATE == STATE_VEL) {
+        float4 *lcv = s_dyn, *lcw = s_dyn + L, *lsv = s_dyn + 2 * L;
+        for (int i = tid; i < nbw; i += nt) {
+            const V3 sw = ld3(B.sw, b0 + i);
+            lcv[i] = f4(ld3(B.cv, b0 + i), sw.x);
+            lcw[i] = f4(ld3(B.cw, b0 + i), sw.y);
+            lsv[i] = f4(ld3(B.sv, b0 + i), sw.z);
+        }
+        BS.cv = lcv; BS.cw = lcw; BS.sv = BS.sw = lsv;   // (sw: in the w lanes)
+        BS.iw0 = B.iw0 + b0; BS.iw1 = B.iw1 + b0; BS.iw2 = B.iw2 + b0;
+        BS.flags = B.flags + b0;
+        BS.vbase = b0;
+    }
+    const int ub = b0 - BS.vbase;   // first body of the group in the state arrays
+    __syncthreads();
+    int nc = 0;   // colours of the group (dense from 0)
+    while (nc < kMaxColors && uniform(s_seg[nc]) < m1) nc++;
+
+    // ---------------- warm start: contacts colour by colour (CS.cpp:326-476), then joints slot by slot
+    for (int c = 0; c < nc; c++) {
+        const int lo = s_seg[c], hi = s_seg[c + 1];
+        for (int i = lo + tid; i < hi; i += nt) sv_warmstart_one(A, i);
+        phase_barrier<STATE>();
+    }
+    bool unit = true;
+    for (int i = tid; i < nbw; i += nt) unit = unit && (BS.flags[ub + i] & BF_UNIT_LOCKS);
+    const bool fast = __syncthreads_and(unit && m1 - m0 <= mcap);   // (and the impulses written above are visible)
+    if (fast)
+        for (int r = tid; r < m1 - m0; r += nt) {
+            const int i = m0 + r;
+            const int2 bb = F.A.S.bodies[i];
+            s_lq[2 * r] = F.A.S.lq[2 * (size_t)i];
+            s_lq[2 * r + 1] = F.A.S.lq[2 * (size_t)i + 1];
+            s_ih[r] = f4(ld3(F.A.S.imp, i), __uint_as_float(row_header(bb.x - b0, bb.y - b0, F.A.S.npts[i])));
+        }
+    for (int s = 0; s < nslots; s++) {
         const int2 r = jr[s];
         if (r.x == r.y) continue;
         for (int j = r.x + tid; j < r.y; j += nt) jt_warmstart_one(BS, F.J, j);
-        __syncthreads();
+        phase_barrier<STATE>();
     }
     const bool residual = F.res_thr > 0.0f;
     // residual mode with several worlds: each world stops on its own residual (mask of converged worlds)
     const bool masked = residual && ngw > 1;
     const unsigned long long all = ngw >= 64 ? ~0ull : (1ull << ngw) - 1ull;
     unsigned long long done = 0;
-    // world of body b within the group
-    auto wk = [&](int b) { return staged ? (BS.flags[b - BS.vbase] >> kGroupShift) & 63 : B.world[b] - w0; };
+    // world (within the group) of the body at index u of the state arrays
+    auto world_of = [&](int u) {
+        if constexpr (STATE == STATE_LDS) return (BS.flags[u] >> kGroupShift) & 63;
+        else return B.world[u - ub + b0] - w0;
+    };
+    // velocities after the previous sweep: the thread's first body in registers, the others in HBM
+    V3 pv0 = v3(0.f, 0.f, 0.f), pw0 = pv0;
     if (residual) {
-        for (int i = b0 + tid; i < b1; i += nt) {
-            PV[i - b0] = BS.cv[i - BS.vbase];
-            PW[i - b0] = BS.cw[i - BS.vbase];
+        if (tid < nbw) {
+            pv0 = ld3(BS.cv, ub + tid);
+            pw0 = ld3(BS.cw, ub + tid);
+        }
+        for (int i = tid + nt; i < nbw; i += nt) {
+            F.pv[b0 + i] = BS.cv[ub + i];
+            F.pw[b0 + i] = BS.cw[ub + i];
         }
         if (masked)
             for (int k = tid; k < ngw; k += nt) {
@@ -84,40 +262,100 @@ __device__ __forceinline__ void group_sweeps(const FusedArgs& F, const SvArgs& A
                 F.world_iters[w0 + k] = 0;
                 F.world_res[w0 + k] = 0.0f;
             }
-        __syncthreads();
     }
+    __syncthreads();
+
+    // ---------------- velocity iterations: joints, then contacts (ConstraintSolverSystem, CS.cpp:479-759)
+    const int nq = nt >> 2, wave = uniform(tid / kWave);
+    // one velocity iteration over the contact rows, colour by colour; FAST: every row's impulses and header
+    // are in LDS and every body of the group has unit lock factors.  Rows are contiguous over the colours,
+    // so a quad's first row of colour c + 1 is at that colour's start; each quad loads its next row before
+    // it solves the current one.
+    auto contact_sweep = [&](auto fast_tag) {
+        constexpr bool FAST = decltype(fast_tag)::value;
+        const DevSolver S = phase_args().A.S;
+        const int t0 = phase_thread(wave), qd = t0 >> 2;
+        const QuadSrc Q(S, t0);
+        auto fetch = [&](int i, QuadRow& R, unsigned int& hd) {
+            if constexpr (FAST) {
+                hd = __float_as_uint(s_ih[i - m0].w);
+            } else {
+                const int2 bb = S.bodies[i];
+                hd = row_header(bb.x - b0, bb.y - b0, S.npts[i]);
+            }
+            Q.load(i, header_points(hd), R);
+        };
+        QuadRow R;
+        unsigned int hd = 0;
+        int lo = m0, hi = nc ? uniform(s_seg[1]) : m0;
+        if (lo + qd < hi) fetch(lo + qd, R, hd);
+        for (int c = 0; c < nc; c++) {
+            const int hi2 = c + 1 < nc ? uniform(s_seg[c + 2]) : hi;
+            int i = lo + qd;
+            bool more = true;
+            while (more) {
+                const QuadRow cur = R;
+                const unsigned int h = hd;
+                const int ic = i;
+                i += nq;
+                more = i < hi;
+                const int nx = more ? i : hi + qd;
+                if (nx < (more ? hi : hi2)) fetch(nx, R, hd);
+                if (ic >= hi) continue;
+                if (masked && ((done >> world_of(ub + (int)(h & 0x3fffu))) & 1ull)) continue;
+                const int rel = (int)((Q.side ? h >> 14 : h) & 0x3fffu);
+                float4* lq = FAST ? s_lq + 2 * (ic - m0) + Q.part : S.lq + 2 * (size_t)ic + Q.part;
+                float4* ih = FAST ? s_ih + (ic - m0) : S.imp + ic;
+                float4 lam = *lq;
+                V3 imp = xyz(*ih);
+                quad_sweep<STATE, !FAST, SPLIT>(A, Q, cur, ub + rel, b0 + rel, header_points(h), lam, imp, F.beta_dt);
+                if (Q.side) {
+                    if (SPLIT || !Q.part) *lq = lam;
+                    if (!Q.part) st3(ih, 0, imp);
+                }
+            }
+            phase_barrier<STATE>();
+            lo = hi;
+            hi = hi2;
+        }
+    };
     int it = 0;
     float res = 0.0f;
     while (it < F.max_iters) {
-        for (int s = 0; s < F.jt_slots; s++) {
-            const int2 r = jr[s];
+        for (int s = 0; s < nslots; s++) {
+            const FusedArgs& FP = phase_args();
+            const int2 r = FP.jt_wr[(size_t)g * FP.jt_slots + s];
             if (r.x == r.y) continue;
-            for (int j = r.x + tid; j < r.y; j += nt) {
-                if (masked && ((done >> wk(F.J.bodies[j].x)) & 1ull)) continue;
-                jt_solve_velocity_one(BS, F.J, j, F.dt);
+            const int t0 = phase_thread(wave);
+            for (int j = r.x + (t0 >> 1); j < r.y; j += nt >> 1) {
+                if (masked && ((done >> world_of(FP.J.bodies[j].x - BS.vbase)) & 1ull)) continue;
+                jt_solve_velocity_pair(BS, FP.J, FP.jt_kind[s], j, t0 & 1, FP.dt);
             }
-            __syncthreads();
+            phase_barrier<STATE>();
         }
-        for (int c = 0; c < kMaxColors; c++) {
-            const int lo = seg[c], hi = seg[c + 1];
-            if (lo == m1) break;
-            for (int i = lo + tid; i < hi; i += nt) {
-                if (masked && ((done >> wk(A.S.bodies[i].x)) & 1ull)) continue;
-                solve_manifold<SPLIT>(A, i, F.beta_dt);
-            }
-            __syncthreads();
-        }
+        if (fast) contact_sweep(std::true_type{});
+        else contact_sweep(std::false_type{});
         it++;
         if (residual) {
             float r = 0.0f;
-            for (int i = b0 + tid; i < b1; i += nt) {
-                if (!dyn_body(B, i)) continue;
+            for (int i = tid; i < nbw; i += nt) {
+                if (!(BS.flags[ub + i] & BF_DYNAMIC)) continue;
                 int k = 0;
                 if (masked) {
-                    k = wk(i);
+                    k = world_of(ub + i);
                     if ((done >> k) & 1ull) continue;
                 }
-                const float4 v = BS.cv[i - BS.vbase], wv = BS.cw[i - BS.vbase], pv = PV[i - b0], pw = PW[i - b0];
+                const V3 v = ld3(BS.cv, ub + i), wv = ld3(BS.cw, ub + i);
+                V3 pv = pv0, pw = pw0;
+                if (i != tid) {
+                    pv = ld3(F.pv, b0 + i);
+                    pw = ld3(F.pw, b0 + i);
+                    F.pv[b0 + i] = f4(v, 0.f);
+                    F.pw[b0 + i] = f4(wv, 0.f);
+                } else {
+                    pv0 = v;
+                    pw0 = wv;
+                }
                 float d = fabsf(v.x - pv.x);
                 d = fmaxf(d, fabsf(v.y - pv.y));
                 d = fmaxf(d, fabsf(v.z - pv.z));
@@ -126,14 +364,12 @@ __device__ __forceinline__ void group_sweeps(const FusedArgs& F, const SvArgs& A
                 d = fmaxf(d, fabsf(wv.z - pw.z));
                 if (masked) atomicMax(&s_wres[k], __float_as_uint(d));   // d >= 0: bit order = value order
                 else r = fmaxf(r, d);
-                PV[i - b0] = v;
-                PW[i - b0] = wv;
             }
             if (!masked) {
                 res = block_maxf(r, red);
                 if (res < F.res_thr) break;
             } else {
-                __syncthreads();
+                phase_barrier<STATE>();
                 if (tid < kWave) {
                     bool fin = false;
                     if (tid < ngw && !((done >> tid) & 1ull)) {
@@ -144,23 +380,32 @@ __device__ __forceinline__ void group_sweeps(const FusedArgs& F, const SvArgs& A
                         F.world_res[w0 + tid] = rk;
                     }
                     const unsigned long long bal = __ballot(fin);
-                    if (tid == 0) *s_done = done | bal;
+                    if (tid == 0) s_done = done | bal;
                 }
-                __syncthreads();
-                done = *s_done;
+                phase_barrier<STATE>();
+                done = uniform(s_done);
                 if (done == all) break;
             }
         }
     }
-    // storeImpulses (CS.cpp:763-785)
-    for (int i = seg[0] + tid; i < m1; i += nt) sv_store_one(A, i);
-    if (staged) {
-        __syncthreads();
+    // ---------------- storeImpulses (CS.cpp:763-785) and the solved velocities
+    __syncthreads();
+    if (fast)
+        for (int r = tid; r < m1 - m0; r += nt) {
+            const int i = m0 + r;
+            F.A.S.lq[2 * (size_t)i] = s_lq[2 * r];
+            F.A.S.lq[2 * (size_t)i + 1] = s_lq[2 * r + 1];
+            st3(F.A.S.imp, i, xyz(s_ih[r]));
+        }
+    for (int i = m0 + tid; i < m1; i += nt) sv_store_one(F.A, i);   // row i is this thread's in both loops
+    if constexpr (STATE != STATE_HBM) {
         for (int i = tid; i < nbw; i += nt) {
-            B.cv[b0 + i] = BS.cv[i];
-            B.cw[b0 + i] = BS.cw[i];
-            B.sv[b0 + i] = BS.sv[i];
-            B.sw[b0 + i] = BS.sw[i];
+            const float4 cv = BS.cv[i], cw = BS.cw[i], sv = BS.sv[i];
+            B.cv[b0 + i] = f4(xyz(cv), 0.f);
+            B.cw[b0 + i] = f4(xyz(cw), 0.f);
+            B.sv[b0 + i] = f4(xyz(sv), 0.f);
+            if constexpr (STATE == STATE_VEL) B.sw[b0 + i] = make_float4(cv.w, cw.w, sv.w, 0.f);
+            else B.sw[b0 + i] = f4(ld3(BS.sw, i), 0.f);
         }
     }
     if (!masked)
@@ -169,112 +414,14 @@ __device__ __forceinline__ void group_sweeps(const FusedArgs& F, const SvArgs& A
             F.world_res[w0 + k] = res;
         }
 }
+template __global__ void sv_world_solve<true, STATE_LDS>(FusedArgs F);
+template __global__ void sv_world_solve<true, STATE_VEL>(FusedArgs F);
+template __global__ void sv_world_solve<true, STATE_HBM>(FusedArgs F);
+template __global__ void sv_world_solve<false, STATE_LDS>(FusedArgs F);
+template __global__ void sv_world_solve<false, STATE_VEL>(FusedArgs F);
+template __global__ void sv_world_solve<false, STATE_HBM>(FusedArgs F);
 
-template <bool SPLIT>
-__global__ __launch_bounds__(kFusedMaxBlock) void sv_world_solve(FusedArgs F) {
-    __shared__ float red[16];
-    __shared__ unsigned int s_wres[kGroupMaxWorlds];   // residual of each world of the group (float bits)
-    __shared__ unsigned long long s_done;               // converged worlds of the group
-    extern __shared__ float4 s_vel[];   // [6][lds_bodies] cv, cw, sv, sw (w: third inertia row), iw0, iw1;
-                                        // [lds_bodies] flags; with lds_residual [2][lds_bodies] previous cv, cw
-    const SvArgs& AG = F.A;
-    const DevBodies& B = AG.B;
-    const int g = F.block_world[blockIdx.x];
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int w0 = F.gworld[g], ngw = F.gworld[g + 1] - w0;
-    const int b0 = F.wbody[w0], b1 = F.wbody[w0 + ngw];
-    const int* seg = F.seg_start + (size_t)g * kMaxColors;
-    const int m0 = seg[0], m1 = seg[kMaxColors];
-    const int2* jr = F.jt_wr + (size_t)g * F.jt_slots;
-    const int j0 = F.jt_slots ? jr[0].x : 0, j1 = F.jt_slots ? jr[F.jt_slots - 1].y : 0;
-
-    if (F.phase != 1) {
-        // PhysicsWorld.cpp:266-272: inverse world inertia tensors and velocity integration
-        for (int i = b0 + tid; i < b1; i += nt) dyn_integrate_velocities_one(B, F.settings, F.dt, i);
-        if (F.J.bfirst)
-            for (int w = tid; w < ngw; w += nt) F.J.bfirst[w0 + w] = INT_MAX;
-        __syncthreads();
-        // ContactSolverSystem::init (rows); ConstraintSolverSystem::initialize (initBeforeSolve)
-        const SvArgs& A = AG;
-        for (int i = m0 + tid; i < m1; i += nt) sv_prepare_one(A, i);
-        for (int j = j0 + tid; j < j1; j += nt) jt_init_one(B, F.J, j, F.dt);
-        if (F.feats) {
-            // feature rows of the points without a cached impulse; same manifold -> thread mapping as
-            // above, so every thread reads only rows it wrote itself
-            const int lane = lane_id();
-            for (int base = m0 + (tid & ~(kWave - 1)); base < m1; base += nt) {
-                const int i = base + lane;
-                int k = 0;
-                if (i < m1) {
-                    const int np = A.S.npts[i];
-                    for (int p = 0; p < np; p++) k += A.S.lam[4 * i + p].z == 0.0f ? 1 : 0;
-                }
-                const int incl = wave_incl_scan(k);
-                int start = 0;
-                if (lane == kWave - 1 && incl > 0) start = atomicAdd(F.nrows, incl);
-                start = __shfl(start, kWave - 1, kWave) + incl - k;
-                if (i < m1) {
-                    const int np = A.S.npts[i];
-                    for (int p = 0; p < np; p++) {
-                        const int q = 4 * i + p;
-                        if (A.S.lam[q].z != 0.0f) continue;
-                        A.S.pred[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if (start < F.feat_cap) {
-                            float f[kFeatures];
-                            sv_point_features(A, i, p, f);
-                            for (int e = 0; e < kFeatures; e++) F.feats[(size_t)start * kFeatures + e] = f[e];
-                            F.row_slot[start] = q;
-                        }
-                        start++;
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        if (F.phase == 0) return;
-    }
-    // stage the group's solver velocities, world inverse inertia rows and flags in LDS for the sweeps
-    // (the rows and the rest of the body data stay in HBM); the third inertia row rides in the w lanes of
-    // cw, sv and sw: 100 bytes a body, so six 256-body groups fit the 160 KB of a CU (five at 116 bytes)
-    const int nbw = b1 - b0;
-    if (nbw <= F.lds_bodies) {
-        const int L = F.lds_bodies;
-        float4 *lcv = s_vel, *lcw = s_vel + L, *lsv = s_vel + 2 * L, *lsw = s_vel + 3 * L;
-        float4 *li0 = s_vel + 4 * L, *li1 = s_vel + 5 * L;
-        int* lfl = reinterpret_cast<int*>(s_vel + 6 * L);
-        for (int i = tid; i < nbw; i += nt) {
-            lfl[i] = B.flags[b0 + i] | ((B.world[b0 + i] - w0) << kGroupShift);
-            const float4 r2 = B.iw2[b0 + i];
-            float4 t = B.cw[b0 + i];
-            t.w = r2.x;
-            lcw[i] = t;
-            t = B.sv[b0 + i];
-            t.w = r2.y;
-            lsv[i] = t;
-            t = B.sw[b0 + i];
-            t.w = r2.z;
-            lsw[i] = t;
-            lcv[i] = B.cv[b0 + i];
-            li0[i] = B.iw0[b0 + i];
-            li1[i] = B.iw1[b0 + i];
-        }
-        SvArgs A = AG;
-        A.B.cv = lcv; A.B.cw = lcw; A.B.sv = lsv; A.B.sw = lsw;
-        A.B.iw0 = li0; A.B.iw1 = li1; A.B.iw2 = nullptr;
-        A.B.flags = lfl;
-        A.B.vbase = b0;
-        float4* lpv = F.lds_residual ? reinterpret_cast<float4*>(lfl + L) : F.pv + b0;
-        float4* lpw = F.lds_residual ? lpv + L : F.pw + b0;
-        __syncthreads();
-        group_sweeps<SPLIT>(F, A, B, true, w0, ngw, b0, b1, m1, seg, jr, red, s_wres, &s_done, lpv, lpw);
-    } else {
-        group_sweeps<SPLIT>(F, AG, B, false, w0, ngw, b0, b1, m1, seg, jr, red, s_wres, &s_done, F.pv + b0, F.pw + b0);
-    }
-}
-template __global__ void sv_world_solve<true>(FusedArgs F);
-template __global__ void sv_world_solve<false>(FusedArgs F);
-
-__global__ __launch_bounds__(kFusedMaxBlock) void world_position(FusedArgs F) {
+__global__ __launch_bounds__(kPositionMaxBlock) void world_position(FusedArgs F) {
     const DevBodies& B = F.A.B;
     const int g = F.block_world[blockIdx.x];
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -311,7 +458,7 @@ __global__ void sv_log_samples(FusedArgs F, float* log_feats, float* log_targets
         const float4 imp = F.A.S.imp[i];
         const float inv_np = 1.0f / (float)F.A.S.npts[i];
         for (int e = 0; e < kFeatures; e++) log_feats[dst * kFeatures + e] = F.feats[(size_t)r * kFeatures + e];
-        log_targets[dst * 3 + 0] = F.A.S.lam[q].x;
+        log_targets[dst * 3 + 0] = reinterpret_cast<const float*>(F.A.S.lq)[8 * (size_t)i + (q & 3)];
         log_targets[dst * 3 + 1] = imp.x * inv_np;
         log_targets[dst * 3 + 2] = imp.y * inv_np;
     }

@@ -34,8 +34,7 @@ struct DevJoints {
     float4 *impT, *impR, *impL;   // accumulated impulses: translation, rotation, (lower, upper, motor)
                                   // (ball-and-socket: impL.x = cone limit; slider: impT.xy = 2 rows)
     // per-step rows
-    float4 *i1r0, *i1r1, *i1r2, *i2r0, *i2r1, *i2r2;
-    float4 *r1, *r2;
+    float4 *r1, *r2;              // lever arms; w: inverse mass of the body
     float4 *kt0, *kt1, *kt2;      // inverse translation mass matrix (slider: 2x2 in kt0)
     float4 *kr0, *kr1, *kr2;      // inverse rotation mass matrix (fixed, slider: 3x3, hinge: 2x2 in kr0)
     float4 *a1, *b2xa1, *c2xa1;   // hinge axes; ball-socket: cone axis in a1; slider: axis, n1, n2
@@ -58,9 +57,8 @@ struct DevJoints {
     int* bfirst;
 };
 
-__global__ void jt_init(DevBodies B, DevJoints J, float dt);
 __global__ void jt_warmstart(DevBodies B, DevJoints J, const int* range, int slot);
-__global__ void jt_solve_velocity(DevBodies B, DevJoints J, const int* range, int slot, float dt);
+__global__ void jt_solve_velocity(DevBodies B, DevJoints J, const int* range, int slot, int kind, float dt);
 __global__ void jt_solve_position(DevBodies B, DevJoints J, const int* range, int slot);
 
 }  // namespace rp3dg

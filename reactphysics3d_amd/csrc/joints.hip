@@ -8,18 +8,15 @@
 
 namespace rp3dg {
 
-__global__ void jt_init(DevBodies B, DevJoints J, float dt) {
-    RP3DG_GRID_STRIDE(j, J.n) jt_init_one(B, J, j, dt);
-}
-
 __global__ void jt_warmstart(DevBodies B, DevJoints J, const int* range, int slot) {
     const int lo = range[2 * slot], hi = range[2 * slot + 1];
     RP3DG_GRID_STRIDE(t, hi - lo) jt_warmstart_one(B, J, lo + t);
 }
 
-__global__ void jt_solve_velocity(DevBodies B, DevJoints J, const int* range, int slot, float dt) {
+// two lanes per joint
+__global__ void jt_solve_velocity(DevBodies B, DevJoints J, const int* range, int slot, int kind, float dt) {
     const int lo = range[2 * slot], hi = range[2 * slot + 1];
-    RP3DG_GRID_STRIDE(t, hi - lo) jt_solve_velocity_one(B, J, lo + t, dt);
+    RP3DG_GRID_STRIDE(t, 2 * (hi - lo)) jt_solve_velocity_pair(B, J, kind, lo + (t >> 1), t & 1, dt);
 }
 
 __global__ void jt_solve_position(DevBodies B, DevJoints J, const int* range, int slot) {

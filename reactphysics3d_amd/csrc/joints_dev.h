@@ -16,6 +16,7 @@
 #include "joints.h"
 #include "kcommon.h"
 #include "solver_dev.h"
+#include "solver_quad.h"
 
 namespace rp3dg {
 
@@ -132,15 +133,13 @@ __device__ __forceinline__ void jt_init_one(const DevBodies& B, const DevJoints&
         const int b1 = bb.x, b2 = bb.y;
         if (!joint_enabled(B, b1, b2)) return;
         const int t = J.type[j];
-        const M3 I1 = ldm(B.iw0, B.iw1, B.iw2, b1), I2 = ldm(B.iw0, B.iw1, B.iw2, b2);
-        stm(J.i1r0, J.i1r1, J.i1r2, j, I1);
-        stm(J.i2r0, J.i2r1, J.i2r2, j, I2);
+        const M3 I1 = body_iw_setup(B, b1), I2 = body_iw_setup(B, b2);
         const Q4 q1 = ldq(B.q, b1), q2 = ldq(B.q, b2);
         const V3 r1 = qrot(q1, ld3(J.la1, j) - ld3(B.com, b1));
         const V3 r2 = qrot(q2, ld3(J.la2, j) - ld3(B.com, b2));
-        J.r1[j] = f4(r1, 0.f);
-        J.r2[j] = f4(r2, 0.f);
         const float im1 = B.ii[b1].w, im2 = B.ii[b2].w;
+        J.r1[j] = f4(r1, im1);
+        J.r2[j] = f4(r2, im2);
         const bool anyDyn = ((body_flags(B, b1) | body_flags(B, b2)) & BF_DYNAMIC) != 0;
         bool ok;
         const M3 Kt = translation_inverse_mass(im1 + im2, r1, r2, I1, I2, anyDyn, ok);
@@ -316,7 +315,7 @@ __device__ __forceinline__ void jt_warmstart_one(const DevBodies& B, const DevJo
         V3 ll1, al1, ll2, al2;
         body_locks(B, b1, ll1, al1);
         body_locks(B, b2, ll2, al2);
-        const M3 I1 = ldm(J.i1r0, J.i1r1, J.i1r2, j), I2 = ldm(J.i2r0, J.i2r1, J.i2r2, j);
+        const M3 I1 = body_iw(B, b1), I2 = body_iw(B, b2);   // as jt_init_one's: the state's rows do not change in a step
         const V3 r1 = ld3(J.r1, j), r2 = ld3(J.r2, j);
         const V3 it = ld3(J.impT, j);
         if (type == JT_BALLSOCKET) {   // SolveBallAndSocketJointSystem.cpp:196-241
@@ -388,217 +387,213 @@ __device__ __forceinline__ void jt_warmstart_one(const DevBodies& B, const DevJo
             v2 += lock_mul((im2 * ll2), li2);
             w2 += cmul(al2, mvmul(I2, ai2));
         }
-        B.cv[u1] = f4(v1, 0.f); st3(B.cw, u1, w1);
-        B.cv[u2] = f4(v2, 0.f); st3(B.cw, u2, w2);
+        st3(B.cv, u1, v1); st3(B.cw, u1, w1);
+        st3(B.cv, u2, v2); st3(B.cw, u2, w2);
     }
 }
 
 // ------------------------------------------------------------------------------------------------
-// velocity constraints (per colour)
+// velocity constraints (per colour), two lanes per joint: the even lane holds body 1, the odd lane body 2
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void jt_solve_velocity_one(const DevBodies& B, const DevJoints& J, int j, float dt) {
-    {
-        const int2 bb = J.bodies[j];
-        const int b1 = bb.x, b2 = bb.y;
-        if (!joint_enabled(B, b1, b2)) return;
-        const int type = J.type[j];
-        const int u1 = b1 - B.vbase, u2 = b2 - B.vbase;
-        V3 v1 = ld3(B.cv, u1), w1 = ld3(B.cw, u1), v2 = ld3(B.cv, u2), w2 = ld3(B.cw, u2);
-        const float im1 = B.ii[b1].w, im2 = B.ii[b2].w;
-        V3 ll1, al1, ll2, al2;
-        body_locks(B, b1, ll1, al1);
-        body_locks(B, b2, ll2, al2);
-        const M3 I1 = ldm(J.i1r0, J.i1r1, J.i1r2, j), I2 = ldm(J.i2r0, J.i2r1, J.i2r2, j);
-        const V3 r1 = ld3(J.r1, j), r2 = ld3(J.r2, j);
+// A joint row is a dependent chain like a contact's (solver_quad.h) and a colour has few joints, so the two
+// bodies' halves run side by side: each lane keeps its body's velocities, inertia and lever arm and does
+// half of the arithmetic, in the reference's operations and order; the row's impulse is computed in body 2's
+// lane and passed by DPP, and body 1's sign is applied by flipping sign bits (exact).
+struct JointBody {
+    V3 v, w, iml, al;   // velocities; inverse mass x linear lock factors, angular lock factors
+    M3 I;
+    unsigned int s1, s2;   // sign bits: s1 flips in body 1's lane, s2 in body 2's
+};
+__device__ __forceinline__ V3 flip3(V3 a, unsigned int m) { return v3(flip(a.x, m), flip(a.y, m), flip(a.z, m)); }
+__device__ __forceinline__ V3 pair_from1(V3 a) { return v3(dpp<kQuadFrom1>(a.x), dpp<kQuadFrom1>(a.y), dpp<kQuadFrom1>(a.z)); }
+__device__ __forceinline__ V3 pair_from2(V3 a) { return v3(dpp<kQuadFrom2>(a.x), dpp<kQuadFrom2>(a.y), dpp<kQuadFrom2>(a.z)); }
+__device__ __forceinline__ void joint_spin(JointBody& b, V3 angular) { b.w += cmul(b.al, mvmul(b.I, angular)); }
+
+// v2 + w2 x r2 - v1 - w1 x r1 (valid in body 2's lane)
+__device__ __forceinline__ V3 joint_rel_vel(const JointBody& b, V3 r) {
+    const V3 c = cross(b.w, r);
+    return b.v + c - pair_from1(b.v) - pair_from1(c);
+}
+// translation impulse dl (of body 2's lane) of the three point-to-point rows
+__device__ __forceinline__ void joint_push(JointBody& b, V3 r, V3 dl2) {
+    const V3 dl = pair_from2(dl2);
+    b.v += lock_mul(b.iml, flip3(dl, b.s1));
+    joint_spin(b, flip3(cross(dl, r), b.s2));
+}
+
+// kind: the joint kind of the slot (uniform)
+__device__ __forceinline__ void jt_solve_velocity_pair(const DevBodies& B, const DevJoints& J, int kind, int j, int side,
+                                                       float dt) {
+    const int2 bb = J.bodies[j];
+    const int bi = side ? bb.y : bb.x, u = bi - B.vbase;
+    const int fl = J.flags[j];
+    const float4 r4 = side ? J.r2[j] : J.r1[j];   // w: inverse mass
+    float4 it = J.impT[j];
+    if (!joint_enabled(B, bb.x, bb.y)) return;
+    const V3 r = xyz(r4);
+    JointBody b;
+    b.v = ld3(B.cv, u);
+    b.w = ld3(B.cw, u);
+    b.I = body_iw(B, bi);
+    V3 ll;
+    body_locks(B, bi, ll, b.al);
+    b.iml = r4.w * ll;
+    b.s1 = side ? 0u : 0x80000000u;
+    b.s2 = side ? 0x80000000u : 0u;
+    // Baumgarte biases; zero under non-linear Gauss-Seidel position correction
+    float4 bias0 = make_float4(0.f, 0.f, 0.f, 0.f), bias1 = bias0;
+    if (fl & JF_BAUMGARTE) {
+        bias0 = J.bias0[j];
+        bias1 = J.bias1[j];
+    }
+    const V3 bt = v3(bias0.x, bias0.y, bias0.z);
+    if (kind == JT_BALLSOCKET) {   // SolveBallAndSocketJointSystem.cpp:245-308
         const M3 Kt = ldm(J.kt0, J.kt1, J.kt2, j);
-        // Baumgarte biases; zero under non-linear Gauss-Seidel position correction
-        float4 bias0 = make_float4(0.f, 0.f, 0.f, 0.f), bias1 = bias0;
-        if (J.flags[j] & JF_BAUMGARTE) {
-            bias0 = J.bias0[j];
-            bias1 = J.bias1[j];
+        if ((fl & (JF_LIMIT | JF_LOWER_VIOLATED)) == (JF_LIMIT | JF_LOWER_VIOLATED)) {
+            const V3 acb = ld3(J.a1, j);
+            const float JvC = dot(acb, pair_from1(b.w) - b.w);
+            float d = J.imlm[j] * (-JvC - bias0.w);
+            float4 il = J.impL[j];
+            const float lt = il.x;
+            il.x = fmax_s(il.x + d, 0.0f);
+            d = dpp<kQuadFrom2>(il.x - lt);
+            if (side) J.impL[j] = il;
+            joint_spin(b, flip(d, b.s2) * acb);
         }
-        const V3 bt = v3(bias0.x, bias0.y, bias0.z);
-        if (type == JT_BALLSOCKET) {   // SolveBallAndSocketJointSystem.cpp:245-308
-            if ((J.flags[j] & (JF_LIMIT | JF_LOWER_VIOLATED)) == (JF_LIMIT | JF_LOWER_VIOLATED)) {
-                const V3 acb = ld3(J.a1, j);
-                const float JvC = dot(acb, w1 - w2);
-                float d = J.imlm[j] * (-JvC - bias0.w);
-                float4 il = J.impL[j];
-                const float lt = il.x;
-                il.x = fmax_s(il.x + d, 0.0f);
-                d = il.x - lt;
-                J.impL[j] = il;
-                w1 += cmul(al1, mvmul(I1, d * acb));
-                w2 += cmul(al2, mvmul(I2, (-d) * acb));
-            }
-            const V3 Jv = v2 + cross(w2, r2) - v1 - cross(w1, r1);
-            const V3 dl = mvmul(Kt, -Jv - bt);
-            J.impT[j] = f4(ld3(J.impT, j) + dl, 0.f);
-            const V3 li1 = -dl;
-            const V3 ai1 = cross(dl, r1);
-            v1 += lock_mul((im1 * ll1), li1);
-            w1 += cmul(al1, mvmul(I1, ai1));
-            const V3 ai2 = -cross(dl, r2);
-            v2 += lock_mul((im2 * ll2), dl);
-            w2 += cmul(al2, mvmul(I2, ai2));
-        } else if (type == JT_FIXED) {   // SolveFixedJointSystem.cpp:189-262
-            const V3 Jvt = v2 + cross(w2, r2) - v1 - cross(w1, r1);
-            const V3 dl = mvmul(Kt, -Jvt - bt);
-            J.impT[j] = f4(ld3(J.impT, j) + dl, 0.f);
-            const V3 li1 = -dl;
-            V3 ai1 = cross(dl, r1);
-            v1 += lock_mul((im1 * ll1), li1);
-            w1 += cmul(al1, mvmul(I1, ai1));
-            const V3 ai2 = -cross(dl, r2);
-            v2 += lock_mul((im2 * ll2), dl);
-            w2 += cmul(al2, mvmul(I2, ai2));
-            const V3 Jvr = w2 - w1;
-            const M3 Kr = ldm(J.kr0, J.kr1, J.kr2, j);
-            const V3 dl2 = mvmul(Kr, -Jvr - v3(bias1.x, bias1.y, bias1.z));
-            J.impR[j] = f4(ld3(J.impR, j) + dl2, 0.f);
-            ai1 = -dl2;
-            w1 += cmul(al1, mvmul(I1, ai1));
-            w2 += cmul(al2, mvmul(I2, dl2));
-        } else if (type == JT_HINGE) {   // SolveHingeJointSystem.cpp:273-440
-            const V3 a1 = ld3(J.a1, j);
-            const int fl = J.flags[j];
+        const V3 dl = mvmul(Kt, -joint_rel_vel(b, r) - bt);
+        if (side) J.impT[j] = f4(xyz(it) + dl, 0.f);
+        joint_push(b, r, dl);
+    } else if (kind == JT_FIXED) {   // SolveFixedJointSystem.cpp:189-262
+        const M3 Kt = ldm(J.kt0, J.kt1, J.kt2, j), Kr = ldm(J.kr0, J.kr1, J.kr2, j);
+        const V3 ir = ld3(J.impR, j);
+        const V3 dl = mvmul(Kt, -joint_rel_vel(b, r) - bt);
+        if (side) J.impT[j] = f4(xyz(it) + dl, 0.f);
+        joint_push(b, r, dl);
+        const V3 Jvr = b.w - pair_from1(b.w);
+        const V3 dl2 = mvmul(Kr, -Jvr - v3(bias1.x, bias1.y, bias1.z));
+        if (side) J.impR[j] = f4(ir + dl2, 0.f);
+        joint_spin(b, flip3(pair_from2(dl2), b.s1));
+    } else if (kind == JT_HINGE) {   // SolveHingeJointSystem.cpp:273-440
+        const M3 Kt = ldm(J.kt0, J.kt1, J.kt2, j);
+        const V3 a1 = ld3(J.a1, j), bxa = ld3(J.b2xa1, j), cxa = ld3(J.c2xa1, j);
+        const float4 kr = J.kr0[j];
+        float4 ir = J.impR[j];
+        if (fl & (JF_LIMIT | JF_MOTOR)) {
             float4 il = J.impL[j];
             const float imlm = J.imlm[j];
             if (fl & JF_LIMIT) {
                 if (fl & JF_LOWER_VIOLATED) {
-                    const float JvL = dot(w2 - w1, a1);
+                    const float JvL = dot(b.w - pair_from1(b.w), a1);
                     float d = imlm * (-JvL - bias1.z);
                     const float lt = il.x;
                     il.x = fmax_s(il.x + d, 0.0f);
-                    d = il.x - lt;
-                    const V3 ai1 = (-d) * a1;
-                    w1 += cmul(al1, mvmul(I1, ai1));
-                    const V3 ai2 = d * a1;
-                    w2 += cmul(al2, mvmul(I2, ai2));
+                    d = dpp<kQuadFrom2>(il.x - lt);
+                    joint_spin(b, flip(d, b.s1) * a1);
                 }
                 if (fl & JF_UPPER_VIOLATED) {
-                    const float JvU = -dot(w2 - w1, a1);
+                    const float JvU = -dot(b.w - pair_from1(b.w), a1);
                     float d = imlm * (-JvU - bias1.w);
                     const float lt = il.y;
                     il.y = fmax_s(il.y + d, 0.0f);
-                    d = il.y - lt;
-                    const V3 ai1 = d * a1;
-                    w1 += cmul(al1, mvmul(I1, ai1));
-                    const V3 ai2 = (-d) * a1;
-                    w2 += cmul(al2, mvmul(I2, ai2));
+                    d = dpp<kQuadFrom2>(il.y - lt);
+                    joint_spin(b, flip(d, b.s2) * a1);
                 }
             }
             if (fl & JF_MOTOR) {
                 const float4 lim = J.lim[j];
-                const float JvM = dot(a1, w1 - w2);
+                const float JvM = dot(a1, pair_from1(b.w) - b.w);
                 const float maxI = lim.w * dt;
                 float d = imlm * (-JvM - lim.z);
                 const float lt = il.z;
                 il.z = clampf(il.z + d, -maxI, maxI);
-                d = il.z - lt;
-                const V3 ai1 = (-d) * a1;
-                w1 += cmul(al1, mvmul(I1, ai1));
-                const V3 ai2 = d * a1;
-                w2 += cmul(al2, mvmul(I2, ai2));
+                d = dpp<kQuadFrom2>(il.z - lt);
+                joint_spin(b, flip(d, b.s1) * a1);
             }
-            J.impL[j] = il;
-            const V3 bxa = ld3(J.b2xa1, j), cxa = ld3(J.c2xa1, j);
-            const float jr0 = -dot(bxa, w1) + dot(bxa, w2);
-            const float jr1 = -dot(cxa, w1) + dot(cxa, w2);
-            const float4 kr = J.kr0[j];
-            const float x0 = -jr0 - bias1.x, x1 = -jr1 - bias1.y;
-            const float d0 = kr.x * x0 + kr.y * x1;
-            const float d1 = kr.z * x0 + kr.w * x1;
-            float4 ir = J.impR[j];
-            ir.x += d0;
-            ir.y += d1;
-            J.impR[j] = ir;
-            V3 ai1 = (-bxa) * d0 - cxa * d1;
-            w1 += cmul(al1, mvmul(I1, ai1));
-            V3 ai2 = bxa * d0 + cxa * d1;
-            w2 += cmul(al2, mvmul(I2, ai2));
-            const V3 Jvt = v2 + cross(w2, r2) - v1 - cross(w1, r1);
-            const V3 dl = mvmul(Kt, -Jvt - bt);
-            J.impT[j] = f4(ld3(J.impT, j) + dl, 0.f);
-            const V3 li1 = -dl;
-            ai1 = cross(dl, r1);
-            v1 += lock_mul((im1 * ll1), li1);
-            w1 += cmul(al1, mvmul(I1, ai1));
-            ai2 = -cross(dl, r2);
-            v2 += lock_mul((im2 * ll2), dl);
-            w2 += cmul(al2, mvmul(I2, ai2));
-        } else {   // slider, SolveSliderJointSystem.cpp:317-510
-            const V3 ax = ld3(J.a1, j), ua = ld3(J.ua, j), ra = ld3(J.ra, j);
-            const int fl = J.flags[j];
+            if (side) J.impL[j] = il;
+        }
+        const float db = dot(bxa, b.w), dc = dot(cxa, b.w);
+        const float jr0 = -dpp<kQuadFrom1>(db) + db;
+        const float jr1 = -dpp<kQuadFrom1>(dc) + dc;
+        const float x0 = -jr0 - bias1.x, x1 = -jr1 - bias1.y;
+        float d0 = kr.x * x0 + kr.y * x1;
+        float d1 = kr.z * x0 + kr.w * x1;
+        ir.x += d0;
+        ir.y += d1;
+        if (side) J.impR[j] = ir;
+        d0 = dpp<kQuadFrom2>(d0);
+        d1 = dpp<kQuadFrom2>(d1);
+        joint_spin(b, flip3(bxa, b.s1) * d0 + flip3(cxa, b.s1) * d1);
+        const V3 dl = mvmul(Kt, -joint_rel_vel(b, r) - bt);
+        if (side) J.impT[j] = f4(xyz(it) + dl, 0.f);
+        joint_push(b, r, dl);
+    } else {   // slider, SolveSliderJointSystem.cpp:317-510
+        const V3 ax = ld3(J.a1, j), arm = side ? ld3(J.ra, j) : ld3(J.ua, j);
+        const M3 Kr = ldm(J.kr0, J.kr1, J.kr2, j);
+        const V3 ir = ld3(J.impR, j);
+        if (fl & (JF_LIMIT | JF_MOTOR)) {
             float4 il = J.impL[j];
             if (fl & JF_LIMIT) {
                 const float imlm = J.imlm[j];
                 if (fl & JF_LOWER_VIOLATED) {
-                    const float JvL = dot(ax, v2) + dot(ra, w2) - dot(ax, v1) - dot(ua, w1);
+                    const float dv = dot(ax, b.v), dw = dot(arm, b.w);
+                    const float JvL = dv + dw - dpp<kQuadFrom1>(dv) - dpp<kQuadFrom1>(dw);
                     float d = imlm * (-JvL - bias0.z);
                     const float lt = il.x;
                     il.x = fmax_s(il.x + d, 0.0f);
-                    d = il.x - lt;
-                    v1 += lock_mul((im1 * ll1), (-d) * ax);
-                    w1 += cmul(al1, mvmul(I1, (-d) * ua));
-                    v2 += lock_mul((im2 * ll2), d * ax);
-                    w2 += cmul(al2, mvmul(I2, d * ra));
+                    d = flip(dpp<kQuadFrom2>(il.x - lt), b.s1);
+                    b.v += lock_mul(b.iml, d * ax);
+                    joint_spin(b, d * arm);
                 }
                 if (fl & JF_UPPER_VIOLATED) {
-                    const float JvU = dot(ax, v1) + dot(ua, w1) - dot(ax, v2) - dot(ra, w2);
+                    const float dv = dot(ax, b.v), dw = dot(arm, b.w);
+                    const float JvU = dpp<kQuadFrom1>(dv + dw) - dv - dw;
                     float d = imlm * (-JvU - bias0.w);
                     const float lt = il.y;
                     il.y = fmax_s(il.y + d, 0.0f);
-                    d = il.y - lt;
-                    v1 += lock_mul((im1 * ll1), d * ax);
-                    w1 += cmul(al1, mvmul(I1, d * ua));
-                    v2 += lock_mul((im2 * ll2), (-d) * ax);
-                    w2 += cmul(al2, mvmul(I2, (-d) * ra));
+                    d = flip(dpp<kQuadFrom2>(il.y - lt), b.s2);
+                    b.v += lock_mul(b.iml, d * ax);
+                    joint_spin(b, d * arm);
                 }
             }
             if (fl & JF_MOTOR) {
                 const float4 lim = J.lim[j];
-                const float JvM = dot(ax, v1) - dot(ax, v2);
+                const float dv = dot(ax, b.v);
+                const float JvM = dpp<kQuadFrom1>(dv) - dv;
                 const float maxI = lim.w * dt;
                 float d = J.imm[j] * (-JvM - lim.z);
                 const float lt = il.z;
                 il.z = clampf(il.z + d, -maxI, maxI);
-                d = il.z - lt;
-                v1 += lock_mul((im1 * ll1), d * ax);
-                v2 += lock_mul((im2 * ll2), (-d) * ax);
+                d = flip(dpp<kQuadFrom2>(il.z - lt), b.s2);
+                b.v += lock_mul(b.iml, d * ax);
             }
-            J.impL[j] = il;
-            // 3 rotation rows
-            const V3 Jvr = w2 - w1;
-            const M3 Kr = ldm(J.kr0, J.kr1, J.kr2, j);
-            const V3 dr = mvmul(Kr, -Jvr - v3(bias1.x, bias1.y, bias1.z));
-            J.impR[j] = f4(ld3(J.impR, j) + dr, 0.f);
-            w1 += cmul(al1, mvmul(I1, -dr));
-            w2 += cmul(al2, mvmul(I2, dr));
-            // 2 translation rows
-            const V3 n1 = ld3(J.b2xa1, j), n2 = ld3(J.c2xa1, j);
-            const V3 un1 = ld3(J.un1, j), un2 = ld3(J.un2, j), rn1 = ld3(J.rn1, j), rn2 = ld3(J.rn2, j);
-            const float el1 = -dot(n1, v1) - dot(w1, un1) + dot(n1, v2) + dot(w2, rn1);
-            const float el2 = -dot(n2, v1) - dot(w1, un2) + dot(n2, v2) + dot(w2, rn2);
-            const float x0 = -el1 - bias0.x, x1 = -el2 - bias0.y;
-            const float4 kt = J.kt0[j];
-            const float d0 = kt.x * x0 + kt.y * x1;
-            const float d1 = kt.z * x0 + kt.w * x1;
-            float4 it = J.impT[j];
-            it.x += d0;
-            it.y += d1;
-            J.impT[j] = it;
-            const V3 li1 = (-n1) * d0 - n2 * d1;
-            const V3 ai1 = (-un1) * d0 - un2 * d1;
-            v1 += lock_mul((im1 * ll1), li1);
-            w1 += cmul(al1, mvmul(I1, ai1));
-            const V3 ai2 = rn1 * d0 + rn2 * d1;
-            v2 += lock_mul((im2 * ll2), -li1);
-            w2 += cmul(al2, mvmul(I2, ai2));
+            if (side) J.impL[j] = il;
         }
-        B.cv[u1] = f4(v1, 0.f); st3(B.cw, u1, w1);
-        B.cv[u2] = f4(v2, 0.f); st3(B.cw, u2, w2);
+        // 3 rotation rows
+        const V3 Jvr = b.w - pair_from1(b.w);
+        const V3 dr = mvmul(Kr, -Jvr - v3(bias1.x, bias1.y, bias1.z));
+        if (side) J.impR[j] = f4(ir + dr, 0.f);
+        joint_spin(b, flip3(pair_from2(dr), b.s1));
+        // 2 translation rows
+        const V3 n1 = ld3(J.b2xa1, j), n2 = ld3(J.c2xa1, j);
+        const V3 arm1 = side ? ld3(J.rn1, j) : ld3(J.un1, j), arm2 = side ? ld3(J.rn2, j) : ld3(J.un2, j);
+        const float p1 = dot(n1, b.v), q1 = dot(b.w, arm1), p2 = dot(n2, b.v), q2 = dot(b.w, arm2);
+        const float el1 = -dpp<kQuadFrom1>(p1) - dpp<kQuadFrom1>(q1) + p1 + q1;
+        const float el2 = -dpp<kQuadFrom1>(p2) - dpp<kQuadFrom1>(q2) + p2 + q2;
+        const float x0 = -el1 - bias0.x, x1 = -el2 - bias0.y;
+        const float4 kt = J.kt0[j];
+        float d0 = kt.x * x0 + kt.y * x1;
+        float d1 = kt.z * x0 + kt.w * x1;
+        it.x += d0;
+        it.y += d1;
+        if (side) J.impT[j] = it;
+        d0 = dpp<kQuadFrom2>(d0);
+        d1 = dpp<kQuadFrom2>(d1);
+        const V3 li1 = (-n1) * d0 - n2 * d1;
+        b.v += lock_mul(b.iml, flip3(li1, b.s2));
+        joint_spin(b, flip3(arm1, b.s1) * d0 + flip3(arm2, b.s1) * d1);
     }
+    st3(B.cv, u, b.v);
+    st3(B.cw, u, b.w);
 }
 
 // ------------------------------------------------------------------------------------------------

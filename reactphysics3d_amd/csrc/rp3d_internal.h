@@ -187,7 +187,10 @@ struct DevSolver {
     // per point [4*m + k]
     float4 *pn;                // normal xyz, penetration depth
     float4 *r1, *r2;           // w: inverse penetration mass | restitution bias
-    float4 *lam;               // penetration impulse, split impulse, resting flag (warm-start transfer)
+    float4 *i1, *i2;           // inverse inertia x (lever arm x normal) of body 1 / 2, constant over the sweeps
+    float4 *lam;               // cached penetration impulse, 0, resting flag (warm-start transfer)
+    float4 *lq;                // [2*m] penetration impulses of the four points, [2*m+1] their split impulses:
+                               // the accumulators of the sweeps
     float4 *pred;              // learned warm start: predicted normal impulse, friction 1, friction 2
 };
 

@@ -20,10 +20,8 @@ struct SvArgs {
     float restitution_threshold;
     int learned;          // learned warm start for points without a cached impulse
     const int* adj_offs;  // body -> manifold adjacency offsets (manifold count of a dynamic body)
-    int split;            // split impulses (1) or Baumgarte contacts (0), PhysicsWorld.h:599-607
 };
 
-__global__ void dyn_integrate_velocities(DevBodies B, Settings S, float dt);
 __global__ void dyn_integrate_positions(DevBodies B, float dt, float split_factor);
 __global__ void dyn_update_state(DevBodies B);
 __global__ void sv_flag_manifolds(const int* ncp, const int* xm, const int* nb_pairs, int* flag);
@@ -43,9 +41,9 @@ __global__ void sv_group_color(const int2* mb, const int* wmstart, const int* gw
                                int* color, int* order, uint64_t* keys, int* seg_start, int* ncolors, int* status);
 __global__ void sv_color_keys(const int* color, const int* nm_ptr, DevColliders C, DevPairs P, const int* mlist,
                               const int* world_group, uint64_t* keys, int* vals, int* seg_cnt, int* ncolors);
-__global__ void sv_prepare(SvArgs A);
 __global__ void sv_warmstart(SvArgs A, int color);
-__global__ void sv_solve_color(SvArgs A, int color, float beta_dt);
+template <bool SPLIT>
+__global__ void sv_solve_color(SvArgs A, int color, float beta_dt);   // one quad of lanes per manifold
 __global__ void sv_store(SvArgs A);
 
 }  // namespace rp3dg

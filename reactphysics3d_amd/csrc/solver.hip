@@ -12,16 +12,13 @@
 #include "rp3d_internal.h"
 #include "solver.h"
 #include "solver_dev.h"
+#include "solver_quad.h"
 
 namespace rp3dg {
 
 // ------------------------------------------------------------------------------------------------
 // Integration and per-colour rows (bodies in solver_dev.h)
 // ------------------------------------------------------------------------------------------------
-
-__global__ void dyn_integrate_velocities(DevBodies B, Settings S, float dt) {
-    RP3DG_GRID_STRIDE(i, B.n) dyn_integrate_velocities_one(B, S, dt, i);
-}
 
 __global__ void dyn_integrate_positions(DevBodies B, float dt, float split_factor) {
     RP3DG_GRID_STRIDE(i, B.n) dyn_integrate_positions_one(B, dt, i, split_factor);
@@ -31,26 +28,22 @@ __global__ void dyn_update_state(DevBodies B) {
     RP3DG_GRID_STRIDE(i, B.n) dyn_update_state_one(B, i);
 }
 
-__global__ void sv_prepare(SvArgs A) {
-    const int nm = *A.nm;
-    RP3DG_GRID_STRIDE(i, nm) sv_prepare_one(A, i);
-}
-
 __global__ void sv_warmstart(SvArgs A, int color) {
     if (color >= *A.ncolors) return;
     const int lo = A.cstart[color], hi = A.cstart[color + 1];
     RP3DG_GRID_STRIDE(t, hi - lo) sv_warmstart_one(A, lo + t);
 }
 
-__global__ void sv_solve_color(SvArgs A, int color, float beta_dt) {
+// four lanes a manifold (solver_quad.h)
+template <bool SPLIT>
+__global__ __launch_bounds__(512) void sv_solve_color(SvArgs A, int color, float beta_dt) {
     if (color >= *A.ncolors) return;
-    const int lo = A.cstart[color], hi = A.cstart[color + 1];
-    if (A.split) {
-        RP3DG_GRID_STRIDE(t, hi - lo) solve_manifold<true>(A, lo + t, beta_dt);
-    } else {
-        RP3DG_GRID_STRIDE(t, hi - lo) solve_manifold<false>(A, lo + t, beta_dt);
-    }
+    const int lo = A.cstart[color], n = 4 * (A.cstart[color + 1] - lo);
+    const QuadSrc Q(A.S, threadIdx.x);
+    RP3DG_GRID_STRIDE(t, n) quad_sweep_row<STATE_HBM, SPLIT>(A, Q, lo + (t >> 2), beta_dt);
 }
+template __global__ void sv_solve_color<true>(SvArgs A, int color, float beta_dt);
+template __global__ void sv_solve_color<false>(SvArgs A, int color, float beta_dt);
 
 __global__ void sv_store(SvArgs A) {
     const int nm = *A.nm;

@@ -119,12 +119,27 @@ __device__ __forceinline__ void dyn_update_state_one(const DevBodies& B, int i) 
 
 // world inverse inertia rows, indexed [body - vbase] like the velocities (staged in LDS per world)
 // World inverse inertia of body b.  Staged in LDS (iw2 == nullptr), its third row lives in the w lanes of
-// cw, sv and sw, which the solver rows therefore store with st3 (x, y, z only).
+// cw, sv and sw.  The w lanes of the staged velocities are in use in every staged layout (solver_quad.h),
+// so the solver rows store velocities with st3 (x, y, z only).
 __device__ __forceinline__ M3 body_iw(const DevBodies& B, int b) {
     const int u = b - B.vbase;
     M3 m;
     m.r[0] = ld3(B.iw0, u); m.r[1] = ld3(B.iw1, u);
     m.r[2] = B.iw2 ? ld3(B.iw2, u) : v3(B.cw[u].w, B.sv[u].w, B.sw[u].w);
+    return m;
+}
+
+// World inverse inertia of body b at the start of a step, in a launch that also runs its velocity
+// integration (sv_setup): computed here from the orientation by the integration's own operations for an
+// enabled body, whose stored rows that launch rewrites; a disabled body keeps the stored rows.
+__device__ __forceinline__ M3 body_iw_setup(const DevBodies& B, int b) {
+    M3 m;
+    if (B.flags[b] & BF_ENABLED) {
+        const float4 ii = B.ii[b];
+        m = world_inv_inertia(qmat(ldq(B.q, b)), v3(ii.x, ii.y, ii.z));
+    } else {
+        m.r[0] = ld3(B.iw0, b); m.r[1] = ld3(B.iw1, b); m.r[2] = ld3(B.iw2, b);
+    }
     return m;
 }
 
@@ -156,7 +171,7 @@ __device__ __forceinline__ void sv_prepare_one(const SvArgs& A, int i) {
         const int2 c = P.col[k];
         const int b1 = C.body[c.x], b2 = C.body[c.y];
         const V3 x1 = ld3(B.x, b1), x2 = ld3(B.x, b2);
-        const M3 I1 = body_iw(B, b1), I2 = body_iw(B, b2);
+        const M3 I1 = body_iw_setup(B, b1), I2 = body_iw_setup(B, b2);
         const float im1 = B.ii[b1].w, im2 = B.ii[b2].w;
         const float2 m1 = C.mat[c.x], m2 = C.mat[c.y];
         const float mu = m1.x * m2.x;
@@ -189,7 +204,9 @@ __device__ __forceinline__ void sv_prepare_one(const SvArgs& A, int i) {
             S.pn[4 * i + p] = pn;
             S.r1[4 * i + p] = f4(r1, imp);
             S.r2[4 * i + p] = f4(r2, rb);
-            // lam: cached normal impulse, split impulse, resting flag from the warm-start transfer
+            S.i1[4 * i + p] = f4(i1n, 0.f);
+            S.i2[4 * i + p] = f4(i2n, 0.f);
+            // lam: cached normal impulse and resting flag from the warm-start transfer
             S.lam[4 * i + p] = make_float4(l1.w, 0.0f, l2.w, 0.f);
         }
         const float fn = (float)np;
@@ -214,8 +231,6 @@ __device__ __forceinline__ void sv_prepare_one(const SvArgs& A, int i) {
         S.r2f[i] = f4(r2f, im2);
         S.t1[i] = f4(t1, f1m > 0.0f ? 1.0f / f1m : 0.0f);
         S.t2[i] = f4(t2, f2m > 0.0f ? 1.0f / f2m : 0.0f);
-        // r x t and I (r x n) are recomputed by the sweeps (same operations, same bits) instead of
-        // being stored: every iteration re-reads the rows, so smaller rows mean less traffic
         const float4 fi = P.fimp[k];
         S.imp[i] = make_float4(fi.x, fi.y, fi.z, twm > 0.0f ? 1.0f / twm : 0.0f);   // w: inverse twist mass
         S.oldt1[i] = P.fv1[k];
@@ -252,6 +267,8 @@ __device__ __forceinline__ void sv_warmstart_one(const SvArgs& A, int i) {
         body_locks(B, b2, ll2, al2);
         const int np = S.npts[i];
         const M3 I1 = body_iw(B, b1), I2 = body_iw(B, b2);
+        float* lq = reinterpret_cast<float*>(S.lq + 2 * (size_t)i);
+        S.lq[2 * (size_t)i + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
         bool any = false;
         float plx = 0.0f, ply = 0.0f;   // learned friction impulses summed over the new points
         for (int p = 0; p < np; p++) {
@@ -265,19 +282,19 @@ __device__ __forceinline__ void sv_warmstart_one(const SvArgs& A, int i) {
                 } else {   // learned warm start of a point with no cached impulse
                     const float4 pr = S.pred[q];
                     lam = fmax_s(pr.x, 0.0f);
-                    S.lam[q].x = lam;
                     plx += pr.y;
                     ply += pr.z;
                 }
+                lq[p] = lam;
                 const V3 n = xyz(S.pn[q]);
-                const V3 i1n = mvmul(I1, cross(ld3(S.r1, q), n)), i2n = mvmul(I2, cross(ld3(S.r2, q), n));
+                const V3 i1n = ld3(S.i1, q), i2n = ld3(S.i2, q);
                 const V3 ip = v3(n.x * lam, n.y * lam, n.z * lam);
                 v1.x -= im1 * ip.x * ll1.x; v1.y -= im1 * ip.y * ll1.y; v1.z -= im1 * ip.z * ll1.z;
                 w1.x -= i1n.x * al1.x * lam; w1.y -= i1n.y * al1.y * lam; w1.z -= i1n.z * al1.z * lam;
                 v2.x += im2 * ip.x * ll2.x; v2.y += im2 * ip.y * ll2.y; v2.z += im2 * ip.z * ll2.z;
                 w2.x += i2n.x * al2.x * lam; w2.y += i2n.y * al2.y * lam; w2.z += i2n.z * al2.z * lam;
             } else {
-                S.lam[q].x = 0.0f;
+                lq[p] = 0.0f;
             }
         }
         float4 imp = S.imp[i];
@@ -323,8 +340,8 @@ __device__ __forceinline__ void sv_warmstart_one(const SvArgs& A, int i) {
             imp.x = imp.y = imp.z = 0.0f;
         }
         S.imp[i] = imp;
-        if (d1) { B.cv[u1] = f4(v1, 0.f); st3(B.cw, u1, w1); }
-        if (d2) { B.cv[u2] = f4(v2, 0.f); st3(B.cw, u2, w2); }
+        if (d1) { st3(B.cv, u1, v1); st3(B.cw, u1, w1); }
+        if (d2) { st3(B.cv, u2, v2); st3(B.cw, u2, w2); }
     }
 }
 
@@ -367,159 +384,15 @@ __device__ __forceinline__ void sv_point_features(const SvArgs& A, int i, int p,
     f[23] = 1.0f / (float)S.npts[i];
 }
 
-// ContactSolverSystem::solve (CS.cpp:479-759), for one colour: with split impulses the penetration bias
-// drives the split row; with Baumgarte contacts it joins the restitution bias in the main row
-// LK = false: both bodies have unit lock factors, and every multiplication by a factor (x * 1 = x
-// exactly) is left out; LK = true multiplies as the reference does.  SPLIT: split impulses (the
-// default technique) or Baumgarte contacts, a separate copy each so that the default's sweep keeps
-// its own registers and schedule.
-template <bool LK, bool SPLIT>
-__device__ __forceinline__ void solve_manifold_t(const SvArgs& A, int i, float beta_dt) {
-    const DevBodies& B = A.B;
-    const DevSolver& S = A.S;
-    const int2 bb = S.bodies[i];
-    const int b1 = bb.x, b2 = bb.y;
-    const bool d1 = dyn_body(B, b1), d2 = dyn_body(B, b2);
-    const int u1 = b1 - B.vbase, u2 = b2 - B.vbase;
-    V3 v1 = ld3(B.cv, u1), w1 = ld3(B.cw, u1), v2 = ld3(B.cv, u2), w2 = ld3(B.cw, u2);
-    V3 sv1 = ld3(B.sv, u1), sw1 = ld3(B.sw, u1), sv2 = ld3(B.sv, u2), sw2 = ld3(B.sw, u2);
-    const float im1 = S.r1f[i].w, im2 = S.r2f[i].w;
-    V3 ll1 = v3(1.0f, 1.0f, 1.0f), al1 = ll1, ll2 = ll1, al2 = ll1;
-    if constexpr (LK) {
-        body_locks(B, b1, ll1, al1);
-        body_locks(B, b2, ll2, al2);
-    }
-    const int np = S.npts[i];
-    const M3 I1 = body_iw(B, b1), I2 = body_iw(B, b2);
-    float sumPen = 0.0f;
-    for (int p = 0; p < np; p++) {
-        const int q = 4 * i + p;
-        const float4 pn = S.pn[q];
-        const V3 n = xyz(pn);
-        const float4 r14 = S.r1[q], r24 = S.r2[q];
-        const V3 r1 = xyz(r14), r2 = xyz(r24);
-        const V3 i1n = mvmul(I1, cross(r1, n)), i2n = mvmul(I2, cross(r2, n));
-        const float ipm = r14.w, rb = r24.w;
-        float4 lam = S.lam[q];
-        const V3 dv = rel_vel(v1, w1, v2, w2, r1, r2);
-        const float Jv = dv.x * n.x + dv.y * n.y + dv.z * n.z;
-        float biasPen = 0.0f;
-        if (pn.w > 0.01f) biasPen = -(beta_dt) * fmax_s(0.0f, pn.w - 0.01f);
-        float dl = SPLIT ? -(Jv + rb) * ipm : -(Jv + (biasPen + rb)) * ipm;
-        float lt = lam.x;
-        lam.x = fmax_s(lam.x + dl, 0.0f);
-        dl = lam.x - lt;
-        const V3 li = v3(n.x * dl, n.y * dl, n.z * dl);
-        v1.x -= lk<LK>(im1 * li.x, ll1.x); v1.y -= lk<LK>(im1 * li.y, ll1.y); v1.z -= lk<LK>(im1 * li.z, ll1.z);
-        w1.x -= lk<LK>(i1n.x, al1.x) * dl; w1.y -= lk<LK>(i1n.y, al1.y) * dl; w1.z -= lk<LK>(i1n.z, al1.z) * dl;
-        v2.x += lk<LK>(im2 * li.x, ll2.x); v2.y += lk<LK>(im2 * li.y, ll2.y); v2.z += lk<LK>(im2 * li.z, ll2.z);
-        w2.x += lk<LK>(i2n.x, al2.x) * dl; w2.y += lk<LK>(i2n.y, al2.y) * dl; w2.z += lk<LK>(i2n.z, al2.z) * dl;
-        sumPen += lam.x;
-        if constexpr (!SPLIT) {
-            S.lam[q] = lam;
-            continue;
-        }
-        // split impulse row
-        const V3 dvs = rel_vel(sv1, sw1, sv2, sw2, r1, r2);
-        const float Jvs = dvs.x * n.x + dvs.y * n.y + dvs.z * n.z;
-        float dls = -(Jvs + biasPen) * ipm;
-        const float lts = lam.y;
-        lam.y = fmax_s(lam.y + dls, 0.0f);
-        dls = lam.y - lts;
-        const V3 ls = v3(n.x * dls, n.y * dls, n.z * dls);
-        sv1.x -= lk<LK>(im1 * ls.x, ll1.x); sv1.y -= lk<LK>(im1 * ls.y, ll1.y); sv1.z -= lk<LK>(im1 * ls.z, ll1.z);
-        sw1.x -= lk<LK>(i1n.x, al1.x) * dls; sw1.y -= lk<LK>(i1n.y, al1.y) * dls; sw1.z -= lk<LK>(i1n.z, al1.z) * dls;
-        sv2.x += lk<LK>(im2 * ls.x, ll2.x); sv2.y += lk<LK>(im2 * ls.y, ll2.y); sv2.z += lk<LK>(im2 * ls.z, ll2.z);
-        sw2.x += lk<LK>(i2n.x, al2.x) * dls; sw2.y += lk<LK>(i2n.y, al2.y) * dls; sw2.z += lk<LK>(i2n.z, al2.z) * dls;
-        S.lam[q] = lam;
-    }
-    const V3 r1f = ld3(S.r1f, i), r2f = ld3(S.r2f, i);
-    const float4 t14 = S.t1[i], t24 = S.t2[i], n4 = S.n[i];
-    const V3 t1 = xyz(t14), t2 = xyz(t24), n = xyz(n4);
-    const float mu = n4.w;
-    float4 imp = S.imp[i];
-    // friction 1
-    {
-        const V3 dv = rel_vel(v1, w1, v2, w2, r1f, r2f);
-        const float Jv = dv.x * t1.x + dv.y * t1.y + dv.z * t1.z;
-        float dl = -Jv * t14.w;
-        const float lim = mu * sumPen;
-        const float lt = imp.x;
-        imp.x = fmax_s(-lim, fmin_s(imp.x + dl, lim));
-        dl = imp.x - lt;
-        const V3 r1ct1 = cross(r1f, t1), r2ct1 = cross(r2f, t1);
-        const V3 a1 = v3(-r1ct1.x * dl, -r1ct1.y * dl, -r1ct1.z * dl);
-        const V3 l2 = v3(t1.x * dl, t1.y * dl, t1.z * dl);
-        const V3 a2 = v3(r2ct1.x * dl, r2ct1.y * dl, r2ct1.z * dl);
-        v1.x -= lk<LK>(im1 * l2.x, ll1.x); v1.y -= lk<LK>(im1 * l2.y, ll1.y); v1.z -= lk<LK>(im1 * l2.z, ll1.z);
-        const V3 aw1 = lkv<LK>(al1, mvmul(I1, a1));
-        w1.x += aw1.x; w1.y += aw1.y; w1.z += aw1.z;
-        v2.x += lk<LK>(im2 * l2.x, ll2.x); v2.y += lk<LK>(im2 * l2.y, ll2.y); v2.z += lk<LK>(im2 * l2.z, ll2.z);
-        const V3 aw2 = lkv<LK>(al2, mvmul(I2, a2));
-        w2.x += aw2.x; w2.y += aw2.y; w2.z += aw2.z;
-    }
-    // friction 2
-    {
-        const V3 dv = rel_vel(v1, w1, v2, w2, r1f, r2f);
-        const float Jv = dv.x * t2.x + dv.y * t2.y + dv.z * t2.z;
-        float dl = -Jv * t24.w;
-        const float lim = mu * sumPen;
-        const float lt = imp.y;
-        imp.y = fmax_s(-lim, fmin_s(imp.y + dl, lim));
-        dl = imp.y - lt;
-        const V3 r1ct2 = cross(r1f, t2), r2ct2 = cross(r2f, t2);
-        const V3 a1 = v3(-r1ct2.x * dl, -r1ct2.y * dl, -r1ct2.z * dl);
-        const V3 l2 = v3(t2.x * dl, t2.y * dl, t2.z * dl);
-        const V3 a2 = v3(r2ct2.x * dl, r2ct2.y * dl, r2ct2.z * dl);
-        v1.x -= lk<LK>(im1 * l2.x, ll1.x); v1.y -= lk<LK>(im1 * l2.y, ll1.y); v1.z -= lk<LK>(im1 * l2.z, ll1.z);
-        const V3 aw1 = lkv<LK>(al1, mvmul(I1, a1));
-        w1.x += aw1.x; w1.y += aw1.y; w1.z += aw1.z;
-        v2.x += lk<LK>(im2 * l2.x, ll2.x); v2.y += lk<LK>(im2 * l2.y, ll2.y); v2.z += lk<LK>(im2 * l2.z, ll2.z);
-        const V3 aw2 = lkv<LK>(al2, mvmul(I2, a2));
-        w2.x += aw2.x; w2.y += aw2.y; w2.z += aw2.z;
-    }
-    // twist
-    {
-        const V3 dv = w2 - w1;
-        const float Jv = dv.x * n.x + dv.y * n.y + dv.z * n.z;
-        float dl = -Jv * imp.w;   // inverse twist mass
-        const float lim = mu * sumPen;
-        const float lt = imp.z;
-        imp.z = fmax_s(-lim, fmin_s(imp.z + dl, lim));
-        dl = imp.z - lt;
-        const V3 a2 = v3(n.x * dl, n.y * dl, n.z * dl);
-        const V3 aw1 = lkv<LK>(al1, mvmul(I1, a2));
-        w1.x -= aw1.x; w1.y -= aw1.y; w1.z -= aw1.z;
-        const V3 aw2 = lkv<LK>(al2, mvmul(I2, a2));
-        w2.x += aw2.x; w2.y += aw2.y; w2.z += aw2.z;
-    }
-    S.imp[i] = imp;
-    if (d1) {
-        B.cv[u1] = f4(v1, 0.f); st3(B.cw, u1, w1);
-        st3(B.sv, u1, sv1); st3(B.sw, u1, sw1);
-    }
-    if (d2) {
-        B.cv[u2] = f4(v2, 0.f); st3(B.cw, u2, w2);
-        st3(B.sv, u2, sv2); st3(B.sw, u2, sw2);
-    }
-}
-
-// SPLIT = A.split, fixed by the caller's kernel instance (the fused solver kernel has one per technique)
-template <bool SPLIT>
-__device__ __forceinline__ void solve_manifold(const SvArgs& A, int i, float beta_dt) {
-    const int2 bb = A.S.bodies[i];
-    if (body_flags(A.B, bb.x) & body_flags(A.B, bb.y) & BF_UNIT_LOCKS) solve_manifold_t<false, SPLIT>(A, i, beta_dt);
-    else solve_manifold_t<true, SPLIT>(A, i, beta_dt);
-}
-
 // ContactSolverSystem::storeImpulses (CS.cpp:763-785); initializeForIsland marks every point resting (:161)
 __device__ __forceinline__ void sv_store_one(const SvArgs& A, int i) {
     {
         const int k = A.S.pair[i];
         const int np = A.S.npts[i];
+        const float* lq = reinterpret_cast<const float*>(A.S.lq + 2 * (size_t)i);
         for (int p = 0; p < np; p++) {
             float4 l1 = A.P.pl1[4 * k + p];
-            l1.w = A.S.lam[4 * i + p].x;
+            l1.w = lq[p];
             A.P.pl1[4 * k + p] = l1;
             float4 l2 = A.P.pl2[4 * k + p];
             l2.w = 1.0f;
