@@ -1303,8 +1303,14 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     if (fused) {
         // greedy colouring per world group in LDS, rows placed colour by colour within each group
         LAUNCH_T("sv_world_ranges", mg, 256, sv_world_ranges, B, C, N, m_list, nm_ptr, nworlds, mb, d_wmstart);
-        LAUNCH_TS("sv_group_color", ngroups, kWave, sizeof(unsigned long long) * max_group_bodies, sv_group_color, mb,
-                  d_wmstart, d_gworld, d_wbody, ngroups, color, cvals, ckeys, seg_start, &counters->nb_colors, dstatus);
+        // LDS for three manifolds a body when the groups share the CUs, all there is for a few large groups
+        const int lds_max = std::min(max_lds_per_block, max_lds_per_cu) - 8192;   // (static LDS)
+        const int lds_want = ngroups > 256 ? color_body_bytes(max_group_bodies) + color_manifold_bytes(3 * max_group_bodies + 64)
+                                           : lds_max;
+        ColorArgs K{mb, d_wmstart, d_gworld, d_wbody, ngroups, std::min(lds_want, lds_max), color, cvals, ckeys, seg_start,
+                    &counters->nb_colors, dstatus, adj, cvtmp};
+        LAUNCH_TS("sv_group_color", ngroups, std::min(1024, (max_group_bodies + kWave - 1) / kWave * kWave), K.lds_bytes,
+                  sv_group_color, K);
     } else {
         // Jones-Plassmann over the whole batch, then a radix sort of the rows by colour
         fill_int<<<grid_for(nb), 256, 0, stream>>>(adj_cursor, nb, 0);

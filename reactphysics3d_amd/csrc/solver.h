@@ -37,8 +37,27 @@ __global__ void sv_color_finish(const int2* mb, const int* nm_ptr, const int* of
                                 const int* left_prev, int* rounds, int* status);
 __global__ void sv_world_ranges(DevBodies B, DevColliders C, DevPairs P, const int* list, const int* nm_ptr, int nw,
                                 int2* mb, int* wmstart);
-__global__ void sv_group_color(const int2* mb, const int* wmstart, const int* gworld, const int* wbody, int ngroups,
-                               int* color, int* order, uint64_t* keys, int* seg_start, int* ncolors, int* status);
+// Arguments of the group colouring (solver.hip).
+struct ColorArgs {
+    const int2* mb;        // dynamic bodies of every manifold (-1: none)
+    const int* wmstart;    // [nw + 1] first manifold of every world
+    const int* gworld;
+    const int* wbody;
+    int ngroups;
+    int lds_bytes;         // dynamic LDS of the launch
+    int *color, *order;
+    uint64_t* keys;
+    int* seg_start;
+    int *ncolors, *status;
+    int *list, *pend;      // HBM scratch: [2 * manifolds] and [manifolds]
+};
+
+// LDS of a group besides its manifolds: colour mask, list head and end, two work lists, per body
+__host__ __device__ constexpr int color_body_bytes(int bodies) { return bodies * (8 + 4 + 4 + 2 * 4); }
+// per manifold: bodies (16 bits each), its two list entries, and two bits
+__host__ __device__ constexpr int color_manifold_bytes(int m) { return m * 8 + (m + 15) / 16 * 4; }
+
+__global__ void sv_group_color(ColorArgs A);
 __global__ void sv_color_keys(const int* color, const int* nm_ptr, DevColliders C, DevPairs P, const int* mlist,
                               const int* world_group, uint64_t* keys, int* vals, int* seg_cnt, int* ncolors);
 __global__ void sv_warmstart(SvArgs A, int color);

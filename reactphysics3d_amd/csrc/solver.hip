@@ -230,137 +230,205 @@ __global__ void sv_world_ranges(DevBodies B, DevColliders C, DevPairs P, const i
     }
 }
 
-// One 64-lane workgroup per world group.  Lane k colours the manifolds of world k of the group
-// greedily in manifold order (smallest colour unused at either dynamic body; worlds share no body, so
-// this equals greedy colouring of the whole group in manifold order), then the group's manifolds are
-// placed colour by colour, in manifold order within a colour: order[row] = manifold, keys[row] =
-// group * kMaxColors + colour, seg_start[group * kMaxColors + c] = first row of colour c.
-// Dynamic LDS: one 64-bit colour mask per body of the largest group.
-__global__ __launch_bounds__(kWave) void sv_group_color(const int2* mb, const int* wmstart, const int* gworld,
-                                                        const int* wbody, int ngroups, int* color, int* order,
-                                                        uint64_t* keys, int* seg_start, int* ncolors, int* status) {
-    extern __shared__ unsigned long long s_mask[];
-    __shared__ int s_hist[kMaxColors];
-    const int g = blockIdx.x;
-    const int lane = threadIdx.x;
-    const int w0 = gworld[g], w1 = gworld[g + 1];
-    const int b0 = wbody[w0], nbg = wbody[w1] - b0;
-    const int ma = wmstart[w0], mz = wmstart[w1];
-    for (int i = lane; i < nbg; i += kWave) s_mask[i] = 0ull;
-    s_hist[lane] = 0;
+// Greedy colouring of a group of worlds: manifolds in order, each the smallest colour unused at either of
+// its dynamic bodies; then the rows are placed colour by colour, in manifold order within a colour:
+// order[row] = manifold, keys[row] = group * kMaxColors + colour, seg_start[group * kMaxColors + c] = first
+// row of colour c of the group.
+//
+// A manifold's colour depends on the earlier manifolds of its two bodies alone, so it can be chosen as soon
+// as it heads both bodies' lists of uncoloured manifolds (kept in manifold order); choosing it makes the
+// next manifold of each list a candidate.  Every round colours all manifolds that are ready, and the colours
+// are the sequential pass's.  The rounds are as many as the longest chain of manifolds in which each shares
+// a body with an earlier one: a few dozen where the sequential pass takes one step per manifold.
+// One workgroup per group; bodies' masks and lists, and the manifolds' bodies, in LDS, or (LDS == false,
+// groups whose manifolds do not fit) the lists and counts in HBM scratch.
+template <bool LDS>
+__device__ __forceinline__ void color_group(const ColorArgs& A, char* lds, int b0, int nb, int ma, int nm, int* s_n) {
+    const int tid = threadIdx.x, nt = blockDim.x;
+    unsigned long long* mask = reinterpret_cast<unsigned long long*>(lds);
+    int* head = reinterpret_cast<int*>(mask + nb);
+    int* end = head + nb;
+    int* work = end + nb;   // [2][nb]
+    unsigned int* s_mb = reinterpret_cast<unsigned int*>(work + 2 * nb);
+    unsigned int* s_pend = s_mb + nm;
+    unsigned short* s_list = reinterpret_cast<unsigned short*>(s_pend + (nm + 15) / 16);
+    int* g_list = A.list + 2 * (size_t)ma;
+    int* g_pend = A.pend + ma;
+    constexpr unsigned int kNone = 0xffffu;
+    auto bodies_of = [&](int m) -> unsigned int {   // body 1 | body 2 << 16, relative to the group
+        if constexpr (LDS) return s_mb[m];
+        const int2 bb = A.mb[ma + m];
+        return (bb.x >= 0 ? (unsigned)(bb.x - b0) : kNone) | (bb.y >= 0 ? (unsigned)(bb.y - b0) : kNone) << 16;
+    };
+    auto list_at = [&](int k) -> int { if constexpr (LDS) return s_list[k]; else return g_list[k]; };
+    auto put_list = [&](int k, int m) { if constexpr (LDS) s_list[k] = (unsigned short)m; else g_list[k] = m; };
+    for (int i = tid; i < nb; i += nt) {
+        mask[i] = 0ull;
+        head[i] = 0;
+    }
+    if (tid < 3) s_n[tid] = 0;
     __syncthreads();
-    // greedy colouring, one world per lane.  The chain of colour decisions is serial; the body pairs of
-    // the next kAhead manifolds are loaded while the current kAhead are coloured, so a global load's
-    // latency is paid once per world rather than once per batch.
-    constexpr int kAhead = 16;
-    int cmax = -1;
-    if (w1 - w0 == 1 && mz - ma > 2 * kWave) {
-        // A group of one large world: the wave colours 64 manifolds at a time.  A manifold's colour is
-        // the smallest one used neither at its bodies by earlier chunks (the masks) nor by the earlier
-        // manifolds of its chunk that share a body with it.  Those dependencies point backwards, so
-        // iterating every lane's choice to a fixed point (at most one round per manifold of the chunk,
-        // plus one that sees no change) gives the colours of the sequential greedy pass.
-        for (int i0 = ma; i0 < mz; i0 += kWave) {
-            const int i = i0 + lane;
-            const int2 bb = i < mz ? mb[i] : make_int2(-1, -1);
-            unsigned long long pre = 0ull;
-            if (bb.x >= 0) pre |= s_mask[bb.x - b0];
-            if (bb.y >= 0) pre |= s_mask[bb.y - b0];
-            unsigned long long dep = 0ull;   // earlier lanes of the chunk sharing a dynamic body
-            for (int k = 0; k < kWave; k++) {
-                const int kx = __shfl(bb.x, k, kWave), ky = __shfl(bb.y, k, kWave);
-                const bool share = (kx >= 0 && (kx == bb.x || kx == bb.y)) || (ky >= 0 && (ky == bb.x || ky == bb.y));
-                if (k < lane && share) dep |= 1ull << k;
-            }
-            const int nd = wave_max(__popcll(dep));
-            unsigned long long used = pre;
-            int c = ~used ? __ffsll(~used) - 1 : kMaxColors - 1;
-            for (int round = 0; round <= kWave; round++) {
-                used = pre;
-                unsigned long long d = dep;
-                for (int t = 0; t < nd; t++) {   // every lane takes part in each shuffle
-                    const int k = d ? __ffsll(d) - 1 : lane;
-                    const int ck = __shfl(c, k, kWave);
-                    if (d) { used |= 1ull << ck; d &= d - 1; }
-                }
-                const int cn = ~used ? __ffsll(~used) - 1 : kMaxColors - 1;
-                const bool changed = cn != c;
-                c = cn;
-                if (!__ballot(changed)) break;
-            }
-            if (i < mz) {
-                if (!~used) atomicOr(status, STATUS_COLOR_OVERFLOW);
-                const unsigned long long bit = 1ull << c;
-                if (bb.x >= 0) atomicOr(&s_mask[bb.x - b0], bit);
-                if (bb.y >= 0) atomicOr(&s_mask[bb.y - b0], bit);
-                color[i] = c;
-                cmax = c > cmax ? c : cmax;
-            }
-            __syncthreads();
+    // lists: count, scan, fill, sort
+    for (int m = tid; m < nm; m += nt) {
+        unsigned int bb;
+        if constexpr (LDS) {
+            const int2 g = A.mb[ma + m];
+            bb = (g.x >= 0 ? (unsigned)(g.x - b0) : kNone) | (g.y >= 0 ? (unsigned)(g.y - b0) : kNone) << 16;
+            s_mb[m] = bb;
+        } else {
+            bb = bodies_of(m);
         }
-    } else if (lane < w1 - w0) {
-        const int s = wmstart[w0 + lane], e = wmstart[w0 + lane + 1];
-        int2 cur[kAhead], nxt[kAhead];
-#pragma unroll
-        for (int u = 0; u < kAhead; u++) cur[u] = s + u < e ? mb[s + u] : make_int2(-1, -1);
-        for (int i = s; i < e; i += kAhead) {
-#pragma unroll
-            for (int u = 0; u < kAhead; u++) nxt[u] = i + kAhead + u < e ? mb[i + kAhead + u] : make_int2(-1, -1);
-#pragma unroll
-            for (int u = 0; u < kAhead; u++) {
-                if (i + u >= e) break;
-                const int2 bb = cur[u];
-                unsigned long long used = 0ull;
-                if (bb.x >= 0) used |= s_mask[bb.x - b0];
-                if (bb.y >= 0) used |= s_mask[bb.y - b0];
-                int c = ~used ? __ffsll(~used) - 1 : kMaxColors;
-                if (c >= kMaxColors) {
-                    atomicOr(status, STATUS_COLOR_OVERFLOW);
-                    c = kMaxColors - 1;
-                }
-                const unsigned long long bit = 1ull << c;
-                if (bb.x >= 0) s_mask[bb.x - b0] |= bit;
-                if (bb.y >= 0) s_mask[bb.y - b0] |= bit;
-                color[i + u] = c;
-                cmax = c > cmax ? c : cmax;
-            }
-#pragma unroll
-            for (int u = 0; u < kAhead; u++) cur[u] = nxt[u];
+        if ((bb & kNone) != kNone) atomicAdd(&head[bb & kNone], 1);
+        if (bb >> 16 != kNone) atomicAdd(&head[bb >> 16], 1);
+        if constexpr (!LDS) g_pend[m] = ((bb & kNone) != kNone ? 1 : 0) | (bb >> 16 != kNone ? 2 : 0);
+    }
+    if constexpr (LDS)
+        for (int k = tid; k < (nm + 15) / 16; k += nt) s_pend[k] = 0u;
+    __syncthreads();
+    {
+        int carry = 0;
+        for (int base = 0; base < nb; base += nt) {
+            const int i = base + tid;
+            const int c = i < nb ? head[i] : 0;
+            int total;
+            const int e = block_excl_scan(c, s_n + 8, &total) + carry + c;
+            if (i < nb) head[i] = end[i] = e;
+            carry += total;
         }
     }
-    cmax = wave_max(cmax);
-    if (lane == 0 && cmax >= 0) atomicMax(ncolors, cmax + 1);
-    __syncthreads();   // the colours written above are read back by other lanes of this workgroup
-    for (int i = ma + lane; i < mz; i += kWave) atomicAdd(&s_hist[color[i]], 1);
     __syncthreads();
-    // segment starts: exclusive prefix of the colour counts
-    const int cnt = s_hist[lane];
-    const int base = ma + wave_incl_scan(cnt) - cnt;
-    seg_start[(size_t)g * kMaxColors + lane] = base;
-    if (g == ngroups - 1 && lane == 0) seg_start[(size_t)ngroups * kMaxColors] = wmstart[gworld[ngroups]];
-    __syncthreads();
-    s_hist[lane] = base;   // running cursor of each colour
-    __syncthreads();
-    // stable placement, 64 manifolds at a time: lanes of equal colour take consecutive rows
-    const unsigned long long below = (1ull << lane) - 1ull;
-    for (int i0 = ma; i0 < mz; i0 += kWave) {
-        const int i = i0 + lane;
-        const int c = i < mz ? color[i] : -1;
-        unsigned long long pending = __ballot(c >= 0);
-        while (pending) {
-            const int leader = __ffsll(pending) - 1;
-            const int cl = __shfl(c, leader, kWave);
-            const unsigned long long same = __ballot(c == cl);
-            if (c == cl) {
-                const int row = s_hist[cl] + __popcll(same & below);
-                order[row] = i;
-                keys[row] = (uint64_t)g * kMaxColors + cl;
-            }
-            pending &= ~same;
-            __syncthreads();
-            if (lane == leader) s_hist[cl] += __popcll(same);
-            __syncthreads();
+    for (int m = tid; m < nm; m += nt) {
+        const unsigned int bb = bodies_of(m);
+        if ((bb & kNone) != kNone) put_list(atomicSub(&head[bb & kNone], 1) - 1, m);
+        if (bb >> 16 != kNone) put_list(atomicSub(&head[bb >> 16], 1) - 1, m);
+        if constexpr (LDS) {
+            const unsigned int bits = ((bb & kNone) != kNone ? 1u : 0u) | (bb >> 16 != kNone ? 2u : 0u);
+            if (bits) atomicOr(&s_pend[m >> 4], bits << (2 * (m & 15)));
         }
+        if (bb == 0xffffffffu) A.color[ma + m] = 0;   // no dynamic body
+    }
+    __syncthreads();
+    // the manifold m became the first uncoloured one of body b: true when it is of both its bodies
+    auto arrive = [&](int m, unsigned int b) -> bool {
+        const unsigned int bb = bodies_of(m), bit = (bb & kNone) == b ? 1u : 2u;
+        if constexpr (LDS) {
+            const int sh = 2 * (m & 15);
+            const unsigned int left = atomicAnd(&s_pend[m >> 4], ~(bit << sh)) & ~(bit << sh);
+            return ((left >> sh) & 3u) == 0u;
+        } else {
+            return (atomicAnd((unsigned int*)&g_pend[m], ~bit) & ~bit) == 0u;
+        }
+    };
+    for (int b = tid; b < nb; b += nt) {
+        const int s = head[b], e = end[b];
+        for (int i = s + 1; i < e; i++) {   // insertion sort: lists are short
+            const int m = list_at(i);
+            int j = i;
+            for (; j > s && list_at(j - 1) > m; j--) put_list(j, list_at(j - 1));
+            put_list(j, m);
+        }
+        if (s < e) {
+            const int m = list_at(s);
+            if (arrive(m, (unsigned)b)) work[atomicAdd(&s_n[0], 1)] = m;
+        }
+    }
+    __syncthreads();
+    // rounds.  A ready manifold owns its bodies, so their masks and heads need no atomics; at most one ready
+    // manifold per body bounds the work lists.
+    for (int round = 0;; round++) {
+        const int cur = round % 3, nxt = (round + 1) % 3;
+        const int n = s_n[cur];
+        if (n == 0) break;
+        const int* wl = work + (round & 1) * nb;
+        int* wn = work + ((round + 1) & 1) * nb;
+        if (tid == 0) s_n[(round + 2) % 3] = 0;
+        for (int t = tid; t < n; t += nt) {
+            const int m = wl[t];
+            const unsigned int bb = bodies_of(m), x = bb & kNone, y = bb >> 16;
+            unsigned long long used = 0ull;
+            if (x != kNone) used |= mask[x];
+            if (y != kNone) used |= mask[y];
+            int c = ~used ? __ffsll(~used) - 1 : kMaxColors;
+            if (c >= kMaxColors) {
+                atomicOr(A.status, STATUS_COLOR_OVERFLOW);
+                c = kMaxColors - 1;
+            }
+            A.color[ma + m] = c;
+            for (int k = 0; k < 2; k++) {
+                const unsigned int b = k ? y : x;
+                if (b == kNone) continue;
+                mask[b] |= 1ull << c;
+                const int h = head[b] + 1;
+                head[b] = h;
+                if (h < end[b]) {
+                    const int q = list_at(h);
+                    if (arrive(q, b)) wn[atomicAdd(&s_n[nxt], 1)] = q;
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(1024) void sv_group_color(ColorArgs A) {
+    extern __shared__ char s_color[];
+    __shared__ int s_n[8 + 17];          // work list lengths; scan scratch
+    __shared__ int s_base[kMaxColors];   // next row of each colour
+    __shared__ int s_wave[16][kMaxColors];
+    const int g = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+    const int w0 = A.gworld[g], w1 = A.gworld[g + 1];
+    const int b0 = A.wbody[w0], nb = A.wbody[w1] - b0;
+    const int ma = A.wmstart[w0], nm = A.wmstart[w1] - ma;
+    if (tid < kMaxColors) s_base[tid] = 0;
+    if (color_body_bytes(nb) + color_manifold_bytes(nm) <= A.lds_bytes && nm <= 0x7fff)
+        color_group<true>(A, s_color, b0, nb, ma, nm, s_n);
+    else
+        color_group<false>(A, s_color, b0, nb, ma, nm, s_n);
+    // rows: colour counts, their exclusive prefix, then stable ranks tile by tile (a wavefront's lanes of one
+    // colour by ballots, the wavefronts of the tile in order)
+    for (int m = tid; m < nm; m += nt) atomicAdd(&s_base[A.color[ma + m]], 1);
+    __syncthreads();
+    if (tid < kWave) {
+        const int cnt = s_base[tid];
+        const int base = ma + wave_incl_scan(cnt) - cnt;
+        A.seg_start[(size_t)g * kMaxColors + tid] = base;
+        s_base[tid] = base;
+        const unsigned long long present = __ballot(cnt > 0);
+        if (tid == 0 && present) atomicMax(A.ncolors, 64 - __clzll((long long)present));
+        if (g == A.ngroups - 1 && tid == 0) A.seg_start[(size_t)A.ngroups * kMaxColors] = A.wmstart[A.gworld[A.ngroups]];
+    }
+    const int wave = tid / kWave, lane = tid & (kWave - 1), nwave = nt / kWave;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (int t0 = 0; t0 < nm; t0 += nt) {
+        const int m = t0 + tid;
+        const int c = m < nm ? A.color[ma + m] : -1;
+        s_wave[wave][lane] = 0;
+        __syncthreads();
+        unsigned long long same = __ballot(c >= 0);
+#pragma unroll
+        for (int b = 0; b < 6; b++) {
+            const unsigned long long bal = __ballot((c >> b) & 1);
+            same &= ((c >> b) & 1) ? bal : ~bal;
+        }
+        const int rank = __popcll(same & below);
+        if (c >= 0 && rank == 0) s_wave[wave][c] = __popcll(same);
+        __syncthreads();
+        if (tid < kMaxColors) {   // first row of each wavefront's share
+            int run = s_base[tid];
+            for (int w = 0; w < nwave; w++) {
+                const int n = s_wave[w][tid];
+                s_wave[w][tid] = run;
+                run += n;
+            }
+            s_base[tid] = run;
+        }
+        __syncthreads();
+        if (c >= 0) {
+            const int row = s_wave[wave][c] + rank;
+            A.order[row] = ma + m;
+            A.keys[row] = (uint64_t)g * kMaxColors + c;
+        }
+        __syncthreads();
     }
 }
 
