@@ -70,14 +70,12 @@ def bytes_per_launch(name, c, ndyn, nj):
         return 192 * ndyn + 48 * ncl
     if name in ("sv_solve_color", "sv_warmstart"):
         return (48 * p + 88 * m + 140 * 2 * m) / ncol
-    if name == "sv_prepare":
-        return 420 * m + 160 * p
-    if name == "bp_traverse":
-        return 48 * ncl + 4 * ncl + 8 * npairs / 2
+    if name == "sv_setup":   # velocity integration and contact rows
+        return nb * (16 * 9 + 16 * 5) + 420 * m + 256 * p
+    if name == "bp_pairs":   # boxes in, partner lists out
+        return 48 * ncl + 8 * npairs
     if name == "bp_merge":
         return 112 * npairs   # keys, pair records and the link to the previous cache; caches are not copied
-    if name == "dyn_integrate_velocities":
-        return nb * (16 * 9 + 16 * 5)
     if name == "dyn_integrate_positions":
         return nb * (16 * 6 + 16 * 2)
     if name == "dyn_update_state":
@@ -119,14 +117,13 @@ BYTE_MODEL = {
     "np_box_box": "176 B/test + 40 B/contact point",
 }
 
-KERNELS = ["bp_bounds", "bp_morton", "bp_sort", "bp_karras", "bp_fit", "bp_world_roots", "bp_traverse", "bp_copy_pairs",
-           "bp_walk_again", "bp_world_scan",
+KERNELS = ["bp_bounds", "bp_morton", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
            "bp_merge",
            "np_classify", "np_sphere_sphere", "np_sphere_capsule", "np_capsule_capsule", "np_sphere_poly",
            "np_capsule_poly", "np_box_box", "np_poly_poly", "sv_flag", "sv_compact", "sv_adj_count", "sv_adj_fill",
            "sv_color_round", "sv_color_finish", "sv_color_keys", "sv_color_sort", "sv_world_ranges", "sv_group_color",
-           "sv_world_prepare", "mlp_infer", "sv_world_solve", "sv_log_samples", "world_position",
-           "dyn_integrate_velocities", "sv_prepare", "sv_warmstart", "sv_solve_color", "sv_store", "jt_init",
+           "sv_setup", "sv_features", "mlp_infer", "sv_world_solve", "sv_log_samples", "world_position",
+           "sv_warmstart", "sv_solve_color", "sv_store",
            "jt_warmstart", "jt_solve_velocity", "jt_solve_position", "dyn_integrate_positions", "dyn_update_state",
            "bp_refit"]
 
@@ -418,7 +415,7 @@ def main():
         # warm start
         choice, ms = dev.autotune(DT, 2)
         tuned = {"choice": choice, "ms_per_step": round(ms, 3), "trials": [[c, round(t, 3)] for c, t in dev.tune_table()],
-                 "meaning": ("world-class workgroup = clamp(bodies bound / choice, 64, 256)" if graph
+                 "meaning": ("world-class workgroup = clamp(2 x bodies bound / choice, 64, 1024)" if graph
                              else "threads per block of the colour kernels"),
                  "applied_to": "plain and learned"}
         if dev_l is not None:

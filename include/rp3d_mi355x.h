@@ -256,10 +256,10 @@ rp3dg_batch* rp3dg_batch_create(rp3dg_world* const* worlds, int32_t nb_worlds);
 /* Solver layout of a batch. */
 #define RP3DG_SOLVER_AUTO 0   /* FUSED when every world has at most 4096 bodies, else PER_COLOR */
 #define RP3DG_SOLVER_PER_COLOR 1  /* one launch per colour over all worlds (large worlds) */
-#define RP3DG_BROADPHASE_AUTO 0        /* world scan when it applies and pays (>= 64 worlds, or worlds of <= 256 colliders), else the tree */
-#define RP3DG_BROADPHASE_TREE 1        /* linear BVH over all colliders, rebuilt every step */
+#define RP3DG_BROADPHASE_AUTO 0        /* world scan when it applies and pays (>= 64 worlds, or worlds of <= 256 colliders), else tiles */
+#define RP3DG_BROADPHASE_TREE 1        /* tiles of 64 colliders in spatial order under their union boxes, rebuilt every step */
 #define RP3DG_BROADPHASE_WORLD_SCAN 2  /* fused layout, worlds of <= 1024 colliders: every collider tests its
-                                          world's boxes in LDS (no tree) */
+                                          world's boxes in LDS */
 #define RP3DG_SOLVER_FUSED 2  /* one workgroup per group of small worlds runs the whole solver phase (worlds up to 4096 bodies) */
 
 typedef struct rp3dg_batch_options {
@@ -461,7 +461,7 @@ int rp3dg_batch_get_kernel_times(rp3dg_batch* batch, const char* kernel, double*
 /* Autotuner: times each candidate launch shape of the solver over steps_per_trial real steps of the
  * batch (the steps advance the simulation) and keeps the fastest; returns the choice and its time.
  * Fused layout: worlds run in size classes (bodies in (L/2, L], L = 64 .. 4096), one concurrent launch
- * each; the candidates are the divisor d of the class workgroup clamp(L / d, 64, 256), d = 1, 2, 4, 8, 16.
+ * each; the candidates are the divisor d of the class workgroup clamp(2 L / d, 64, 1024), d = 1, 2, 4, 8, 16.
  * Per-colour layout: threads per block of the colour kernels, 64..512. */
 int rp3dg_batch_autotune(rp3dg_batch* batch, float time_step, int32_t steps_per_trial, int32_t* chosen,
                          double* best_ms_per_step);

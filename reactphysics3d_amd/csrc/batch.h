@@ -88,7 +88,7 @@ struct rp3dg_batch {
     int *d_gworld = nullptr, *d_world_group = nullptr;
     int* d_wmstart = nullptr;            // [nworlds + 1] first manifold of each world (fused colouring)
     int max_group_bodies = 0;
-    bool world_scan = false;             // broadphase by per-world box scans in LDS instead of the tree
+    bool world_scan = false;             // broadphase by per-world box scans in LDS instead of tiles
     int max_group_colliders = 0;
     float4 *res_pv = nullptr, *res_pw = nullptr;
     int* world_iters = nullptr;
@@ -169,14 +169,14 @@ struct rp3dg_batch {
 
     // broadphase scratch
     uint64_t *bp_keys = nullptr, *bp_ktmp = nullptr, *bp_out = nullptr;
-    uint64_t* bp_slab = nullptr;       // first kTravSlab partners of every collider (first traversal pass)
-    int* bp_walk = nullptr;            // colliders walked again after the scan (more partners than the slab)
+    float4 *bp_smn = nullptr, *bp_smx = nullptr;   // boxes in tile order
+    float4 *bp_tmn = nullptr, *bp_tmx = nullptr;   // union boxes of the tiles
+    int* bp_slab = nullptr;            // first kSlab partners of every collider
+    int* bp_large = nullptr;           // colliders with more
     int *bp_vals = nullptr, *bp_vtmp = nullptr;
-    int2 *bp_child = nullptr, *bp_range = nullptr;
-    int *bp_parent = nullptr, *bp_root = nullptr, *bp_count = nullptr;
+    int* bp_count = nullptr;
     int* bp_offs_ab[2] = {nullptr, nullptr};   // per-collider segment starts of pair table A / B
-    float4 *fit_min = nullptr, *fit_max = nullptr;   // unions of aligned 64 / 4096 / 262144-leaf blocks
-    float4 *bp_nmin = nullptr, *bp_nmax = nullptr, *bp_partial = nullptr;
+    float4* bp_partial = nullptr;
     // narrowphase
     int *np_lists = nullptr, *np_counts = nullptr;
     // manifolds / colouring
@@ -216,7 +216,8 @@ struct rp3dg_batch {
     int step_graph(float dt, int n);
     void drop_graphs();
     int scan(const int* in, int n, const int* nptr, int* out, hipStream_t s);
-    int sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr, int bits, hipStream_t s);
+    int sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr,
+             int first_bit, int bits, hipStream_t s);
     void timer_begin(const char* name);
     void timer_end();
     void timer_flush();

@@ -29,26 +29,19 @@ namespace rp3dg {
 __global__ void bp_refit(DevBodies B, DevColliders C, const float4* hull_bounds, int init);
 __global__ void bp_bounds(DevColliders C, float4* partial);
 __global__ void bp_morton(DevColliders C, const float4* partial, int nparts, uint64_t* keys, int* vals);
+template <int ITEMS>
 __global__ void rs_hist(const uint64_t* keys, int n, const int* nptr, int shift, int* hist, int nblocks);
+template <int ITEMS>
 __global__ void rs_scatter(const uint64_t* kin, const int* vin, uint64_t* kout, int* vout, int n, const int* nptr,
                            int shift, const int* offs, int nblocks);
-__global__ void bp_karras(const uint64_t* k, int n, int2* child, int* parent, int2* range);
-__global__ void bp_leaves(DevColliders C, const int* sorted, int n, float4* nmin, float4* nmax, float4* bmin,
-                          float4* bmax);
-__global__ void bp_blocks(const float4* imin, const float4* imax, int nin, float4* omin, float4* omax);
-__global__ void bp_internal(int n, const int2* range, float4* nmin, float4* nmax, const float4* b1min,
-                            const float4* b1max, const float4* b2min, const float4* b2max, const float4* b3min,
-                            const float4* b3max);
-__global__ void bp_world_roots(const uint64_t* k, int n, const int2* range, int* root);
-__global__ void bp_traverse(DevColliders C, const int* sorted, int n, const int2* child, const float4* nmin,
-                            const float4* nmax, const int* root, NoColLists nc, int* count,
-                            const int* offset, uint64_t* out_keys, uint64_t* slab, int capacity, int pass,
-                            int* walk_list, int* walk_count, int* status);
-__global__ void bp_walk_wave(DevColliders C, const int* sorted, int n, const int2* child, const float4* nmin,
-                             const float4* nmax, const int* root, NoColLists ncl, const int* offset, uint64_t* out_keys,
-                             int capacity, const int* walk_list, const int* walk_count, int* status);
-__global__ void bp_copy_slabs(DevColliders C, int n, const int* count, const int* offset, const uint64_t* slab,
-                              uint64_t* out_keys, int capacity, int* status);
+__global__ void bp_tiles(DevColliders C, const int* sorted, int n, float4* smn, float4* smx, float4* tmn, float4* tmx);
+__global__ void bp_pairs(DevColliders C, int n, const float4* smn, const float4* smx, const float4* tmn,
+                         const float4* tmx, const int* wcoll, NoColLists L, int* count, int* slab, int* large,
+                         int* nb_large);
+__global__ void bp_emit(DevColliders C, int n, const int* count, const int* offset, const int* slab, uint64_t* out_keys,
+                        int capacity, int* status);
+__global__ void bp_emit_large(DevColliders C, const int* wcoll, NoColLists L, const int* offset, uint64_t* out_keys,
+                              int capacity, const int* large, const int* nb_large, int* status);
 __global__ void bp_world_scan(DevColliders C, const int* gworld, const int* wcoll, const int* block_group, NoColLists L,
                               int* count, const int* offset, uint64_t* out_keys, int capacity, int pass, int* status);
 __global__ void bp_merge(DevColliders C, const uint64_t* keys, const int* nkeys_ptr, int capacity, DevPairs O,
@@ -58,6 +51,9 @@ __global__ void bp_merge(DevColliders C, const uint64_t* keys, const int* nkeys_
 // exclusive scan (out has n+1 entries; out[n] = total).  With nptr the element count is
 // min(n, *nptr), read on the device, and n is only the capacity the grid was sized for.
 // ---------------------------------------------------------------------------------------------
+// Colliders whose broadphase tiles stay in index order (no Morton sort).
+constexpr int kIndexOrderColliders = 8192;
+
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -255,22 +251,30 @@ int rp3dg_batch::scan(const int* in, int n, const int* nptr, int* out, hipStream
     return RP3DG_OK;
 }
 
-// Stable LSD radix sort of (keys, vals) over the low `bits` bits; n keys, or min(n, *nptr) when the
-// count lives on the device.  The result is in (*keys, *vals), which may be the tmp buffers.
-int rp3dg_batch::sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr, int bits,
-                      hipStream_t s) {
+// Keys a thread of the radix sort (tiles of 256 times that): 4 for up to 2^18 keys, so that the sort of a
+// few ten thousand has blocks for every CU.
+static int sort_items(int n) { return n <= (1 << 18) ? 4 : 16; }
+static int sort_blocks(int n) { return (n + 256 * sort_items(n) - 1) / (256 * sort_items(n)); }
+
+// Stable LSD radix sort of (keys, vals) over the bits [first_bit, first_bit + bits); n keys, or min(n, *nptr)
+// when the count lives on the device.  The result is in (*keys, *vals), which may be the tmp buffers.
+int rp3dg_batch::sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr, int first_bit,
+                      int bits, hipStream_t s) {
     if (n <= 1) return RP3DG_OK;
-    const int nblocks = (n + 4095) / 4096;
+    const int nblocks = sort_blocks(n);
     if (nblocks * 256 > sort_hist_cap) return RP3DG_EOVERFLOW;
     uint64_t* ki = *keys;
     int* vi = *vals;
     uint64_t* ko = ktmp;
     int* vo = vtmp;
-    for (int shift = 0; shift < bits; shift += 8) {
-        rs_hist<<<nblocks, 256, 0, s>>>(ki, n, nptr, shift, sort_hist, nblocks);
+    for (int shift = first_bit; shift < first_bit + bits; shift += 8) {
+        const bool few = sort_items(n) == 4;
+        if (few) rs_hist<4><<<nblocks, 256, 0, s>>>(ki, n, nptr, shift, sort_hist, nblocks);
+        else rs_hist<16><<<nblocks, 256, 0, s>>>(ki, n, nptr, shift, sort_hist, nblocks);
         int r = scan(sort_hist, nblocks * 256, nullptr, sort_offs, s);
         if (r) return r;
-        rs_scatter<<<nblocks, 256, 0, s>>>(ki, vi, ko, vo, n, nptr, shift, sort_offs, nblocks);
+        if (few) rs_scatter<4><<<nblocks, 256, 0, s>>>(ki, vi, ko, vo, n, nptr, shift, sort_offs, nblocks);
+        else rs_scatter<16><<<nblocks, 256, 0, s>>>(ki, vi, ko, vo, n, nptr, shift, sort_offs, nblocks);
         std::swap(ki, ko);
         std::swap(vi, vo);
     }
@@ -915,26 +919,25 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
         TA.edges = d_edges; TA.vidx = d_vidx;
         TA.face_edge0[0] = tfe[0]; TA.face_edge0[1] = tfe[1];
     }
-    const int nn = std::max(1, 2 * nc);
-    bp_keys = dalloc<uint64_t>(this, nc); bp_vals = dalloc<int>(this, nc);
-    bp_ktmp = dalloc<uint64_t>(this, nc); bp_vtmp = dalloc<int>(this, nc);
-    bp_child = dalloc<int2>(this, nn); bp_parent = dalloc<int>(this, nn); bp_range = dalloc<int2>(this, nn);
-    bp_nmin = dalloc<float4>(this, nn); bp_nmax = dalloc<float4>(this, nn);
-    {
-        const int nb1 = (nc + 63) / 64, nb2 = (nb1 + 63) / 64, nb3 = (nb2 + 63) / 64;
-        fit_min = dalloc<float4>(this, nb1 + nb2 + nb3);
-        fit_max = dalloc<float4>(this, nb1 + nb2 + nb3);
+    if (!world_scan) {
+        const int nt = (nc + 63) / 64;
+        if (nc > kIndexOrderColliders) {
+            bp_keys = dalloc<uint64_t>(this, nc); bp_vals = dalloc<int>(this, nc);
+            bp_ktmp = dalloc<uint64_t>(this, nc); bp_vtmp = dalloc<int>(this, nc);
+            bp_partial = dalloc<float4>(this, 2 * 256);
+        }
+        bp_smn = dalloc<float4>(this, nc); bp_smx = dalloc<float4>(this, nc);
+        bp_tmn = dalloc<float4>(this, nt); bp_tmx = dalloc<float4>(this, nt);
+        bp_slab = dalloc<int>(this, (size_t)nc * kSlab);
+        bp_large = dalloc<int>(this, nc);
+        if (!bp_large || !bp_slab || !bp_tmx) { set_error("device allocation failed (broadphase)"); return RP3DG_EHIP; }
     }
-    bp_root = dalloc<int>(this, (size_t)1 << world_bits);
-    bp_partial = dalloc<float4>(this, 2 * 256);
     bp_count = dalloc<int>(this, nc + 1);
     for (int t = 0; t < 2; t++) {
         bp_offs_ab[t] = dalloc<int>(this, nc + 1);
         if (bp_offs_ab[t]) HIPCHECK(hipMemset(bp_offs_ab[t], 0, sizeof(int) * (nc + 1)));
     }
     bp_out = dalloc<uint64_t>(this, pair_cap);
-    bp_slab = dalloc<uint64_t>(this, (size_t)nc * kTravSlab);
-    bp_walk = dalloc<int>(this, nc);
     np_lists = dalloc<int>(this, (size_t)kNpListSlots * pair_cap);
     np_counts = dalloc<int>(this, ALGO_COUNT);
     m_flag = dalloc<int>(this, pair_cap); m_offs = dalloc<int>(this, pair_cap + 1);
@@ -1017,7 +1020,8 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     S.lq = dalloc<float4>(this, 2 * (size_t)man_cap);
     scan_sums_cap = 1 << 16;
     scan_sums_buf = dalloc<int>(this, scan_sums_cap);
-    sort_hist_cap = 256 * (std::max(man_cap, nc) / 4096 + 2);
+    sort_hist_cap = 0;
+    for (int n : {nc, man_cap}) sort_hist_cap = std::max(sort_hist_cap, 256 * (sort_blocks(n) + 1));
     if ((sort_hist_cap + kScanTile - 1) / kScanTile > scan_sums_cap || (man_cap + kScanTile - 1) / kScanTile > scan_sums_cap) {
         set_error("batch too large for the scan workspace");
         return RP3DG_EOVERFLOW;
@@ -1119,39 +1123,33 @@ int rp3dg_batch::enqueue_broadphase(bool capturing, const DevEvents& E, int pg) 
     const int* old_offs = bp_offs_ab[cur_is_a ? 0 : 1];   // segments of the previous table
     int* dstatus = &counters->status;
     int r;
-    uint64_t* k = bp_keys;
-    int* vls = bp_vals;
     const size_t scan_lds = 2 * sizeof(float4) * max_group_colliders;
     if (world_scan) {
         // small worlds: every dynamic collider tests the boxes of its world in LDS
         LAUNCH_TS("bp_world_scan", ngroups, 256, scan_lds, bp_world_scan, C, d_gworld, d_wcoll, d_block_world,
                   nocol_lists, bp_count, bp_offs, bp_out, pair_cap, 0, dstatus);
     } else {
-        const int nparts = std::min(256, grid_for(nc));
-        LAUNCH_T("bp_bounds", nparts, 256, bp_bounds, C, bp_partial);
-        LAUNCH_T("bp_morton", grid_for(nc), 256, bp_morton, C, bp_partial, nparts, bp_keys, bp_vals);
-        timer_begin("bp_sort");
-        r = sort(&k, &vls, bp_ktmp, bp_vtmp, nc, nullptr, 30 + world_bits, stream);
-        timer_end();
-        if (r) { set_error("radix sort overflow"); return r; }
-        if (nc > 1) LAUNCH_T("bp_karras", grid_for(nc - 1), 256, bp_karras, k, nc, bp_child, bp_parent, bp_range);
-        {
-            const int nb1 = (nc + 63) / 64, nb2 = (nb1 + 63) / 64;
-            timer_begin("bp_fit");
-            bp_leaves<<<grid_for(nc), 256, 0, stream>>>(C, vls, nc, bp_nmin, bp_nmax, fit_min, fit_max);
-            bp_blocks<<<grid_for(nb1), 256, 0, stream>>>(fit_min, fit_max, nb1, fit_min + nb1, fit_max + nb1);
-            bp_blocks<<<grid_for(nb2), 256, 0, stream>>>(fit_min + nb1, fit_max + nb1, nb2, fit_min + nb1 + nb2,
-                                                          fit_max + nb1 + nb2);
-            if (nc > 1)
-                bp_internal<<<grid_for(nc - 1), 256, 0, stream>>>(nc, bp_range, bp_nmin, bp_nmax, fit_min, fit_max,
-                                                                  fit_min + nb1, fit_max + nb1, fit_min + nb1 + nb2,
-                                                                  fit_max + nb1 + nb2);
+        // tiles of 64 colliders in spatial order; up to kIndexOrderColliders in index order, where testing
+        // more tiles costs less than the launches of the sort
+        const int* order = nullptr;
+        if (nc > kIndexOrderColliders) {
+            const int nparts = std::min(256, grid_for(nc));
+            LAUNCH_T("bp_bounds", nparts, 256, bp_bounds, C, bp_partial);
+            LAUNCH_T("bp_morton", grid_for(nc), 256, bp_morton, C, bp_partial, nparts, bp_keys, bp_vals);
+            // cells of 16 Morton bits (2 passes), 24 where 64-collider tiles need finer ones
+            const int cell_bits = nc <= (1 << 18) ? 16 : 24;
+            uint64_t* k = bp_keys;
+            int* v = bp_vals;
+            timer_begin("bp_sort");
+            r = sort(&k, &v, bp_ktmp, bp_vtmp, nc, nullptr, 30 - cell_bits, cell_bits + world_bits, stream);
             timer_end();
+            if (r) { set_error("radix sort overflow"); return r; }
+            order = v;
         }
-        LAUNCH_T("bp_world_roots", grid_for(2 * nc - 1), 256, bp_world_roots, k, nc, bp_range, bp_root);
-        LAUNCH_T("bp_traverse", grid_for(nc, kTravBlock, 1 << 20), kTravBlock, bp_traverse, C, vls, nc, bp_child,
-                 bp_nmin, bp_nmax, bp_root, nocol_lists, bp_count, bp_offs, bp_out, bp_slab, pair_cap, 0, bp_walk,
-                 &counters->nb_walk_again, dstatus);
+        const int ntiles = (nc + 63) / 64;
+        LAUNCH_T("bp_tiles", grid_for(nc), 256, bp_tiles, C, order, nc, bp_smn, bp_smx, bp_tmn, bp_tmx);
+        LAUNCH_T("bp_pairs", ntiles, ntiles > 512 ? 256 : 1024, bp_pairs, C, nc, bp_smn, bp_smx, bp_tmn, bp_tmx, d_wcoll,
+                 nocol_lists, bp_count, bp_slab, bp_large, &counters->nb_large);
     }
     r = scan(bp_count, nc, nullptr, bp_offs, stream);
     if (r) { set_error("scan overflow"); return r; }
@@ -1159,12 +1157,11 @@ int rp3dg_batch::enqueue_broadphase(bool capturing, const DevEvents& E, int pg) 
         LAUNCH_TS("bp_world_scan", ngroups, 256, scan_lds, bp_world_scan, C, d_gworld, d_wcoll, d_block_world,
                   nocol_lists, bp_count, bp_offs, bp_out, pair_cap, 1, dstatus);
     } else {
-        LAUNCH_T("bp_copy_pairs", grid_for(nc * kTravSlab, 256, 1 << 20), 256, bp_copy_slabs, C, nc, bp_count, bp_offs,
-                 bp_slab, bp_out, pair_cap, dstatus);
-        const int hw = capturing ? nc : std::min(nc, last.nb_walk_again + last.nb_walk_again / 4 + 256);
-        LAUNCH_T("bp_walk_again", std::max(1, std::min(hw, 1 << 16)), kWave, bp_walk_wave, C, vls, nc, bp_child,
-                 bp_nmin, bp_nmax, bp_root, nocol_lists, bp_offs, bp_out, pair_cap, bp_walk, &counters->nb_walk_again,
-                 dstatus);
+        LAUNCH_T("bp_emit", grid_for(nc * 8, 256, 1 << 20), 256, bp_emit, C, nc, bp_count, bp_offs, bp_slab, bp_out,
+                 pair_cap, dstatus);
+        const int hl = capturing ? 256 : std::min(nc, last.nb_large + last.nb_large / 4 + 16);
+        LAUNCH_T("bp_emit_large", std::max(1, std::min(hl, 1024)), 1024, bp_emit_large, C, d_wcoll, nocol_lists, bp_offs,
+                 bp_out, pair_cap, bp_large, &counters->nb_large, dstatus);
     }
     if (events_on) fill_int_n<<<pg, 256, 0, stream>>>(O.kept, pair_cap, old_count, 0);
     LAUNCH_T("bp_merge", pg, 256, bp_merge, C, bp_out, bp_offs + nc, pair_cap, O, old_count, old_offs, N, new_count,
@@ -1328,7 +1325,7 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         int sbits = 0;
         while ((1 << sbits) < nseg) sbits++;
         timer_begin("sv_color_sort");
-        r = sort(&ck, &cv, cktmp, cvtmp, man_cap, nm_ptr, sbits, stream);
+        r = sort(&ck, &cv, cktmp, cvtmp, man_cap, nm_ptr, 0, sbits, stream);
         timer_end();
         if (r) { set_error("sort overflow"); return r; }
         r = scan(seg_cnt, nseg, nullptr, seg_start, stream);
@@ -2650,7 +2647,7 @@ int64_t rp3dg_batch_get_log(rp3dg_batch* b, float* feats, float* targets, int64_
 
 // Autotuner: times every candidate launch shape of the solver over a few real steps of this batch
 // (the steps are not undone) and keeps the fastest.  Fused layout: workgroup size of each world
-// class = clamp(bodies bound / d, 64, 256) for d = 1, 2, 4, 8, 16 (the choice returned is d); per-colour
+// class = clamp(2 x bodies bound / d, 64, 1024) for d = 1, 2, 4, 8, 16 (the choice returned is d); per-colour
 // layout: threads per block of the colour kernels.
 int rp3dg_batch_autotune(rp3dg_batch* b, float dt, int32_t steps_per_trial, int32_t* chosen, double* best_ms) {
     if (!b || !(dt > 0.f) || steps_per_trial < 1 || steps_per_trial > 1000) return RP3DG_EINVAL;

@@ -8,15 +8,15 @@
 // filtered by different-body / category masks / no-collision body pairs
 // (CollisionDetectionSystem.cpp:270-343).  We therefore keep the persistent
 // fat AABB per collider (same FP32 refit as BroadPhaseSystem.cpp:155-185) and
-// rebuild a linear BVH over them every step:
-//   bp_bounds -> bp_morton -> radix sort (LDS, stable, 8-bit digits)
-//   -> bp_karras (Karras 2012 radix tree) -> node boxes as unions over leaf ranges
-//      (bp_leaves, bp_blocks, bp_internal; no inter-thread synchronisation)
-//   -> bp_traverse (count, first 8 partners sorted into a slab) -> scan
-//   -> bp_copy_slabs (slab -> per-collider sorted segment) + bp_traverse again
-//      for the few colliders with more partners
-//   -> bp_merge (carry orientation, temporal-coherence record and contact cache
-//      of surviving pairs; orient new pairs like the reference).
+// find the overlaps of the current boxes anew every step, without a tree:
+//   bp_tiles  boxes in spatial order (Morton cells, radix sort) or, up to a few
+//             thousand colliders, in index order; the union box of every 64
+//   bp_pairs  one workgroup per tile of 64 colliders against the tiles it meets
+//   scan of the partner counts
+//   bp_emit   partners -> each collider's sorted segment of the pair keys
+//   bp_merge  carries orientation, temporal-coherence record and contact cache
+//             of surviving pairs; orients new pairs like the reference.
+// Batches of many small worlds scan each world in LDS instead (bp_world_scan).
 #include <hip/hip_runtime.h>
 
 #include "kcommon.h"
@@ -29,9 +29,55 @@ __global__ void bp_refit(DevBodies B, DevColliders C, const float4* hull_bounds,
     RP3DG_GRID_STRIDE(i, C.n) refit_one(B, C, hull_bounds, init, i);
 }
 
+__device__ __forceinline__ void box_union(float4& mn, float4& mx, float4 bmn, float4 bmx) {
+    mn = make_float4(fminf(mn.x, bmn.x), fminf(mn.y, bmn.y), fminf(mn.z, bmn.z), 0.f);
+    mx = make_float4(fmaxf(mx.x, bmx.x), fmaxf(mx.y, bmx.y), fmaxf(mx.z, bmx.z), 0.f);
+}
+
+__device__ __forceinline__ void wave_box_union(float4& mn, float4& mx) {
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        float4 omn, omx;
+        omn.x = __shfl_xor(mn.x, off, kWave); omn.y = __shfl_xor(mn.y, off, kWave); omn.z = __shfl_xor(mn.z, off, kWave);
+        omx.x = __shfl_xor(mx.x, off, kWave); omx.y = __shfl_xor(mx.y, off, kWave); omx.z = __shfl_xor(mx.z, off, kWave);
+        box_union(mn, mx, omn, omx);
+    }
+}
+
+__device__ __forceinline__ bool aabb_overlap(float4 amn, float4 amx, float4 bmn, float4 bmx) {
+    // AABB::testCollision (AABB.h:179-187), closed intervals
+    if (amx.x < bmn.x || bmx.x < amn.x) return false;
+    if (amx.y < bmn.y || bmx.y < amn.y) return false;
+    if (amx.z < bmn.z || bmx.z < amn.z) return false;
+    return true;
+}
+
+// Body pairs that must not collide (joints with collideConnected = false): per-body partner lists
+__device__ __forceinline__ bool no_collision(const NoColLists& L, int ba, int bb) {
+    const int e = L.offs[ba + 1];
+    for (int k = L.offs[ba]; k < e; k++)
+        if (L.list[k] == bb) return true;
+    return false;
+}
+
+__device__ __forceinline__ bool filters_pass(uint32_t fa, uint32_t fb) {
+    const uint32_t cata = fa & 0xffffu, maska = fa >> 16, catb = fb & 0xffffu, maskb = fb >> 16;
+    return (maska & catb) != 0 && (cata & maskb) != 0;
+}
+
+// Pair filter of CollisionDetectionSystem::updateOverlappingPairs (CD.cpp:284-331): different bodies, no
+// joint excluding the pair, collision category / mask, at least one convex shape (:324-331)
+__device__ __forceinline__ bool pair_allowed(const DevColliders& C, int a, int b, const NoColLists& L) {
+    const int ba = C.body[a], bb = C.body[b];
+    if (ba == bb) return false;
+    if (no_collision(L, ba, bb)) return false;
+    if (shape_is_concave(C.type[a]) && shape_is_concave(C.type[b])) return false;
+    return filters_pass(C.filter[a], C.filter[b]);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Morton keys over fat-AABB centres; the world id sits above the 30 Morton bits so that every
-// world occupies a contiguous key range and owns one subtree of the radix tree.
+// world occupies a contiguous key range.
 // ---------------------------------------------------------------------------------------------
 
 __global__ void bp_bounds(DevColliders C, float4* partial) {
@@ -72,17 +118,16 @@ __device__ inline uint32_t expand10(uint32_t v) {
     return v;
 }
 
-__global__ void bp_morton(DevColliders C, const float4* partial, int nparts, uint64_t* keys, int* vals) {
+__global__ __launch_bounds__(256) void bp_morton(DevColliders C, const float4* partial, int nparts, uint64_t* keys, int* vals) {
     __shared__ float4 bmn, bmx;
-    if (threadIdx.x == 0) {
-        float4 mn = partial[0], mx = partial[1];
-        for (int p = 1; p < nparts; p++) {
-            const float4 a = partial[2 * p], b = partial[2 * p + 1];
-            mn.x = fminf(mn.x, a.x); mn.y = fminf(mn.y, a.y); mn.z = fminf(mn.z, a.z);
-            mx.x = fmaxf(mx.x, b.x); mx.y = fmaxf(mx.y, b.y); mx.z = fmaxf(mx.z, b.z);
+    if (threadIdx.x < kWave) {
+        float4 mn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), mx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+        for (int p = threadIdx.x; p < nparts; p += kWave) box_union(mn, mx, partial[2 * p], partial[2 * p + 1]);
+        wave_box_union(mn, mx);
+        if (threadIdx.x == 0) {
+            bmn = mn;
+            bmx = mx;
         }
-        bmn = mn;
-        bmx = mx;
     }
     __syncthreads();
     const float sx = bmx.x > bmn.x ? 1023.0f / (bmx.x - bmn.x) : 0.f;
@@ -101,24 +146,24 @@ __global__ void bp_morton(DevColliders C, const float4* partial, int nparts, uin
 }
 
 // ---------------------------------------------------------------------------------------------
-// Stable LSD radix sort, 8-bit digits.  Tiles of kSortTile keys per block; inside a tile keys are
+// Stable LSD radix sort, 8-bit digits.  Tiles of 256 x ITEMS keys per block; inside a tile keys are
 // ranked by wave-level multisplit (8 ballots give the lanes sharing a digit) and cross-wave
 // prefix counts in LDS, so equal digits keep their input order.
 // ---------------------------------------------------------------------------------------------
 
 constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortThreads * kSortItems;
 
-// n: key count, or its upper bound when nptr (the count in device memory) is given.
+// n: key count, or its upper bound when nptr (the count in device memory) is given.  ITEMS: keys a thread; 16,
+// or 4 for a sort that would otherwise run on a fraction of the CUs.
+template <int ITEMS>
 __global__ __launch_bounds__(kSortThreads) void rs_hist(const uint64_t* keys, int n, const int* nptr, int shift, int* hist,
                                                         int nblocks) {
     if (nptr) n = min(n, *nptr);
     __shared__ int h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    const int base = blockIdx.x * kSortTile;
-    for (int k = 0; k < kSortItems; k++) {
+    const int base = blockIdx.x * kSortThreads * ITEMS;
+    for (int k = 0; k < ITEMS; k++) {
         const int i = base + k * kSortThreads + threadIdx.x;
         if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xff], 1);
     }
@@ -131,6 +176,7 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
+template <int ITEMS>
 __global__ __launch_bounds__(kSortThreads) void rs_scatter(const uint64_t* kin, const int* vin, uint64_t* kout,
                                                            int* vout, int n, const int* nptr, int shift, const int* offs,
                                                            int nblocks) {
@@ -140,8 +186,8 @@ __global__ __launch_bounds__(kSortThreads) void rs_scatter(const uint64_t* kin, 
     const int t = threadIdx.x;
     base[t] = offs[t * nblocks + blockIdx.x];
     const int wid = t / kWave;
-    const int blk = blockIdx.x * kSortTile;
-    for (int k = 0; k < kSortItems; k++) {
+    const int blk = blockIdx.x * kSortThreads * ITEMS;
+    for (int k = 0; k < ITEMS; k++) {
         for (int w = 0; w < kSortThreads / kWave; w++) wcnt[w][t] = 0;
         __syncthreads();
         const int i = blk + k * kSortThreads + t;
@@ -179,396 +225,234 @@ __global__ __launch_bounds__(kSortThreads) void rs_scatter(const uint64_t* kin, 
     }
 }
 
+#define RS_INSTANCE(I)                                                                                            \
+    template __global__ void rs_hist<I>(const uint64_t*, int, const int*, int, int*, int);                        \
+    template __global__ void rs_scatter<I>(const uint64_t*, const int*, uint64_t*, int*, int, const int*, int,     \
+                                           const int*, int);
+RS_INSTANCE(4)
+RS_INSTANCE(16)
+#undef RS_INSTANCE
+
 // ---------------------------------------------------------------------------------------------
-// Karras (2012) radix tree: internal nodes [0, n-1), leaf of sorted position s is node n-1+s.
+// Overlaps.  Each overlapping pair is emitted by exactly one of its colliders (the pair key's high word):
+//   moving vs moving -> the lower collider index; moving vs static -> the moving one;
+//   static vs static -> the lower index, from the constant list built at creation.
+// Each emitter's partners end sorted ascending in its segment, so the pair table is sorted by key.
 // ---------------------------------------------------------------------------------------------
 
-__device__ __forceinline__ int delta(const uint64_t* k, int n, int i, int j) {
-    if (j < 0 || j >= n) return -1;
-    const uint64_t a = k[i], b = k[j];
-    if (a == b) return 64 + __clz((uint32_t)(i ^ j));
-    return __clzll(a ^ b);
-}
+constexpr int kTile = kWave;   // colliders per tile
 
-__global__ void bp_karras(const uint64_t* k, int n, int2* child, int* parent, int2* range) {
-    RP3DG_GRID_STRIDE(i, n - 1) {
-        const int d = (delta(k, n, i, i + 1) - delta(k, n, i, i - 1)) >= 0 ? 1 : -1;
-        const int dmin = delta(k, n, i, i - d);
-        int lmax = 2;
-        while (delta(k, n, i, i + lmax * d) > dmin) lmax <<= 1;
-        int l = 0;
-        for (int t = lmax >> 1; t >= 1; t >>= 1)
-            if (delta(k, n, i, i + (l + t) * d) > dmin) l += t;
-        const int j = i + l * d;
-        const int dnode = delta(k, n, i, j);
-        int s = 0;
-        int t = l;
-        do {
-            t = (t + 1) >> 1;
-            if (delta(k, n, i, i + (s + t) * d) > dnode) s += t;
-        } while (t > 1);
-        const int g = i + s * d + (d < 0 ? d : 0);
-        const int lo = min(i, j), hi = max(i, j);
-        const int left = (lo == g) ? (n - 1 + g) : g;
-        const int right = (hi == g + 1) ? (n - 1 + g + 1) : (g + 1);
-        child[i] = make_int2(left, right);
-        parent[left] = i;
-        parent[right] = i;
-        range[i] = make_int2(lo, hi);
-    }
-}
-
-// Synchronisation-free fit.  An internal node's box is the union of the fat AABBs of its leaf range
-// [lo, hi] (range[i] from bp_karras).  Min / max are exact, so any union order gives the same bits
-// as a bottom-up fit.  Unions over aligned blocks of 64, 4096 and 262144 sorted leaves are
-// precomputed, so a range costs at most ~64 reads per level.
-constexpr int kFitBlock = 64;
-
-__device__ __forceinline__ void box_union(float4& mn, float4& mx, float4 bmn, float4 bmx) {
-    mn = make_float4(fminf(mn.x, bmn.x), fminf(mn.y, bmn.y), fminf(mn.z, bmn.z), 0.f);
-    mx = make_float4(fmaxf(mx.x, bmx.x), fmaxf(mx.y, bmx.y), fmaxf(mx.z, bmx.z), 0.f);
-}
-
-__device__ __forceinline__ void wave_box_union(float4& mn, float4& mx) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        float4 omn, omx;
-        omn.x = __shfl_xor(mn.x, off, kWave); omn.y = __shfl_xor(mn.y, off, kWave); omn.z = __shfl_xor(mn.z, off, kWave);
-        omx.x = __shfl_xor(mx.x, off, kWave); omx.y = __shfl_xor(mx.y, off, kWave); omx.z = __shfl_xor(mx.z, off, kWave);
-        box_union(mn, mx, omn, omx);
-    }
-}
-
-// Leaves (node n-1+s = sorted collider s) and the unions of aligned blocks of 64 leaves.
-__global__ void bp_leaves(DevColliders C, const int* sorted, int n, float4* nmin, float4* nmax, float4* bmin,
-                          float4* bmax) {
-    const int nb = (n + kWave - 1) / kWave;
-    for (int base = (blockIdx.x * blockDim.x + threadIdx.x) & ~(kWave - 1); base < nb * kWave;
+// Boxes in the order of `sorted` (null: index order), the union of every tile and its range of worlds.
+// smn.w = collider, smx.w = world * 2 + static (int bits); tmn.w / tmx.w = first / last world of the tile.
+__global__ __launch_bounds__(256) void bp_tiles(DevColliders C, const int* sorted, int n, float4* smn, float4* smx,
+                                                float4* tmn, float4* tmx) {
+    const int nt = (n + kTile - 1) / kTile;
+    for (int base = (blockIdx.x * blockDim.x + threadIdx.x) & ~(kTile - 1); base < nt * kTile;
          base += gridDim.x * blockDim.x) {
         const int s = base + lane_id();
         float4 mn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), mx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+        int w = 0;
         if (s < n) {
-            const int c = sorted[s];
+            const int c = sorted ? sorted[s] : s;
             mn = C.amin[c];
             mx = C.amax[c];
-            nmin[n - 1 + s] = mn;
-            nmax[n - 1 + s] = mx;
+            w = C.world[c];
+            smn[s] = make_float4(mn.x, mn.y, mn.z, __int_as_float(c));
+            smx[s] = make_float4(mx.x, mx.y, mx.z, __int_as_float(2 * w + (C.is_static[c] ? 1 : 0)));
         }
         wave_box_union(mn, mx);
+        const int last = min(n - base, kTile) - 1;   // worlds ascend in either order
+        const int w0 = __shfl(w, 0, kWave), w1 = __shfl(w, last, kWave);
         if (lane_id() == 0) {
-            bmin[base / kWave] = mn;
-            bmax[base / kWave] = mx;
+            tmn[base / kTile] = make_float4(mn.x, mn.y, mn.z, __int_as_float(w0));
+            tmx[base / kTile] = make_float4(mx.x, mx.y, mx.z, __int_as_float(w1));
         }
     }
 }
 
-// Unions of aligned groups of 64 entries of the level below.
-__global__ void bp_blocks(const float4* imin, const float4* imax, int nin, float4* omin, float4* omax) {
-    const int nout = (nin + kWave - 1) / kWave;
-    for (int base = (blockIdx.x * blockDim.x + threadIdx.x) & ~(kWave - 1); base < nout * kWave;
-         base += gridDim.x * blockDim.x) {
-        const int s = base + lane_id();
-        float4 mn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), mx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
-        if (s < nin) { mn = imin[s]; mx = imax[s]; }
-        wave_box_union(mn, mx);
-        if (lane_id() == 0) {
-            omin[base / kWave] = mn;
-            omax[base / kWave] = mx;
-        }
-    }
+__device__ __forceinline__ float4 wave_read4(float4 v, int lane) {
+    return make_float4(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.x), lane)),
+                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.y), lane)),
+                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.z), lane)),
+                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.w), lane)));
 }
 
-// Internal nodes: union over the leaf range with the largest aligned blocks that fit.
-__global__ void bp_internal(int n, const int2* range, float4* nmin, float4* nmax, const float4* b1min,
-                            const float4* b1max, const float4* b2min, const float4* b2max, const float4* b3min,
-                            const float4* b3max) {
-    RP3DG_GRID_STRIDE(i, n - 1) {
-        const int2 r = range[i];
-        int s = r.x;
-        const int e = r.y + 1;   // exclusive
-        float4 mn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), mx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
-        while (s < e) {
-            if ((s & (262144 - 1)) == 0 && s + 262144 <= e) {
-                box_union(mn, mx, b3min[s >> 18], b3max[s >> 18]);
-                s += 262144;
-            } else if ((s & (4096 - 1)) == 0 && s + 4096 <= e) {
-                box_union(mn, mx, b2min[s >> 12], b2max[s >> 12]);
-                s += 4096;
-            } else if ((s & (kFitBlock - 1)) == 0 && s + kFitBlock <= e) {
-                box_union(mn, mx, b1min[s >> 6], b1max[s >> 6]);
-                s += kFitBlock;
-            } else {
-                box_union(mn, mx, nmin[n - 1 + s], nmax[n - 1 + s]);
-                s += 1;
+// Does collider c emit the pair (c, o)?  (Their boxes overlap; both are of one world.)
+__device__ __forceinline__ bool emits(const DevColliders& C, int c, int o, const NoColLists& L) {
+    return o != c && (C.is_static[o] || o > c) && pair_allowed(C, c, o, L);
+}
+
+// One workgroup per tile of 64 querying colliders, one per lane, the same in every wavefront.  The
+// wavefronts share the tiles whose box meets the queries': a wavefront loads a tile's boxes (one per lane),
+// drops those outside the queries' union, and every lane tests its box against the others one by one from
+// scalar registers.  A tree walk is a chain of dependent loads per collider with most lanes of a wavefront
+// waiting for the deepest; here every load is a full tile, and the arithmetic grows with the overlapping
+// tiles only.  Overlaps are collected in LDS, filtered (pair_allowed), sorted by rank and written to the
+// collider's slab; count[c] = its partners.  A collider with more overlaps than the slab holds is counted
+// by the whole workgroup and listed for bp_emit_large.
+__global__ __launch_bounds__(1024) void bp_pairs(DevColliders C, int n, const float4* smn, const float4* smx,
+                                                 const float4* tmn, const float4* tmx, const int* wcoll, NoColLists L,
+                                                 int* count, int* slab, int* large, int* nb_large) {
+    __shared__ int s_cnt[kTile], s_id[kTile];
+    __shared__ int s_list[kTile][kSlab];
+    __shared__ int s_total;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, nw = blockDim.x / kWave;
+    const int nt = (n + kTile - 1) / kTile;
+    const int s0 = blockIdx.x * kTile + lane;
+    float4 qmn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), qmx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    int c = -1, world = 0;
+    bool query = false;
+    if (s0 < n) {
+        qmn = smn[s0];
+        qmx = smx[s0];
+        c = __float_as_int(qmn.w);
+        const int t = __float_as_int(qmx.w);
+        world = t >> 1;
+        query = !(t & 1);
+        if (!query && wave == 0) count[c] = C.ss_offs[c + 1] - C.ss_offs[c];
+    }
+    if (!query) {   // overlaps nothing
+        qmn = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+        qmx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    }
+    if (wave == 0) {
+        s_cnt[lane] = 0;
+        s_id[lane] = query ? c : -1;
+    }
+    if (!__ballot(query)) return;   // (the same in every wavefront)
+    float4 umn = qmn, umx = qmx;
+    wave_box_union(umn, umx);
+    int wlo = query ? world : 0x7fffffff, whi = query ? world : -1;
+    whi = wave_max(whi);
+    wlo = -wave_max(-wlo);
+    __syncthreads();
+    int seen = 0;   // tiles that meet the queries so far
+    for (int T0 = 0; T0 < nt; T0 += kWave) {
+        const int T = T0 + lane;
+        bool meets = false;
+        if (T < nt) {
+            const float4 a = tmn[T], b = tmx[T];
+            meets = __float_as_int(a.w) <= whi && __float_as_int(b.w) >= wlo && aabb_overlap(umn, umx, a, b);
+        }
+        unsigned long long m = __ballot(meets);
+        while (m) {
+            const int k = __ffsll(m) - 1;
+            m &= m - 1;
+            if ((seen++ & (nw - 1)) != wave) continue;   // (a power of two)
+            const int s = (T0 + k) * kTile + lane;
+            float4 bmn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), bmx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+            if (s < n) {
+                bmn = smn[s];
+                bmx = smx[s];
             }
-        }
-        nmin[i] = mn;
-        nmax[i] = mx;
-    }
-}
-
-// Root node of every world: the node whose leaf range is exactly the world's key range.
-__global__ void bp_world_roots(const uint64_t* k, int n, const int2* range, int* root) {
-    RP3DG_GRID_STRIDE(i, 2 * n - 1) {
-        int lo, hi;
-        if (i < n - 1) { const int2 r = range[i]; lo = r.x; hi = r.y; }
-        else { lo = hi = i - (n - 1); }
-        const uint32_t w = (uint32_t)(k[lo] >> 30);
-        if ((uint32_t)(k[hi] >> 30) != w) continue;
-        if (lo > 0 && (uint32_t)(k[lo - 1] >> 30) == w) continue;
-        if (hi < n - 1 && (uint32_t)(k[hi + 1] >> 30) == w) continue;
-        root[w] = i;
-    }
-}
-
-__device__ __forceinline__ bool aabb_overlap(float4 amn, float4 amx, float4 bmn, float4 bmx) {
-    // AABB::testCollision (AABB.h:179-187), closed intervals
-    if (amx.x < bmn.x || bmx.x < amn.x) return false;
-    if (amx.y < bmn.y || bmx.y < amn.y) return false;
-    if (amx.z < bmn.z || bmx.z < amn.z) return false;
-    return true;
-}
-
-// Body pairs that must not collide (joints with collideConnected = false): per-body partner lists
-__device__ __forceinline__ bool no_collision(const NoColLists& L, int ba, int bb) {
-    const int e = L.offs[ba + 1];
-    for (int k = L.offs[ba]; k < e; k++)
-        if (L.list[k] == bb) return true;
-    return false;
-}
-
-__device__ __forceinline__ bool filters_pass(uint32_t fa, uint32_t fb) {
-    const uint32_t cata = fa & 0xffffu, maska = fa >> 16, catb = fb & 0xffffu, maskb = fb >> 16;
-    return (maska & catb) != 0 && (cata & maskb) != 0;
-}
-
-// Pair filter of CollisionDetectionSystem::updateOverlappingPairs (CD.cpp:284-331): different bodies, no
-// joint excluding the pair, collision category / mask, at least one convex shape (:324-331)
-__device__ __forceinline__ bool pair_allowed(const DevColliders& C, int a, int b, const NoColLists& L) {
-    const int ba = C.body[a], bb = C.body[b];
-    if (ba == bb) return false;
-    if (no_collision(L, ba, bb)) return false;
-    if (shape_is_concave(C.type[a]) && shape_is_concave(C.type[b])) return false;
-    return filters_pass(C.filter[a], C.filter[b]);
-}
-
-constexpr int kTravStack = 64;   // traversal stack depth (per thread)
-
-// Each overlapping pair is emitted by exactly one of its colliders (the pair key's high word):
-//   moving vs moving -> the lower collider index; moving vs static -> the moving one;
-//   static vs static -> the lower index, from the constant list built at creation (statics never
-//   traverse: a floor's AABB overlaps most of the tree and would serialise one thread over it).
-// Pass 0 counts, pass 1 writes each emitter's partner list sorted ascending into its segment, so the
-// pair table is sorted by key.
-// Pass 0 traverses once (colliders in Morton order, so neighbouring lanes walk similar paths),
-// counts every collider's partners and keeps the first kTravSlab of them, sorted, in a
-// per-collider slab.  Pass 1 (after the scan of the counts) runs over colliders in index order,
-// copies the slabs into the emitters' segments of the pair-key table (coalesced), and traverses
-// again only for colliders with more partners than the slab holds.
-__global__ __launch_bounds__(kTravBlock) void bp_traverse(DevColliders C, const int* sorted, int n, const int2* child,
-                                                          const float4* nmin, const float4* nmax, const int* root,
-                                                          NoColLists nc, int* count, const int* offset,
-                                                          uint64_t* out_keys, uint64_t* slab, int capacity, int pass,
-                                                          int* walk_list, int* walk_count, int* status) {
-    const int nw = pass ? *walk_count : n;
-    RP3DG_GRID_STRIDE(s, nw) {
-        const int c = pass ? walk_list[s] : sorted[s];
-        const int base = pass ? offset[c] : 0;
-        if (!pass && C.is_static[c]) {
-            count[c] = C.ss_offs[c + 1] - C.ss_offs[c];
-            continue;
-        }
-        uint64_t* sl = slab + (size_t)c * kTravSlab;
-        const float4 amn = C.amin[c], amx = C.amax[c];
-        int stack[kTravStack];
-        int sp = 0;
-        stack[sp++] = root[C.world[c]];
-        int cnt = 0;
-        while (sp > 0) {
-            const int node = stack[--sp];
-            if (!aabb_overlap(amn, amx, nmin[node], nmax[node])) continue;
-            if (node >= n - 1) {
-                const int o = sorted[node - (n - 1)];
-                if (o == c) continue;
-                if (!C.is_static[o] && o < c) continue;
-                if (!pair_allowed(C, c, o, nc)) continue;
-                const uint64_t key = ((uint64_t)(uint32_t)c << 32) | (uint32_t)o;
-                if (pass) {
-                    int pos = base + cnt;
-                    if (pos < capacity) {
-                        // insertion into the sorted segment
-                        while (pos > base && out_keys[pos - 1] > key) {
-                            out_keys[pos] = out_keys[pos - 1];
-                            pos--;
-                        }
-                        out_keys[pos] = key;
-                    } else {
-                        atomicOr(status, STATUS_PAIR_OVERFLOW);
-                    }
-                } else if (cnt < kTravSlab) {
-                    int pos = cnt;
-                    while (pos > 0 && sl[pos - 1] > key) {
-                        sl[pos] = sl[pos - 1];
-                        pos--;
-                    }
-                    sl[pos] = key;
+            unsigned long long cand = __ballot(s < n && aabb_overlap(umn, umx, bmn, bmx));
+            while (cand) {
+                const int q = __ffsll(cand) - 1;
+                cand &= cand - 1;
+                const float4 amn = wave_read4(bmn, q), amx = wave_read4(bmx, q);
+                const int o = __float_as_int(amn.w), t = __float_as_int(amx.w);
+                if (aabb_overlap(qmn, qmx, amn, amx) && (t >> 1) == world && o != c && ((t & 1) || o > c)) {
+                    const int pos = atomicAdd(&s_cnt[lane], 1);
+                    if (pos < kSlab) s_list[lane][pos] = o;
                 }
-                cnt++;
-            } else {
-                if (sp + 2 > kTravStack) { atomicOr(status, STATUS_STACK_OVERFLOW); break; }
-                const int2 ch = child[node];
-                stack[sp++] = ch.x;
-                stack[sp++] = ch.y;
             }
         }
-        if (!pass) {
-            count[c] = cnt;
-            if (cnt > kTravSlab) walk_list[atomicAdd(walk_count, 1)] = c;   // walked again after the scan
-        }
     }
-}
-
-// Second traversal pass, one wavefront per collider whose partners overflowed its slab (a ground or
-// wall overlapping hundreds of bodies).  The overlapping top of the tree is expanded breadth-first
-// into at most 64 subtrees, each lane walks one with the filters of bp_traverse, the keys go to the
-// collider's segment, and the segment is sorted: in LDS by a bitonic network when it fits, else by
-// lane 0.  Keys are unique (each leaf is reached once), so the segment equals the one pass 1 of
-// bp_traverse produces.
-constexpr int kWalkSort = 4096;   // keys sorted in LDS (32 KB)
-__global__ __launch_bounds__(kWave) void bp_walk_wave(DevColliders C, const int* sorted, int n, const int2* child,
-                                                      const float4* nmin, const float4* nmax, const int* root,
-                                                      NoColLists ncl, const int* offset, uint64_t* out_keys,
-                                                      int capacity, const int* walk_list, const int* walk_count,
-                                                      int* status) {
-    __shared__ uint64_t s_keys[kWalkSort];
-    __shared__ int s_front[2 * kWave];
-    __shared__ int s_nf, s_cnt;
-    const int lane = threadIdx.x;
-    const int nw = *walk_count;
-    for (int s = blockIdx.x; s < nw; s += gridDim.x) {
-        const int c = walk_list[s];
-        const int base = offset[c];
-        const float4 amn = C.amin[c], amx = C.amax[c];
-        if (lane == 0) { s_front[0] = root[C.world[c]]; s_nf = 1; s_cnt = 0; }
+    __syncthreads();
+    // filters, one entry a thread
+    constexpr int kDrop = 0x7fffffff;
+    for (int e = tid; e < kTile * kSlab; e += blockDim.x) {
+        const int q = e / kSlab, k = e % kSlab;
+        if (k >= s_cnt[q] || s_cnt[q] > kSlab) s_list[q][k] = kDrop;
+        else if (!pair_allowed(C, s_id[q], s_list[q][k], L)) s_list[q][k] = kDrop;
+    }
+    __syncthreads();
+    for (int q = wave; q < kTile; q += nw) {   // rank sort; ids are unique
+        const int cq = s_id[q], len = s_cnt[q];
+        if (cq < 0 || len > kSlab) continue;
+        const int id = lane < kSlab ? s_list[q][lane] : kDrop;
+        int rank = 0;
+        const int ulen = __builtin_amdgcn_readfirstlane(len);
+        for (int k = 0; k < ulen; k++) rank += __builtin_amdgcn_readlane(id, k) < id ? 1 : 0;
+        if (id != kDrop) slab[(size_t)cq * kSlab + rank] = id;
+        const int total = __popcll(__ballot(id != kDrop));
+        if (lane == 0) count[cq] = total;
+    }
+    // colliders with more overlaps than their slab holds: exact count by the whole workgroup
+    for (int q = 0; q < kTile; q++) {
+        const int cq = s_id[q];
+        if (cq < 0 || s_cnt[q] <= kSlab) continue;
         __syncthreads();
-        // breadth-first expansion while the frontier holds at most kWave / 2 nodes and some are internal
-        for (int level = 0; level < 64; level++) {
-            const int nf = s_nf;
-            const int node = lane < nf ? s_front[lane] : -1;
-            const bool internal = node >= 0 && node < n - 1;
-            if (nf > kWave / 2 || !__ballot(internal)) break;
-            const bool ov = node >= 0 && aabb_overlap(amn, amx, nmin[node], nmax[node]);
-            const int emit = !ov ? 0 : (internal ? 2 : 1);
-            const int incl = wave_incl_scan(emit);
-            const int off = incl - emit;
-            const int tot = __shfl(incl, kWave - 1, kWave);
-            __syncthreads();   // every lane has read the frontier
-            if (emit == 1) s_front[off] = node;
-            if (emit == 2) {
-                const int2 ch = child[node];
-                s_front[off] = ch.x;
-                s_front[off + 1] = ch.y;
-            }
-            if (lane == 0) s_nf = tot;
-            __syncthreads();
-        }
-        const int nf = s_nf;
-        for (int f = lane; f < nf; f += kWave) {
-            int stack[kTravStack];
-            int sp = 0;
-            stack[sp++] = s_front[f];
-            while (sp > 0) {
-                const int node = stack[--sp];
-                if (!aabb_overlap(amn, amx, nmin[node], nmax[node])) continue;
-                if (node >= n - 1) {
-                    const int o = sorted[node - (n - 1)];
-                    if (o == c) continue;
-                    if (!C.is_static[o] && o < c) continue;
-                    if (!pair_allowed(C, c, o, ncl)) continue;
-                    const uint64_t key = ((uint64_t)(uint32_t)c << 32) | (uint32_t)o;
-                    const int pos = atomicAdd(&s_cnt, 1);
-                    if (pos < kWalkSort) s_keys[pos] = key;
-                    if (base + pos < capacity) out_keys[base + pos] = key;
-                    else atomicOr(status, STATUS_PAIR_OVERFLOW);
-                } else {
-                    if (sp + 2 > kTravStack) { atomicOr(status, STATUS_STACK_OVERFLOW); break; }
-                    const int2 ch = child[node];
-                    stack[sp++] = ch.x;
-                    stack[sp++] = ch.y;
-                }
-            }
-        }
+        if (tid == 0) s_total = 0;
         __syncthreads();
-        const int nk = s_cnt;
-        const int nsort = min(nk, capacity - base);   // keys present in the segment
-        if (nk <= kWalkSort) {
-            int P = 1;
-            while (P < nk) P <<= 1;
-            for (int i = nk + lane; i < P; i += kWave) s_keys[i] = ~0ull;
-            __syncthreads();
-            for (int k = 2; k <= P; k <<= 1)
-                for (int j = k >> 1; j > 0; j >>= 1) {
-                    for (int i = lane; i < P; i += kWave) {
-                        const int ixj = i ^ j;
-                        if (ixj > i) {
-                            const uint64_t a = s_keys[i], b = s_keys[ixj];
-                            if ((a > b) == ((i & k) == 0)) { s_keys[i] = b; s_keys[ixj] = a; }
-                        }
-                    }
-                    __syncthreads();
-                }
-            for (int i = lane; i < nsort; i += kWave) out_keys[base + i] = s_keys[i];
-        } else if (lane == 0) {
-            for (int i = 1; i < nsort; i++) {
-                const uint64_t key = out_keys[base + i];
-                int pos = base + i;
-                while (pos > base && out_keys[pos - 1] > key) {
-                    out_keys[pos] = out_keys[pos - 1];
-                    pos--;
-                }
-                out_keys[pos] = key;
-            }
+        const float4 amn = C.amin[cq], amx = C.amax[cq];
+        const int w = C.world[cq];
+        int mine = 0;
+        for (int o = wcoll[w] + tid; o < wcoll[w + 1]; o += blockDim.x)
+            if (aabb_overlap(amn, amx, C.amin[o], C.amax[o]) && emits(C, cq, o, L)) mine++;
+        mine = wave_sum(mine);
+        if (lane == 0 && mine) atomicAdd(&s_total, mine);
+        __syncthreads();
+        if (tid == 0) {
+            count[cq] = s_total;
+            slab[(size_t)cq * kSlab] = -1;
+            large[atomicAdd(nb_large, 1)] = cq;
         }
-        __syncthreads();   // the frontier and keys of this collider are done before the next one
     }
 }
 
-// Second traversal pass for the colliders with at most kTravSlab partners: their sorted partners are
-// in the slab; eight lanes per collider copy them to the collider's segment of the key array.  Static
-// colliders copy their static-static partner list.
-__global__ void bp_copy_slabs(DevColliders C, int n, const int* count, const int* offset, const uint64_t* slab,
-                              uint64_t* out_keys, int capacity, int* status) {
-    RP3DG_GRID_STRIDE(t, n * kTravSlab) {
-        const int c = t / kTravSlab, k = t % kTravSlab;
-        const int base = offset[c];
-        if (C.is_static[c]) {
-            if (k != 0) continue;
-            const int b = C.ss_offs[c], e = C.ss_offs[c + 1];
-            for (int q = b; q < e; q++)
-                if (base + q - b < capacity) out_keys[base + q - b] = ((uint64_t)(uint32_t)c << 32) | (uint32_t)C.ss_list[q];
-            if (base + e - b > capacity) atomicOr(status, STATUS_PAIR_OVERFLOW);
-            continue;
-        }
-        const int total = count[c];
-        if (total > kTravSlab || k >= total) continue;
+// Partners from the slabs (eight lanes per collider) and the static colliders' lists to the segments of the
+// key array.
+__global__ void bp_emit(DevColliders C, int n, const int* count, const int* offset, const int* slab, uint64_t* out_keys,
+                        int capacity, int* status) {
+    constexpr int kLanes = 8;
+    RP3DG_GRID_STRIDE(t, n * kLanes) {
+        const int c = t / kLanes;
+        const int base = offset[c], total = count[c];
+        const bool fixed = C.is_static[c];
+        const int* src = fixed ? C.ss_list + C.ss_offs[c] : slab + (size_t)c * kSlab;
+        if (!fixed && total > 0 && src[0] < 0) continue;   // bp_emit_large's
         // past the capacity the table is truncated (and the step reports the overflow), but every entry
         // below it is written, since the merge reads all of them
-        if (base + k >= capacity) {
-            atomicOr(status, STATUS_PAIR_OVERFLOW);
-            continue;
+        for (int k = t % kLanes; k < total; k += kLanes) {
+            if (base + k < capacity) out_keys[base + k] = ((uint64_t)(uint32_t)c << 32) | (uint32_t)src[k];
+            else atomicOr(status, STATUS_PAIR_OVERFLOW);
         }
-        out_keys[base + k] = slab[(size_t)c * kTravSlab + k];
+    }
+}
+
+// Colliders with more overlaps than a slab: one workgroup each walks the colliders of its world in index
+// order, so that the partners come out sorted.
+__global__ __launch_bounds__(1024) void bp_emit_large(DevColliders C, const int* wcoll, NoColLists L, const int* offset,
+                                                      uint64_t* out_keys, int capacity, const int* large,
+                                                      const int* nb_large, int* status) {
+    __shared__ int sm[17];
+    const int nl = *nb_large;
+    for (int i = blockIdx.x; i < nl; i += gridDim.x) {
+        const int c = large[i], w = C.world[c];
+        const float4 amn = C.amin[c], amx = C.amax[c];
+        int base = offset[c];
+        for (int o0 = wcoll[w]; o0 < wcoll[w + 1]; o0 += blockDim.x) {
+            const int o = o0 + threadIdx.x;
+            const bool hit = o < wcoll[w + 1] && aabb_overlap(amn, amx, C.amin[o], C.amax[o]) && emits(C, c, o, L);
+            int total;
+            const int pos = base + block_excl_scan(hit ? 1 : 0, sm, &total);
+            if (hit) {
+                if (pos < capacity) out_keys[pos] = ((uint64_t)(uint32_t)c << 32) | (uint32_t)o;
+                else atomicOr(status, STATUS_PAIR_OVERFLOW);
+            }
+            base += total;
+        }
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// Batches of small worlds: no tree.  One workgroup per world group stages the fat AABBs of its
+// Batches of small worlds.  One workgroup per world group stages the fat AABBs of its
 // colliders in LDS and every dynamic collider tests the boxes of all colliders of its own world in
 // index order, so its partners come out sorted; the scan runs twice (count, then write after the
-// prefix sum of the counts).  The pair set is the tree query's (the same
+// prefix sum of the counts).  The pair set is bp_pairs' (the same
 // AABB::testCollision on the same boxes, the same emitter rule and filters); the cost is
-// sum over worlds of (colliders)^2 box tests, cheaper than building and walking a tree per world up to
-// about a thousand colliders.  LDS per collider: min (w = body | static << 31), max (w = filter bits).
+// sum over worlds of (colliders)^2 box tests in one launch for thousands of worlds.  LDS per collider: min (w = body | static << 31), max (w = filter bits).
 // ---------------------------------------------------------------------------------------------
 // pass 0 writes the partner count of every collider, pass 1 (after the scan) its sorted keys.
 __global__ __launch_bounds__(256) void bp_world_scan(DevColliders C, const int* gworld, const int* wcoll,

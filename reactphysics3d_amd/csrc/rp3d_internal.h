@@ -60,8 +60,7 @@ __host__ __device__ inline uint32_t lf_face(uint32_t w) { return (w >> 8) & 0xff
 __host__ __device__ inline uint32_t lf_edge1(uint32_t w) { return (w >> 16) & 0xffu; }
 __host__ __device__ inline uint32_t lf_edge2(uint32_t w) { return (w >> 24) & 0xffu; }
 
-constexpr int kTravBlock = 128;       // threads per block of the broadphase traversal
-constexpr int kTravSlab = 8;          // partners kept per collider by the first traversal pass
+constexpr int kSlab = 64;             // partners kept per collider by the broadphase's overlap pass
 constexpr int kMaxRawContacts = 16;   // NB_MAX_CONTACT_POINTS_IN_NARROWPHASE_INFO (configuration.h:134)
 constexpr int kMaxManifoldPoints = 4; // MAX_CONTACT_POINTS_IN_MANIFOLD
 // Hull faces have at most this many vertices: clipping an incident face by the side planes of a
@@ -227,7 +226,7 @@ struct DevCounters {
     int nb_box_tests;          // box-box subset of nb_tests[ALGO_POLY_POLY] that collided last step
     int nb_box_sep_tests;      // box-box pairs that did not (cheap temporal-coherence rejects, listed apart)
     int nb_hull_tests;         // the rest of nb_tests[ALGO_POLY_POLY] (a convex mesh involved)
-    int nb_walk_again;         // colliders with more partners than the traversal slab holds
+    int nb_large;              // colliders with more overlaps than their broadphase slab holds
     int nb_events;             // contact events of the step (may exceed the event buffer)
     int nb_concave_tests;      // triangle tests of the convex vs concave pairs
     int nb_concave_points;     // contact points of those tests

@@ -1,0 +1,44 @@
+"""The tile broadphase (index order up to 8,192 colliders, Morton cells beyond) lists the same oriented pairs as
+the per-world box scan, step after step: sizes around a tile, several worlds per tile, more colliders
+than the index order takes, and moving bodies that overlap more colliders than a slab holds."""
+import numpy as np
+import pytest
+
+from reactphysics3d_amd import scene as S
+
+pytestmark = pytest.mark.gpu
+
+
+def _heap(n, seed):
+    side = max(6.0, float(np.sqrt(n * 0.6)))
+    return S.mixed_container(n, extent=(side, side, 12.0), seed=seed)
+
+
+def _plate(n, seed):
+    """A wide moving plate among n spheres: it overlaps most of them at once."""
+    sc = _heap(n, seed)
+    b = sc.add_body(S.DYNAMIC, (0.0, 0.0, 6.0))
+    sc.add_collider(b, S.BOX, (6.0, 6.0, 5.0))
+    return sc
+
+
+@pytest.mark.parametrize("name,worlds", [
+    ("one", lambda: [_heap(1, 3)]),
+    ("tile edge", lambda: [_heap(59, 3), _heap(58, 4), _heap(1, 5)]),
+    ("tiles", lambda: [_heap(700, 6)]),
+    ("plate over a slab", lambda: [_plate(150, 7), _plate(64, 8)]),
+    ("plates, many", lambda: [_plate(400, 9 + k) for k in range(4)]),
+    ("Morton order", lambda: [_heap(380, 20 + k) for k in range(22)] + [_plate(300, 50)]),
+], ids=lambda x: x if isinstance(x, str) else "")
+def test_tiles_list_the_scans_pairs(name, worlds):
+    from reactphysics3d_amd.lib import Batch
+    scenes = worlds()
+    a = Batch(scenes, solver="fused", broadphase="tree", pairs_per_collider=64)
+    b = Batch(scenes, solver="fused", broadphase="world_scan", pairs_per_collider=64)
+    for k in range(12):
+        a.step(1.0 / 60.0)
+        b.step(1.0 / 60.0)
+        for x, y in zip(a.pairs(), b.pairs()):
+            assert np.array_equal(x, y), f"step {k}: pairs differ"
+    for x, y in zip(a.bodies(), b.bodies()):
+        assert np.array_equal(x, y)
