@@ -6,9 +6,13 @@
 // fraction, a set that does not depend on the visiting order).  Only world-query colliders whose
 // category passes the mask are tested (BroadPhaseRaycastCallback, BroadPhaseSystem.cpp:224-241).
 //
-// A thread walks the colliders of its ray's world in index order instead of the tree: every collider
-// whose fat AABB the (clipped) ray crosses (AABB::testRayIntersect, AABB.h:285-313) and whose category
-// passes the mask is tested against its shape in the collider's space, and each reported hit clips the
+// A thread walks the colliders of its ray's world in index order instead of the tree, 64 at a time: the box
+// tests of a block give a mask, and the shapes of its set bits are tested afterwards, so that the lanes of
+// a wavefront run their shape tests side by side (tested as they come, nearly every collider costs the
+// whole wavefront a shape test for one or two rays).  The boxes of a block come from LDS when the rays of
+// the workgroup belong to one world.
+// Every collider whose fat AABB the (clipped) ray crosses (AABB::testRayIntersect, AABB.h:285-313) and whose
+// category passes the mask is tested against its shape in the collider's space, and each reported hit clips the
 // ray.  The closest hit is the same in any visiting order; only hits at exactly equal fractions (the
 // box and convex-mesh tests accept a hit at the current fraction, the sphere and capsule tests do not)
 // may be reported in a different order than the tree visits them.  A hit at fraction 0 ends the ray,
@@ -21,6 +25,8 @@
 namespace rp3dg {
 
 namespace {
+
+constexpr int kRayChunk = 512;   // colliders whose boxes are staged in LDS at a time
 
 struct Hit {
     float t;
@@ -206,51 +212,130 @@ __device__ bool ray_collider(const RayArgs& A, int c, uint32_t mask, V3 p1, V3 p
 
 }  // namespace
 
+// Visits, in index order, every collider of the ray's world whose box the ray crosses within maxf (read anew
+// before each visit, so the visitor may clip it); visit(collider) returns false to end the walk.  All threads
+// of the workgroup call it (a thread without a ray with c0 == c1).
+template <class Visit>
+__device__ __forceinline__ void walk_boxes(const RayArgs& A, int c0, int c1, uint32_t mask, V3 p1, V3 inv, const float& maxf,
+                                           Visit visit) {
+    __shared__ float4 s_mn[kRayChunk], s_mx[kRayChunk];
+    __shared__ int s_range[2];
+    if (threadIdx.x == 0) {
+        s_range[0] = 0x7fffffff;
+        s_range[1] = 0;
+    }
+    __syncthreads();
+    if (c0 < c1) {
+        atomicMin(&s_range[0], c0);
+        atomicMax(&s_range[1], c0);
+    }
+    __syncthreads();
+    const int first = s_range[0];
+    const bool one_world = first == s_range[1];   // a world's rays share c0
+    auto box = [&](int c, float4& mn, float4& mx) {   // min box, max box; mx.w = 1 when the ray may hit it
+        mn = A.C.amin[c];
+        mx = A.C.amax[c];
+        mx.w = ((A.C.filter[c] & mask & 0xffffu) != 0u && (A.C.kind[c] & CK_WORLD_QUERY)) ? 1.0f : 0.0f;
+    };
+    bool open = c0 < c1;
+    if (one_world) {
+        const int end = A.wcoll[A.C.world[first] + 1];
+        for (int base = first; base < end; base += kRayChunk) {
+            __syncthreads();
+            for (int k = threadIdx.x; k < kRayChunk && base + k < end; k += blockDim.x) box(base + k, s_mn[k], s_mx[k]);
+            __syncthreads();
+            for (int b = 0; b < kRayChunk && base + b < end; b += 64) {
+                const int n = min(64, end - base - b);
+                unsigned long long hits = 0ull;
+                if (open)
+                    for (int k = 0; k < n; k++) {
+                        const float4 mn = s_mn[b + k], mx = s_mx[b + k];
+                        if (mx.w != 0.0f && ray_aabb(xyz(mn), xyz(mx), p1, inv, maxf)) hits |= 1ull << k;
+                    }
+                while (hits) {
+                    const int k = __ffsll(hits) - 1;
+                    hits &= hits - 1;
+                    if (!visit(base + b + k)) {
+                        open = false;
+                        hits = 0ull;
+                    }
+                }
+            }
+        }
+    } else {
+        for (int base = c0; open && base < c1; base += 64) {
+            const int n = min(64, c1 - base);
+            unsigned long long hits = 0ull;
+            for (int k = 0; k < n; k++) {
+                float4 mn, mx;
+                box(base + k, mn, mx);
+                if (mx.w != 0.0f && ray_aabb(xyz(mn), xyz(mx), p1, inv, maxf)) hits |= 1ull << k;
+            }
+            while (hits && open) {
+                const int k = __ffsll(hits) - 1;
+                hits &= hits - 1;
+                open = visit(base + k);
+            }
+        }
+    }
+    __syncthreads();   // s_range is written again by the next call
+}
+
 // Every hit of every ray: hits are appended at an atomically reserved slot (those past cap are counted,
 // not written); *count ends as the number of hits.
-__global__ void rc_all(RayArgs A, const int* ray_world, const float4* p1s, const float4* p2s, int n, uint32_t mask,
-                       int2* hit_ray_collider, float4* hit_point, float4* hit_normal, int cap, int* count) {
-    RP3DG_GRID_STRIDE(i, n) {
-        const float4 a = p1s[i], b = p2s[i];
+__global__ __launch_bounds__(256) void rc_all(RayArgs A, const int* ray_world, const float4* p1s, const float4* p2s, int n,
+                                              uint32_t mask, int2* hit_ray_collider, float4* hit_point, float4* hit_normal,
+                                              int cap, int* count) {
+    const int rounds = (n + gridDim.x * blockDim.x - 1) / (gridDim.x * blockDim.x);
+    for (int r = 0; r < rounds; r++) {
+        const int i = (r * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+        const bool ray = i < n;
+        const float4 a = ray ? p1s[i] : make_float4(0.f, 0.f, 0.f, 0.f), b = ray ? p2s[i] : a;
         const V3 p1 = v3(a.x, a.y, a.z), p2 = v3(b.x, b.y, b.z);
         const float maxf = b.w;
         const V3 dir = p2 - p1;
         const V3 inv = v3(1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z);
-        const int w = ray_world[i];
-        for (int c = A.wcoll[w]; c < A.wcoll[w + 1]; c++) {
+        const int w = ray ? ray_world[i] : 0;
+        walk_boxes(A, ray ? A.wcoll[w] : 0, ray ? A.wcoll[w + 1] : 0, mask, p1, inv, maxf, [&](int c) {
             Hit h;
-            if (!ray_collider(A, c, mask, p1, p2, inv, maxf, h)) continue;
+            if (!ray_collider(A, c, mask, p1, p2, inv, maxf, h)) return true;
             const int slot = atomicAdd(count, 1);
             if (slot < cap) {
                 hit_ray_collider[slot] = make_int2(i, c);
                 hit_point[slot] = make_float4(h.p.x, h.p.y, h.p.z, h.t);
                 hit_normal[slot] = make_float4(h.n.x, h.n.y, h.n.z, 0.f);
             }
-        }
+            return true;
+        });
     }
 }
 
-__global__ void rc_closest(RayArgs A, const int* ray_world, const float4* p1s, const float4* p2s, int n, uint32_t mask,
-                           int* hit_collider, float4* hit_point, float4* hit_normal) {
-    RP3DG_GRID_STRIDE(i, n) {
-        const float4 a = p1s[i], b = p2s[i];
+__global__ __launch_bounds__(256) void rc_closest(RayArgs A, const int* ray_world, const float4* p1s, const float4* p2s,
+                                                  int n, uint32_t mask, int* hit_collider, float4* hit_point,
+                                                  float4* hit_normal) {
+    const int rounds = (n + gridDim.x * blockDim.x - 1) / (gridDim.x * blockDim.x);
+    for (int r = 0; r < rounds; r++) {
+        const int i = (r * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+        const bool ray = i < n;
+        const float4 a = ray ? p1s[i] : make_float4(0.f, 0.f, 0.f, 0.f), b = ray ? p2s[i] : a;
         const V3 p1 = v3(a.x, a.y, a.z), p2 = v3(b.x, b.y, b.z);
         float maxf = b.w;
         const V3 dir = p2 - p1;
         const V3 inv = v3(1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z);
-        const int w = ray_world[i];
-        const int c0 = A.wcoll[w], c1 = A.wcoll[w + 1];
+        const int w = ray ? ray_world[i] : 0;
         int best = -1;
         Hit hb{0.f, v3(0.f, 0.f, 0.f), v3(0.f, 0.f, 0.f)};
-        for (int c = c0; c < c1; c++) {
+        walk_boxes(A, ray ? A.wcoll[w] : 0, ray ? A.wcoll[w + 1] : 0, mask, p1, inv, maxf, [&](int c) {
             Hit h;
-            if (!ray_collider(A, c, mask, p1, p2, inv, maxf, h)) continue;
+            if (!ray_collider(A, c, mask, p1, p2, inv, maxf, h)) return true;
             hb = h;
             best = c;
             // DynamicAABBTree::raycast (DynamicAABBTree.cpp:705-721) with the closest-hit callback
-            if (h.t == 0.0f) break;
+            if (h.t == 0.0f) return false;
             if (h.t > 0.0f && h.t < maxf) maxf = h.t;
-        }
+            return true;
+        });
+        if (!ray) continue;
         hit_collider[i] = best;
         hit_point[i] = make_float4(hb.p.x, hb.p.y, hb.p.z, hb.t);
         hit_normal[i] = make_float4(hb.n.x, hb.n.y, hb.n.z, 0.f);
