@@ -140,17 +140,35 @@ __global__ __launch_bounds__(256) void mlp_infer(MlpDev M, const float* feats, c
 // ---------------------------------------------------------------------------------------------
 constexpr int kChunk = 64;
 constexpr int kGradTiles = 16 + 64 + 8;   // dW1 (2 x 8), dW2 (8 x 8), dW3 (8 x 1) tiles of 16 x 16
-constexpr int kTilesPerWave = kGradTiles / 4;
+constexpr int kGradThreads = 512;         // 4 wavefronts for the samples, 8 for the weight gradients
+constexpr int kTilesPerWave = kGradTiles / (kGradThreads / kWave);
 
+// Activations and errors of the chunk with the samples along the rows: an MFMA operand of the weight
+// gradients (four consecutive samples of one feature) is one 8-byte load, and the 16 samples that a
+// wavefront's lanes store are consecutive.  The row pitch of 68 spreads the four feature rows of a store over
+// the banks.
+constexpr int kPitch = kChunk + 4;
 struct GradLds {
-    uint16_t x[kChunk][kMlpInPad];
-    uint16_t h1[kChunk][kMlpHid];
-    uint16_t h2[kChunk][kMlpHid];
-    uint16_t dz1[kChunk][kMlpHid];
-    uint16_t dz2[kChunk][kMlpHid];
-    uint16_t dy[kChunk][kMlpOutPad];
+    uint16_t x[kMlpInPad][kPitch];
+    uint16_t h1[kMlpHid][kPitch];
+    uint16_t h2[kMlpHid][kPitch];
+    uint16_t dz1[kMlpHid][kPitch];
+    uint16_t dz2[kMlpHid][kPitch];
+    uint16_t dy[kMlpOutPad][kPitch];
     float red[4];
 };
+
+// sum of the chunk's samples of one feature, in sample order
+__device__ __forceinline__ float sum_samples(const uint16_t* row) {
+    float s = 0.0f;
+#pragma unroll
+    for (int q = 0; q < kChunk / 4; q++) {
+        const v4s v = ld4(row + 4 * q);
+#pragma unroll
+        for (int j = 0; j < 4; j++) s += bf2f((uint16_t)v[j]);
+    }
+    return s;
+}
 
 __device__ __forceinline__ void tile_of(int tidx, int& layer, int& ti, int& to) {
     if (tidx < 16) { layer = 0; ti = tidx >> 3; to = tidx & 7; }
@@ -158,17 +176,17 @@ __device__ __forceinline__ void tile_of(int tidx, int& layer, int& ti, int& to) 
     else { layer = 2; ti = tidx - 80; to = 0; }
 }
 
-__global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, const float* targets, const int* idx,
+__global__ __launch_bounds__(kGradThreads) void mlp_grad(MlpDev M, const float* feats, const float* targets, const int* idx,
                                                 int n, float* partial, float* loss_partial) {
-    __shared__ GradLds L;
+    __shared__ __align__(16) GradLds L;
     const int tid = threadIdx.x, w = tid / kWave, l = lane_id(), r = l & 15, g = l >> 4;
     const float inv_n = 1.0f / (float)n;
     const int srow = 16 * w + r;
     const int s = blockIdx.x * kChunk + srow;
-    const bool valid = s < n;
+    const bool valid = srow < kChunk && s < n;
     const int si = valid ? (idx ? idx[s] : s) : 0;
     float loss = 0.0f;
-    {
+    if (w < kChunk / 16) {
         v4s xb[2];
         float xn[8];
         load_x(M, feats, si, valid, xb, xn);
@@ -177,13 +195,13 @@ __global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, co
 #pragma unroll
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) L.x[srow][16 * kt + 4 * g + j] = (uint16_t)xb[kt][j];
+            for (int j = 0; j < 4; j++) L.x[16 * kt + 4 * g + j][srow] = (uint16_t)xb[kt][j];
 #pragma unroll
         for (int t = 0; t < 8; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                L.h1[srow][16 * t + 4 * g + i] = (uint16_t)F.h1[t][i];
-                L.h2[srow][16 * t + 4 * g + i] = (uint16_t)F.h2[t][i];
+                L.h1[16 * t + 4 * g + i][srow] = (uint16_t)F.h1[t][i];
+                L.h2[16 * t + 4 * g + i][srow] = (uint16_t)F.h2[t][i];
             }
         // output error (lanes with g == 0 hold outputs 0..3 of sample r)
         float dyv[4];
@@ -201,7 +219,7 @@ __global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, co
         }
         const v4s dyb = pack4(dyv[0], dyv[1], dyv[2], dyv[3]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) L.dy[srow][4 * g + i] = (uint16_t)dyb[i];
+        for (int i = 0; i < 4; i++) L.dy[4 * g + i][srow] = (uint16_t)dyb[i];
         // dz2 = (W3 dy) * silu'(z2)
         v4s dz2b[8];
 #pragma unroll
@@ -216,7 +234,7 @@ __global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, co
             }
             dz2b[t] = pack4(d[0], d[1], d[2], d[3]);
 #pragma unroll
-            for (int i = 0; i < 4; i++) L.dz2[srow][16 * t + 4 * g + i] = (uint16_t)dz2b[t][i];
+            for (int i = 0; i < 4; i++) L.dz2[16 * t + 4 * g + i][srow] = (uint16_t)dz2b[t][i];
         }
         // dz1 = (W2 dz2) * silu'(z1)
 #pragma unroll
@@ -227,7 +245,7 @@ __global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, co
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float z = F.z1[t][i], sg = sigm(z);
-                L.dz1[srow][16 * t + 4 * g + i] = f2bf(a[i] * (sg * (1.0f + z * (1.0f - sg))));
+                L.dz1[16 * t + 4 * g + i][srow] = f2bf(a[i] * (sg * (1.0f + z * (1.0f - sg))));
             }
         }
     }
@@ -236,21 +254,13 @@ __global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, co
     float* P = partial + (size_t)blockIdx.x * kMlpParams;
     for (int k = 0; k < kTilesPerWave; k++) {
         int layer, ti, to;
-        tile_of(w + 4 * k, layer, ti, to);
+        tile_of(w + kGradThreads / kWave * k, layer, ti, to);
+        const uint16_t* in_row = layer == 0 ? L.x[16 * ti + r] : (layer == 1 ? L.h1[16 * ti + r] : L.h2[16 * ti + r]);
+        const uint16_t* out_row = layer == 0 ? L.dz1[16 * to + r] : (layer == 1 ? L.dz2[16 * to + r] : L.dy[r]);
         v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kc = 0; kc < kChunk / 16; kc++) {
-            v4s a, b;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int ss = 16 * kc + 4 * g + j;
-                uint16_t av, bv;
-                if (layer == 0) { av = L.x[ss][16 * ti + r]; bv = L.dz1[ss][16 * to + r]; }
-                else if (layer == 1) { av = L.h1[ss][16 * ti + r]; bv = L.dz2[ss][16 * to + r]; }
-                else { av = L.h2[ss][16 * ti + r]; bv = L.dy[ss][r]; }
-                a[j] = (short)av;
-                b[j] = (short)bv;
-            }
+            const v4s a = ld4(in_row + 16 * kc + 4 * g), b = ld4(out_row + 16 * kc + 4 * g);
             acc = mfma(a, b, acc);
         }
 #pragma unroll
@@ -263,38 +273,63 @@ __global__ __launch_bounds__(256) void mlp_grad(MlpDev M, const float* feats, co
     }
     // bias gradients from the same bf16 errors, fixed sample order
     if (tid < kMlpHid) {
-        float db = 0.0f;
-        for (int ss = 0; ss < kChunk; ss++) db += bf2f(L.dz1[ss][tid]);
-        P[kP_B1 + tid] = db;
-        if (tid < kMlpOut) {
-            float db3 = 0.0f;
-            for (int ss = 0; ss < kChunk; ss++) db3 += bf2f(L.dy[ss][tid]);
-            P[kP_B3 + tid] = db3;
-        }
-    } else {
-        float db = 0.0f;
-        for (int ss = 0; ss < kChunk; ss++) db += bf2f(L.dz2[ss][tid - kMlpHid]);
-        P[kP_B2 + tid - kMlpHid] = db;
+        P[kP_B1 + tid] = sum_samples(L.dz1[tid]);
+        if (tid < kMlpOut) P[kP_B3 + tid] = sum_samples(L.dy[tid]);
+    } else if (tid < 2 * kMlpHid) {
+        P[kP_B2 + tid - kMlpHid] = sum_samples(L.dz2[tid - kMlpHid]);
     }
     // loss: block sum in a fixed order
     loss = wave_sumf(loss);
-    if (l == 0) L.red[w] = loss;
+    if (l == 0 && w < 4) L.red[w] = loss;
     __syncthreads();
     if (tid == 0) loss_partial[blockIdx.x] = (L.red[0] + L.red[1]) + (L.red[2] + L.red[3]);
 }
 
-__global__ void mlp_reduce_adam(float* params, const float* partial, int nparts, float* grad, float* m, float* v,
-                                float lr, float beta1, float beta2, float eps, float bc1, float bc2) {
+// bf16 copies of parameter p in the layouts the kernels read (the padding is set once, by mlp_refresh)
+struct MlpCopies {
+    uint16_t *w1t, *w2t, *w2n, *w3t, *w3n;
+};
+__device__ __forceinline__ void copy_param(const MlpCopies& W, int p, float v) {
+    const uint16_t h = f2bf(v);
+    if (p < kP_B1) {
+        const int i = (p - kP_W1) / kMlpHid, o = (p - kP_W1) % kMlpHid;
+        W.w1t[o * kMlpInPad + i] = h;
+    } else if (p >= kP_W2 && p < kP_B2) {
+        const int e = p - kP_W2, i = e / kMlpHid, o = e % kMlpHid;
+        W.w2n[e] = h;
+        W.w2t[o * kMlpHid + i] = h;
+    } else if (p >= kP_W3 && p < kP_B3) {
+        const int i = (p - kP_W3) / kMlpOut, o = (p - kP_W3) % kMlpOut;
+        W.w3t[o * kMlpHid + i] = h;
+        W.w3n[i * kMlpOutPad + o] = h;
+    }
+}
+
+// Sum of the partial gradients in block order, and (lr > 0) the Adam update with the bf16 copies.  Loads run
+// eight partials ahead of the additions.
+__global__ __launch_bounds__(64) void mlp_reduce_adam(float* params, const float* partial, int nparts, float* grad,
+                                                      float* m, float* v, float lr, float beta1, float beta2, float eps,
+                                                      float bc1, float bc2, MlpCopies W) {
     RP3DG_GRID_STRIDE(p, kMlpParams) {
         float gsum = 0.0f;
-        for (int b = 0; b < nparts; b++) gsum += partial[(size_t)b * kMlpParams + p];
+        int b = 0;
+        for (; b + 8 <= nparts; b += 8) {
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) x[k] = partial[(size_t)(b + k) * kMlpParams + p];
+#pragma unroll
+            for (int k = 0; k < 8; k++) gsum += x[k];
+        }
+        for (; b < nparts; b++) gsum += partial[(size_t)b * kMlpParams + p];
         if (grad) grad[p] = gsum;
         if (lr > 0.0f) {
             const float mm = beta1 * m[p] + (1.0f - beta1) * gsum;
             const float vv = beta2 * v[p] + (1.0f - beta2) * gsum * gsum;
             m[p] = mm;
             v[p] = vv;
-            params[p] -= lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+            const float np = params[p] - lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+            params[p] = np;
+            copy_param(W, p, np);
         }
     }
 }
@@ -343,6 +378,7 @@ struct rp3dg_mlp {
         d.out_scale = norm + 2 * kMlpIn;
         return d;
     }
+    MlpCopies copies() const { return {w1t, w2t, w2n, w3t, w3n}; }
     ~rp3dg_mlp() {
         for (void* p : allocs) hipFree(p);
         if (stream) hipStreamDestroy(stream);
@@ -437,7 +473,7 @@ static int mlp_grad_step(rp3dg_mlp* m, const float* dfeats, const float* dtarget
     if (nparts > kMaxParts) { set_error("too many samples for one gradient pass"); return RP3DG_EINVAL; }
     int r = mlp_ensure_parts(m, nparts);
     if (r) return r;
-    mlp_grad<<<nparts, 256, 0, m->stream>>>(m->view(), dfeats, dtargets, didx, n, m->partial, m->loss_partial);
+    mlp_grad<<<nparts, kGradThreads, 0, m->stream>>>(m->view(), dfeats, dtargets, didx, n, m->partial, m->loss_partial);
     float bc1 = 1.0f, bc2 = 1.0f;
     const float b1 = 0.9f, b2 = 0.999f;
     if (lr > 0.0f) {
@@ -445,9 +481,8 @@ static int mlp_grad_step(rp3dg_mlp* m, const float* dfeats, const float* dtarget
         bc1 = 1.0f - std::pow(b1, (float)m->adam_t);
         bc2 = 1.0f - std::pow(b2, (float)m->adam_t);
     }
-    mlp_reduce_adam<<<(kMlpParams + 255) / 256, 256, 0, m->stream>>>(m->params, m->partial, nparts, m->grad, m->m, m->v,
-                                                                      lr, b1, b2, 1e-8f, bc1, bc2);
-    if (lr > 0.0f && (r = mlp_refresh_copies(m))) return r;
+    mlp_reduce_adam<<<(kMlpParams + 63) / 64, 64, 0, m->stream>>>(m->params, m->partial, nparts, m->grad, m->m, m->v, lr,
+                                                                   b1, b2, 1e-8f, bc1, bc2, m->copies());
     MLPCHECK(hipGetLastError());
     if (host_loss) {
         std::vector<float> lp(nparts);
@@ -595,9 +630,9 @@ int rp3dg_mlp_gradient_noalloc(rp3dg_mlp* m, const float* feats, const float* ta
     float* partial = m->noalloc_scratch;
     float* loss_partial = partial + (size_t)kNoAllocParts * kMlpParams;
     const int nparts = (int)((n + kChunk - 1) / kChunk);
-    mlp_grad<<<nparts, 256, 0, m->stream>>>(m->view(), feats, targets, nullptr, (int)n, partial, loss_partial);
-    mlp_reduce_adam<<<(kMlpParams + 255) / 256, 256, 0, m->stream>>>(m->params, partial, nparts, grad, nullptr, nullptr,
-                                                                      0.0f, 0.9f, 0.999f, 1e-8f, 1.0f, 1.0f);
+    mlp_grad<<<nparts, kGradThreads, 0, m->stream>>>(m->view(), feats, targets, nullptr, (int)n, partial, loss_partial);
+    mlp_reduce_adam<<<(kMlpParams + 63) / 64, 64, 0, m->stream>>>(m->params, partial, nparts, grad, nullptr, nullptr,
+                                                                   0.0f, 0.9f, 0.999f, 1e-8f, 1.0f, 1.0f, m->copies());
     mlp_loss_mean<<<1, 64, 0, m->stream>>>(loss_partial, nparts, (int)n, loss);
     MLPCHECK(hipGetLastError());
     MLPCHECK(hipStreamSynchronize(m->stream));
