@@ -117,7 +117,7 @@ BYTE_MODEL = {
     "np_box_box": "176 B/test + 40 B/contact point",
 }
 
-KERNELS = ["bp_bounds", "bp_morton", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
+KERNELS = ["bp_bounds", "bp_cells", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
            "bp_merge",
            "np_classify", "np_sphere_sphere", "np_sphere_capsule", "np_capsule_capsule", "np_sphere_poly",
            "np_capsule_poly", "np_box_box", "np_poly_poly", "sv_flag", "sv_compact", "sv_adj_count", "sv_adj_fill",

@@ -216,8 +216,7 @@ struct rp3dg_batch {
     int step_graph(float dt, int n);
     void drop_graphs();
     int scan(const int* in, int n, const int* nptr, int* out, hipStream_t s);
-    int sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr,
-             int first_bit, int bits, hipStream_t s);
+    int sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr, int bits, hipStream_t s);
     void timer_begin(const char* name);
     void timer_end();
     void timer_flush();

@@ -28,7 +28,8 @@ namespace rp3dg {
 // broadphase.hip
 __global__ void bp_refit(DevBodies B, DevColliders C, const float4* hull_bounds, int init);
 __global__ void bp_bounds(DevColliders C, float4* partial);
-__global__ void bp_morton(DevColliders C, const float4* partial, int nparts, uint64_t* keys, int* vals);
+__global__ void bp_cells(DevColliders C, const float4* partial, int nparts, float world_colliders, uint64_t* keys,
+                         int* vals);
 template <int ITEMS>
 __global__ void rs_hist(const uint64_t* keys, int n, const int* nptr, int shift, int* hist, int nblocks);
 template <int ITEMS>
@@ -51,7 +52,7 @@ __global__ void bp_merge(DevColliders C, const uint64_t* keys, const int* nkeys_
 // exclusive scan (out has n+1 entries; out[n] = total).  With nptr the element count is
 // min(n, *nptr), read on the device, and n is only the capacity the grid was sized for.
 // ---------------------------------------------------------------------------------------------
-// Colliders whose broadphase tiles stay in index order (no Morton sort).
+// Colliders whose broadphase tiles stay in index order (no sort).
 constexpr int kIndexOrderColliders = 8192;
 
 constexpr int kScanThreads = 256;
@@ -256,10 +257,10 @@ int rp3dg_batch::scan(const int* in, int n, const int* nptr, int* out, hipStream
 static int sort_items(int n) { return n <= (1 << 18) ? 4 : 16; }
 static int sort_blocks(int n) { return (n + 256 * sort_items(n) - 1) / (256 * sort_items(n)); }
 
-// Stable LSD radix sort of (keys, vals) over the bits [first_bit, first_bit + bits); n keys, or min(n, *nptr)
-// when the count lives on the device.  The result is in (*keys, *vals), which may be the tmp buffers.
-int rp3dg_batch::sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr, int first_bit,
-                      int bits, hipStream_t s) {
+// Stable LSD radix sort of (keys, vals) over the low `bits` bits; n keys, or min(n, *nptr) when the
+// count lives on the device.  The result is in (*keys, *vals), which may be the tmp buffers.
+int rp3dg_batch::sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, int n, const int* nptr, int bits,
+                      hipStream_t s) {
     if (n <= 1) return RP3DG_OK;
     const int nblocks = sort_blocks(n);
     if (nblocks * 256 > sort_hist_cap) return RP3DG_EOVERFLOW;
@@ -267,7 +268,7 @@ int rp3dg_batch::sort(uint64_t** keys, int** vals, uint64_t* ktmp, int* vtmp, in
     int* vi = *vals;
     uint64_t* ko = ktmp;
     int* vo = vtmp;
-    for (int shift = first_bit; shift < first_bit + bits; shift += 8) {
+    for (int shift = 0; shift < bits; shift += 8) {
         const bool few = sort_items(n) == 4;
         if (few) rs_hist<4><<<nblocks, 256, 0, s>>>(ki, n, nptr, shift, sort_hist, nblocks);
         else rs_hist<16><<<nblocks, 256, 0, s>>>(ki, n, nptr, shift, sort_hist, nblocks);
@@ -1135,13 +1136,12 @@ int rp3dg_batch::enqueue_broadphase(bool capturing, const DevEvents& E, int pg) 
         if (nc > kIndexOrderColliders) {
             const int nparts = std::min(256, grid_for(nc));
             LAUNCH_T("bp_bounds", nparts, 256, bp_bounds, C, bp_partial);
-            LAUNCH_T("bp_morton", grid_for(nc), 256, bp_morton, C, bp_partial, nparts, bp_keys, bp_vals);
-            // cells of 16 Morton bits (2 passes), 24 where 64-collider tiles need finer ones
-            const int cell_bits = nc <= (1 << 18) ? 16 : 24;
+            LAUNCH_T("bp_cells", grid_for(nc), 256, bp_cells, C, bp_partial, nparts,
+                     (float)std::max(1, nc / nworlds), bp_keys, bp_vals);
             uint64_t* k = bp_keys;
             int* v = bp_vals;
             timer_begin("bp_sort");
-            r = sort(&k, &v, bp_ktmp, bp_vtmp, nc, nullptr, 30 - cell_bits, cell_bits + world_bits, stream);
+            r = sort(&k, &v, bp_ktmp, bp_vtmp, nc, nullptr, kCellBits + world_bits, stream);
             timer_end();
             if (r) { set_error("radix sort overflow"); return r; }
             order = v;
@@ -1325,7 +1325,7 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         int sbits = 0;
         while ((1 << sbits) < nseg) sbits++;
         timer_begin("sv_color_sort");
-        r = sort(&ck, &cv, cktmp, cvtmp, man_cap, nm_ptr, 0, sbits, stream);
+        r = sort(&ck, &cv, cktmp, cvtmp, man_cap, nm_ptr, sbits, stream);
         timer_end();
         if (r) { set_error("sort overflow"); return r; }
         r = scan(seg_cnt, nseg, nullptr, seg_start, stream);

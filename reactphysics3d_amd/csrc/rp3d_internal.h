@@ -61,6 +61,8 @@ __host__ __device__ inline uint32_t lf_edge1(uint32_t w) { return (w >> 16) & 0x
 __host__ __device__ inline uint32_t lf_edge2(uint32_t w) { return (w >> 24) & 0xffu; }
 
 constexpr int kSlab = 64;             // partners kept per collider by the broadphase's overlap pass
+constexpr int kStripBits = 8;         // broadphase order: strip, and 16 bits of position in it, below the world id
+constexpr int kCellBits = kStripBits + 16;
 constexpr int kMaxRawContacts = 16;   // NB_MAX_CONTACT_POINTS_IN_NARROWPHASE_INFO (configuration.h:134)
 constexpr int kMaxManifoldPoints = 4; // MAX_CONTACT_POINTS_IN_MANIFOLD
 // Hull faces have at most this many vertices: clipping an incident face by the side planes of a
@@ -119,7 +121,7 @@ struct DevColliders {
     int *moved;                // fat AABB recomputed by the last refit (BroadPhaseSystem moved set)
     int *rank;                 // position of the collider in the moved-set iteration order
     int *world;
-    int *is_static;            // collider of a static body (never moves, never traverses the BVH)
+    int *is_static;            // collider of a static body (never moves, starts no pair)
     int *ss_offs;              // static-static overlapping partners (CSR, constant after creation)
     int *ss_list;
     int n;
