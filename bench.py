@@ -65,9 +65,9 @@ def bytes_per_launch(name, c, ndyn, nj):
         # whole velocity solver of a step, one launch: 48 B / contact point + 88 B / manifold +
         # 140 B / dynamic body + 200 B / joint
         return 48 * p + 88 * m + 140 * ndyn + 200 * nj
-    if name == "world_position":
-        # position integration + commit (192 B / dynamic body) and fat-AABB refit (48 B / collider)
-        return 192 * ndyn + 48 * ncl
+    if name in ("world_position", "body_position"):
+        # position integration + commit (192 B / dynamic body), world_position also refits (48 B / collider)
+        return 192 * ndyn + (48 * ncl if name == "world_position" else 0)
     if name in ("sv_solve_color", "sv_warmstart"):
         return (48 * p + 88 * m + 140 * 2 * m) / ncol
     if name == "sv_setup":   # velocity integration and contact rows
@@ -123,6 +123,7 @@ KERNELS = ["bp_bounds", "bp_cells", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit"
            "np_capsule_poly", "np_box_box", "np_poly_poly", "sv_flag", "sv_compact", "sv_adj_count", "sv_adj_fill",
            "sv_color_round", "sv_color_finish", "sv_color_keys", "sv_color_sort", "sv_world_ranges", "sv_group_color",
            "sv_setup", "sv_features", "mlp_infer", "sv_world_solve", "sv_log_samples", "world_position",
+           "body_position",
            "sv_warmstart", "sv_solve_color", "sv_store",
            "jt_warmstart", "jt_solve_velocity", "jt_solve_position", "dyn_integrate_positions", "dyn_update_state",
            "bp_refit"]

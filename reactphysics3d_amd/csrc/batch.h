@@ -43,10 +43,11 @@ struct rp3dg_batch {
     int ev_cap = 0;
     bool events_on = false;
     int* jt_ranges = nullptr;          // [2*slot] colour ranges of the joint rows, slots in solve order
-    int2* jt_wr = nullptr;             // fused solver: [w * jt_slots + slot] joint rows of world w
+    int4* jt_segs = nullptr;           // fused solver: the strands of every group (fused.h)
+    int* jt_strands = nullptr;
+    int jt_waves = 1;                  // wavefronts that the fullest group's strands or slots take
     int jt_slots = 0;
     std::vector<int> jt_kind;          // [slot] joint kind (JT_*) of the slot
-    int* d_jt_kind = nullptr;
     std::vector<int> joint_order;      // global joint index of each joint row
     bool cur_is_a = true;
     int pair_cap = 0;
@@ -207,6 +208,7 @@ struct rp3dg_batch {
     ~rp3dg_batch();
     int upload(rp3dg_world* const* worlds, int n, const rp3dg_batch_options* opt);
     void set_class_blocks();
+    int class_block(int max_bodies) const;
     int launch_world_classes(const char* name, const rp3dg::FusedArgs& F);
     int upload_joints(rp3dg_world* const* worlds, int n);
     void enqueue_sleep(float dt, const rp3dg::DevPairs& N, int pair_grid);

@@ -355,7 +355,7 @@ static void moved_ranks(int n, std::vector<int>& rank) {
 // (BallAndSocketJoint.cpp:38-53, FixedJoint.cpp:36-56, HingeJoint.cpp:36-80, SliderJoint.cpp:38-91); the
 // rows are sorted by (kind in solve order, colour, creation index) with a greedy colouring over all bodies.
 int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
-    struct Row { int kind, color, order, b1, b2, group, slot, world; float4 la1, la2, ax1, ax2, qinit, lim; int flags; };
+    struct Row { int kind, color, order, b1, b2, group, slot, world, strand, srank; float4 la1, la2, ax1, ax2, qinit, lim; int flags; };
     std::vector<Row> rows;
     int jbase = 0;
     for (int wi = 0; wi < nw; wi++) {
@@ -436,30 +436,127 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     for (int k = 0; k < JT_KINDS * 64; k++)
         if (slot_of[k] >= 0) jt_kind.push_back(k / 64);
     for (Row& r : rows) r.slot = slot_of[r.kind * 64 + r.color];
+    const int n = (int)rows.size();
     const bool wmajor = fused;
+    // order of the solve: (group,) slot, creation index
     std::stable_sort(rows.begin(), rows.end(), [wmajor](const Row& a, const Row& b) {
         if (wmajor && a.group != b.group) return a.group < b.group;
         if (a.slot != b.slot) return a.slot < b.slot;
         return a.order < b.order;
     });
-    const int n = (int)rows.size();
+    // slider ranks in each world's solve order
+    std::vector<int> nsl(nw, 0);
+    joint_order.resize(n);
+    for (int i = 0; i < n; i++) {
+        rows[i].srank = rows[i].kind == JT_SLIDER ? nsl[rows[i].world]++ : -1;
+        joint_order[i] = rows[i].order;
+    }
     std::vector<int> ranges;   // per-colour kernels: [2*slot] = [first, end) over all worlds
-    std::vector<int2> wr((size_t)ngroups * std::max(jt_slots, 1), make_int2(0, 0));   // fused: per group and slot
+    std::vector<int4> segs;    // fused: the strands' runs of joints
+    std::vector<int> strands(1, 0);
     if (!wmajor) {
         for (int i = 0; i < n; i++) {
             if (i == 0 || rows[i].slot != rows[i - 1].slot) ranges.push_back(i);
             if (i == n - 1 || rows[i + 1].slot != rows[i].slot) ranges.push_back(i + 1);
         }
     } else {
-        std::vector<int> cnt((size_t)ngroups * std::max(jt_slots, 1), 0);
-        for (const Row& r : rows) cnt[(size_t)r.group * jt_slots + r.slot]++;
-        int run = 0;
-        for (size_t k = 0; k < cnt.size(); k++) {
-            wr[k] = make_int2(run, run + cnt[k]);
-            run += cnt[k];
+        // Strands (fused.h): the connected components of a group's joints, packed so that the longest strand,
+        // in phases of 32 joints of a slot, is as short as its longest component allows.
+        struct Comp {
+            int first, end;   // in `parts`
+            int phases;
+        };
+        struct Part {
+            int root, slot, count;
+        };
+        std::vector<int> root(nb);
+        for (int i = 0; i < nb; i++) root[i] = i;
+        auto find = [&](int i) {
+            while (root[i] != i) i = root[i] = root[root[i]];
+            return i;
+        };
+        for (const Row& r : rows) root[find(r.b1)] = find(r.b2);
+        auto phases = [](int joints, int lanes) { return (joints + lanes - 1) / lanes; };
+        jt_waves = 1;
+        std::vector<int> strand_of(nb, 0);   // by root
+        for (int g = 0, i0 = 0; g < ngroups; g++) {
+            int i1 = i0;
+            while (i1 < n && rows[i1].group == g) i1++;
+            std::vector<Part> parts;
+            for (int i = i0; i < i1; i++) parts.push_back({find(rows[i].b1), rows[i].slot, 1});
+            std::sort(parts.begin(), parts.end(), [](const Part& a, const Part& b) {
+                return a.root != b.root ? a.root < b.root : a.slot < b.slot;
+            });
+            std::vector<Comp> comps;
+            size_t np = 0;
+            for (size_t k = 0; k < parts.size(); k++) {
+                const Part p = parts[k];
+                const bool same_comp = np > 0 && parts[np - 1].root == p.root;
+                if (same_comp && parts[np - 1].slot == p.slot) parts[np - 1].count++;
+                else {
+                    if (!same_comp) comps.push_back({(int)np, 0, 0});
+                    parts[np++] = p;
+                }
+                comps.back().end = (int)np;
+            }
+            int longest = 0, nseg = 0;
+            for (Comp& c : comps) {
+                for (int k = c.first; k < c.end; k++) c.phases += phases(parts[k].count, 32);
+                longest = std::max(longest, c.phases);
+            }
+            std::stable_sort(comps.begin(), comps.end(), [](const Comp& a, const Comp& b) { return a.phases > b.phases; });
+            int L = 64;   // as wclasses: the solver's threads for a group of this size
+            while (L < body_base[group_world[g + 1]] - body_base[group_world[g]]) L *= 2;
+            const int waves = class_block(L) / kWave, most = std::min(kJointStrands, waves);
+            std::vector<std::vector<int>> load(most, std::vector<int>(jt_slots, 0));   // [strand][slot] joints
+            std::vector<int> cost(most, 0);
+            for (const Comp& c : comps) {
+                int best = 0, best_cost = INT_MAX;
+                for (int s = 0; s < most; s++) {
+                    int v = cost[s];
+                    for (int k = c.first; k < c.end; k++) {
+                        const int l = load[s][parts[k].slot];
+                        v += phases(l + parts[k].count, 32) - phases(l, 32);
+                    }
+                    if (v <= longest) v = longest;   // the first strand that stays within the longest component
+                    if (v < best_cost) { best = s; best_cost = v; }
+                }
+                strand_of[parts[c.first].root] = best;
+                for (int k = c.first; k < c.end; k++) {
+                    int& l = load[best][parts[k].slot];
+                    cost[best] += phases(l + parts[k].count, 32) - phases(l, 32);
+                    l += parts[k].count;
+                }
+            }
+            int together = 0, fullest = 0, used = 0;
+            for (int s = 0; s < jt_slots; s++) {
+                int all = 0;
+                for (int k = 0; k < most; k++) {
+                    all += load[k][s];
+                    nseg += load[k][s] > 0;
+                }
+                together += phases(all, 32 * waves);
+                fullest = std::max(fullest, all);
+            }
+            for (int k = 0; k < most; k++) used += cost[k] > 0;
+            const bool wide = *std::max_element(cost.begin(), cost.end()) > together || nseg > kMaxJointSegs;
+            jt_waves = std::max(jt_waves, wide ? phases(fullest, 32) : used);
+            for (int i = i0; i < i1; i++) rows[i].strand = wide ? 0 : strand_of[find(rows[i].b1)];
+            std::stable_sort(rows.begin() + i0, rows.begin() + i1, [](const Row& a, const Row& b) {
+                return a.strand != b.strand ? a.strand < b.strand : a.slot < b.slot;
+            });
+            int i = i0;
+            for (int s = 0; s < kJointStrands; s++) {
+                while (i < i1 && rows[i].strand == s) {
+                    const int lo = i;
+                    while (i < i1 && rows[i].strand == s && rows[i].slot == rows[lo].slot) i++;
+                    segs.push_back(make_int4(lo, i, rows[lo].kind, wide));
+                }
+                strands.push_back((int)segs.size());
+            }
+            i0 = i1;
         }
     }
-    joint_order.resize(n);
     J.n = n;
     const size_t m = std::max(1, n);
     J.type = dalloc<int>(this, m); J.bodies = dalloc<int2>(this, m); J.flags = dalloc<int>(this, m);
@@ -470,13 +567,11 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     J.bias1 = dalloc<float4>(this, m);
     J.srank = dalloc<int>(this, m);
     if (!J.bias0 || !J.bias1 || !J.srank) { set_error("device allocation failed (joints)"); return RP3DG_EHIP; }
-    // slider ranks in each world's solve order (rows are sorted by slot, then creation index, within a world)
-    std::vector<int> srank(m, -1), nsl(nw, 0);
+    std::vector<int> srank(m, -1);
     bool any_bslider = false;
     for (int i = 0; i < n; i++) {
-        if (rows[i].kind != JT_SLIDER) continue;
-        srank[i] = nsl[rows[i].world]++;
-        any_bslider |= (rows[i].flags & JF_BAUMGARTE) != 0;
+        srank[i] = rows[i].srank;
+        any_bslider |= rows[i].kind == JT_SLIDER && (rows[i].flags & JF_BAUMGARTE) != 0;
     }
     J.bfirst = nullptr;
     if (any_bslider) {
@@ -486,9 +581,10 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     J.imlm = dalloc<float>(this, m);
     J.imm = dalloc<float>(this, m);
     jt_ranges = dalloc<int>(this, std::max<size_t>(2, ranges.size()));
-    jt_wr = dalloc<int2>(this, wr.size());
-    d_jt_kind = dalloc<int>(this, jt_kind.size());
-    if (!J.imlm || !J.imm || !jt_ranges || !jt_wr || !d_jt_kind) { set_error("device allocation failed (joints)"); return RP3DG_EHIP; }
+    jt_segs = dalloc<int4>(this, std::max<size_t>(1, segs.size()));
+    jt_strands = dalloc<int>(this, strands.size());
+    if (!J.imlm || !J.imm || !jt_ranges || !jt_segs || !jt_strands) { set_error("device allocation failed (joints)"); return RP3DG_EHIP; }
+    HIPCHECK(hipMemcpy(jt_strands, strands.data(), sizeof(int) * strands.size(), hipMemcpyHostToDevice));
     if (n == 0) return RP3DG_OK;
     std::vector<int> type(n), flags(n);
     std::vector<int2> bodies(n);
@@ -497,7 +593,6 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
         const Row& r = rows[i];
         type[i] = r.kind; flags[i] = r.flags; bodies[i] = make_int2(r.b1, r.b2);
         la1[i] = r.la1; la2[i] = r.la2; ax1[i] = r.ax1; ax2[i] = r.ax2; qinit[i] = r.qinit; lim[i] = r.lim;
-        joint_order[i] = r.order;
     }
     HIPCHECK(hipMemcpy(J.type, type.data(), 4 * n, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(J.flags, flags.data(), 4 * n, hipMemcpyHostToDevice));
@@ -515,8 +610,7 @@ int rp3dg_batch::upload_joints(rp3dg_world* const* ws, int nw) {
     HIPCHECK(hipMemset(J.imlm, 0, sizeof(float) * n));
     HIPCHECK(hipMemset(J.imm, 0, sizeof(float) * n));
     if (!ranges.empty()) HIPCHECK(hipMemcpy(jt_ranges, ranges.data(), sizeof(int) * ranges.size(), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(jt_wr, wr.data(), sizeof(int2) * wr.size(), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(d_jt_kind, jt_kind.data(), sizeof(int) * jt_kind.size(), hipMemcpyHostToDevice));
+    if (!segs.empty()) HIPCHECK(hipMemcpy(jt_segs, segs.data(), sizeof(int4) * segs.size(), hipMemcpyHostToDevice));
     return RP3DG_OK;
 }
 
@@ -1352,9 +1446,8 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         F.J = J;
         F.settings = settings;
         F.seg_start = seg_start;
-        F.jt_wr = jt_wr;
-        F.jt_kind = d_jt_kind;
-        F.jt_slots = jt_slots;
+        F.jt_segs = jt_segs;
+        F.jt_strands = jt_strands;
         F.wbody = d_wbody;
         F.wcoll = d_wcoll;
         F.block_world = d_block_world;
@@ -1394,7 +1487,19 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
                      log_cap);
             sv_log_advance<<<1, 1, 0, stream>>>(&counters->nb_new_points, feat_cap, log_count, log_cap);
         }
-        LAUNCH_T("world_position", ngroups, fused_block, world_position, F);
+        if (J.n == 0) {
+            LAUNCH_T("body_position", grid_for(nb), 256, body_position, B, dt, settings.split_impulse ? 1.0f : 0.0f);
+            LAUNCH_T("bp_refit", grid_for(nc), 256, bp_refit, B, C, d_hbounds, 0);
+        } else {
+            // Bodies in LDS unless they would keep a batch of many groups from having 4 workgroups on a CU.
+            // (block_world may be the residual mode's order; the first class has the largest group)
+            F.lds_bodies = wclasses[0].largest;
+            const int block = user_block ? user_block : std::min(kPositionMaxBlock, std::max(fused_block, kWave * jt_waves));
+            const size_t lds = (size_t)F.lds_bodies * kPositionLds, own = 64;
+            if (lds + own <= std::min<size_t>(max_lds_per_block, max_lds_per_cu / std::max(1, std::min(4, (ngroups + 255) / 256))))
+                LAUNCH_TS("world_position", ngroups, block, lds, world_position<true>, F);
+            else LAUNCH_T("world_position", ngroups, block, world_position<false>, F);
+        }
         enqueue_sleep(dt, N, pg);
         return RP3DG_OK;
     }
@@ -1428,7 +1533,7 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     LAUNCH_T("dyn_integrate_positions", bg, 256, dyn_integrate_positions, B, dt, settings.split_impulse ? 1.0f : 0.0f);
     for (int it = 0; it < settings.pos_iters; it++)
         for (int s = 0; s < jt_slots; s++)
-            LAUNCH_T("jt_solve_position", jg, 256, jt_solve_position, B, J, jt_ranges, s);
+            LAUNCH_T("jt_solve_position", jg2, 256, jt_solve_position, B, J, jt_ranges, s, jt_kind[s]);
     LAUNCH_T("dyn_update_state", bg, 256, dyn_update_state, B);
     LAUNCH_T("bp_refit", grid_for(nc), 256, bp_refit, B, C, d_hbounds, 0);
     enqueue_sleep(dt, N, pg);
@@ -1452,7 +1557,12 @@ static const SolveKernel kSolveKernels[2][3] = {   // [split impulses][STATE_*]
 // a world of n bodies has about n / 6 to n / 4 manifolds a colour, so L threads fill the colour phases.
 void rp3dg_batch::set_class_blocks() {
     for (WorldClass& c : wclasses)
-        c.block = user_block ? user_block : std::max(64, std::min(kFusedMaxBlock, 2 * c.max_bodies / block_div));
+        c.block = class_block(c.max_bodies);
+}
+int rp3dg_batch::class_block(int L) const {
+    // (with a CU for every group, a wavefront for every strand of joints costs nothing)
+    const int least = jt_slots > 0 && ngroups <= 256 ? kWave * kJointStrands : kWave;
+    return user_block ? user_block : std::max(least, std::min(kFusedMaxBlock, 2 * L / block_div));
 }
 
 // LDS of a class's workgroups.  The body state is staged whole when it fits (100 B a body, up to about

@@ -135,6 +135,35 @@ __device__ __forceinline__ unsigned long long uniform(unsigned long long x) {
            (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)x);
 }
 
+// Tables that no kernel writes, read through the scalar cache.
+template <class T>
+using Table = const __attribute__((address_space(4))) T*;
+template <class T>
+__device__ __forceinline__ Table<T> table(const T* p) { return (Table<T>)(uintptr_t)p; }
+
+// Calls f(arguments, segment, all) for the segments of this wavefront's strands of group g, or of the whole
+// group's (all); ends with a barrier if there were any.
+template <int STATE, class F>
+__device__ __forceinline__ void joint_strands(int g, int wave, int waves, F&& f) {
+    const FusedArgs& P = phase_args();
+    const Table<int> st = table(P.jt_strands) + (size_t)g * kJointStrands;
+    const int first = st[0];
+    if (first == st[kJointStrands]) return;
+    const bool all = table(&P.jt_segs[first].w)[0] != 0;
+    for (int s = all ? 0 : wave; s < (all ? 1 : kJointStrands); s += waves) {
+        const int end = st[s + 1];
+        for (int k = st[s]; k < end; k++) {
+            const FusedArgs& FP = phase_args();
+            const Table<int> e = table(&FP.jt_segs[k].x);
+            const int4 r = make_int4(e[0], e[1], e[2], 0);
+            f(FP, r, all);
+            if (all) phase_barrier<STATE>();
+            else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+    if (!all) phase_barrier<STATE>();
+}
+
 // Header of a row: bodies relative to the group's first (14 bits each), points (3 bits).
 __device__ __forceinline__ unsigned int row_header(int u1, int u2, int np) {
     return (unsigned)u1 | (unsigned)u2 << 14 | (unsigned)np << 28;
@@ -163,8 +192,6 @@ __global__ __launch_bounds__(kFusedMaxBlock) void sv_world_solve(FusedArgs F) {
     const int b0 = F.wbody[w0], b1 = F.wbody[w0 + ngw], nbw = b1 - b0;
     const int* seg = F.seg_start + (size_t)g * kMaxColors;
     const int m0 = seg[0], m1 = seg[kMaxColors];
-    const int2* jr = F.jt_wr + (size_t)g * F.jt_slots;
-    const int nslots = F.jt_slots && jr[0].x < jr[F.jt_slots - 1].y ? F.jt_slots : 0;
     const int mcap = F.lds_rows;
 
     // ---------------- staging
@@ -229,12 +256,9 @@ __global__ __launch_bounds__(kFusedMaxBlock) void sv_world_solve(FusedArgs F) {
             s_lq[2 * r + 1] = F.A.S.lq[2 * (size_t)i + 1];
             s_ih[r] = f4(ld3(F.A.S.imp, i), __uint_as_float(row_header(bb.x - b0, bb.y - b0, F.A.S.npts[i])));
         }
-    for (int s = 0; s < nslots; s++) {
-        const int2 r = jr[s];
-        if (r.x == r.y) continue;
-        for (int j = r.x + tid; j < r.y; j += nt) jt_warmstart_one(BS, F.J, j);
-        phase_barrier<STATE>();
-    }
+    joint_strands<STATE>(g, uniform(tid / kWave), nt / kWave, [&](const FusedArgs& FP, const int4& r, bool all) {
+        for (int j = r.x + (all ? tid : tid & (kWave - 1)); j < r.y; j += all ? nt : kWave) jt_warmstart_one(BS, FP.J, j);
+    });
     const bool residual = F.res_thr > 0.0f;
     // residual mode with several worlds: each world stops on its own residual (mask of converged worlds)
     const bool masked = residual && ngw > 1;
@@ -322,17 +346,13 @@ __global__ __launch_bounds__(kFusedMaxBlock) void sv_world_solve(FusedArgs F) {
     int it = 0;
     float res = 0.0f;
     while (it < F.max_iters) {
-        for (int s = 0; s < nslots; s++) {
-            const FusedArgs& FP = phase_args();
-            const int2 r = FP.jt_wr[(size_t)g * FP.jt_slots + s];
-            if (r.x == r.y) continue;
-            const int t0 = phase_thread(wave);
-            for (int j = r.x + (t0 >> 1); j < r.y; j += nt >> 1) {
+        joint_strands<STATE>(g, wave, nt / kWave, [&](const FusedArgs& FP, const int4& r, bool all) {
+            const int t0 = phase_thread(all ? wave : 0), kind = r.z;
+            for (int j = r.x + (t0 >> 1); j < r.y; j += (all ? nt : kWave) >> 1) {
                 if (masked && ((done >> world_of(FP.J.bodies[j].x - BS.vbase)) & 1ull)) continue;
-                jt_solve_velocity_pair(BS, FP.J, FP.jt_kind[s], j, t0 & 1, FP.dt);
+                jt_solve_velocity_pair(BS, FP.J, kind, j, t0 & 1, FP.dt);
             }
-            phase_barrier<STATE>();
-        }
+        });
         if (fast) contact_sweep(std::true_type{});
         else contact_sweep(std::false_type{});
         it++;
@@ -421,30 +441,96 @@ template __global__ void sv_world_solve<false, STATE_LDS>(FusedArgs F);
 template __global__ void sv_world_solve<false, STATE_VEL>(FusedArgs F);
 template __global__ void sv_world_solve<false, STATE_HBM>(FusedArgs F);
 
+// Position integration, joint position correction, body state and refit of a group of worlds with joints
+// (PhysicsWorld.cpp:275-288).  A strand of joints is a chain of short phases, each of them one joint's
+// dependent chain for its lanes, so the length of that chain sets the time: two lanes share a joint
+// (joints_dev.h), the bodies are staged in LDS, and the next segment's joints are loaded while the current
+// ones are solved.  64 joints of 3 kinds (88 bodies), 5 iterations: 181 us with one lane a joint, positions
+// in HBM and a barrier after each kind and colour, 119 with two lanes and LDS, 61 with strands; 1024 worlds
+// of 8 to 128 bodies: 123, 103, 78.
+template <bool STAGED>
 __global__ __launch_bounds__(kPositionMaxBlock) void world_position(FusedArgs F) {
+    extern __shared__ float4 s_pos[];
     const DevBodies& B = F.A.B;
     const int g = F.block_world[blockIdx.x];
     const int tid = threadIdx.x, nt = blockDim.x;
     const int w0 = F.gworld[g], w1 = F.gworld[g + 1];
     const int b0 = F.wbody[w0], b1 = F.wbody[w1];
     const int c0 = F.wcoll[w0], c1 = F.wcoll[w1];
-    const int2* jr = F.jt_wr + (size_t)g * F.jt_slots;
-    // PhysicsWorld.cpp:275-288: integrate positions, joint position correction, update body state
     const float split_factor = F.settings.split_impulse ? 1.0f : 0.0f;
     for (int i = b0 + tid; i < b1; i += nt) dyn_integrate_positions_one(B, F.dt, i, split_factor);
-    __syncthreads();
-    for (int it = 0; it < F.settings.pos_iters; it++) {
-        for (int s = 0; s < F.jt_slots; s++) {
-            const int2 r = jr[s];
-            if (r.x == r.y) continue;
-            for (int j = r.x + tid; j < r.y; j += nt) jt_solve_position_one(B, F.J, j);
-            __syncthreads();
+    PosBodies<STAGED> P;
+    if constexpr (STAGED) {
+        float4* com = s_pos + 3 * F.lds_bodies;
+        P = {s_pos, s_pos + F.lds_bodies, s_pos + 2 * F.lds_bodies, com, nullptr, b0};
+        for (int i = b0 + tid; i < b1; i += nt) {   // each thread reads what it wrote
+            P.x[i - b0] = f4(ld3(B.cx, i), __int_as_float(B.flags[i]));
+            P.q[i - b0] = B.cq[i];
+            s_pos[2 * F.lds_bodies + i - b0] = B.ii[i];
+            com[i - b0] = B.com[i];
         }
+    } else {
+        P = {B.cx, B.cq, B.ii, B.com, B.flags, 0};
     }
-    for (int i = b0 + tid; i < b1; i += nt) dyn_update_state_one(B, i);
+    __syncthreads();
+    const Table<int> st = table(F.jt_strands) + (size_t)g * kJointStrands;
+    const int first = st[0];
+    if (first != st[kJointStrands]) {
+        const Table<int> segs = table(&F.jt_segs[0].x);   // 4 ints each
+        const bool all = segs[4 * (size_t)first + 3] != 0;
+        const int wave = uniform(tid / kWave), side = tid & 1, step = (all ? nt : kWave) >> 1;
+        const int turn = (all ? tid : tid & (kWave - 1)) >> 1;
+        for (int s = all ? 0 : wave; s < (all ? 1 : kJointStrands); s += nt / kWave) {
+            const int k0 = st[s], k1 = st[s + 1], total = (k1 - k0) * F.settings.pos_iters;
+            JointPos next;
+            if (total > 0) {
+                const Table<int> e = segs + 4 * (size_t)k0;
+                next = jt_position_load(F.J, min(e[0] + turn, e[1] - 1), side);
+            }
+            for (int n = 0, k = k0; n < total; n++) {
+                const Table<int> e = segs + 4 * (size_t)k;
+                const int last = e[1], kind = e[2];
+                JointPos p = next;
+                int j = e[0] + turn;
+                k = k + 1 < k1 ? k + 1 : k0;
+                if (n + 1 < total) {
+                    const Table<int> e2 = segs + 4 * (size_t)k;
+                    next = jt_position_load(F.J, min(e2[0] + turn, e2[1] - 1), side);
+                }
+                while (j < last) {   // (rarely more than once: one copy of the code)
+                    jt_solve_position_pair(B, P, F.J, kind, j, side, p);
+                    j += step;
+                    if (j < last) p = jt_position_load(F.J, j, side);
+                }
+                if (all) phase_barrier<STAGED ? STATE_LDS : STATE_HBM>();
+                else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = b0 + tid; i < b1; i += nt) {
+        if constexpr (STAGED) {
+            B.cx[i] = f4(xyz(P.x[i - b0]), 0.f);
+            B.cq[i] = P.q[i - b0];
+        }
+        dyn_update_state_one(B, i);
+    }
     __syncthreads();
     // collider transforms and fat AABBs for the next broadphase
     for (int i = c0 + tid; i < c1; i += nt) refit_one(B, F.A.C, F.hull_bounds, 0, i);
+}
+template __global__ void world_position<true>(FusedArgs F);
+template __global__ void world_position<false>(FusedArgs F);
+
+// Positions and state of the bodies of worlds without joints, whatever world they are in.  One thread a body
+// over the whole batch, and the colliders after it in a launch of their own: a workgroup per group of worlds
+// leaves the chip idle with few groups and waits for its slowest load three times over with many.  1001
+// bodies: 30 us in one workgroup, 6 and 7 us in the two launches.
+__global__ __launch_bounds__(256) void body_position(DevBodies B, float dt, float split_factor) {
+    RP3DG_GRID_STRIDE(i, B.n) {
+        dyn_integrate_positions_one(B, dt, i, split_factor);
+        dyn_update_state_one(B, i);
+    }
 }
 
 __global__ void sv_log_samples(FusedArgs F, float* log_feats, float* log_targets, const unsigned long long* logged,

@@ -59,6 +59,6 @@ struct DevJoints {
 
 __global__ void jt_warmstart(DevBodies B, DevJoints J, const int* range, int slot);
 __global__ void jt_solve_velocity(DevBodies B, DevJoints J, const int* range, int slot, int kind, float dt);
-__global__ void jt_solve_position(DevBodies B, DevJoints J, const int* range, int slot);
+__global__ void jt_solve_position(DevBodies B, DevJoints J, const int* range, int slot, int kind);
 
 }  // namespace rp3dg

@@ -82,7 +82,7 @@ __device__ inline Q4 nudge(Q4 q, V3 w) {
 // ---- hinge angle (SolveHingeJointSystem.cpp:733-799) ----
 __device__ inline float normalized_angle(float a) {
     const float twopi = 2.0f * kPi;
-    a = fmodf(a, twopi);
+    if (!(fabsf(a) < twopi)) a = fmodf(a, twopi);   // (fmodf returns a itself below 2 pi)
     if (a < -kPi) return a + twopi;
     if (a > kPi) return a - twopi;
     return a;
@@ -597,247 +597,237 @@ __device__ __forceinline__ void jt_solve_velocity_pair(const DevBodies& B, const
 }
 
 // ------------------------------------------------------------------------------------------------
-// non-linear Gauss-Seidel position correction (per colour)
+// non-linear Gauss-Seidel position correction (per colour), two lanes per joint as above
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void jt_solve_position_one(const DevBodies& B, const DevJoints& J, int j) {
-    {
-        const int2 bb = J.bodies[j];
-        const int b1 = bb.x, b2 = bb.y;
-        if (!joint_enabled(B, b1, b2)) return;
-        const int type = J.type[j];
-        // only non-linear Gauss-Seidel joints (SolveBallAndSocketJointSystem.cpp:309,
-        // SolveFixedJointSystem.cpp:299, SolveHingeJointSystem.cpp:479); the slider system stops at its
-        // first Baumgarte joint (SolveSliderJointSystem.cpp:527)
-        if (J.flags[j] & JF_BAUMGARTE) return;
-        if (type == JT_SLIDER && J.bfirst && J.srank[j] >= J.bfirst[B.world[b1]]) return;
-        Q4 q1 = ldq(B.cq, b1), q2 = ldq(B.cq, b2);
-        V3 x1 = ld3(B.cx, b1), x2 = ld3(B.cx, b2);
-        const float4 ii1 = B.ii[b1], ii2 = B.ii[b2];
-        const float im1 = ii1.w, im2 = ii2.w;
-        V3 ll1, al1, ll2, al2;
-        body_locks(B, b1, ll1, al1);
-        body_locks(B, b2, ll2, al2);
-        const bool anyDyn = ((body_flags(B, b1) | body_flags(B, b2)) & BF_DYNAMIC) != 0;
-        M3 I1 = world_inv_inertia(qmat(q1), v3(ii1.x, ii1.y, ii1.z));
-        M3 I2 = world_inv_inertia(qmat(q2), v3(ii2.x, ii2.y, ii2.z));
-        const V3 r1 = qrot(q1, ld3(J.la1, j) - ld3(B.com, b1));
-        const V3 r2 = qrot(q2, ld3(J.la2, j) - ld3(B.com, b2));
-        if (type == JT_BALLSOCKET) {   // SolveBallAndSocketJointSystem.cpp:312-445
-            int fl = J.flags[j];
-            if (fl & JF_LIMIT) {
-                const V3 r1u = unit(r1), r2u = -unit(r2);
-                const V3 acb = cross(r1u, r2u);
-                const float err = J.lim[j].x - ref_acosf(dot(r1u, r2u));
-                fl = err < 0.0f ? (fl | JF_LOWER_VIOLATED) : (fl & ~JF_LOWER_VIOLATED);
-                J.flags[j] = fl;
-                if (fl & JF_LOWER_VIOLATED) {
-                    const float m = dot(acb, mvmul(I1, acb)) + dot(acb, mvmul(I2, acb));
-                    const float l = (m > 0.0f ? 1.0f / m : 0.0f) * (-err);
-                    q1 = nudge(q1, cmul(al1, mvmul(I1, l * acb)));
-                    q2 = nudge(q2, cmul(al2, mvmul(I2, (-l) * acb)));
-                }
+// Constrained positions and what the correction reads of a body, indexed [body - base]: arrays of the whole
+// batch, or staged in LDS with the body's flags in the w lanes of x (STAGED).
+template <bool STAGED>
+struct PosBodies {
+    float4 *x, *q;
+    const float4 *ii, *com;
+    const int* flags;   // unless STAGED
+    int base;
+    __device__ __forceinline__ int body_flags(int u) const {
+        if constexpr (STAGED) return __float_as_int(x[u].w);
+        else return flags[u];
+    }
+};
+
+// What the correction reads of a joint and does not change, loaded ahead of its turn.
+struct JointPos {
+    int2 bodies;
+    int fl;              // the violation bits may be old: they are found anew
+    V3 la, ax;           // this side's anchor and axis
+    Q4 qinit;
+    float4 lim;
+};
+__device__ __forceinline__ JointPos jt_position_load(const DevJoints& J, int j, int side) {
+    JointPos p;
+    p.bodies = J.bodies[j];
+    p.fl = J.flags[j];
+    p.la = side ? ld3(J.la2, j) : ld3(J.la1, j);
+    p.ax = side ? ld3(J.ax2, j) : ld3(J.ax1, j);
+    p.qinit = ldq(J.qinit, j);
+    p.lim = J.lim[j];
+    return p;
+}
+
+__device__ __forceinline__ float pair_other(float a) { return dpp<kQuadOther>(a); }
+__device__ __forceinline__ float pair_from1(float a) { return dpp<kQuadFrom1>(a); }
+__device__ __forceinline__ float pair_from2(float a) { return dpp<kQuadFrom2>(a); }
+__device__ __forceinline__ Q4 pair_from1(Q4 a) { return q4(dpp<kQuadFrom1>(a.x), dpp<kQuadFrom1>(a.y), dpp<kQuadFrom1>(a.z), dpp<kQuadFrom1>(a.w)); }
+__device__ __forceinline__ Q4 pair_from2(Q4 a) { return q4(dpp<kQuadFrom2>(a.x), dpp<kQuadFrom2>(a.y), dpp<kQuadFrom2>(a.z), dpp<kQuadFrom2>(a.w)); }
+__device__ __forceinline__ M3 pair_from1(const M3& a) { M3 m; for (int i = 0; i < 3; i++) m.r[i] = pair_from1(a.r[i]); return m; }
+__device__ __forceinline__ M3 pair_from2(const M3& a) { M3 m; for (int i = 0; i < 3; i++) m.r[i] = pair_from2(a.r[i]); return m; }
+
+struct JointSide {
+    V3 x, r, iml, al;   // position, lever arm; inverse mass x linear lock factors, angular lock factors
+    Q4 q;
+    M3 I;
+    unsigned int s1, s2;
+};
+__device__ __forceinline__ void side_turn(JointSide& b, V3 angular) { b.q = nudge(b.q, cmul(b.al, mvmul(b.I, angular))); }
+
+// x2 + r2 - x1 - r1
+__device__ __forceinline__ V3 side_gap(const JointSide& b) {
+    return pair_from2(b.x + b.r) - pair_from1(b.x) - pair_from1(b.r);
+}
+
+// the three point-to-point rows
+__device__ __forceinline__ void side_translation(JointSide& b, float imsum, bool anyDyn) {
+    const M3 U = skew(b.r);
+    const M3 A = mmul(mmul(U, b.I), mtranspose(U));
+    const M3 K = madd(madd(m3(imsum, 0, 0, 0, imsum, 0, 0, 0, imsum), pair_from1(A)), pair_from2(A));
+    const float det = mdet(K);
+    if (fabsf(det) > kMachineEps) {
+        const M3 Kt = anyDyn ? minv(K, det) : mzero();
+        const V3 lam = mvmul(Kt, -side_gap(b));
+        const V3 turn = flip3(cross(lam, b.r), b.s2);
+        b.x += lock_mul(b.iml, flip3(lam, b.s1));
+        side_turn(b, turn);
+    }
+}
+
+// the three rotation rows of a fixed or slider joint
+__device__ __forceinline__ void side_rotation(JointSide& b, Q4 qinit, bool anyDyn) {
+    M3 Kr = madd(pair_from1(b.I), pair_from2(b.I));
+    const float det = mdet(Kr);
+    if (fabsf(det) > kMachineEps) {
+        if (anyDyn) Kr = minv(Kr, det);
+        const Q4 qe = qmul(qmul(pair_from2(b.q), qinit), qconj(pair_from1(b.q)));
+        const V3 er = 2.0f * v3(qe.x, qe.y, qe.z);
+        side_turn(b, flip3(mvmul(Kr, -er), b.s1));
+    }
+}
+
+// B: the batch's bodies (absolute indices); P: their positions; kind: the joint kind of the slot (uniform)
+template <bool STAGED>
+__device__ __forceinline__ void jt_solve_position_pair(const DevBodies& B, const PosBodies<STAGED>& P, const DevJoints& J,
+                                                       int kind, int j, int side, const JointPos& p) {
+    const int b1 = p.bodies.x, bi = side ? p.bodies.y : b1, u = bi - P.base;
+    const int fo = P.body_flags(u), fa = fo | P.body_flags((side ? b1 : p.bodies.y) - P.base);
+    if (!(fa & BF_ENABLED)) return;
+    // only non-linear Gauss-Seidel joints (SolveBallAndSocketJointSystem.cpp:309,
+    // SolveFixedJointSystem.cpp:299, SolveHingeJointSystem.cpp:479); the slider system stops at its
+    // first Baumgarte joint (SolveSliderJointSystem.cpp:527)
+    int fl = p.fl;
+    if (fl & JF_BAUMGARTE) return;
+    if (kind == JT_SLIDER && J.bfirst && J.srank[j] >= J.bfirst[B.world[b1]]) return;
+    const bool anyDyn = (fa & BF_DYNAMIC) != 0;
+    const float4 ii = P.ii[u];
+    JointSide b;
+    b.x = ld3(P.x, u);
+    b.q = ldq(P.q, u);
+    V3 ll = v3(1.0f, 1.0f, 1.0f);
+    b.al = ll;
+    if (!(fo & BF_UNIT_LOCKS)) {
+        ll = ld3(B.llock, bi);
+        b.al = ld3(B.alock, bi);
+    }
+    b.iml = ii.w * ll;
+    b.s1 = side ? 0u : 0x80000000u;
+    b.s2 = side ? 0x80000000u : 0u;
+    b.I = world_inv_inertia(qmat(b.q), v3(ii.x, ii.y, ii.z));
+    b.r = qrot(b.q, p.la - ld3(P.com, u));
+    const float ims = ii.w + pair_other(ii.w);
+    if (kind == JT_BALLSOCKET) {   // SolveBallAndSocketJointSystem.cpp:312-445
+        if (fl & JF_LIMIT) {
+            const V3 ru = flip3(unit(b.r), b.s2);
+            const V3 r1u = pair_from1(ru), r2u = pair_from2(ru);
+            const V3 acb = cross(r1u, r2u);
+            const float err = p.lim.x - ref_acosf(dot(r1u, r2u));
+            fl = err < 0.0f ? (fl | JF_LOWER_VIOLATED) : (fl & ~JF_LOWER_VIOLATED);
+            if (side) J.flags[j] = fl;
+            if (fl & JF_LOWER_VIOLATED) {
+                const float d = dot(acb, mvmul(b.I, acb));
+                const float m = d + pair_other(d);
+                const float l = (m > 0.0f ? 1.0f / m : 0.0f) * (-err);
+                side_turn(b, flip(l, b.s2) * acb);
             }
-            bool ok;
-            const M3 Kt = translation_inverse_mass(im1 + im2, r1, r2, I1, I2, anyDyn, ok);
-            if (ok) {
-                const V3 err = x2 + r2 - x1 - r1;
-                const V3 lam = mvmul(Kt, -err);
-                const V3 li1 = -lam;
-                const V3 ai1 = cross(lam, r1);
-                const V3 dv1 = lock_mul((im1 * ll1), li1);
-                const V3 dw1 = cmul(al1, mvmul(I1, ai1));
-                x1 += dv1;
-                q1 = nudge(q1, dw1);
-                const V3 ai2 = -cross(lam, r2);
-                const V3 dv2 = lock_mul((im2 * ll2), lam);
-                const V3 dw2 = cmul(al2, mvmul(I2, ai2));
-                x2 += dv2;
-                q2 = nudge(q2, dw2);
-            }
-        } else if (type == JT_FIXED) {   // SolveFixedJointSystem.cpp:266-448
-            bool ok;
-            const M3 Kt = translation_inverse_mass(im1 + im2, r1, r2, I1, I2, anyDyn, ok);
-            if (ok) {
-                const V3 err = x2 + r2 - x1 - r1;
-                const V3 lam = mvmul(Kt, -err);
-                const V3 li1 = -lam;
-                const V3 ai1 = cross(lam, r1);
-                const V3 dv1 = lock_mul((im1 * ll1), li1);
-                const V3 dw1 = cmul(al1, mvmul(I1, ai1));
-                x1 += dv1;
-                q1 = nudge(q1, dw1);
-                const V3 ai2 = -cross(lam, r2);
-                const V3 dv2 = lock_mul((im2 * ll2), lam);
-                const V3 dw2 = cmul(al2, mvmul(I2, ai2));
-                x2 += dv2;
-                q2 = nudge(q2, dw2);
-            }
-            M3 Kr = madd(I1, I2);
-            const float det = mdet(Kr);
-            if (fabsf(det) > kMachineEps) {
-                if (anyDyn) Kr = minv(Kr, det);
-                const Q4 qe = qmul(qmul(q2, ldq(J.qinit, j)), qconj(q1));
-                const V3 er = 2.0f * v3(qe.x, qe.y, qe.z);
-                const V3 lr = mvmul(Kr, -er);
-                const V3 ai1 = -lr;
-                const V3 dw1 = cmul(al1, mvmul(I1, ai1));
-                q1 = nudge(q1, dw1);
-                const V3 dw2 = cmul(al2, mvmul(I2, lr));
-                q2 = nudge(q2, dw2);
-            }
-        } else if (type == JT_HINGE) {   // SolveHingeJointSystem.cpp:444-730
-            V3 a1 = normalized(qrot(q1, ld3(J.ax1, j)));
-            const V3 a2 = normalized(qrot(q2, ld3(J.ax2, j)));
-            const V3 b2v = one_unit_orthogonal(a2);
-            const V3 c2v = cross(a2, b2v);
-            const V3 bxa = cross(b2v, a1), cxa = cross(c2v, a1);
+        }
+        side_translation(b, ims, anyDyn);
+    } else if (kind == JT_FIXED) {   // SolveFixedJointSystem.cpp:266-448
+        side_translation(b, ims, anyDyn);
+        side_rotation(b, p.qinit, anyDyn);
+    } else if (kind == JT_HINGE) {   // SolveHingeJointSystem.cpp:444-730
+        const V3 a = normalized(qrot(b.q, p.ax));
+        const V3 a1 = pair_from1(a), a2 = pair_from2(a);
+        const V3 b2v = one_unit_orthogonal(a2);
+        const V3 c2v = cross(a2, b2v);
+        const V3 bxa = cross(b2v, a1), cxa = cross(c2v, a1);
+        if (side) {
             J.a1[j] = f4(a1, 0.f);
             J.b2xa1[j] = f4(bxa, 0.f);
             J.c2xa1[j] = f4(cxa, 0.f);
-            int fl = J.flags[j];
-            const float4 lim = J.lim[j];
-            if (fl & (JF_LIMIT | JF_MOTOR)) {
-                const float ang = hinge_angle(q1, q2, ldq(J.qinit, j), a1, lim.x, lim.y);
-                const float le = ang - lim.x, ue = lim.y - ang;
-                fl = le <= 0 ? (fl | JF_LOWER_VIOLATED) : (fl & ~JF_LOWER_VIOLATED);
-                fl = ue <= 0 ? (fl | JF_UPPER_VIOLATED) : (fl & ~JF_UPPER_VIOLATED);
-                J.flags[j] = fl;
-                if (fl & JF_LIMIT) {
-                    const float imlm_old = J.imlm[j];
-                    if (fl & (JF_LOWER_VIOLATED | JF_UPPER_VIOLATED)) {
-                        const float m = dot(a1, mvmul(I1, a1)) + dot(a1, mvmul(I2, a1));
-                        J.imlm[j] = imlm_old > 0.0f ? 1.0f / m : 0.0f;   // reference tests the old value
-                    }
-                    if (fl & JF_LOWER_VIOLATED) {
-                        const float l = imlm_old * (-le);
-                        q1 = nudge(q1, cmul(al1, mvmul(I1, (-l) * a1)));
-                        q2 = nudge(q2, cmul(al2, mvmul(I2, l * a1)));
-                    }
-                    if (fl & JF_UPPER_VIOLATED) {
-                        const float l = imlm_old * (-ue);
-                        q1 = nudge(q1, cmul(al1, mvmul(I1, l * a1)));
-                        q2 = nudge(q2, cmul(al2, mvmul(I2, (-l) * a1)));
-                    }
-                }
-            }
-            const V3 i1b = mvmul(I1, bxa), i1c = mvmul(I1, cxa), i2b = mvmul(I2, bxa), i2c = mvmul(I2, cxa);
-            const float e11 = dot(bxa, i1b) + dot(bxa, i2b);
-            const float e12 = dot(bxa, i1c) + dot(bxa, i2c);
-            const float e21 = dot(cxa, i1b) + dot(cxa, i2b);
-            const float e22 = dot(cxa, i1c) + dot(cxa, i2c);
-            const float det = e11 * e22 - e21 * e12;
-            if (fabsf(det) > kMachineEps) {
-                float k00 = 0, k01 = 0, k10 = 0, k11 = 0;
-                if (anyDyn) {
-                    const float id = 1.0f / det;
-                    k00 = e22 * id; k01 = -e12 * id; k10 = -e21 * id; k11 = e11 * id;
-                }
-                const float er0 = dot(a1, b2v), er1 = dot(a1, c2v);
-                const float x0 = -er0, x1v = -er1;
-                const float l0 = k00 * x0 + k01 * x1v;
-                const float l1 = k10 * x0 + k11 * x1v;
-                const V3 ai1 = (-bxa) * l0 - cxa * l1;
-                q1 = nudge(q1, cmul(al1, mvmul(I1, ai1)));
-                const V3 ai2 = bxa * l0 + cxa * l1;
-                q2 = nudge(q2, cmul(al2, mvmul(I2, ai2)));
-            }
-            bool ok;
-            const M3 Kt = translation_inverse_mass(im1 + im2, r1, r2, I1, I2, anyDyn, ok);
-            if (ok) {
-                const V3 err = x2 + r2 - x1 - r1;
-                const V3 lam = mvmul(Kt, -err);
-                const V3 li1 = -lam;
-                const V3 ai1 = cross(lam, r1);
-                const V3 dv1 = lock_mul((im1 * ll1), li1);
-                const V3 dw1 = cmul(al1, mvmul(I1, ai1));
-                x1 += dv1;
-                q1 = nudge(q1, dw1);
-                const V3 ai2 = -cross(lam, r2);
-                const V3 dv2 = lock_mul((im2 * ll2), lam);
-                const V3 dw2 = cmul(al2, mvmul(I2, ai2));
-                x2 += dv2;
-                q2 = nudge(q2, dw2);
-            }
-        } else {   // slider, SolveSliderJointSystem.cpp:514-826
-            const V3 u = x2 + r2 - x1 - r1;
-            const V3 ax = normalized(qrot(q1, ld3(J.ax1, j)));
-            const V3 n1 = one_unit_orthogonal(ax);
-            const V3 n2 = cross(ax, n1);
-            const float4 lim = J.lim[j];
-            const float ud = dot(u, ax);
-            int fl = J.flags[j];
-            fl = (ud - lim.x) <= 0 ? (fl | JF_LOWER_VIOLATED) : (fl & ~JF_LOWER_VIOLATED);
-            fl = (lim.y - ud) <= 0 ? (fl | JF_UPPER_VIOLATED) : (fl & ~JF_UPPER_VIOLATED);
-            J.flags[j] = fl;
-            const V3 rn1 = cross(r2, n1), rn2 = cross(r2, n2), ra = cross(r2, ax);
-            J.ra[j] = f4(ra, 0.f);   // read by the next step's limit inverse mass
-            const V3 rpu = r1 + u;
-            const V3 un1 = cross(rpu, n1), un2 = cross(rpu, n2), ua = cross(rpu, ax);
-            const float ims = im1 + im2;
-            if (fl & JF_LIMIT) {
-                float imlm = J.imlm[j];
-                if (fl & (JF_LOWER_VIOLATED | JF_UPPER_VIOLATED)) {
-                    const float m = ims + dot(ua, mvmul(I1, ua)) + dot(ra, mvmul(I2, ra));
-                    imlm = m > 0.0f ? 1.0f / m : 0.0f;
-                    J.imlm[j] = imlm;
-                }
-                if (fl & JF_LOWER_VIOLATED) {
-                    const float err = dot(x2 + r2 - x1 - r1, ax) - lim.x;
-                    const float l = imlm * (-err);
-                    x1 += lock_mul((im1 * ll1), (-l) * ax);
-                    q1 = nudge(q1, cmul(al1, mvmul(I1, (-l) * ua)));
-                    x2 += lock_mul((im2 * ll2), l * ax);
-                    q2 = nudge(q2, cmul(al2, mvmul(I2, l * ra)));
-                }
-                if (fl & JF_UPPER_VIOLATED) {
-                    const float err = lim.y - dot(x2 + r2 - x1 - r1, ax);
-                    const float l = imlm * (-err);
-                    x1 += lock_mul((im1 * ll1), l * ax);
-                    q1 = nudge(q1, cmul(al1, mvmul(I1, l * ua)));
-                    x2 += lock_mul((im2 * ll2), (-l) * ax);
-                    q2 = nudge(q2, cmul(al2, mvmul(I2, (-l) * ra)));
-                }
-            }
-            // 3 rotation rows
-            M3 Kr = madd(I1, I2);
-            const float detr = mdet(Kr);
-            if (fabsf(detr) > kMachineEps) {
-                if (anyDyn) Kr = minv(Kr, detr);
-                const Q4 qe = qmul(qmul(q2, ldq(J.qinit, j)), qconj(q1));
-                const V3 er = 2.0f * v3(qe.x, qe.y, qe.z);
-                const V3 lr = mvmul(Kr, -er);
-                q1 = nudge(q1, cmul(al1, mvmul(I1, -lr)));
-                q2 = nudge(q2, cmul(al2, mvmul(I2, lr)));
-            }
-            // 2 translation rows (with u and the cross products from before the corrections above)
-            const V3 i1n1 = mvmul(I1, un1), i1n2 = mvmul(I1, un2), i2n1 = mvmul(I2, rn1), i2n2 = mvmul(I2, rn2);
-            const float e11 = ims + dot(un1, i1n1) + dot(rn1, i2n1);
-            const float e12 = dot(un1, i1n2) + dot(rn1, i2n2);
-            const float e21 = dot(un2, i1n1) + dot(rn2, i2n1);
-            const float e22 = ims + dot(un2, i1n2) + dot(rn2, i2n2);
-            const float det = e11 * e22 - e21 * e12;
-            if (fabsf(det) > kMachineEps) {
-                float k00 = 0, k01 = 0, k10 = 0, k11 = 0;
-                if (anyDyn) {
-                    const float id = 1.0f / det;
-                    k00 = e22 * id; k01 = -e12 * id; k10 = -e21 * id; k11 = e11 * id;
-                }
-                const float t0 = -dot(u, n1), t1 = -dot(u, n2);
-                const float l0 = k00 * t0 + k01 * t1;
-                const float l1 = k10 * t0 + k11 * t1;
-                const V3 li1 = (-n1) * l0 - n2 * l1;
-                const V3 ai1 = (-un1) * l0 - un2 * l1;
-                x1 += lock_mul((im1 * ll1), li1);
-                q1 = nudge(q1, cmul(al1, mvmul(I1, ai1)));
-                const V3 li2 = n1 * l0 + n2 * l1;
-                const V3 ai2 = rn1 * l0 + rn2 * l1;
-                x2 += lock_mul((im2 * ll2), li2);
-                q2 = nudge(q2, cmul(al2, mvmul(I2, ai2)));
+        }
+        if (fl & (JF_LIMIT | JF_MOTOR)) {
+            const float ang = hinge_angle(pair_from1(b.q), pair_from2(b.q), p.qinit, a1, p.lim.x, p.lim.y);
+            const float le = ang - p.lim.x, ue = p.lim.y - ang;
+            fl = le <= 0 ? (fl | JF_LOWER_VIOLATED) : (fl & ~JF_LOWER_VIOLATED);
+            fl = ue <= 0 ? (fl | JF_UPPER_VIOLATED) : (fl & ~JF_UPPER_VIOLATED);
+            if (side) J.flags[j] = fl;
+            if ((fl & JF_LIMIT) && (fl & (JF_LOWER_VIOLATED | JF_UPPER_VIOLATED))) {
+                const float imlm_old = J.imlm[j];
+                const float d = dot(a1, mvmul(b.I, a1));
+                const float m = pair_from1(d) + pair_from2(d);
+                if (side) J.imlm[j] = imlm_old > 0.0f ? 1.0f / m : 0.0f;   // reference tests the old value
+                if (fl & JF_LOWER_VIOLATED) side_turn(b, flip(imlm_old * (-le), b.s1) * a1);
+                if (fl & JF_UPPER_VIOLATED) side_turn(b, flip(imlm_old * (-ue), b.s2) * a1);
             }
         }
-        B.cx[b1] = f4(x1, 0.f); B.cq[b1] = f4q(q1);
-        B.cx[b2] = f4(x2, 0.f); B.cq[b2] = f4q(q2);
+        const V3 ib = mvmul(b.I, bxa), ic = mvmul(b.I, cxa);
+        const float d11 = dot(bxa, ib), d12 = dot(bxa, ic), d21 = dot(cxa, ib), d22 = dot(cxa, ic);
+        const float e11 = d11 + pair_other(d11);
+        const float e12 = d12 + pair_other(d12);
+        const float e21 = d21 + pair_other(d21);
+        const float e22 = d22 + pair_other(d22);
+        const float det = e11 * e22 - e21 * e12;
+        if (fabsf(det) > kMachineEps) {
+            float k00 = 0, k01 = 0, k10 = 0, k11 = 0;
+            if (anyDyn) {
+                const float id = 1.0f / det;
+                k00 = e22 * id; k01 = -e12 * id; k10 = -e21 * id; k11 = e11 * id;
+            }
+            const float x0 = -dot(a1, b2v), x1 = -dot(a1, c2v);
+            const float l0 = k00 * x0 + k01 * x1;
+            const float l1 = k10 * x0 + k11 * x1;
+            side_turn(b, flip3(bxa, b.s1) * l0 + flip3(cxa, b.s1) * l1);
+        }
+        side_translation(b, ims, anyDyn);
+    } else {   // slider, SolveSliderJointSystem.cpp:514-826
+        const V3 u21 = side_gap(b);
+        const V3 ax = pair_from1(normalized(qrot(b.q, p.ax)));
+        const V3 n1 = one_unit_orthogonal(ax);
+        const V3 n2 = cross(ax, n1);
+        const float ud = dot(u21, ax);
+        fl = (ud - p.lim.x) <= 0 ? (fl | JF_LOWER_VIOLATED) : (fl & ~JF_LOWER_VIOLATED);
+        fl = (p.lim.y - ud) <= 0 ? (fl | JF_UPPER_VIOLATED) : (fl & ~JF_UPPER_VIOLATED);
+        const V3 arm = side ? b.r : b.r + u21;   // r2, r1 + u
+        const V3 m1 = cross(arm, n1), m2 = cross(arm, n2), ma = cross(arm, ax);
+        if (side) {
+            J.flags[j] = fl;
+            J.ra[j] = f4(ma, 0.f);   // read by the next step's limit inverse mass
+        }
+        if ((fl & JF_LIMIT) && (fl & (JF_LOWER_VIOLATED | JF_UPPER_VIOLATED))) {
+            const float d = dot(ma, mvmul(b.I, ma));
+            const float m = ims + pair_from1(d) + pair_from2(d);
+            const float imlm = m > 0.0f ? 1.0f / m : 0.0f;
+            if (side) J.imlm[j] = imlm;
+            if (fl & JF_LOWER_VIOLATED) {
+                const float l = flip(imlm * (-(dot(side_gap(b), ax) - p.lim.x)), b.s1);
+                b.x += lock_mul(b.iml, l * ax);
+                side_turn(b, l * ma);
+            }
+            if (fl & JF_UPPER_VIOLATED) {
+                const float l = flip(imlm * (-(p.lim.y - dot(side_gap(b), ax))), b.s2);
+                b.x += lock_mul(b.iml, l * ax);
+                side_turn(b, l * ma);
+            }
+        }
+        side_rotation(b, p.qinit, anyDyn);
+        // 2 translation rows (with u and the cross products from before the corrections above)
+        const V3 i1 = mvmul(b.I, m1), i2 = mvmul(b.I, m2);
+        const float d11 = dot(m1, i1), d12 = dot(m1, i2), d21 = dot(m2, i1), d22 = dot(m2, i2);
+        const float e11 = ims + pair_from1(d11) + pair_from2(d11);
+        const float e12 = d12 + pair_other(d12);
+        const float e21 = d21 + pair_other(d21);
+        const float e22 = ims + pair_from1(d22) + pair_from2(d22);
+        const float det = e11 * e22 - e21 * e12;
+        if (fabsf(det) > kMachineEps) {
+            float k00 = 0, k01 = 0, k10 = 0, k11 = 0;
+            if (anyDyn) {
+                const float id = 1.0f / det;
+                k00 = e22 * id; k01 = -e12 * id; k10 = -e21 * id; k11 = e11 * id;
+            }
+            const float t0 = -dot(u21, n1), t1 = -dot(u21, n2);
+            const float l0 = k00 * t0 + k01 * t1;
+            const float l1 = k10 * t0 + k11 * t1;
+            b.x += lock_mul(b.iml, flip3(n1, b.s1) * l0 + flip3(n2, b.s1) * l1);
+            side_turn(b, flip3(m1, b.s1) * l0 + flip3(m2, b.s1) * l1);
+        }
     }
+    P.x[u] = f4(b.x, STAGED ? __int_as_float(fo) : 0.f);
+    P.q[u] = f4q(b.q);
 }
 
 }  // namespace rp3dg

@@ -43,6 +43,7 @@ __device__ __forceinline__ float dpp(float x) {
 }
 constexpr int kQuadFrom1 = 0 | 0 << 2 | 2 << 4 | 2 << 6;   // body 1's lane of the same half
 constexpr int kQuadFrom2 = 1 | 1 << 2 | 3 << 4 | 3 << 6;   // body 2's lane of the same half
+constexpr int kQuadOther = 1 | 0 << 2 | 3 << 4 | 2 << 6;   // the other body's lane of the same half
 constexpr int kQuadLow = 0 | 1 << 2 | 0 << 4 | 1 << 6;     // the velocity lane of the same body
 constexpr int kQuadHigh = 2 | 3 << 2 | 2 << 4 | 3 << 6;    // the split lane of the same body
 template <int K>
