@@ -144,7 +144,6 @@ struct rp3dg_batch {
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     hipGraph_t graph[2] = {nullptr, nullptr};
     float graph_dt = 0.0f;
-    int graph_rounds = 0;
 
     // hull arena
     rp3dg::HullHeader* d_hulls = nullptr;

@@ -1407,15 +1407,14 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         fill_int<<<grid_for(nb), 256, 0, stream>>>(adj_cursor, nb, 0);
         LAUNCH_T("sv_adj_fill", mg, 256, sv_adj_fill, B, C, N, m_list, nm_ptr, adj_offs, adj_cursor, adj, mb);
         fill_int_n<<<mg, 256, 0, stream>>>(color, man_cap, nm_ptr, -1);
-        const int rounds = capturing ? graph_rounds : std::min(kColorRoundsMax, std::max(4, hint_rounds));
+        const int rounds = std::min(kColorRoundsMax, std::max(2, hint_rounds));
         for (int q = 0; q < rounds; q++)
             LAUNCH_T("sv_color_round", mg, 256, sv_color_round, mb, nm_ptr, adj_offs, adj, color,
                      q ? &counters->color_left[q - 1] : nullptr, &counters->color_left[q], dstatus);
         LAUNCH_T("sv_color_finish", 1, 1024, sv_color_finish, mb, nm_ptr, adj_offs, adj, color,
                  rounds ? &counters->color_left[rounds - 1] : nullptr, &counters->finish_rounds, dstatus);
         fill_int<<<grid_for(nseg + 1), 256, 0, stream>>>(seg_cnt, nseg + 1, 0);
-        LAUNCH_T("sv_color_keys", mg, 256, sv_color_keys, color, nm_ptr, C, N, m_list, nullptr, ckeys, cvals, seg_cnt,
-                 &counters->nb_colors);
+        LAUNCH_T("sv_color_keys", mg, 256, sv_color_keys, color, nm_ptr, ckeys, cvals, seg_cnt, &counters->nb_colors);
         int sbits = 0;
         while ((1 << sbits) < nseg) sbits++;
         timer_begin("sv_color_sort");
@@ -1680,7 +1679,6 @@ int rp3dg_batch::step_graph(float dt, int n) {
     }
     if (graph_exec[0] && graph_dt != dt) drop_graphs();
     if (!graph_exec[0]) {
-        graph_rounds = std::min(kColorRoundsMax, std::max(8, hint_rounds + 4));
         const bool start = cur_is_a;
         for (int p = 0; p < 2; p++) {
             const int parity = start == (p == 0) ? 0 : 1;   // parity 0: a -> b

@@ -224,7 +224,7 @@ struct DevCounters {
     int status;
     int finish_rounds;         // rounds taken by the single-workgroup colouring finisher
     int nb_new_points;         // contact points without a cached impulse
-    int color_left[kColorRoundsMax];   // manifolds still uncoloured after each parallel round
+    int color_left[kColorRoundsMax];   // set: manifolds left uncoloured by each colouring launch
     int nb_box_tests;          // box-box subset of nb_tests[ALGO_POLY_POLY] that collided last step
     int nb_box_sep_tests;      // box-box pairs that did not (cheap temporal-coherence rejects, listed apart)
     int nb_hull_tests;         // the rest of nb_tests[ALGO_POLY_POLY] (a convex mesh involved)

@@ -58,8 +58,7 @@ __host__ __device__ constexpr int color_body_bytes(int bodies) { return bodies *
 __host__ __device__ constexpr int color_manifold_bytes(int m) { return m * 8 + (m + 15) / 16 * 4; }
 
 __global__ void sv_group_color(ColorArgs A);
-__global__ void sv_color_keys(const int* color, const int* nm_ptr, DevColliders C, DevPairs P, const int* mlist,
-                              const int* world_group, uint64_t* keys, int* vals, int* seg_cnt, int* ncolors);
+__global__ void sv_color_keys(const int* color, const int* nm_ptr, uint64_t* keys, int* vals, int* seg_cnt, int* ncolors);
 __global__ void sv_warmstart(SvArgs A, int color);
 template <bool SPLIT>
 __global__ void sv_solve_color(SvArgs A, int color, float beta_dt);   // one quad of lanes per manifold

@@ -137,6 +137,12 @@ __device__ __forceinline__ bool higher(uint32_t a, uint32_t b) {  // priority of
 // Tries to colour manifold m (color[m] == -1 while uncoloured).  Returns false when a
 // higher-priority neighbour is still uncoloured.  A neighbour coloured concurrently is read either
 // as -1 or as its final colour, so the result does not depend on timing.
+__device__ __forceinline__ void jp_choose(int m, uint64_t used, int* color, int* status) {
+    const uint64_t freem = ~used;
+    int c = freem ? __ffsll((unsigned long long)freem) - 1 : 64;
+    if (c >= kMaxColors) { atomicOr(status, STATUS_COLOR_OVERFLOW); c = kMaxColors - 1; }
+    __atomic_store_n(&color[m], c, __ATOMIC_RELAXED);
+}
 __device__ __forceinline__ bool jp_try(int m, const int2* mb, const int* offs, const int* adj, int* color, int* status) {
     const int2 bb = mb[m];
     uint64_t used = 0;
@@ -154,25 +160,77 @@ __device__ __forceinline__ bool jp_try(int m, const int2* mb, const int* offs, c
             }
         }
     }
-    const uint64_t freem = ~used;
-    int c = freem ? __ffsll((unsigned long long)freem) - 1 : 64;
-    if (c >= kMaxColors) { atomicOr(status, STATUS_COLOR_OVERFLOW); c = kMaxColors - 1; }
-    __atomic_store_n(&color[m], c, __ATOMIC_RELAXED);
+    jp_choose(m, used, color, status);
     return true;
 }
 
-// One parallel round; left_prev = manifolds left after the previous round (nullptr for the first).
-__global__ void sv_color_round(const int2* mb, const int* nm_ptr, const int* offs, const int* adj, int* color,
-                               const int* left_prev, int* left, int* status) {
+// One launch colours as far as the waiting goes; left[0] != 0 afterwards if manifolds are left
+// (left_prev: the last launch's, nullptr for the first).
+//
+// A manifold waits for the neighbours of higher priority, and the longest such chain is some 25 manifolds.
+// A launch per link of that chain, each looking at every neighbour of every manifold that is left, took 26 us
+// a launch (65,536-body heap, 120,000 manifolds, 25 launches) and 13 us (6,000 hulls, 20).  Here a lane walks
+// its manifold's neighbours once, eight at a time, and stays at eight while one of them has no colour yet:
+// a link costs a store and a load that reaches it, and one launch does nearly all (114 and 77 us, and an
+// empty launch to confirm it).  The lanes of a wavefront step together, so none keeps another from going on, and a wavefront gives up after kColorPolls steps in
+// which none of its lanes got further: nothing depends on workgroups running side by side.
+constexpr int kColorPolls = 48, kColorChunk = 8;
+__global__ __launch_bounds__(256) void sv_color_round(const int2* mb, const int* nm_ptr, const int* offs, const int* adj,
+                                                      int* color, const int* left_prev, int* left, int* status) {
     if (left_prev && *left_prev == 0) return;
     const int nm = *nm_ptr;
-    int n_left = 0;
-    RP3DG_GRID_STRIDE(m, nm) {
-        if (color[m] >= 0) continue;
-        if (!jp_try(m, mb, offs, adj, color, status)) n_left++;
+    bool any_left = false;
+    for (int m0 = blockIdx.x * blockDim.x; m0 < nm; m0 += gridDim.x * blockDim.x) {
+        const int m = m0 + threadIdx.x;
+        bool todo = m < nm && color[m] < 0;
+        const int2 bb = todo ? mb[m] : make_int2(-1, -1);
+        // both bodies' lists as one: [k1, e1), then [k2, e2)
+        int k1 = 0, e1 = 0, k2 = 0, e2 = 0;
+        if (bb.x >= 0) { k1 = offs[bb.x]; e1 = offs[bb.x + 1]; }
+        if (bb.y >= 0) { k2 = offs[bb.y]; e2 = offs[bb.y + 1]; }
+        uint64_t used = 0;
+        int wait[kColorChunk];   // neighbours of the current chunk that are waited for, -1: none
+        bool fresh = true;
+        for (int polls = 0; polls < kColorPolls && __any(todo);) {
+            bool moved = false;
+            if (todo) {
+                if (fresh) {
+                    const int n1 = min(kColorChunk, e1 - k1), n = n1 + min(kColorChunk - n1, e2 - k2);
+                    moved = true;
+                    if (n == 0) {
+                        jp_choose(m, used, color, status);
+                        todo = false;
+                    } else {
+                        for (int j = 0; j < kColorChunk; j++) wait[j] = adj[j < n1 ? k1 + j : (n > n1 ? k2 + min(j, n - 1) - n1 : k1 + n1 - 1)];
+                        for (int j = 0; j < kColorChunk; j++)
+                            if (j >= n || !higher((uint32_t)wait[j], (uint32_t)m)) wait[j] = -1;   // (m itself is not higher)
+                        k1 += n1;
+                        k2 += n - n1;
+                        fresh = false;
+                    }
+                }
+                if (todo) {
+                    int co[kColorChunk];
+                    for (int j = 0; j < kColorChunk; j++)
+                        co[j] = wait[j] >= 0 ? __hip_atomic_load(&color[wait[j]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 64;
+                    bool all = true;
+                    for (int j = 0; j < kColorChunk; j++) {
+                        if (co[j] < 0) { all = false; continue; }
+                        if (wait[j] >= 0) moved = true;
+                        wait[j] = -1;
+                        if (co[j] < 64) used |= 1ull << co[j];
+                    }
+                    if (all) fresh = moved = true;
+                }
+            }
+            if (!__any(moved)) {
+                polls++;
+                __builtin_amdgcn_s_sleep(2);
+            }
+        }
+        any_left |= __any(todo) != 0;
     }
-    n_left = wave_sum(n_left);
-    if (lane_id() == 0 && n_left) atomicAdd(left, n_left);
+    if (any_left && lane_id() == 0) *left = 1;   // (a flag: counting on one address would cost more than the round)
 }
 
 // Single workgroup: rounds until every manifold is coloured.  Each round colours at least the
@@ -435,33 +493,27 @@ __global__ __launch_bounds__(1024) void sv_group_color(ColorArgs A) {
 // Segment key of every manifold: its colour, or (world group, colour) when the solver runs one workgroup
 // per group of consecutive worlds (world_group != null).  Counts per segment and the number of colours
 // are accumulated for the segment table.
-__global__ void sv_color_keys(const int* color, const int* nm_ptr, DevColliders C, DevPairs P, const int* mlist,
-                              const int* world_group, uint64_t* keys, int* vals, int* seg_cnt, int* ncolors) {
+__global__ __launch_bounds__(256) void sv_color_keys(const int* color, const int* nm_ptr, uint64_t* keys, int* vals,
+                                                     int* seg_cnt, int* ncolors) {
     __shared__ int hist[kMaxColors];
     for (int i = threadIdx.x; i < kMaxColors; i += blockDim.x) hist[i] = 0;
     __syncthreads();
     const int nm = *nm_ptr;
-    int cmax = -1;
     RP3DG_GRID_STRIDE(m, nm) {
         const int c = color[m];
-        uint64_t seg = (uint64_t)c;
-        if (world_group) {
-            const int g = world_group[C.world[P.col[mlist[m]].x]];
-            seg = (uint64_t)g * kMaxColors + c;
-            atomicAdd(&seg_cnt[seg], 1);
-        } else {
-            atomicAdd(&hist[c], 1);
-        }
-        keys[m] = seg;
+        atomicAdd(&hist[c], 1);
+        keys[m] = (uint64_t)c;
         vals[m] = m;
-        cmax = c > cmax ? c : cmax;
     }
-    cmax = wave_max(cmax);
-    if (lane_id() == 0 && cmax >= 0) atomicMax(ncolors, cmax + 1);
     __syncthreads();
-    if (!world_group)
-        for (int i = threadIdx.x; i < kMaxColors; i += blockDim.x)
-            if (hist[i]) atomicAdd(&seg_cnt[i], hist[i]);
+    // the colours in use, once a workgroup: same-address atomics serialise
+    static_assert(kMaxColors == kWave, "one lane a colour");
+    if (threadIdx.x < kWave) {
+        const int n = hist[threadIdx.x];
+        if (n) atomicAdd(&seg_cnt[threadIdx.x], n);
+        const unsigned long long in_use = __ballot(n != 0);
+        if (threadIdx.x == 0 && in_use) atomicMax(ncolors, 64 - __clzll((long long)in_use));
+    }
 }
 
 }  // namespace rp3dg

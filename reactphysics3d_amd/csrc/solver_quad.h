@@ -251,7 +251,7 @@ __device__ __forceinline__ void quad_sweep_row(const SvArgs& A, const QuadSrc& Q
     const int2 bb = S.bodies[i];
     const int np = S.npts[i];
     QuadRow R;
-    Q.load(i, np, R);
+    Q.load(i, 4, R);   // (all four slots, so that these loads do not wait for np; a row's slots share a line)
     const int b = Q.side ? bb.y : bb.x, u = b - A.B.vbase;
     float4 lam = S.lq[2 * (size_t)i + Q.part];
     V3 imp = ld3(S.imp, i);
