@@ -1514,9 +1514,8 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     LAUNCH_T("sv_setup", grid_for(nb + hm + J.n + 128), 256, sv_setup, SA, J, settings, dt);
     // contact solver (PhysicsWorld.cpp:321-345)
     const int jg = grid_for(std::max(J.n, 1)), jg2 = grid_for(std::max(2 * J.n, 1));
-    const int cg = grid_for(hm / std::max(1, ncol) + 1, color_block);
     const int qg = grid_for(4 * (hm / std::max(1, ncol) + 1), color_block);
-    for (int c = 0; c < ncol; c++) LAUNCH_T("sv_warmstart", cg, color_block, sv_warmstart, SA, c);
+    for (int c = 0; c < ncol; c++) LAUNCH_T("sv_warmstart", qg, color_block, sv_warmstart, SA, c);
     // ConstraintSolverSystem::initialize: warm start of every joint kind
     for (int s = 0; s < jt_slots; s++) LAUNCH_T("jt_warmstart", jg, 256, jt_warmstart, B, J, jt_ranges, s);
     for (int it = 0; it < settings.vel_iters; it++) {

@@ -240,10 +240,13 @@ __global__ __launch_bounds__(kFusedMaxBlock) void sv_world_solve(FusedArgs F) {
     while (nc < kMaxColors && uniform(s_seg[nc]) < m1) nc++;
 
     // ---------------- warm start: contacts colour by colour (CS.cpp:326-476), then joints slot by slot
-    for (int c = 0; c < nc; c++) {
-        const int lo = s_seg[c], hi = s_seg[c + 1];
-        for (int i = lo + tid; i < hi; i += nt) sv_warmstart_one(A, i);
-        phase_barrier<STATE>();
+    {
+        const QuadSrc Q(F.A.S, tid);
+        for (int c = 0; c < nc; c++) {
+            const int lo = s_seg[c], hi = s_seg[c + 1];
+            for (int t = tid; t < 4 * (hi - lo); t += nt) quad_warmstart(A, Q, lo + (t >> 2));
+            phase_barrier<STATE>();
+        }
     }
     bool unit = true;
     for (int i = tid; i < nbw; i += nt) unit = unit && (BS.flags[ub + i] & BF_UNIT_LOCKS);

@@ -28,10 +28,11 @@ __global__ void dyn_update_state(DevBodies B) {
     RP3DG_GRID_STRIDE(i, B.n) dyn_update_state_one(B, i);
 }
 
-__global__ void sv_warmstart(SvArgs A, int color) {
+__global__ __launch_bounds__(512) void sv_warmstart(SvArgs A, int color) {
     if (color >= *A.ncolors) return;
-    const int lo = A.cstart[color], hi = A.cstart[color + 1];
-    RP3DG_GRID_STRIDE(t, hi - lo) sv_warmstart_one(A, lo + t);
+    const int lo = A.cstart[color], n = 4 * (A.cstart[color + 1] - lo);
+    const QuadSrc Q(A.S, threadIdx.x);
+    RP3DG_GRID_STRIDE(t, n) quad_warmstart(A, Q, lo + (t >> 2));
 }
 
 // four lanes a manifold (solver_quad.h)

@@ -251,100 +251,6 @@ __device__ __forceinline__ void load_body(const DevBodies& B, int b, const float
     w = ld3(ang, b);
 }
 
-// ContactSolverSystem::warmStart (CS.cpp:326-476) for the manifolds [lo, hi) of one colour
-__device__ __forceinline__ void sv_warmstart_one(const SvArgs& A, int i) {
-    {
-        const DevBodies& B = A.B;
-        const DevSolver& S = A.S;
-        const int2 bb = S.bodies[i];
-        const int b1 = bb.x, b2 = bb.y;
-        const bool d1 = dyn_body(B, b1), d2 = dyn_body(B, b2);
-        const int u1 = b1 - B.vbase, u2 = b2 - B.vbase;
-        V3 v1 = ld3(B.cv, u1), w1 = ld3(B.cw, u1), v2 = ld3(B.cv, u2), w2 = ld3(B.cw, u2);
-        const float im1 = S.r1f[i].w, im2 = S.r2f[i].w;
-        V3 ll1, al1, ll2, al2;
-        body_locks(B, b1, ll1, al1);
-        body_locks(B, b2, ll2, al2);
-        const int np = S.npts[i];
-        const M3 I1 = body_iw(B, b1), I2 = body_iw(B, b2);
-        float* lq = reinterpret_cast<float*>(S.lq + 2 * (size_t)i);
-        S.lq[2 * (size_t)i + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
-        bool any = false;
-        float plx = 0.0f, ply = 0.0f;   // learned friction impulses summed over the new points
-        for (int p = 0; p < np; p++) {
-            const int q = 4 * i + p;
-            const float4 lam4 = S.lam[q];
-            if (lam4.z != 0.0f || A.learned) {
-                float lam;
-                if (lam4.z != 0.0f) {
-                    any = true;
-                    lam = lam4.x;
-                } else {   // learned warm start of a point with no cached impulse
-                    const float4 pr = S.pred[q];
-                    lam = fmax_s(pr.x, 0.0f);
-                    plx += pr.y;
-                    ply += pr.z;
-                }
-                lq[p] = lam;
-                const V3 n = xyz(S.pn[q]);
-                const V3 i1n = ld3(S.i1, q), i2n = ld3(S.i2, q);
-                const V3 ip = v3(n.x * lam, n.y * lam, n.z * lam);
-                v1.x -= im1 * ip.x * ll1.x; v1.y -= im1 * ip.y * ll1.y; v1.z -= im1 * ip.z * ll1.z;
-                w1.x -= i1n.x * al1.x * lam; w1.y -= i1n.y * al1.y * lam; w1.z -= i1n.z * al1.z * lam;
-                v2.x += im2 * ip.x * ll2.x; v2.y += im2 * ip.y * ll2.y; v2.z += im2 * ip.z * ll2.z;
-                w2.x += i2n.x * al2.x * lam; w2.y += i2n.y * al2.y * lam; w2.z += i2n.z * al2.z * lam;
-            } else {
-                lq[p] = 0.0f;
-            }
-        }
-        float4 imp = S.imp[i];
-        // learned friction only for a manifold with no resting point (the reference then starts from zero)
-        const bool learned_friction = !any && A.learned && np > 0;
-        if (any || learned_friction) {
-            const V3 t1 = ld3(S.t1, i), t2 = ld3(S.t2, i);
-            if (any) {
-                const V3 ot1 = ld3(S.oldt1, i), ot2 = ld3(S.oldt2, i);
-                const V3 oi = v3(imp.x * ot1.x + imp.y * ot2.x, imp.x * ot1.y + imp.y * ot2.y, imp.x * ot1.z + imp.y * ot2.z);
-                imp.x = dot(oi, t1);
-                imp.y = dot(oi, t2);
-            } else {
-                imp.x = plx;
-                imp.y = ply;
-                imp.z = 0.0f;
-            }
-            const V3 r1f = ld3(S.r1f, i), r2f = ld3(S.r2f, i);
-            const V3 r1ct1 = cross(r1f, t1), r2ct1 = cross(r2f, t1), r1ct2 = cross(r1f, t2), r2ct2 = cross(r2f, t2);
-            V3 a1 = v3(-r1ct1.x * imp.x, -r1ct1.y * imp.x, -r1ct1.z * imp.x);
-            V3 l2 = v3(t1.x * imp.x, t1.y * imp.x, t1.z * imp.x);
-            V3 a2 = v3(r2ct1.x * imp.x, r2ct1.y * imp.x, r2ct1.z * imp.x);
-            v1 -= cmul(im1 * l2, ll1);
-            w1 += cmul(al1, mvmul(I1, a1));
-            v2 += cmul(im2 * l2, ll2);
-            w2 += cmul(al2, mvmul(I2, a2));
-            a1 = v3(-r1ct2.x * imp.y, -r1ct2.y * imp.y, -r1ct2.z * imp.y);
-            l2 = v3(t2.x * imp.y, t2.y * imp.y, t2.z * imp.y);
-            a2 = v3(r2ct2.x * imp.y, r2ct2.y * imp.y, r2ct2.z * imp.y);
-            v1.x -= im1 * l2.x * ll1.x; v1.y -= im1 * l2.y * ll1.y; v1.z -= im1 * l2.z * ll1.z;
-            w1 += cmul(al1, mvmul(I1, a1));
-            v2.x += im2 * l2.x * ll2.x; v2.y += im2 * l2.y * ll2.y; v2.z += im2 * l2.z * ll2.z;
-            w2 += cmul(al2, mvmul(I2, a2));
-            const V3 n = ld3(S.n, i);
-            a1 = v3(-n.x * imp.z, -n.y * imp.z, -n.z * imp.z);
-            a2 = v3(n.x * imp.z, n.y * imp.z, n.z * imp.z);
-            w1 += cmul(al1, mvmul(I1, a1));
-            w2 += cmul(al2, mvmul(I2, a2));
-            // the reference applies the twist impulse a second time (CS.cpp:457-466)
-            w1 -= cmul(al1, mvmul(I1, a2));
-            w2 += cmul(al2, mvmul(I2, a2));
-        } else {
-            imp.x = imp.y = imp.z = 0.0f;
-        }
-        S.imp[i] = imp;
-        if (d1) { st3(B.cv, u1, v1); st3(B.cw, u1, w1); }
-        if (d2) { st3(B.cv, u2, v2); st3(B.cw, u2, w2); }
-    }
-}
-
 // Learned warm start: the 24 features of contact point p of solver row i (after sv_prepare_one and
 // the velocity integration): normal, r1, r2, relative velocity in the (t1, t2, n) frame, inverse
 // masses, world inverse inertia (xx of each body), the manifold's cached normal impulses (sum over

@@ -23,6 +23,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "kcommon.h"
 #include "rp3d_internal.h"
 #include "solver_dev.h"
@@ -262,6 +264,100 @@ __device__ __forceinline__ void quad_sweep_row(const SvArgs& A, const QuadSrc& Q
     if (Q.side) {
         if (SPLIT || !Q.part) S.lq[2 * (size_t)i + Q.part] = lam;
         if (!Q.part) st3(S.imp, i, imp);
+    }
+}
+
+// ContactSolverSystem::warmStart (CS.cpp:326-476) of row i by its quad: lane k loads point k and one of
+// (t1, t2, normal, impulses), the lanes of one side add up their body's velocities (both halves alike, the
+// velocity lanes store).  On one lane a manifold's points were loaded one after another behind its number of
+// points: 16 us a colour (65,536-body heap) and 13 us (6,000 hulls).
+__device__ __forceinline__ void quad_warmstart(const SvArgs& A, const QuadSrc& Q, int i) {
+    const DevBodies& B = A.B;
+    const DevSolver& S = A.S;
+    const int2 bb = S.bodies[i];
+    const int np = S.npts[i];
+    const size_t o = 4 * (size_t)i;
+    const float4 pn = Q.pn[o + Q.sub], lam4 = S.lam[o + Q.sub];
+    const float4 ra = Q.in[o + Q.part], rb = Q.in[o + Q.part + 2];
+    const float4 tn = Q.tn[i], rf4 = Q.rf[i];
+    const float4 ot1 = S.oldt1[i], ot2 = S.oldt2[i];
+    const int b = Q.side ? bb.y : bb.x, u = b - B.vbase;
+    const int flags = B.flags[u];
+    V3 v = ld3(B.cv, u), w = ld3(B.cw, u);
+    const M3 I = body_iw(B, b);
+    V3 ll, al;
+    body_locks(B, b, ll, al);
+    const float im = rf4.w;
+    // this lane's point: resting (its cached impulse), new (a learned one, or none) or absent
+    const bool resting = Q.sub < np && lam4.z != 0.0f, fresh = Q.sub < np && !resting && A.learned;
+    float lam = resting ? lam4.x : 0.0f;
+    float4 pr = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (fresh) {
+        pr = S.pred[o + Q.sub];
+        lam = fmax_s(pr.x, 0.0f);
+    }
+    const float kind = resting ? 1.0f : (fresh ? 2.0f : 0.0f);
+    bool any = false;
+    float plx = 0.0f, ply = 0.0f;   // learned friction impulses summed over the new points
+    float4 lq;
+    auto point = [&](auto P, float4 in4) {
+        constexpr int K = decltype(P)::value, kFrom = (K & 1) ? kQuadHigh : kQuadLow;
+        const float l = quad_lane<K>(lam), k = quad_lane<K>(kind);
+        const V3 n = quad_lane3<K>(pn);
+        const V3 in = v3(dpp<kFrom>(in4.x), dpp<kFrom>(in4.y), dpp<kFrom>(in4.z));
+        const float py = quad_lane<K>(pr.y), pz = quad_lane<K>(pr.z);
+        if (k != 0.0f) {
+            if (k == 1.0f) any = true;
+            else {
+                plx += py;
+                ply += pz;
+            }
+            const float ls = flip(l, Q.smask);
+            v.x += im * (n.x * ls) * ll.x; v.y += im * (n.y * ls) * ll.y; v.z += im * (n.z * ls) * ll.z;
+            w.x += in.x * al.x * ls; w.y += in.y * al.y * ls; w.z += in.z * al.z * ls;
+        }
+        return l;
+    };
+    lq.x = point(std::integral_constant<int, 0>{}, ra);
+    lq.y = point(std::integral_constant<int, 1>{}, ra);
+    lq.z = point(std::integral_constant<int, 2>{}, rb);
+    lq.w = point(std::integral_constant<int, 3>{}, rb);
+    float4 imp = make_float4(quad_lane<3>(tn.x), quad_lane<3>(tn.y), quad_lane<3>(tn.z), quad_lane<3>(tn.w));
+    const V3 t1 = quad_lane3<0>(tn), t2 = quad_lane3<1>(tn), n = quad_lane3<2>(tn);
+    // learned friction only for a manifold with no resting point (the reference then starts from zero)
+    if (any || (A.learned && np > 0)) {
+        if (any) {
+            const V3 oi = v3(imp.x * ot1.x + imp.y * ot2.x, imp.x * ot1.y + imp.y * ot2.y, imp.x * ot1.z + imp.y * ot2.z);
+            imp.x = dot(oi, t1);
+            imp.y = dot(oi, t2);
+        } else {
+            imp.x = plx;
+            imp.y = ply;
+            imp.z = 0.0f;
+        }
+        const V3 rf = xyz(rf4);
+        const V3 rct1 = cross(rf, t1), rct2 = cross(rf, t2);
+        const float s1 = flip(imp.x, Q.smask), s2 = flip(imp.y, Q.smask), s3 = flip(imp.z, Q.smask);
+        v += cmul(im * v3(t1.x * s1, t1.y * s1, t1.z * s1), ll);
+        w += cmul(al, mvmul(I, v3(rct1.x * s1, rct1.y * s1, rct1.z * s1)));
+        v += cmul(im * v3(t2.x * s2, t2.y * s2, t2.z * s2), ll);
+        w += cmul(al, mvmul(I, v3(rct2.x * s2, rct2.y * s2, rct2.z * s2)));
+        w += cmul(al, mvmul(I, v3(n.x * s3, n.y * s3, n.z * s3)));
+        // the reference applies the twist impulse a second time (CS.cpp:457-466)
+        const V3 tw = cmul(al, mvmul(I, v3(n.x * imp.z, n.y * imp.z, n.z * imp.z)));
+        w += v3(flip(tw.x, Q.smask), flip(tw.y, Q.smask), flip(tw.z, Q.smask));
+    } else {
+        imp.x = imp.y = imp.z = 0.0f;
+    }
+    if (Q.part) {
+        if (Q.side) S.imp[i] = imp;
+        else S.lq[2 * (size_t)i + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
+    if (!Q.side) S.lq[2 * (size_t)i] = lq;
+    if (flags & BF_DYNAMIC) {
+        st3(B.cv, u, v);
+        st3(B.cw, u, w);
     }
 }
 
