@@ -59,7 +59,7 @@ struct rp3dg_batch {
     // rows; otherwise one launch per colour over colour-major rows.
     bool fused = false;
     int fused_block = 64;              // threads per world of the position kernel (and of the single-class solve)
-    int color_block = 256;             // per-colour layout: threads per block of the colour kernels
+    int color_block = 64;              // per-colour layout: threads per block of the colour kernels (autotuned)
     // fused layout: worlds grouped into size classes (bodies in (L/2, L], L = 64, 128, ... 4096), largest
     // first, `largest` bodies the largest); each class is one launch with its own workgroup size and LDS, the
     // classes run concurrently
@@ -195,6 +195,7 @@ struct rp3dg_batch {
 
     rp3dg::DevCounters* counters = nullptr;
     rp3dg::DevCounters* hcounters = nullptr;
+    int* hseg = nullptr;               // per-colour layout: first row of every colour
 
     bool profiling = false;
     std::string profile_only;          // time only this kernel (empty: all)

@@ -1127,6 +1127,7 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     allocs.push_back(counters);
     alloc_bytes.push_back(sizeof(DevCounters));
     HIPCHECK(hipHostMalloc(&hcounters, sizeof(DevCounters), hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc(&hseg, sizeof(int) * (kMaxColors + 1), hipHostMallocDefault));
     HIPCHECK(hipMemsetAsync(counters, 0, sizeof(DevCounters), stream));
     if (!sort_offs || !S.lam || !S.lq) { set_error("device allocation failed (pair arenas)"); return RP3DG_EHIP; }
     // collider creation: world transforms, initial fat AABBs, all colliders in the moved set
@@ -1506,24 +1507,37 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     // ---------------- per-colour layout: the colour count decides the launches
     if (capturing) { set_error("graph capture needs the fused solver layout"); return RP3DG_EUNSUPPORTED; }
     HIPCHECK(hipMemcpyAsync(&hcounters->nb_colors, &counters->nb_colors, sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIPCHECK(hipMemcpyAsync(hseg, seg_start, sizeof(int) * (kMaxColors + 1), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
     const int ncol = hcounters->nb_colors;
+    // The last colours, at most kTailRows rows each, go to one workgroup in one launch (one such colour would
+    // gain nothing), the others to a launch each that has a quad for every row.  65,536-body heap, 16 colours
+    // of 31,890 to 4 rows: 10 us a launch with the grid of a mean colour
+    int tail = ncol;
+    while (tail > 0 && hseg[tail] - hseg[tail - 1] <= kTailRows) tail--;
+    if (ncol - tail < 2) tail = ncol;
+    auto color_grid = [&](int c) { return grid_for(4 * (hseg[c + 1] - hseg[c]), color_block, 1 << 16); };
     const int bg = grid_for(nb);
     // inverse world inertia + velocity integration (PhysicsWorld.cpp:266-272), contact and joint rows
     if (J.bfirst) LAUNCH_T("fill_int", grid_for(nworlds), 256, fill_int, J.bfirst, nworlds, INT_MAX);
     LAUNCH_T("sv_setup", grid_for(nb + hm + J.n + 128), 256, sv_setup, SA, J, settings, dt);
     // contact solver (PhysicsWorld.cpp:321-345)
     const int jg = grid_for(std::max(J.n, 1)), jg2 = grid_for(std::max(2 * J.n, 1));
-    const int qg = grid_for(4 * (hm / std::max(1, ncol) + 1), color_block);
-    for (int c = 0; c < ncol; c++) LAUNCH_T("sv_warmstart", qg, color_block, sv_warmstart, SA, c);
+    for (int c = 0; c < tail; c++) LAUNCH_T("sv_warmstart", color_grid(c), color_block, sv_warmstart, SA, c);
+    if (tail < ncol) LAUNCH_T("sv_warmstart", 1, 4 * kTailRows, sv_warmstart_tail, SA, tail, ncol);
     // ConstraintSolverSystem::initialize: warm start of every joint kind
     for (int s = 0; s < jt_slots; s++) LAUNCH_T("jt_warmstart", jg, 256, jt_warmstart, B, J, jt_ranges, s);
     for (int it = 0; it < settings.vel_iters; it++) {
         for (int s = 0; s < jt_slots; s++)
             LAUNCH_T("jt_solve_velocity", jg2, 256, jt_solve_velocity, B, J, jt_ranges, s, jt_kind[s], dt);
-        for (int c = 0; c < ncol; c++) {
-            if (settings.split_impulse) LAUNCH_T("sv_solve_color", qg, color_block, sv_solve_color<true>, SA, c, beta_dt);
-            else LAUNCH_T("sv_solve_color", qg, color_block, sv_solve_color<false>, SA, c, beta_dt);
+        for (int c = 0; c < tail; c++) {
+            if (settings.split_impulse)
+                LAUNCH_T("sv_solve_color", color_grid(c), color_block, sv_solve_color<true>, SA, c, beta_dt);
+            else LAUNCH_T("sv_solve_color", color_grid(c), color_block, sv_solve_color<false>, SA, c, beta_dt);
+        }
+        if (tail < ncol) {
+            if (settings.split_impulse) LAUNCH_T("sv_solve_color", 1, 4 * kTailRows, sv_solve_tail<true>, SA, tail, ncol, beta_dt);
+            else LAUNCH_T("sv_solve_color", 1, 4 * kTailRows, sv_solve_tail<false>, SA, tail, ncol, beta_dt);
         }
     }
     LAUNCH_T("sv_store", mg, 256, sv_store, SA);
@@ -1804,6 +1818,7 @@ rp3dg_batch::~rp3dg_batch() {
     for (hipEvent_t ev : event_pool) hipEventDestroy(ev);
     for (void* p : allocs) hipFree(p);
     if (hcounters) hipHostFree(hcounters);
+    if (hseg) hipHostFree(hseg);
     if (stream) hipStreamDestroy(stream);
 }
 

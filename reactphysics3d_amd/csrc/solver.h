@@ -60,6 +60,10 @@ __host__ __device__ constexpr int color_manifold_bytes(int m) { return m * 8 + (
 __global__ void sv_group_color(ColorArgs A);
 __global__ void sv_color_keys(const int* color, const int* nm_ptr, uint64_t* keys, int* vals, int* seg_cnt, int* ncolors);
 __global__ void sv_warmstart(SvArgs A, int color);
+constexpr int kTailRows = 256;   // rows at most of a colour that one workgroup takes in a pass
+template <bool SPLIT>
+__global__ void sv_solve_tail(SvArgs A, int c0, int c1, float beta_dt);
+__global__ void sv_warmstart_tail(SvArgs A, int c0, int c1);
 template <bool SPLIT>
 __global__ void sv_solve_color(SvArgs A, int color, float beta_dt);   // one quad of lanes per manifold
 __global__ void sv_store(SvArgs A);
