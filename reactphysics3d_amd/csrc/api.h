@@ -35,4 +35,21 @@ struct ApiArgs {
 
 __global__ void api_apply_ops(ApiArgs A, const ApiOp* ops, int n);
 
+// State of bodies [first, first + n) as packed arrays (host memory of the batch; null: not wanted).
+__global__ void api_pack_bodies(DevBodies B, int first, int n, float* pos, float* ori, float* lin, float* ang);
+// Adds packed forces and torques (host memory of the batch, or null) to bodies [first, first + n); *woke = 1 if
+// a sleeping body was woken.
+__global__ void api_add_forces(DevBodies B, int first, int n, const float* force, const float* torque, float* sleep_time,
+                               int* woke);
+
+// One array of a snapshot: its first piece of kCopyPiece bytes in the launch.
+struct CopyArray {
+    char *a, *b;
+    size_t bytes;
+    int first, pad;
+};
+constexpr int kCopyPiece = 32768, kCopyArrays = 1024;   // arrays a launch at most
+// a -> b, or b -> a (back); `skip`: an array that is left out, or -1
+__global__ void api_copy_arrays(const CopyArray* arrays, int n, int pieces, int back, int skip);
+
 }  // namespace rp3dg

@@ -99,4 +99,92 @@ __global__ void api_apply_ops(ApiArgs A, const ApiOp* ops, int n) {
     }
 }
 
+// The host's arrays have 3 floats a vector and the device's 4.  Packing on the device and writing over the bus
+// costs one launch: 21 us a call for 28 bodies and 224 us for 65,541 (most of it the caller's memory), where
+// copying the four arrays whole and packing on the host took 53 and 460 us.  Consecutive lanes write
+// consecutive words.
+__global__ __launch_bounds__(256) void api_pack_bodies(DevBodies B, int first, int n, float* pos, float* ori, float* lin,
+                                                       float* ang) {
+    const float* src[4] = {reinterpret_cast<const float*>(B.p + first), reinterpret_cast<const float*>(B.q + first),
+                           reinterpret_cast<const float*>(B.v + first), reinterpret_cast<const float*>(B.w + first)};
+    float* const dst[4] = {pos, ori, lin, ang};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        if (!dst[k]) continue;
+        if (k == 1) {
+            RP3DG_GRID_STRIDE(t, 4 * n) dst[k][t] = src[k][t];
+        } else {
+            RP3DG_GRID_STRIDE(t, 3 * n) {
+                const int i = t / 3;
+                dst[k][t] = src[k][4 * i + (t - 3 * i)];
+            }
+        }
+    }
+}
+
+// RigidBody::applyWorldForceAtCenterOfMass / applyWorldTorque (RigidBody.cpp:298-311) on every body
+__global__ __launch_bounds__(256) void api_add_forces(DevBodies B, int first, int n, const float* force, const float* torque,
+                                                      float* sleep_time, int* woke) {
+    __shared__ float s_in[2][3 * 256];   // (so that the host's memory is read in whole lines, once)
+    for (int i0 = blockIdx.x * 256; i0 < n; i0 += gridDim.x * 256) {
+        for (int k = threadIdx.x; k < 3 * 256; k += 256) {
+            const bool in = k < 3 * (n - i0);
+            s_in[0][k] = in && force ? force[3 * (size_t)i0 + k] : 0.f;
+            s_in[1][k] = in && torque ? torque[3 * (size_t)i0 + k] : 0.f;
+        }
+        __syncthreads();
+        const int l = threadIdx.x, i = first + i0 + l;
+        if (i0 + l < n) {
+            const V3 f = v3(s_in[0][3 * l], s_in[0][3 * l + 1], s_in[0][3 * l + 2]);
+            const V3 t = v3(s_in[1][3 * l], s_in[1][3 * l + 1], s_in[1][3 * l + 2]);
+            const bool nf = f.x != 0.f || f.y != 0.f || f.z != 0.f, nt = t.x != 0.f || t.y != 0.f || t.z != 0.f;
+            const int fl = B.flags[i];
+            if ((fl & BF_DYNAMIC) && (nf || nt)) {   // only dynamic bodies take forces
+                if (!(fl & BF_ENABLED)) {            // asleep: setIsSleeping(false)
+                    B.flags[i] = fl | BF_ENABLED | BF_WOKEN;
+                    if (sleep_time) sleep_time[i] = 0.0f;
+                    *woke = 1;
+                }
+                if (nf) st3(B.force, i, ld3(B.force, i) + f);
+                if (nt) st3(B.torque, i, ld3(B.torque, i) + t);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Every array of a snapshot in one launch: a copy of its own for each of about 150 took 500 us to put a world
+// of 88 bodies back.
+__global__ __launch_bounds__(256) void api_copy_arrays(const CopyArray* arrays, int n, int pieces, int back, int skip) {
+    __shared__ int s_first[kCopyArrays];
+    for (int k = threadIdx.x; k < n; k += 256) s_first[k] = arrays[k].first;
+    __syncthreads();
+    for (int p = blockIdx.x; p < pieces; p += gridDim.x) {
+        int lo = 0, hi = n;   // the last array that starts at or before the piece
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) / 2;
+            if (s_first[mid] <= p) lo = mid;
+            else hi = mid;
+        }
+        if (lo == skip) continue;
+        const CopyArray A = arrays[lo];
+        const size_t off = (size_t)(p - s_first[lo]) * kCopyPiece;
+        const size_t bytes = min((size_t)kCopyPiece, A.bytes - off);
+        const char* src = (back ? A.b : A.a) + off;
+        char* dst = (back ? A.a : A.b) + off;
+        const int vecs = (int)(bytes / 16);   // (arrays start at multiples of 256 bytes)
+        const float4* s4 = reinterpret_cast<const float4*>(src);
+        float4* d4 = reinterpret_cast<float4*>(dst);
+        for (int k = threadIdx.x; k < vecs; k += 4 * 256) {
+            float4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = s4[min(k + 256 * j, vecs - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (k + 256 * j < vecs) d4[k + 256 * j] = v[j];
+        }
+        for (int k = 16 * vecs + threadIdx.x; k < (int)bytes; k += 256) dst[k] = src[k];
+    }
+}
+
 }  // namespace rp3dg

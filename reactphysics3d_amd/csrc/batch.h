@@ -37,6 +37,11 @@ struct rp3dg_batch {
     rp3dg::DevSolver S{};
     rp3dg::DevJoints J{};
     rp3dg::DevIslands isl{};           // allocated when the worlds have sleeping enabled
+    // pinned host memory through which bodies, forces and rays pass, in parts of at most kStageBytes
+    static constexpr size_t kStageBytes = (size_t)16 << 20;
+    char* stage = nullptr;
+    size_t stage_cap = 0;
+    int stage_reserve(size_t bytes);
     void* ray_buf = nullptr;           // raycast staging (grown on demand, freed with the batch)
     size_t ray_cap = 0;
     int4* ev_buf = nullptr;            // contact events of the last step (allocated when first enabled)

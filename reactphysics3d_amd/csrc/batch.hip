@@ -1807,6 +1807,18 @@ int rp3dg_batch::flush_api() {
     return RP3DG_OK;
 }
 
+// The caller has waited for whatever used the memory before.
+int rp3dg_batch::stage_reserve(size_t bytes) {
+    if (bytes <= stage_cap) return RP3DG_OK;
+    if (stage) HIPCHECK(hipHostFree(stage));
+    stage = nullptr;
+    stage_cap = 0;
+    const size_t want = std::max<size_t>(bytes, 65536);
+    HIPCHECK(hipHostMalloc((void**)&stage, want, hipHostMallocDefault));
+    stage_cap = want;
+    return RP3DG_OK;
+}
+
 rp3dg_batch::~rp3dg_batch() {
     drop_graphs();
     for (hipStream_t s : side_streams) hipStreamDestroy(s);
@@ -1819,6 +1831,7 @@ rp3dg_batch::~rp3dg_batch() {
     for (void* p : allocs) hipFree(p);
     if (hcounters) hipHostFree(hcounters);
     if (hseg) hipHostFree(hseg);
+    if (stage) hipHostFree(stage);
     if (stream) hipStreamDestroy(stream);
 }
 
@@ -1869,6 +1882,8 @@ struct rp3dg_snapshot {
     size_t nallocs = 0;
     std::vector<size_t> offs, sizes;
     char* dev = nullptr;
+    CopyArray* table = nullptr;      // the arrays, kCopyArrays a launch
+    std::vector<int> pieces;         // of each launch
     size_t bytes = 0;
     DevCounters last{};
     bool cur_is_a = true, contacts_is_a = true, ev_pending = false, query_points = false;
@@ -1880,6 +1895,19 @@ struct rp3dg_snapshot {
 static int sync_all_streams(rp3dg_batch* b) {
     HIPCHECK(hipStreamSynchronize(b->stream));
     for (hipStream_t st : b->side_streams) HIPCHECK(hipStreamSynchronize(st));
+    return RP3DG_OK;
+}
+
+// Copies the batch's arrays into the snapshot, or back (all but array `skip`).
+static int copy_snapshot(rp3dg_batch* b, const rp3dg_snapshot* s, bool back, int skip) {
+    for (size_t i = 0, l = 0; i < s->nallocs; i += kCopyArrays, l++) {
+        const int n = (int)std::min<size_t>(kCopyArrays, s->nallocs - i);
+        const int sk = skip >= (int)i && skip < (int)i + n ? skip - (int)i : -1;
+        if (s->pieces[l] > 0)
+            api_copy_arrays<<<std::min(s->pieces[l], 4096), 256, 0, b->stream>>>(s->table + i, n, s->pieces[l], back, sk);
+        HIPCHECK(hipGetLastError());
+    }
+    HIPCHECK(hipStreamSynchronize(b->stream));
     return RP3DG_OK;
 }
 
@@ -1906,13 +1934,16 @@ int rp3dg_batch_snapshot(rp3dg_batch* b, rp3dg_snapshot** out) {
         set_error("device allocation failed (snapshot of " + std::to_string(b->bytes) + " bytes)");
         return RP3DG_EHIP;
     }
-    for (size_t i = 0; i < s->nallocs; i++)
-        if (hipMemcpyAsync(s->dev + s->offs[i], b->allocs[i], s->sizes[i], hipMemcpyDeviceToDevice, b->stream) != hipSuccess) {
-            rp3dg_snapshot_destroy(s);
-            set_error("snapshot copy failed");
-            return RP3DG_EHIP;
-        }
-    if (hipStreamSynchronize(b->stream) != hipSuccess) {
+    std::vector<CopyArray> table(s->nallocs);
+    for (size_t i = 0; i < s->nallocs; i++) {
+        if (i % kCopyArrays == 0) s->pieces.push_back(0);
+        table[i] = {(char*)b->allocs[i], s->dev + s->offs[i], s->sizes[i], s->pieces.back(), 0};
+        s->pieces.back() += (int)((s->sizes[i] + kCopyPiece - 1) / kCopyPiece);
+    }
+    if (hipMalloc((void**)&s->table, sizeof(CopyArray) * std::max<size_t>(1, s->nallocs)) != hipSuccess ||
+        hipMemcpy(s->table, table.data(), sizeof(CopyArray) * s->nallocs, hipMemcpyHostToDevice) != hipSuccess ||
+        copy_snapshot(b, s, false, -1) != RP3DG_OK) {
+        (void)hipGetLastError();
         rp3dg_snapshot_destroy(s);
         set_error("snapshot copy failed");
         return RP3DG_EHIP;
@@ -1941,11 +1972,11 @@ int rp3dg_batch_restore(rp3dg_batch* b, const rp3dg_snapshot* s) {
     if (r) return r;
     b->api_ops.clear();   // calls queued since the snapshot belong to the state it replaces
     b->api_sleep_op = false;
-    for (size_t i = 0; i < s->nallocs; i++) {
-        if (b->allocs[i] == (void*)b->log_count) continue;   // the sample log is not simulation state
-        HIPCHECK(hipMemcpyAsync(b->allocs[i], s->dev + s->offs[i], s->sizes[i], hipMemcpyDeviceToDevice, b->stream));
-    }
-    HIPCHECK(hipStreamSynchronize(b->stream));
+    int skip = -1;   // the sample log is not simulation state
+    for (size_t i = 0; i < s->nallocs; i++)
+        if (b->allocs[i] == (void*)b->log_count) skip = (int)i;
+    r = copy_snapshot(b, s, true, skip);
+    if (r) return r;
     b->last = s->last;
     b->cur_is_a = s->cur_is_a; b->contacts_is_a = s->contacts_is_a;
     b->ev_pending = s->ev_pending; b->query_points = s->query_points;
@@ -1962,6 +1993,7 @@ int64_t rp3dg_snapshot_bytes(const rp3dg_snapshot* s) { return s ? (int64_t)s->b
 void rp3dg_snapshot_destroy(rp3dg_snapshot* s) {
     if (!s) return;
     if (s->dev) (void)hipFree(s->dev);
+    if (s->table) (void)hipFree(s->table);
     delete s;
 }
 
@@ -2098,36 +2130,25 @@ int rp3dg_batch_apply_forces(rp3dg_batch* b, const float* force, const float* to
     if (!force && !torque) return RP3DG_OK;
     const int fr = b->flush_api();
     if (fr) return fr;
-    const int n = b->nb;
+    constexpr size_t kBody = 6 * sizeof(float);
+    const int part = (int)(rp3dg_batch::kStageBytes / kBody);
+    int* woke_flag = nullptr;
     bool woke = false;
-    std::vector<float4> f(n), t(n);
-    std::vector<int> fl(n);
-    std::vector<float> st;
-    HIPCHECK(hipStreamSynchronize(b->stream));
-    HIPCHECK(hipMemcpy(f.data(), b->B.force, sizeof(float4) * n, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(t.data(), b->B.torque, sizeof(float4) * n, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(fl.data(), b->B.flags, sizeof(int) * n, hipMemcpyDeviceToHost));
-    if (b->settings.sleeping_enabled) {
-        st.resize(n);
-        HIPCHECK(hipMemcpy(st.data(), b->isl.sleep_time, sizeof(float) * n, hipMemcpyDeviceToHost));
+    for (int i = 0; i < b->nb; i += part) {
+        const size_t n = (size_t)std::min(part, b->nb - i);
+        if (const int r = b->stage_reserve(kBody * n + 64)) return r;
+        woke_flag = (int*)b->stage;
+        float *f = (float*)(b->stage + 64), *t = f + 3 * n;
+        *woke_flag = 0;
+        if (force) memcpy(f, force + 3 * (size_t)i, 3 * sizeof(float) * n);
+        if (torque) memcpy(t, torque + 3 * (size_t)i, 3 * sizeof(float) * n);
+        api_add_forces<<<grid_for((int)n), 256, 0, b->stream>>>(b->B, i, (int)n, force ? f : nullptr, torque ? t : nullptr,
+                                                                b->settings.sleeping_enabled ? b->isl.sleep_time : nullptr,
+                                                                woke_flag);
+        HIPCHECK(hipGetLastError());
+        HIPCHECK(hipStreamSynchronize(b->stream));
+        woke = woke || *woke_flag != 0;
     }
-    auto nonzero = [](const float* a, int i) { return a && (a[3 * i] != 0.f || a[3 * i + 1] != 0.f || a[3 * i + 2] != 0.f); };
-    for (int i = 0; i < n; i++) {
-        if (!(fl[i] & BF_DYNAMIC)) continue;   // only dynamic bodies take forces (RigidBody.cpp:298-311)
-        const bool nf = nonzero(force, i), nt = nonzero(torque, i);
-        if (!nf && !nt) continue;
-        if (!(fl[i] & BF_ENABLED)) {   // asleep: setIsSleeping(false)
-            fl[i] |= BF_ENABLED | BF_WOKEN;
-            st[i] = 0.0f;
-            woke = true;
-        }
-        if (nf) { f[i].x += force[3 * i]; f[i].y += force[3 * i + 1]; f[i].z += force[3 * i + 2]; }
-        if (nt) { t[i].x += torque[3 * i]; t[i].y += torque[3 * i + 1]; t[i].z += torque[3 * i + 2]; }
-    }
-    HIPCHECK(hipMemcpy(b->B.force, f.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(b->B.torque, t.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(b->B.flags, fl.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-    if (!st.empty()) HIPCHECK(hipMemcpy(b->isl.sleep_time, st.data(), sizeof(float) * n, hipMemcpyHostToDevice));
     if (woke) {   // askForBroadPhaseCollisionCheck (RigidBody.cpp:1045-1051): the moved set takes their colliders
         bp_refit<<<grid_for(b->nc), 256, 0, b->stream>>>(b->B, b->C, b->d_hbounds, 2);
         HIPCHECK(hipGetLastError());
@@ -2144,47 +2165,43 @@ int rp3dg_batch_raycast(rp3dg_batch* b, int64_t n, const int32_t* world, const f
     if (n > (1 << 26)) { set_error("at most 2^26 rays per call"); return RP3DG_EINVAL; }
     if (b->has_concave) { set_error("raycasts do not take batches with concave shapes yet"); return RP3DG_EUNSUPPORTED; }
     if (const int fr = b->flush_api()) return fr;
-    std::vector<int> wv((size_t)n);
-    std::vector<float4> a((size_t)n), c((size_t)n);
-    for (int64_t i = 0; i < n; i++) {
-        const int w = world ? world[i] : 0;
-        if (w < 0 || w >= b->nworlds) { set_error("raycast: invalid world index"); return RP3DG_EINVAL; }
-        const float mf = max_fraction ? max_fraction[i] : 1.0f;
-        wv[i] = w;
-        a[i] = make_float4(point1[3 * i], point1[3 * i + 1], point1[3 * i + 2], 0.f);
-        c[i] = make_float4(point2[3 * i], point2[3 * i + 1], point2[3 * i + 2], mf);
-    }
-    // staging: p1, p2, hit point, hit normal (float4 each), world, hit collider (int each)
-    const size_t need = (size_t)n * (4 * sizeof(float4) + 2 * sizeof(int));
-    if (need > b->ray_cap) {
-        if (b->ray_buf) HIPCHECK(hipFree(b->ray_buf));
-        b->ray_buf = nullptr;
-        b->ray_cap = 0;
-        HIPCHECK(hipMalloc(&b->ray_buf, need));
-        b->ray_cap = need;
-    }
-    float4* dp1 = (float4*)b->ray_buf;
-    float4* dp2 = dp1 + n;
-    float4* dhp = dp2 + n;
-    float4* dhn = dhp + n;
-    int* dw = (int*)(dhn + n);
-    int* dhc = dw + n;
-    HIPCHECK(hipMemcpyAsync(dp1, a.data(), sizeof(float4) * n, hipMemcpyHostToDevice, b->stream));
-    HIPCHECK(hipMemcpyAsync(dp2, c.data(), sizeof(float4) * n, hipMemcpyHostToDevice, b->stream));
-    HIPCHECK(hipMemcpyAsync(dw, wv.data(), sizeof(int) * n, hipMemcpyHostToDevice, b->stream));
-    RayArgs A{b->C, b->d_hulls, b->d_hverts, b->d_hnormals, b->d_hfverts, b->d_hfvidx, b->d_wcoll};
-    rc_closest<<<grid_for((int)n), 256, 0, b->stream>>>(A, dw, dp1, dp2, (int)n, category_mask, dhc, dhp, dhn);
-    HIPCHECK(hipGetLastError());
-    std::vector<int> hc((size_t)n);
-    HIPCHECK(hipMemcpyAsync(hc.data(), dhc, sizeof(int) * n, hipMemcpyDeviceToHost, b->stream));
-    HIPCHECK(hipMemcpyAsync(a.data(), dhp, sizeof(float4) * n, hipMemcpyDeviceToHost, b->stream));
-    HIPCHECK(hipMemcpyAsync(c.data(), dhn, sizeof(float4) * n, hipMemcpyDeviceToHost, b->stream));
-    HIPCHECK(hipStreamSynchronize(b->stream));
-    for (int64_t i = 0; i < n; i++) {
-        if (collider) collider[i] = hc[i];
-        if (point) { point[3 * i] = a[i].x; point[3 * i + 1] = a[i].y; point[3 * i + 2] = a[i].z; }
-        if (normal) { normal[3 * i] = c[i].x; normal[3 * i + 1] = c[i].y; normal[3 * i + 2] = c[i].z; }
-        if (fraction) fraction[i] = a[i].w;
+    if (world) {
+        for (int64_t i = 0; i < n; i++)
+            if (world[i] < 0 || world[i] >= b->nworlds) { set_error("raycast: invalid world index"); return RP3DG_EINVAL; }
+    } else if (b->nworlds < 1) { set_error("raycast: invalid world index"); return RP3DG_EINVAL; }
+    // rays in: points 1 and 2, world, max fraction; hits out: collider, fraction, point, normal.  The host's
+    // arrays as they are, through pinned memory, and one copy each way.
+    constexpr size_t kIn = 8 * sizeof(float), kOut = 8 * sizeof(float);
+    const int64_t part = (int64_t)(rp3dg_batch::kStageBytes / (kIn + kOut));
+    for (int64_t i = 0; i < n; i += part) {
+        const size_t m = (size_t)std::min(part, n - i);
+        if (const int r = b->stage_reserve((kIn + kOut) * m)) return r;
+        if ((kIn + kOut) * m > b->ray_cap) {
+            if (b->ray_buf) HIPCHECK(hipFree(b->ray_buf));
+            b->ray_buf = nullptr;
+            b->ray_cap = 0;
+            HIPCHECK(hipMalloc(&b->ray_buf, (kIn + kOut) * m));
+            b->ray_cap = (kIn + kOut) * m;
+        }
+        float* h = (float*)b->stage;
+        memcpy(h, point1 + 3 * i, 3 * sizeof(float) * m);
+        memcpy(h + 3 * m, point2 + 3 * i, 3 * sizeof(float) * m);
+        size_t in = 6 * m, owf = 0, omf = 0;   // words
+        if (world) { memcpy(h + (owf = in), world + i, sizeof(int) * m); in += m; }
+        if (max_fraction) { memcpy(h + (omf = in), max_fraction + i, sizeof(float) * m); in += m; }
+        float *d = (float*)b->ray_buf, *dout = d + 8 * m, *hout = h + 8 * m;
+        HIPCHECK(hipMemcpyAsync(d, h, sizeof(float) * in, hipMemcpyHostToDevice, b->stream));
+        RayArgs A{b->C, b->d_hulls, b->d_hverts, b->d_hnormals, b->d_hfverts, b->d_hfvidx, b->d_wcoll};
+        rc_closest<<<grid_for((int)m), 256, 0, b->stream>>>(A, world ? (const int*)(d + owf) : nullptr, d, d + 3 * m,
+                                                             max_fraction ? d + omf : nullptr, (int)m, category_mask,
+                                                             (int*)dout, dout + m, dout + 2 * m, dout + 5 * m);
+        HIPCHECK(hipGetLastError());
+        HIPCHECK(hipMemcpyAsync(hout, dout, sizeof(float) * 8 * m, hipMemcpyDeviceToHost, b->stream));
+        HIPCHECK(hipStreamSynchronize(b->stream));
+        if (collider) memcpy(collider + i, hout, sizeof(int) * m);
+        if (fraction) memcpy(fraction + i, hout + m, sizeof(float) * m);
+        if (point) memcpy(point + 3 * i, hout + 2 * m, 3 * sizeof(float) * m);
+        if (normal) memcpy(normal + 3 * i, hout + 5 * m, 3 * sizeof(float) * m);
     }
     return RP3DG_OK;
 }
@@ -2383,24 +2400,21 @@ int rp3dg_batch_get_sleeping(rp3dg_batch* b, int32_t* sleeping, int64_t capacity
 int rp3dg_batch_get_bodies(rp3dg_batch* b, float* pos, float* ori, float* lin, float* ang) {
     if (!b) return RP3DG_EINVAL;
     if (const int fr = b->flush_api()) return fr;
-    std::vector<float4> t(b->nb);
-    auto grab = [&](const float4* d, float* out, int comps) -> int {
-        if (!out) return RP3DG_OK;
-        HIPCHECK(hipMemcpy(t.data(), d, sizeof(float4) * b->nb, hipMemcpyDeviceToHost));
-        for (int i = 0; i < b->nb; i++) {
-            out[comps * i + 0] = t[i].x;
-            out[comps * i + 1] = t[i].y;
-            out[comps * i + 2] = t[i].z;
-            if (comps == 4) out[comps * i + 3] = t[i].w;
-        }
-        return RP3DG_OK;
-    };
-    HIPCHECK(hipStreamSynchronize(b->stream));
-    int r;
-    if ((r = grab(b->B.p, pos, 3))) return r;
-    if ((r = grab(b->B.q, ori, 4))) return r;
-    if ((r = grab(b->B.v, lin, 3))) return r;
-    if ((r = grab(b->B.w, ang, 3))) return r;
+    constexpr size_t kBody = 13 * sizeof(float);
+    const int part = (int)(rp3dg_batch::kStageBytes / kBody);
+    for (int i = 0; i < b->nb; i += part) {
+        const size_t n = (size_t)std::min(part, b->nb - i);
+        if (const int r = b->stage_reserve(kBody * n)) return r;
+        float *p = (float*)b->stage, *q = p + 3 * n, *v = q + 4 * n, *w = v + 3 * n;
+        api_pack_bodies<<<grid_for((int)n), 256, 0, b->stream>>>(b->B, i, (int)n, pos ? p : nullptr, ori ? q : nullptr,
+                                                                 lin ? v : nullptr, ang ? w : nullptr);
+        HIPCHECK(hipGetLastError());
+        HIPCHECK(hipStreamSynchronize(b->stream));
+        if (pos) memcpy(pos + 3 * (size_t)i, p, 3 * sizeof(float) * n);
+        if (ori) memcpy(ori + 4 * (size_t)i, q, 4 * sizeof(float) * n);
+        if (lin) memcpy(lin + 3 * (size_t)i, v, 3 * sizeof(float) * n);
+        if (ang) memcpy(ang + 3 * (size_t)i, w, 3 * sizeof(float) * n);
+    }
     return RP3DG_OK;
 }
 

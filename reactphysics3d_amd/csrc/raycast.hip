@@ -310,19 +310,22 @@ __global__ __launch_bounds__(256) void rc_all(RayArgs A, const int* ray_world, c
     }
 }
 
-__global__ __launch_bounds__(256) void rc_closest(RayArgs A, const int* ray_world, const float4* p1s, const float4* p2s,
-                                                  int n, uint32_t mask, int* hit_collider, float4* hit_point,
-                                                  float4* hit_normal) {
+__global__ __launch_bounds__(256) void rc_closest(RayArgs A, const int* ray_world, const float* p1s, const float* p2s,
+                                                  const float* max_fraction, int n, uint32_t mask, int* hit_collider,
+                                                  float* hit_fraction, float* hit_point, float* hit_normal) {
     const int rounds = (n + gridDim.x * blockDim.x - 1) / (gridDim.x * blockDim.x);
     for (int r = 0; r < rounds; r++) {
         const int i = (r * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
         const bool ray = i < n;
-        const float4 a = ray ? p1s[i] : make_float4(0.f, 0.f, 0.f, 0.f), b = ray ? p2s[i] : a;
-        const V3 p1 = v3(a.x, a.y, a.z), p2 = v3(b.x, b.y, b.z);
-        float maxf = b.w;
+        V3 p1 = v3(0.f, 0.f, 0.f), p2 = p1;
+        if (ray) {
+            p1 = v3(p1s[3 * (size_t)i], p1s[3 * (size_t)i + 1], p1s[3 * (size_t)i + 2]);
+            p2 = v3(p2s[3 * (size_t)i], p2s[3 * (size_t)i + 1], p2s[3 * (size_t)i + 2]);
+        }
+        float maxf = !ray ? 0.f : (max_fraction ? max_fraction[i] : 1.0f);
         const V3 dir = p2 - p1;
         const V3 inv = v3(1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z);
-        const int w = ray ? ray_world[i] : 0;
+        const int w = ray && ray_world ? ray_world[i] : 0;
         int best = -1;
         Hit hb{0.f, v3(0.f, 0.f, 0.f), v3(0.f, 0.f, 0.f)};
         walk_boxes(A, ray ? A.wcoll[w] : 0, ray ? A.wcoll[w + 1] : 0, mask, p1, inv, maxf, [&](int c) {
@@ -337,8 +340,12 @@ __global__ __launch_bounds__(256) void rc_closest(RayArgs A, const int* ray_worl
         });
         if (!ray) continue;
         hit_collider[i] = best;
-        hit_point[i] = make_float4(hb.p.x, hb.p.y, hb.p.z, hb.t);
-        hit_normal[i] = make_float4(hb.n.x, hb.n.y, hb.n.z, 0.f);
+        hit_fraction[i] = hb.t;
+        const float p[3] = {hb.p.x, hb.p.y, hb.p.z}, m[3] = {hb.n.x, hb.n.y, hb.n.z};
+        for (int k = 0; k < 3; k++) {
+            hit_point[3 * (size_t)i + k] = p[k];
+            hit_normal[3 * (size_t)i + k] = m[k];
+        }
     }
 }
 
