@@ -48,19 +48,10 @@ def bytes_per_launch(name, c, ndyn, nj):
     m, p = c["nb_manifolds"], c["nb_contact_points"]
     ncol = max(1, c["nb_colors"])
     nb, ncl, npairs = c["nb_bodies"], c["nb_colliders"], c["nb_pairs"]
-    np_types = {"np_sphere_sphere": 1, "np_sphere_capsule": 2, "np_capsule_capsule": 3, "np_sphere_poly": 4,
-                "np_capsule_poly": 5, "np_poly_poly": 6}
-    if name == "np_box_box":
-        tests = c["nb_box_tests"]
-        return 176 * tests + 40 * p * (tests / max(1, sum(nt)))
-    if name == "np_poly_poly":
-        # pairs with a convex mesh: bytes of the pair records (the hull data is L2 resident); the kernel is
+    if name == "np_pairs":
+        # the pair records and contact points; with convex meshes (their data is L2 resident) the kernel is
         # rooflined with the VALU FLOP model instead (poly_flops_per_launch)
-        tests = nt[6] - c["nb_box_tests"]
-        return 176 * tests + 40 * p * (tests / max(1, sum(nt)))
-    if name in np_types:
-        tests = nt[np_types[name]]
-        return 176 * tests + 40 * p * (tests / max(1, sum(nt)))
+        return 176 * sum(nt) + 40 * p
     if name == "sv_world_solve":
         # whole velocity solver of a step, one launch: 48 B / contact point + 88 B / manifold +
         # 140 B / dynamic body + 200 B / joint
@@ -113,14 +104,12 @@ VALU_FP32_PEAK = 157.3e12   # FP32 vector, MI355X vendor figure
 BYTE_MODEL = {
     "sv_world_solve": "48 B/contact point + 88 B/manifold + 140 B/dynamic body + 200 B/joint per launch (one step)",
     "world_position": "192 B/dynamic body + 48 B/collider per launch (one step)",
-    "np_poly_poly": "176 B/test + 40 B/contact point",
-    "np_box_box": "176 B/test + 40 B/contact point",
+    "np_pairs": "176 B/test + 40 B/contact point",
 }
 
 KERNELS = ["bp_bounds", "bp_cells", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
            "bp_merge",
-           "np_classify", "np_sphere_sphere", "np_sphere_capsule", "np_capsule_capsule", "np_sphere_poly",
-           "np_capsule_poly", "np_box_box", "np_poly_poly", "sv_flag", "sv_compact", "sv_adj_count", "sv_adj_fill",
+           "np_classify", "np_pairs", "sv_flag", "sv_compact", "sv_adj_count", "sv_adj_fill",
            "sv_color_round", "sv_color_finish", "sv_color_keys", "sv_color_sort", "sv_world_ranges", "sv_group_color",
            "sv_setup", "sv_features", "mlp_infer", "sv_world_solve", "sv_log_samples", "world_position",
            "body_position",
@@ -486,7 +475,7 @@ def main():
             if b is not None:
                 e["gb_s"] = round(b / (ms * 1e-3) / 1e9, 2)
                 e["hbm_frac"] = round(b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 5)
-            if k == "np_poly_poly" and hs:
+            if k == "np_pairs" and hs:
                 fl = poly_flops_per_launch(cp, hs)
                 e["tflop_s"] = round(fl / (ms * 1e-3) / 1e12, 3)
                 e["valu_frac"] = round(fl / (ms * 1e-3) / VALU_FP32_PEAK, 5)
@@ -516,7 +505,7 @@ def main():
                     tj = json.load(f)
                 traffic = tj.get(dominant)
                 traffic_src = tj.get("_measured")
-            if dominant == "np_poly_poly" and hs:
+            if dominant == "np_pairs" and hs:
                 fl = poly_flops_per_launch(cd, hs)
                 achieved = fl / (ms * 1e-3) / 1e12
                 roofline = {"kernel": dominant, "bound": "valu", "achieved": round(achieved, 3),

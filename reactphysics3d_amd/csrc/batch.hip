@@ -1300,34 +1300,30 @@ NpArgs rp3dg_batch::np_args(const DevPairs& P, const DevPairs& O, int query, int
 }
 
 // CollisionDetectionSystem::testNarrowPhaseCollision (CD.cpp:618-665): the pairs are binned by algorithm
-// and each bin is one launch.
+// and one launch takes all bins.
 int rp3dg_batch::enqueue_narrowphase(const NpArgs& A, bool capturing, int pg) {
     LAUNCH_T("np_classify", std::min(pg, 1024), 256, np_classify, A, np_lists, pair_cap, counters->nb_tests,
              &counters->nb_box_tests, &counters->nb_box_sep_tests, &counters->nb_hull_tests);
     int* L = np_lists;
     int* T = counters->nb_tests;
-    auto hint = [&](int n, int block) {
-        const int h = capturing ? pair_cap : std::min(pair_cap, n + n / 4 + 512);
-        return grid_for(h, block);
-    };
-    auto tg = [&](int algo, int block) { return hint(last.nb_tests[algo], block); };
-    LAUNCH_T("np_sphere_sphere", tg(ALGO_SPHERE_SPHERE, 256), 256, np_sphere_sphere, A, L + ALGO_SPHERE_SPHERE * pair_cap, T + ALGO_SPHERE_SPHERE);
-    LAUNCH_T("np_sphere_capsule", tg(ALGO_SPHERE_CAPSULE, 256), 256, np_sphere_capsule, A, L + ALGO_SPHERE_CAPSULE * pair_cap, T + ALGO_SPHERE_CAPSULE);
-    LAUNCH_T("np_capsule_capsule", tg(ALGO_CAPSULE_CAPSULE, 256), 256, np_capsule_capsule, A, L + ALGO_CAPSULE_CAPSULE * pair_cap, T + ALGO_CAPSULE_CAPSULE);
-    LAUNCH_T("np_sphere_poly", tg(ALGO_SPHERE_POLY, 256), 256, np_sphere_poly, A, L + ALGO_SPHERE_POLY * pair_cap, T + ALGO_SPHERE_POLY);
-    LAUNCH_T("np_capsule_poly", tg(ALGO_CAPSULE_POLY, 256), 256, np_capsule_poly, A, L + ALGO_CAPSULE_POLY * pair_cap, T + ALGO_CAPSULE_POLY);
-    LAUNCH_T("np_box_box", hint(last.nb_box_tests, kNpBoxThreads), kNpBoxThreads, np_box_box, A, L + np_list_slot(ALGO_COUNT) * pair_cap,
-             &counters->nb_box_tests);
-    LAUNCH_T("np_box_box", hint(last.nb_box_sep_tests, kNpBoxThreads), kNpBoxThreads, np_box_box, A, L + np_list_slot(ALGO_COUNT + 1) * pair_cap,
-             &counters->nb_box_sep_tests);
-    LAUNCH_T("np_poly_poly", hint(last.nb_hull_tests, 128), 128, np_poly_poly, A, L + ALGO_POLY_POLY * pair_cap,
-             &counters->nb_hull_tests);
-    if (has_concave) {   // convex vs concave pairs: middle phase, triangle tests, manifolds
+    NpLists NL;
+    int tests = 0;
+    for (int i = 0; i < kNpLists; i++) {
+        const int bin = kNpOrder[i];
+        NL.list[i] = L + np_list_slot(bin) * pair_cap;
+        NL.count[i] = bin == ALGO_COUNT ? &counters->nb_box_tests
+                      : bin == ALGO_COUNT + 1 ? &counters->nb_box_sep_tests
+                      : bin == ALGO_POLY_POLY ? &counters->nb_hull_tests : T + bin;
+    }
+    for (int a = 1; a < ALGO_COUNT; a++) tests += last.nb_tests[a];
+    const int hn = capturing ? pair_cap : std::min(pair_cap, tests + tests / 4 + 512);
+    LAUNCH_T("np_pairs", grid_for(hn + kNpLists * kNpThreads, kNpThreads), kNpThreads, np_pairs, A, NL);
+    if (has_concave) {   // convex vs concave pairs: triangle tests, manifolds
         const int* lc = L + np_list_slot(ALGO_CONCAVE) * pair_cap;
-        LAUNCH_T("np_concave_mid", tg(ALGO_CONCAVE, 128), 128, np_concave_mid, A, lc, T + ALGO_CONCAVE);
         const int ht = capturing ? A.CT.cap : std::min(A.CT.cap, last.nb_concave_tests + last.nb_concave_tests / 4 + 512);
         LAUNCH_T("np_concave_tri", grid_for(ht, 128), 128, np_concave_tri, A);
-        LAUNCH_T("np_concave_reduce", tg(ALGO_CONCAVE, 64), 64, np_concave_reduce, A, lc, T + ALGO_CONCAVE);
+        const int hc = capturing ? pair_cap : std::min(pair_cap, last.nb_tests[ALGO_CONCAVE] + last.nb_tests[ALGO_CONCAVE] / 4 + 512);
+        LAUNCH_T("np_concave_reduce", grid_for(hc, 64), 64, np_concave_reduce, A, lc, T + ALGO_CONCAVE);
     }
 
     return RP3DG_OK;

@@ -85,20 +85,21 @@ static_assert(np_list_slot(ALGO_COUNT + 1) < kNpListSlots && np_list_slot(ALGO_C
 
 __global__ void np_classify(NpArgs A, int* lists, int list_stride, int* counts, int* box_count, int* box_sep_count,
                             int* hull_count);
-__global__ void np_sphere_sphere(NpArgs A, const int* list, const int* count);
-__global__ void np_sphere_capsule(NpArgs A, const int* list, const int* count);
-__global__ void np_capsule_capsule(NpArgs A, const int* list, const int* count);
-__global__ void np_sphere_poly(NpArgs A, const int* list, const int* count);
-__global__ void np_capsule_poly(NpArgs A, const int* list, const int* count);
-__global__ void np_poly_poly(NpArgs A, const int* list, const int* count);
-// np_box_box runs in workgroups of exactly this many threads (its clip buffers are sliced from LDS by
+// The lists np_pairs takes and the bins they hold, the longest tests first.
+constexpr int kNpLists = ALGO_COUNT + 1;
+constexpr int kNpOrder[kNpLists] = {ALGO_POLY_POLY, ALGO_CAPSULE_POLY, ALGO_SPHERE_POLY, ALGO_CONCAVE, ALGO_COUNT,
+                                    ALGO_COUNT + 1, ALGO_CAPSULE_CAPSULE, ALGO_SPHERE_CAPSULE, ALGO_SPHERE_SPHERE};
+struct NpLists {
+    const int* list[kNpLists];
+    const int* count[kNpLists];
+};
+// np_pairs runs in workgroups of exactly this many threads (the boxes' clip buffers are sliced from LDS by
 // threadIdx.x)
-constexpr int kNpBoxThreads = 128;
-__global__ void np_box_box(NpArgs A, const int* list, const int* count);
+constexpr int kNpThreads = 128;
+__global__ void np_pairs(NpArgs A, NpLists L);   // convex vs concave pairs: the middle phase (lists the triangle tests)
 void upload_box_topology(const int* edges4, const int* face_edge, const int* face_verts);
-// convex vs concave pairs: middle phase (lists the triangle tests), the tests, then per pair the potential
-// manifolds, their reduction and the warm-start transfer
-__global__ void np_concave_mid(NpArgs A, const int* list, const int* count);
+// convex vs concave pairs: the tests, then per pair the potential manifolds, their reduction and the warm-start
+// transfer
 __global__ void np_concave_tri(NpArgs A);
 __global__ void np_concave_reduce(NpArgs A, const int* list, const int* count);
 

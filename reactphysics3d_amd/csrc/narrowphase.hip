@@ -191,14 +191,14 @@ struct PrivClip {
     __device__ void put(int i, V3 x) { v[i] = x; }
 };
 struct LdsClip {
-    float* p;   // component c of vertex i at p[(3 * i + c) * kNpBoxThreads]
+    float* p;   // component c of vertex i at p[(3 * i + c) * kNpThreads]
     __device__ V3 get(int i) const {
-        return v3(p[(3 * i) * kNpBoxThreads], p[(3 * i + 1) * kNpBoxThreads], p[(3 * i + 2) * kNpBoxThreads]);
+        return v3(p[(3 * i) * kNpThreads], p[(3 * i + 1) * kNpThreads], p[(3 * i + 2) * kNpThreads]);
     }
     __device__ void put(int i, V3 x) {
-        p[(3 * i) * kNpBoxThreads] = x.x;
-        p[(3 * i + 1) * kNpBoxThreads] = x.y;
-        p[(3 * i + 2) * kNpBoxThreads] = x.z;
+        p[(3 * i) * kNpThreads] = x.x;
+        p[(3 * i + 1) * kNpThreads] = x.y;
+        p[(3 * i + 2) * kNpThreads] = x.z;
     }
 };
 
@@ -423,11 +423,11 @@ template <bool BOX, class R>
 __device__ __forceinline__ bool face_contacts(bool refIs1, const Poly& P1, const Poly& P2, const Tf& t12, const Tf& t21,
                                               int minFace, const Tf& T1, const Tf& T2, R& raw) {
     if constexpr (BOX) {
-        // one slice per thread of the np_box_box workgroup (kNpBoxThreads threads), shared by every
+        // one slice per thread of the np_box_box workgroup (kNpThreads threads), shared by every
         // inlined call site of the test
-        __shared__ float s_box_clip[2 * 3 * kBoxClip * kNpBoxThreads];
+        __shared__ float s_box_clip[2 * 3 * kBoxClip * kNpThreads];
         LdsClip bufA{s_box_clip + threadIdx.x};
-        LdsClip bufB{s_box_clip + 3 * kBoxClip * kNpBoxThreads + threadIdx.x};
+        LdsClip bufB{s_box_clip + 3 * kBoxClip * kNpThreads + threadIdx.x};
         return sat_face_contacts_t<kBoxClip>(refIs1, P1, P2, t12, t21, minFace, T1, T2, raw, bufA, bufB);
     } else {
         return sat_face_contacts(refIs1, P1, P2, t12, t21, minFace, T1, T2, raw);
@@ -869,47 +869,38 @@ __global__ __launch_bounds__(256) void np_classify(NpArgs A, int* lists, int lis
     }
 }
 
-__global__ void np_sphere_sphere(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
-        const int k = list[t];
-        const int2 c = A.P.col[k];
-        const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
-        const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
-        Raw raw; raw.n = 0;
-        const bool hit = sphere_sphere(A.C.shape[c.x].x, A.C.shape[c.y].x, T1, T2, raw);
-        A.P.lf[k] = A.lf_update ? lf_after_test(A.P.lf[k], hit) : A.P.lf[k];
-        contact_epilogue(A, k, hit, raw, c.x);
-    }
+__device__ __forceinline__ void np_sphere_sphere(const NpArgs& A, int k) {
+    const int2 c = A.P.col[k];
+    const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
+    const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
+    Raw raw; raw.n = 0;
+    const bool hit = sphere_sphere(A.C.shape[c.x].x, A.C.shape[c.y].x, T1, T2, raw);
+    A.P.lf[k] = A.lf_update ? lf_after_test(A.P.lf[k], hit) : A.P.lf[k];
+    contact_epilogue(A, k, hit, raw, c.x);
 }
 
-__global__ void np_sphere_capsule(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
-        const int k = list[t];
-        const int2 c = A.P.col[k];
-        const bool s1 = A.C.type[c.x] == SHAPE_SPHERE;
-        const int cs = s1 ? c.x : c.y, cc = s1 ? c.y : c.x;
-        const Tf Ts = tf(ld3(A.C.wpos, cs), ldq(A.C.wq, cs));
-        const Tf Tc = tf(ld3(A.C.wpos, cc), ldq(A.C.wq, cc));
-        const float4 cap = A.C.shape[cc];
-        Raw raw; raw.n = 0;
-        const bool hit = sphere_capsule(s1, A.C.shape[cs].x, cap.x, cap.y + cap.y, Ts, Tc, raw);
-        A.P.lf[k] = A.lf_update ? lf_after_test(A.P.lf[k], hit) : A.P.lf[k];
-        contact_epilogue(A, k, hit, raw, c.x);
-    }
+__device__ __forceinline__ void np_sphere_capsule(const NpArgs& A, int k) {
+    const int2 c = A.P.col[k];
+    const bool s1 = A.C.type[c.x] == SHAPE_SPHERE;
+    const int cs = s1 ? c.x : c.y, cc = s1 ? c.y : c.x;
+    const Tf Ts = tf(ld3(A.C.wpos, cs), ldq(A.C.wq, cs));
+    const Tf Tc = tf(ld3(A.C.wpos, cc), ldq(A.C.wq, cc));
+    const float4 cap = A.C.shape[cc];
+    Raw raw; raw.n = 0;
+    const bool hit = sphere_capsule(s1, A.C.shape[cs].x, cap.x, cap.y + cap.y, Ts, Tc, raw);
+    A.P.lf[k] = A.lf_update ? lf_after_test(A.P.lf[k], hit) : A.P.lf[k];
+    contact_epilogue(A, k, hit, raw, c.x);
 }
 
-__global__ void np_capsule_capsule(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
-        const int k = list[t];
-        const int2 c = A.P.col[k];
-        const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
-        const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
-        const float4 s1 = A.C.shape[c.x], s2 = A.C.shape[c.y];
-        Raw raw; raw.n = 0;
-        const bool hit = capsule_capsule(s1.x, s1.y + s1.y, s2.x, s2.y + s2.y, T1, T2, raw);
-        A.P.lf[k] = A.lf_update ? lf_after_test(A.P.lf[k], hit) : A.P.lf[k];
-        contact_epilogue(A, k, hit, raw, c.x);
-    }
+__device__ __forceinline__ void np_capsule_capsule(const NpArgs& A, int k) {
+    const int2 c = A.P.col[k];
+    const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
+    const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
+    const float4 s1 = A.C.shape[c.x], s2 = A.C.shape[c.y];
+    Raw raw; raw.n = 0;
+    const bool hit = capsule_capsule(s1.x, s1.y + s1.y, s2.x, s2.y + s2.y, T1, T2, raw);
+    A.P.lf[k] = A.lf_update ? lf_after_test(A.P.lf[k], hit) : A.P.lf[k];
+    contact_epilogue(A, k, hit, raw, c.x);
 }
 
 // Box-box pairs (the same SAT test with the box topology known at compile time and box-sized buffers)
@@ -1111,127 +1102,112 @@ __device__ __forceinline__ float face_search_result(const EdgeSearch& es, int& f
     return es.pen;
 }
 
-// Polyhedron pairs, one lane per pair.  The edge search of a pair that needs one is shared by the whole
+// Polyhedron pairs list[t], one lane per pair (every lane of the wavefront calls).  The edge search of a pair that needs one is shared by the whole
 // wavefront (each lane takes every 64th edge pair and the results are combined across lanes) while at
 // most coop_max lanes need it; beyond that every such lane walks its own pairs.  Both give the same
 // result.
 template <bool BOX, class R>
-__device__ __forceinline__ void sat_pair_list(const NpArgs& A, const int* list, int n, int coop_max) {
+__device__ __forceinline__ void sat_pairs(const NpArgs& A, const int* list, int n, int t, int coop_max) {
     const int lane = lane_id();
-    for (int base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {   // uniform in the block
-        const int t = base + threadIdx.x;
-        const bool act = t < n;
-        int k = 0;
-        int2 c = make_int2(0, 0);
-        Poly P1{}, P2{};
-        if constexpr (BOX) {   // inactive lanes too: every access folds to the box's implicit topology
-            P1.hull = -1;
-            P2.hull = -1;
-        }
-        Tf T1{}, T2{}, t12{}, t21{};
-        R raw;
-        raw.n = 0;
-        uint32_t lf = 0;
-        int stage = 0;
-        float minPen0 = 0.0f;
-        int minFace = 0;
-        bool isMinFace1 = false;
-        if (act) {
-            k = list[t];
-            c = A.P.col[k];
-            T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
-            T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
-            P1 = BOX ? box_poly(A, c.x) : make_poly(A, c.x);
-            P2 = BOX ? box_poly(A, c.y) : make_poly(A, c.y);
-            lf = A.P.lf[k];
-            t12 = tmul(tinv(T2), T1);
-            t21 = tinv(t12);
-            stage = sat_begin<BOX, BOX>(P1, P2, T1, T2, t12, t21, lf, raw, minPen0, minFace, isMinFace1, A.clip_prev != 0);
-        }
-        if constexpr (!BOX) {
-            // mesh pairs share the two face searches as well (each face's support point walks every
-            // vertex of the other mesh)
-            auto nfaces = [](const Poly& B1, const Poly&) { return B1.nfaces(); };
-            auto face_pen = [](const Poly& B1, const Poly& B2, const Tf& tb, int f, float& p) {
-                p = sat_single_face(B1, B2, tb, f);
-                return true;
-            };
-            EdgeSearch fs;
-            fs.init(kDecimalLargest);
-            shared_search<BOX>(A, __ballot(stage == 3), lane, t12, c.x, c.y, kDecimalLargest, fs, nfaces, face_pen);
-            int face1 = 0, face2 = 0;
-            float pen1 = 0.0f;
-            if (stage == 3) {
-                pen1 = face_search_result(fs, face1);
-                if (fs.sep != INT_MAX) {
-                    lf = lf_set_face(lf, true, face1);
-                    stage = 0;
-                }
-            }
-            fs.init(kDecimalLargest);
-            shared_search<BOX>(A, __ballot(stage == 3), lane, t21, c.y, c.x, kDecimalLargest, fs, nfaces, face_pen);
-            if (stage == 3) {
-                const float pen2 = face_search_result(fs, face2);
-                if (fs.sep != INT_MAX) {
-                    lf = lf_set_face(lf, false, face2);
-                    stage = 0;
-                } else {
-                    minPen0 = fmin_s(pen1, pen2);
-                    isMinFace1 = pen1 < pen2 * kSatRel + kSatAbs;
-                    minFace = isMinFace1 ? face1 : face2;
-                    stage = 2;
-                }
+    const bool act = t < n;
+    int k = 0;
+    int2 c = make_int2(0, 0);
+    Poly P1{}, P2{};
+    if constexpr (BOX) {   // inactive lanes too: every access folds to the box's implicit topology
+        P1.hull = -1;
+        P2.hull = -1;
+    }
+    Tf T1{}, T2{}, t12{}, t21{};
+    R raw;
+    raw.n = 0;
+    uint32_t lf = 0;
+    int stage = 0;
+    float minPen0 = 0.0f;
+    int minFace = 0;
+    bool isMinFace1 = false;
+    if (act) {
+        k = list[t];
+        c = A.P.col[k];
+        T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
+        T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
+        P1 = BOX ? box_poly(A, c.x) : make_poly(A, c.x);
+        P2 = BOX ? box_poly(A, c.y) : make_poly(A, c.y);
+        lf = A.P.lf[k];
+        t12 = tmul(tinv(T2), T1);
+        t21 = tinv(t12);
+        stage = sat_begin<BOX, BOX>(P1, P2, T1, T2, t12, t21, lf, raw, minPen0, minFace, isMinFace1, A.clip_prev != 0);
+    }
+    if constexpr (!BOX) {
+        // mesh pairs share the two face searches as well (each face's support point walks every
+        // vertex of the other mesh)
+        auto nfaces = [](const Poly& B1, const Poly&) { return B1.nfaces(); };
+        auto face_pen = [](const Poly& B1, const Poly& B2, const Tf& tb, int f, float& p) {
+            p = sat_single_face(B1, B2, tb, f);
+            return true;
+        };
+        EdgeSearch fs;
+        fs.init(kDecimalLargest);
+        shared_search<BOX>(A, __ballot(stage == 3), lane, t12, c.x, c.y, kDecimalLargest, fs, nfaces, face_pen);
+        int face1 = 0, face2 = 0;
+        float pen1 = 0.0f;
+        if (stage == 3) {
+            pen1 = face_search_result(fs, face1);
+            if (fs.sep != INT_MAX) {
+                lf = lf_set_face(lf, true, face1);
+                stage = 0;
             }
         }
-        EdgeSearch es;
-        es.init();
-        uint64_t m = __ballot(stage == 2);
-        if (__popcll(m) > coop_max) {
-            if (stage == 2) {
-                int h2;
-                const int np = sat_edge_pairs(P1, P2, h2);
-                for (int kk = 0; kk < np; kk++) {
-                    float p = 0.0f;
-                    const bool v = sat_edge_pair(P1, P2, t12, kk, h2, p);
-                    es.visit(kk, v, p);
-                    if (es.sep != INT_MAX) break;
-                }
+        fs.init(kDecimalLargest);
+        shared_search<BOX>(A, __ballot(stage == 3), lane, t21, c.y, c.x, kDecimalLargest, fs, nfaces, face_pen);
+        if (stage == 3) {
+            const float pen2 = face_search_result(fs, face2);
+            if (fs.sep != INT_MAX) {
+                lf = lf_set_face(lf, false, face2);
+                stage = 0;
+            } else {
+                minPen0 = fmin_s(pen1, pen2);
+                isMinFace1 = pen1 < pen2 * kSatRel + kSatAbs;
+                minFace = isMinFace1 ? face1 : face2;
+                stage = 2;
             }
-        } else {
-            auto npairs = [](const Poly& B1, const Poly& B2) {
-                int h2;
-                return sat_edge_pairs(B1, B2, h2);
-            };
-            auto edge_pen = [](const Poly& B1, const Poly& B2, const Tf& tb, int kk, float& p) {
-                int h2;
-                sat_edge_pairs(B1, B2, h2);
-                return sat_edge_pair(B1, B2, tb, kk, h2, p);
-            };
-            shared_search<BOX>(A, m, lane, t12, c.x, c.y, __builtin_huge_valf(), es, npairs, edge_pen);
-        }
-        if (act) {
-            bool hit = stage == 1;
-            if (stage == 2)
-                hit = sat_finish<BOX>(P1, P2, T1, T2, t12, t21, lf, raw, minPen0, minFace, isMinFace1, es);
-            // ConvexPolyhedronVsConvexPolyhedronAlgorithm.cpp:55-62
-            lf |= LF_WAS_SAT;
-            lf &= ~LF_WAS_GJK;
-            A.P.lf[k] = A.lf_update ? lf_after_test(lf, hit) : lf;
-            contact_epilogue(A, k, hit, raw, c.x);
         }
     }
-}
-
-// Pairs with a convex mesh (the general buffers); their edge searches run over hundreds of pairs, so
-// they are always shared.
-__global__ __launch_bounds__(128) void np_poly_poly(NpArgs A, const int* list, const int* count) {
-    sat_pair_list<false, Raw>(A, list, *count, kWave);
-}
-
-// Box-box pairs: the box topology is known at compile time and the buffers are box-sized.  A lane's own
-// walk over the 144 edge pairs costs about as much as 32 shared searches, hence the limit.
-__global__ __launch_bounds__(kNpBoxThreads) void np_box_box(NpArgs A, const int* list, const int* count) {
-    sat_pair_list<true, RawBoxView>(A, list, *count, 32);
+    EdgeSearch es;
+    es.init();
+    uint64_t m = __ballot(stage == 2);
+    if (__popcll(m) > coop_max) {
+        if (stage == 2) {
+            int h2;
+            const int np = sat_edge_pairs(P1, P2, h2);
+            for (int kk = 0; kk < np; kk++) {
+                float p = 0.0f;
+                const bool v = sat_edge_pair(P1, P2, t12, kk, h2, p);
+                es.visit(kk, v, p);
+                if (es.sep != INT_MAX) break;
+            }
+        }
+    } else {
+        auto npairs = [](const Poly& B1, const Poly& B2) {
+            int h2;
+            return sat_edge_pairs(B1, B2, h2);
+        };
+        auto edge_pen = [](const Poly& B1, const Poly& B2, const Tf& tb, int kk, float& p) {
+            int h2;
+            sat_edge_pairs(B1, B2, h2);
+            return sat_edge_pair(B1, B2, tb, kk, h2, p);
+        };
+        shared_search<BOX>(A, m, lane, t12, c.x, c.y, __builtin_huge_valf(), es, npairs, edge_pen);
+    }
+    if (act) {
+        bool hit = stage == 1;
+        if (stage == 2)
+            hit = sat_finish<BOX>(P1, P2, T1, T2, t12, t21, lf, raw, minPen0, minFace, isMinFace1, es);
+        // ConvexPolyhedronVsConvexPolyhedronAlgorithm.cpp:55-62
+        lf |= LF_WAS_SAT;
+        lf &= ~LF_WAS_GJK;
+        A.P.lf[k] = A.lf_update ? lf_after_test(lf, hit) : lf;
+        contact_epilogue(A, k, hit, raw, c.x);
+    }
 }
 
 void upload_box_topology(const int* edges4, const int* face_edge, const int* face_verts) {
@@ -1722,21 +1698,18 @@ __device__ __forceinline__ bool sphere_poly_test(const Conv& S1, const Conv& S2,
     return hit;
 }
 
-__global__ void np_sphere_poly(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
-        const int k = list[t];
-        const int2 c = A.P.col[k];
-        const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
-        const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
-        const Conv S1 = make_conv(A, c.x), S2 = make_conv(A, c.y);
-        uint32_t lf = A.P.lf[k];
-        float4 axis = A.P.lfaxis[k];
-        Raw raw; raw.n = 0;
-        const bool hit = sphere_poly_test(S1, S2, T1, T2, lf, axis, raw);
-        A.P.lfaxis[k] = axis;
-        A.P.lf[k] = A.lf_update ? lf_after_test(lf, hit) : lf;
-        contact_epilogue(A, k, hit, raw, c.x);
-    }
+__device__ __forceinline__ void np_sphere_poly(const NpArgs& A, int k) {
+    const int2 c = A.P.col[k];
+    const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
+    const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
+    const Conv S1 = make_conv(A, c.x), S2 = make_conv(A, c.y);
+    uint32_t lf = A.P.lf[k];
+    float4 axis = A.P.lfaxis[k];
+    Raw raw; raw.n = 0;
+    const bool hit = sphere_poly_test(S1, S2, T1, T2, lf, axis, raw);
+    A.P.lfaxis[k] = axis;
+    A.P.lf[k] = A.lf_update ? lf_after_test(lf, hit) : lf;
+    contact_epilogue(A, k, hit, raw, c.x);
 }
 
 // CapsuleVsConvexPolyhedronAlgorithm.cpp:42-177
@@ -1785,21 +1758,18 @@ __device__ __forceinline__ bool capsule_poly_test(const Conv& S1, const Conv& S2
     return hit;
 }
 
-__global__ void np_capsule_poly(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
-        const int k = list[t];
-        const int2 c = A.P.col[k];
-        const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
-        const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
-        const Conv S1 = make_conv(A, c.x), S2 = make_conv(A, c.y);
-        uint32_t lf = A.P.lf[k];
-        float4 axis = A.P.lfaxis[k];
-        Raw raw; raw.n = 0;
-        const bool hit = capsule_poly_test(S1, S2, T1, T2, lf, axis, raw, pair_reports(A, k));
-        A.P.lfaxis[k] = axis;
-        A.P.lf[k] = A.lf_update ? lf_after_test(lf, hit) : lf;
-        contact_epilogue(A, k, hit, raw, c.x);
-    }
+__device__ __forceinline__ void np_capsule_poly(const NpArgs& A, int k) {
+    const int2 c = A.P.col[k];
+    const Tf T1 = tf(ld3(A.C.wpos, c.x), ldq(A.C.wq, c.x));
+    const Tf T2 = tf(ld3(A.C.wpos, c.y), ldq(A.C.wq, c.y));
+    const Conv S1 = make_conv(A, c.x), S2 = make_conv(A, c.y);
+    uint32_t lf = A.P.lf[k];
+    float4 axis = A.P.lfaxis[k];
+    Raw raw; raw.n = 0;
+    const bool hit = capsule_poly_test(S1, S2, T1, T2, lf, axis, raw, pair_reports(A, k));
+    A.P.lfaxis[k] = axis;
+    A.P.lf[k] = A.lf_update ? lf_after_test(lf, hit) : lf;
+    contact_epilogue(A, k, hit, raw, c.x);
 }
 
 }  // namespace rp3dg
@@ -1877,60 +1847,101 @@ __device__ __forceinline__ bool mesh_walk(const NpArgs& A, const ConcaveInst& I,
 // Middle phase: the convex shape's AABB in the concave shape's space and the triangles it overlaps
 // (ConcaveShape::computeOverlappingTriangles), listed as this step's tests of the pair, contiguous and in
 // order.
-__global__ void np_concave_mid(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
-        const int k = list[t];
-        const int2 c = A.P.col[k];
-        int cv, cc;
-        bool convex1;
-        concave_sides(A, c, cv, cc, convex1);
-        const Tf Tv = tf(ld3(A.C.wpos, cv), ldq(A.C.wq, cv));
-        const Tf Tc = tf(ld3(A.C.wpos, cc), ldq(A.C.wq, cc));
-        V3 mn, mx;
-        transformed_aabb(A.C.type[cv], A.C.shape[cv], A.hull_bounds, tmul(tinv(Tc), Tv), mn, mx);
-        const ConcaveInst I = A.cinst[(int)A.C.shape[cc].y];
-        int n = 0, base = 0;
-        bool ok = true, reserved = false;
-        if (I.kind == SHAPE_CONCAVE_MESH) {
-            const V3 is = v3(I.isx, I.isy, I.isz);   // AABB::applyScale(1 / scale)
-            mn = cmul(mn, is);
-            mx = cmul(mx, is);
-            ok = mesh_walk(A, I, mn, mx, [&](int i, int) { n = i + 1; });
-            if (ok) {
-                base = n ? atomicAdd(A.CT.count, n) : 0;
-                reserved = n > 0;
-                if (base + n > A.CT.cap) ok = false;
-                else mesh_walk(A, I, mn, mx, [&](int i, int tri) {
-                    A.CT.pair[base + i] = k;
-                    A.CT.tri[base + i] = tri;
-                });
-            }
-        } else {
-            int i0, i1, j0, j1;
-            hf_cells(I, mn, mx, i0, i1, j0, j1);
-            n = (i1 > i0 && j1 > j0) ? 2 * (i1 - i0) * (j1 - j0) : 0;
+__device__ __forceinline__ void np_concave_mid(const NpArgs& A, int k) {
+    const int2 c = A.P.col[k];
+    int cv, cc;
+    bool convex1;
+    concave_sides(A, c, cv, cc, convex1);
+    const Tf Tv = tf(ld3(A.C.wpos, cv), ldq(A.C.wq, cv));
+    const Tf Tc = tf(ld3(A.C.wpos, cc), ldq(A.C.wq, cc));
+    V3 mn, mx;
+    transformed_aabb(A.C.type[cv], A.C.shape[cv], A.hull_bounds, tmul(tinv(Tc), Tv), mn, mx);
+    const ConcaveInst I = A.cinst[(int)A.C.shape[cc].y];
+    int n = 0, base = 0;
+    bool ok = true, reserved = false;
+    if (I.kind == SHAPE_CONCAVE_MESH) {
+        const V3 is = v3(I.isx, I.isy, I.isz);   // AABB::applyScale(1 / scale)
+        mn = cmul(mn, is);
+        mx = cmul(mx, is);
+        ok = mesh_walk(A, I, mn, mx, [&](int i, int) { n = i + 1; });
+        if (ok) {
             base = n ? atomicAdd(A.CT.count, n) : 0;
             reserved = n > 0;
             if (base + n > A.CT.cap) ok = false;
-            else {
-                int q = base;
-                for (int i = i0; i < i1; i++) {
-                    for (int j = j0; j < j1; j++) {
-                        const int id = (j * (I.columns - 1) + i) * 2;   // HeightField::computeTriangleShapeId
-                        A.CT.pair[q] = k; A.CT.tri[q] = id; q++;
-                        A.CT.pair[q] = k; A.CT.tri[q] = id + 1; q++;
-                    }
+            else mesh_walk(A, I, mn, mx, [&](int i, int tri) {
+                A.CT.pair[base + i] = k;
+                A.CT.tri[base + i] = tri;
+            });
+        }
+    } else {
+        int i0, i1, j0, j1;
+        hf_cells(I, mn, mx, i0, i1, j0, j1);
+        n = (i1 > i0 && j1 > j0) ? 2 * (i1 - i0) * (j1 - j0) : 0;
+        base = n ? atomicAdd(A.CT.count, n) : 0;
+        reserved = n > 0;
+        if (base + n > A.CT.cap) ok = false;
+        else {
+            int q = base;
+            for (int i = i0; i < i1; i++) {
+                for (int j = j0; j < j1; j++) {
+                    const int id = (j * (I.columns - 1) + i) * 2;   // HeightField::computeTriangleShapeId
+                    A.CT.pair[q] = k; A.CT.tri[q] = id; q++;
+                    A.CT.pair[q] = k; A.CT.tri[q] = id + 1; q++;
                 }
             }
         }
-        if (!ok) {
-            atomicOr(A.status, STATUS_CONCAVE_OVERFLOW);
-            if (reserved)   // slots reserved but not listed
-                for (int q = base; q < A.CT.cap && q < base + n; q++) A.CT.pair[q] = -1;
-            n = 0;
+    }
+    if (!ok) {
+        atomicOr(A.status, STATUS_CONCAVE_OVERFLOW);
+        if (reserved)   // slots reserved but not listed
+            for (int q = base; q < A.CT.cap && q < base + n; q++) A.CT.pair[q] = -1;
+        n = 0;
+    }
+    A.P.ct0[k] = base;
+    A.P.ctn[k] = n;
+}
+
+// Every pair of the step, 128 of one test list to a workgroup; the workgroups share out the lists by their
+// counts, the longest tests first.  A launch a list took 6 us for each of up to eight lists, empty ones too, and
+// the lists that are there waited for each other's last wavefront: a colliding box pair is a chain of some
+// 30 us however few there are, and so are a capsule's or a mesh's.  All lists' launches before, and now: 27 boxes
+// 99 and 52 us, 1000 boxes 165 and 81, 65,536 spheres, boxes and capsules 360 and 188, 600 bodies on a mesh
+// (middle phase included) 375 and 142.
+// Box-box pairs: the box topology is known at compile time and the buffers are box-sized; a lane's own
+// walk over the 144 edge pairs costs about as much as 32 shared searches, hence the limit.  Pairs with a
+// convex mesh (the general buffers): their edge searches run over hundreds of pairs, so they are always shared.
+__global__ __launch_bounds__(kNpThreads, 3) void np_pairs(NpArgs A, NpLists L) {
+    __shared__ int s_count[kNpLists], s_first[kNpLists + 1];
+    if (threadIdx.x < kNpLists) s_count[threadIdx.x] = *L.count[threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int run = 0;
+        for (int i = 0; i < kNpLists; i++) {
+            s_first[i] = run;
+            run += (s_count[i] + kNpThreads - 1) / kNpThreads;
         }
-        A.P.ct0[k] = base;
-        A.P.ctn[k] = n;
+        s_first[kNpLists] = run;
+    }
+    __syncthreads();
+    const int tiles = s_first[kNpLists];
+    for (int w = blockIdx.x; w < tiles; w += gridDim.x) {
+        int i = 0;
+        while (w >= s_first[i + 1]) i++;
+        i = __builtin_amdgcn_readfirstlane(i);
+        const int n = s_count[i], t = (w - s_first[i]) * kNpThreads + threadIdx.x;
+        const int* list = L.list[i];
+        const int bin = kNpOrder[i];
+        if (bin == ALGO_POLY_POLY) sat_pairs<false, Raw>(A, list, n, t, kWave);
+        else if (bin == ALGO_COUNT || bin == ALGO_COUNT + 1) sat_pairs<true, RawBoxView>(A, list, n, t, 32);
+        else if (t < n) {
+            const int k = list[t];
+            if (bin == ALGO_CAPSULE_POLY) np_capsule_poly(A, k);
+            else if (bin == ALGO_SPHERE_POLY) np_sphere_poly(A, k);
+            else if (bin == ALGO_CONCAVE) np_concave_mid(A, k);
+            else if (bin == ALGO_CAPSULE_CAPSULE) np_capsule_capsule(A, k);
+            else if (bin == ALGO_SPHERE_CAPSULE) np_sphere_capsule(A, k);
+            else np_sphere_sphere(A, k);
+        }
     }
 }
 

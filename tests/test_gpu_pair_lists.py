@@ -1,0 +1,54 @@
+"""One narrowphase launch takes the test lists of all pair types, 128 pairs of a list to a workgroup.  Batches
+with one, almost, exactly and more than a workgroup's pairs of several types at once give every pair the
+contacts it has alone."""
+import numpy as np
+import pytest
+
+from reactphysics3d_amd import scene as S
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {S.SPHERE: (0.5,), S.CAPSULE: (0.3, 0.8), S.BOX: (0.4, 0.5, 0.3), S.HULL: None}
+
+
+def _pair(a, b, k):
+    """Two overlapping bodies of shapes a and b, a little different for every k."""
+    rng = np.random.default_rng(17 * k + 5)
+    sc = S.Scene("pair", S.make_settings(gravity=(0.0, 0.0, 0.0)))
+    for s, x in ((a, 0.0), (b, 0.55)):
+        q = rng.normal(size=4)
+        body = sc.add_body(S.DYNAMIC, (x, 0.0, 0.1 * rng.random()), tuple(q / np.linalg.norm(q)))
+        if s == S.HULL:
+            u = rng.normal(size=(20, 3))
+            h = sc.add_hull_from_points((0.45 * u / np.linalg.norm(u, axis=1)[:, None]).astype(np.float32))
+            sc.add_collider(body, S.HULL, (float(h), 0.0, 0.0))
+        else:
+            sc.add_collider(body, s, SHAPES[s])
+    return sc
+
+
+def _run(scenes):
+    from reactphysics3d_amd.lib import Batch
+    dev = Batch(scenes)
+    dev.step(1.0 / 60.0, 3)
+    ct, state = dev.contacts(), dev.bodies()
+    out = []
+    for w, b0 in enumerate(dev.body_base[:len(scenes)]):
+        m = ct["colliders"][:, 0] // 2 == w   # two colliders a world
+        n = ct["nb_points"][m]
+        out.append([n] + [ct[k][m][:, :n[0] if len(n) else 0] for k in ("normal_depth", "local1", "local2", "impulse")] +
+                   [a[b0:b0 + 2] for a in state])
+    return out
+
+
+@pytest.mark.parametrize("counts", [(1, 1, 1, 1, 1, 1, 1, 1), (127, 0, 129, 0, 1, 0, 128, 0), (0, 130, 0, 128, 0, 300, 0, 1)])
+def test_every_pair_has_the_contacts_it_has_alone(counts):
+    types = [(S.SPHERE, S.SPHERE), (S.SPHERE, S.CAPSULE), (S.CAPSULE, S.CAPSULE), (S.BOX, S.SPHERE),
+             (S.CAPSULE, S.BOX), (S.BOX, S.BOX), (S.HULL, S.BOX), (S.HULL, S.CAPSULE)]
+    kinds = [(t, k % 5) for t, n in enumerate(counts) for k in range(n)]
+    alone = {tk: _run([_pair(*types[tk[0]], tk[1])])[0] for tk in set(kinds)}
+    assert all(len(a[0]) for a in alone.values())
+    order = np.random.default_rng(3).permutation(len(kinds))
+    for i, got in zip(order, _run([_pair(*types[kinds[i][0]], kinds[i][1]) for i in order])):
+        for a, b in zip(alone[kinds[i]], got):
+            assert np.array_equal(a, b), kinds[i]
