@@ -1302,28 +1302,28 @@ NpArgs rp3dg_batch::np_args(const DevPairs& P, const DevPairs& O, int query, int
 // CollisionDetectionSystem::testNarrowPhaseCollision (CD.cpp:618-665): the pairs are binned by algorithm
 // and one launch takes all bins.
 int rp3dg_batch::enqueue_narrowphase(const NpArgs& A, bool capturing, int pg) {
-    LAUNCH_T("np_classify", std::min(pg, 1024), 256, np_classify, A, np_lists, pair_cap, counters->nb_tests,
-             &counters->nb_box_tests, &counters->nb_box_sep_tests, &counters->nb_hull_tests);
+    LAUNCH_T("np_classify", std::min(pg, 1024), 256, np_classify, A, np_lists, pair_cap, counters->nb_bin);
     int* L = np_lists;
-    int* T = counters->nb_tests;
+    int* T = counters->nb_bin;
     NpLists NL;
-    int tests = 0;
+    int tiles = 0;
     for (int i = 0; i < kNpLists; i++) {
         const int bin = kNpOrder[i];
-        NL.list[i] = L + np_list_slot(bin) * pair_cap;
-        NL.count[i] = bin == ALGO_COUNT ? &counters->nb_box_tests
-                      : bin == ALGO_COUNT + 1 ? &counters->nb_box_sep_tests
-                      : bin == ALGO_POLY_POLY ? &counters->nb_hull_tests : T + bin;
+        NL.list[i] = L + (size_t)np_list_slot(bin) * pair_cap;
+        NL.count[i] = T + bin;
     }
-    for (int a = 1; a < ALGO_COUNT; a++) tests += last.nb_tests[a];
-    const int hn = capturing ? pair_cap : std::min(pair_cap, tests + tests / 4 + 512);
-    LAUNCH_T("np_pairs", grid_for(hn + kNpLists * kNpThreads, kNpThreads), kNpThreads, np_pairs, A, NL);
+    // workgroups for the last step's counts and a quarter more
+    auto more = [&](int n) { return capturing ? pair_cap : std::min(pair_cap, n + n / 4 + 64); };
+    for (int i = 0; i < kNpLists; i++) {
+        tiles += np_tiles(kNpOrder[i], more(last.nb_bin[kNpOrder[i]]));
+    }
+    LAUNCH_T("np_pairs", std::min(tiles, 4096), kNpThreads, np_pairs, A, NL);
     if (has_concave) {   // convex vs concave pairs: triangle tests, manifolds
-        const int* lc = L + np_list_slot(ALGO_CONCAVE) * pair_cap;
-        const int ht = capturing ? A.CT.cap : std::min(A.CT.cap, last.nb_concave_tests + last.nb_concave_tests / 4 + 512);
-        LAUNCH_T("np_concave_tri", grid_for(ht, 128), 128, np_concave_tri, A);
-        const int hc = capturing ? pair_cap : std::min(pair_cap, last.nb_tests[ALGO_CONCAVE] + last.nb_tests[ALGO_CONCAVE] / 4 + 512);
-        LAUNCH_T("np_concave_reduce", grid_for(hc, 64), 64, np_concave_reduce, A, lc, T + ALGO_CONCAVE);
+        const int* lc = L + (size_t)np_list_slot(ALGO_CONCAVE) * pair_cap;
+        const int ht = capturing ? A.CT.cap : std::min(A.CT.cap, last.nb_concave_tests + last.nb_concave_tests / 4 + 64);
+        LAUNCH_T("np_concave_tri", std::min(np_tiles(ALGO_CONCAVE, ht), 4096), kNpThreads, np_concave_tri, A);
+        const int hc = more(last.nb_bin[ALGO_CONCAVE]);
+        LAUNCH_T("np_concave_reduce", std::min(2 * np_tiles(ALGO_CONCAVE, hc), 4096), 64, np_concave_reduce, A, lc, T + ALGO_CONCAVE);
     }
 
     return RP3DG_OK;
@@ -2078,14 +2078,18 @@ int rp3dg_batch_get_counts(rp3dg_batch* b, rp3dg_counts* o) {
     o->nb_contact_points = b->last.nb_points;
     o->nb_colors = b->last.nb_colors;
     o->status = b->last.status;
-    for (int a = 0; a < 7; a++) o->nb_tests[a] = b->last.nb_tests[a];
+    const int* t = b->last.nb_bin;
+    for (int a = 0; a < 7; a++) o->nb_tests[a] = t[a];
+    o->nb_tests[ALGO_SPHERE_POLY] += t[BIN_SPHERE_POLY_SEP];
+    o->nb_tests[ALGO_CAPSULE_POLY] += t[BIN_CAPSULE_POLY_SEP];
+    o->nb_tests[ALGO_POLY_POLY] += t[BIN_POLY_POLY_SEP] + t[BIN_BOX] + t[BIN_BOX_SEP];
     unsigned long long tp = 0;
     HIPCHECK(hipMemcpyAsync(&tp, b->total_points, sizeof(tp), hipMemcpyDeviceToHost, b->stream));
     HIPCHECK(hipStreamSynchronize(b->stream));
     o->total_contact_points = (int64_t)tp;
     o->steps = b->steps_done;
     o->nb_new_points = b->last.nb_new_points;
-    o->nb_box_tests = b->last.nb_box_tests + b->last.nb_box_sep_tests;
+    o->nb_box_tests = t[BIN_BOX] + t[BIN_BOX_SEP];
     return RP3DG_OK;
 }
 

@@ -71,24 +71,26 @@ struct NpArgs {
 constexpr int NP_STEP = 0, NP_QUERY_ALL = 1, NP_QUERY_BODIES = 2;
 constexpr int NP_REPORT_NO_TRIGGER = 0, NP_REPORT_ALL = 1, NP_REPORT_NONE = 2;
 
-// Narrowphase test lists: bins 1..5 closed forms, ALGO_POLY_POLY pairs with a convex mesh,
-// ALGO_COUNT box-box pairs colliding last step, ALGO_COUNT + 1 box-box pairs separated last step.
-// List slot of each bin (kNpListSlots lists of the pair capacity each are allocated).
-constexpr int kNpBins = ALGO_COUNT + 2;
-constexpr int kNpListSlots = ALGO_COUNT + 1;
-__host__ __device__ constexpr int np_list_slot(int bin) {
-    return bin == ALGO_COUNT ? 0 : (bin == ALGO_COUNT + 1 ? ALGO_COUNT : bin);
-}
-static_assert(np_list_slot(ALGO_COUNT + 1) < kNpListSlots && np_list_slot(ALGO_COUNT) < kNpListSlots &&
-                  np_list_slot(ALGO_POLY_POLY) < kNpListSlots,
-              "every narrowphase bin needs an allocated list slot");
+// Test lists: one of the pair capacity for each bin but ALGO_NONE, whose slot has BIN_BOX's.
+constexpr int kNpListSlots = kNpBins - 1;
+__host__ __device__ constexpr int np_list_slot(int bin) { return bin < BIN_BOX ? bin : (bin == BIN_BOX ? 0 : bin - 1); }
 
-__global__ void np_classify(NpArgs A, int* lists, int list_stride, int* counts, int* box_count, int* box_sep_count,
-                            int* hull_count);
+__global__ void np_classify(NpArgs A, int* lists, int list_stride, int* counts);
 // The lists np_pairs takes and the bins they hold, the longest tests first.
-constexpr int kNpLists = ALGO_COUNT + 1;
-constexpr int kNpOrder[kNpLists] = {ALGO_POLY_POLY, ALGO_CAPSULE_POLY, ALGO_SPHERE_POLY, ALGO_CONCAVE, ALGO_COUNT,
-                                    ALGO_COUNT + 1, ALGO_CAPSULE_CAPSULE, ALGO_SPHERE_CAPSULE, ALGO_SPHERE_SPHERE};
+constexpr int kNpLists = kNpBins - 1;
+constexpr int kNpOrder[kNpLists] = {ALGO_POLY_POLY, ALGO_CAPSULE_POLY, ALGO_SPHERE_POLY, BIN_BOX, BIN_POLY_POLY_SEP,
+                                    BIN_CAPSULE_POLY_SEP, BIN_SPHERE_POLY_SEP, ALGO_CONCAVE, BIN_BOX_SEP,
+                                    ALGO_CAPSULE_CAPSULE, ALGO_SPHERE_CAPSULE, ALGO_SPHERE_SPHERE};
+// Pairs a wavefront takes of a list of n: a power of two, as few as keep kNpWaves wavefronts for the list.
+// With few pairs the chip has SIMDs to spare, and a wavefront is faster with fewer: it runs the shared searches
+// of polyhedra one pair after another, and pairs that part at a branch one side after the other.  Pairs of 1000
+// boxes (3,952): 81 us with 64 a wavefront, 60 with 8; triangle tests of 600 bodies on a mesh 315 and 248.
+constexpr int kNpWaves = 2048;
+__host__ __device__ inline int np_wave_pairs(int bin, int n) {
+    int p = bin == ALGO_POLY_POLY || bin == BIN_POLY_POLY_SEP ? 2 : 8;
+    while (p < 64 && p * kNpWaves < n) p *= 2;
+    return p;
+}
 struct NpLists {
     const int* list[kNpLists];
     const int* count[kNpLists];
@@ -96,6 +98,10 @@ struct NpLists {
 // np_pairs runs in workgroups of exactly this many threads (the boxes' clip buffers are sliced from LDS by
 // threadIdx.x)
 constexpr int kNpThreads = 128;
+__host__ __device__ inline int np_tiles(int bin, int n) {   // workgroups' worth of a list
+    const int p = np_wave_pairs(bin, n) * (kNpThreads / 64);
+    return (n + p - 1) / p;
+}
 __global__ void np_pairs(NpArgs A, NpLists L);   // convex vs concave pairs: the middle phase (lists the triangle tests)
 void upload_box_topology(const int* edges4, const int* face_edge, const int* face_verts);
 // convex vs concave pairs: the tests, then per pair the potential manifolds, their reduction and the warm-start

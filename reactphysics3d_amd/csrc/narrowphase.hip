@@ -182,6 +182,14 @@ struct IdxList {
     __device__ void set(int i, int x) { v = (v & ~(15ull << (4 * i))) | ((uint64_t)x << (4 * i)); }
 };
 
+// LDS of a narrowphase workgroup: the clip buffers of its box pairs, or the search tables of its mesh pairs
+// (a workgroup has pairs of one kind).
+constexpr int kNpLdsFloats = 2 * 3 * 8 * kNpThreads;
+__device__ __forceinline__ float* np_lds() {
+    __shared__ float4 s_np[kNpLdsFloats / 4];
+    return reinterpret_cast<float*>(s_np);
+}
+
 // Clip buffers of one thread.  General polyhedra keep them in private arrays; the box-box kernel keeps
 // them in a strided slice of its workgroup's LDS, so that it needs no scratch memory.
 template <int CM>
@@ -425,7 +433,7 @@ __device__ __forceinline__ bool face_contacts(bool refIs1, const Poly& P1, const
     if constexpr (BOX) {
         // one slice per thread of the np_box_box workgroup (kNpThreads threads), shared by every
         // inlined call site of the test
-        __shared__ float s_box_clip[2 * 3 * kBoxClip * kNpThreads];
+        float* s_box_clip = np_lds();
         LdsClip bufA{s_box_clip + threadIdx.x};
         LdsClip bufB{s_box_clip + 3 * kBoxClip * kNpThreads + threadIdx.x};
         return sat_face_contacts_t<kBoxClip>(refIs1, P1, P2, t12, t21, minFace, T1, T2, raw, bufA, bufB);
@@ -780,11 +788,9 @@ __device__ inline uint32_t lf_after_test(uint32_t lf, bool colliding) {
 // Middle phase: bucket the tested pairs by algorithm; a pair is tested only if at least one of its
 // bodies is enabled (CD.cpp:391-400).  Untested pairs have no contact pair this step.  The list order
 // is irrelevant because every test writes only its own pair slot.
-// Polyhedron pairs are split further (np_list_slot): box-box pairs that collided in the last step go
-// to list slot 0 (ALGO_NONE is never listed) counted in box_count, the other box-box pairs to slot
-// ALGO_COUNT counted in box_sep_count (a wave of either kind follows one path through the test), pairs
-// with a mesh stay in the ALGO_POLY_POLY slot counted in hull_count; counts[ALGO_POLY_POLY] keeps the
-// total.  Each workgroup counts its pairs per bin first and reserves one contiguous range per bin with
+// Polyhedron tests are split further, by shape and by whether the pair collided in the last step (BIN_*): a
+// wavefront of either kind follows one path through the test, and a separated pair is mostly decided by its
+// cached axis.  Each workgroup counts its pairs per bin first and reserves one contiguous range per bin with
 // a single global atomic (same-address atomics from every wave serialise in the L2), then lists its
 // pairs into those ranges.
 __device__ __forceinline__ int np_bin(const NpArgs& A, int k, bool count_pass) {
@@ -813,59 +819,58 @@ __device__ __forceinline__ int np_bin(const NpArgs& A, int k, bool count_pass) {
         return 0;
     }
     const int a = A.P.algo[k];
-    if (a == ALGO_POLY_POLY && A.C.type[c.x] == SHAPE_BOX && A.C.type[c.y] == SHAPE_BOX)   // box-box
-        return (A.P.lf[k] & LF_WAS_COLLIDING) ? ALGO_COUNT : ALGO_COUNT + 1;
-    return a;
+    if (a != ALGO_POLY_POLY && a != ALGO_CAPSULE_POLY && a != ALGO_SPHERE_POLY) return a;
+    const bool colliding = (A.P.lf[k] & LF_WAS_COLLIDING) != 0;
+    if (a == ALGO_CAPSULE_POLY) return colliding ? a : BIN_CAPSULE_POLY_SEP;
+    if (a == ALGO_SPHERE_POLY) return colliding ? a : BIN_SPHERE_POLY_SEP;
+    if (A.C.type[c.x] == SHAPE_BOX && A.C.type[c.y] == SHAPE_BOX) return colliding ? BIN_BOX : BIN_BOX_SEP;
+    return colliding ? a : BIN_POLY_POLY_SEP;
 }
 
-__global__ __launch_bounds__(256) void np_classify(NpArgs A, int* lists, int list_stride, int* counts, int* box_count,
-                                                   int* box_sep_count, int* hull_count) {
-    constexpr int kBins = kNpBins;
-    __shared__ int s_cnt[kBins];
-    __shared__ int s_base[kBins];
-    __shared__ int s_cur[kBins];
+__global__ __launch_bounds__(256) void np_classify(NpArgs A, int* lists, int list_stride, int* counts) {
+    __shared__ int s_cnt[kNpBins];
+    __shared__ int s_base[kNpBins];
     const int np = *A.nb_pairs;
     const int stride = gridDim.x * blockDim.x;
     const int lane = lane_id();
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    if (threadIdx.x < kBins) {
-        s_cnt[threadIdx.x] = 0;
-        s_cur[threadIdx.x] = 0;
-    }
+    if (threadIdx.x < kNpBins) s_cnt[threadIdx.x] = 0;
     __syncthreads();
-    for (int base = blockIdx.x * blockDim.x; base < np; base += stride) {
+    // calls f(bin, lanes of the wavefront in it) for every bin among the lanes' b
+    auto each_bin = [&](int b, auto f) {
+        uint64_t todo = __ballot(b > 0);
+        while (todo) {
+            const int t = __builtin_amdgcn_readlane(b, __ffsll((unsigned long long)todo) - 1);
+            const uint64_t m = __ballot(b == t);
+            todo &= ~m;
+            f(t, m);
+        }
+    };
+    uint32_t known = 0;   // the bins of the thread's first eight pairs, four bits each
+    static_assert(kNpBins <= 16, "four bits a bin");
+    for (int base = blockIdx.x * blockDim.x, j = 0; base < np; base += stride, j++) {
         const int k = base + threadIdx.x;
         const int b = k < np ? np_bin(A, k, true) : 0;
-        for (int t = 1; t < kBins; t++) {
-            const uint64_t m = __ballot(b == t);
-            if (m && lane == __ffsll((unsigned long long)m) - 1) atomicAdd(&s_cnt[t], __popcll(m));
-        }
+        if (j < 8) known |= (uint32_t)b << (4 * j);
+        each_bin(b, [&](int t, uint64_t m) {
+            if (lane == __ffsll((unsigned long long)m) - 1) atomicAdd(&s_cnt[t], __popcll(m));
+        });
     }
     __syncthreads();
-    if (threadIdx.x < kBins && threadIdx.x > 0) {
+    if (threadIdx.x < kNpBins) {
         const int t = threadIdx.x, n = s_cnt[t];
-        int* ctr = t == ALGO_COUNT ? box_count
-                   : t == ALGO_COUNT + 1 ? box_sep_count
-                   : t == ALGO_POLY_POLY ? hull_count : &counts[t];
-        s_base[t] = n ? atomicAdd(ctr, n) : 0;
-        if (t == ALGO_POLY_POLY) {
-            const int polys = n + s_cnt[ALGO_COUNT] + s_cnt[ALGO_COUNT + 1];
-            if (polys) atomicAdd(&counts[ALGO_POLY_POLY], polys);
-        }
+        s_base[t] = n ? atomicAdd(&counts[t], n) : 0;
     }
     __syncthreads();
-    for (int base = blockIdx.x * blockDim.x; base < np; base += stride) {
+    for (int base = blockIdx.x * blockDim.x, j = 0; base < np; base += stride, j++) {
         const int k = base + threadIdx.x;
-        const int b = k < np ? np_bin(A, k, false) : 0;
-        for (int t = 1; t < kBins; t++) {
-            const uint64_t m = __ballot(b == t);
-            if (m == 0) continue;
+        const int b = j < 8 ? (known >> (4 * j)) & 15 : (k < np ? np_bin(A, k, false) : 0);
+        each_bin(b, [&](int t, uint64_t m) {
             const int leader = __ffsll((unsigned long long)m) - 1;
             int pos = 0;
-            if (lane == leader) pos = atomicAdd(&s_cur[t], __popcll(m));
-            pos = __shfl(pos, leader, kWave) + s_base[t] + __popcll(m & lt);
-            if (b == t) lists[np_list_slot(t) * list_stride + pos] = k;
-        }
+            if (lane == leader) pos = atomicAdd(&s_base[t], __popcll(m));
+            pos = __builtin_amdgcn_readlane(pos, leader) + __popcll(m & ((1ull << lane) - 1ull));
+            if (b == t) lists[(size_t)np_list_slot(t) * list_stride + pos] = k;
+        });
     }
 }
 
@@ -986,19 +991,22 @@ __device__ __forceinline__ int sat_edge_pairs(const Poly& P1, const Poly& P2, in
     h2 = (P2.nhalfedges() + 1) / 2;
     return ((P1.nhalfedges() + 1) / 2) * h2;
 }
-__device__ __forceinline__ bool sat_edge_pair(const Poly& P1, const Poly& P2, const Tf& t12, int k, int h2, float& pen,
-                                              V3* axis_out = nullptr) {
-    const int i = 2 * (k / h2), j = 2 * (k % h2);
-    const int4 e1 = P1.edge(i);
-    const int4 e2 = P2.edge(j);
-    if (!sat_minkowski_face(P1, e1, P2, e2, t12)) return false;
+// penetration along the cross product of edges e1 and e2
+__device__ __forceinline__ float sat_edge_pen(const Poly& P1, const Poly& P2, const Tf& t12, int4 e1, int4 e2, V3& axis) {
     const V3 e1a = tapply(t12, P1.vertex(e1.x));
     const V3 e1b = tapply(t12, P1.vertex(P1.edge(e1.w).x));
     const V3 e2a = P2.vertex(e2.x);
     const V3 e2b = P2.vertex(P2.edge(e2.w).x);
+    return sat_edge_distance(e1a, e2a, tapply(t12, P1.centroid()), e1b - e1a, e2b - e2a, axis, P1.tri(),
+                             P1.tri() ? P2.centroid() : v3zero());
+}
+__device__ __forceinline__ bool sat_edge_pair(const Poly& P1, const Poly& P2, const Tf& t12, int k, int h2, float& pen,
+                                              V3* axis_out = nullptr) {
+    const int4 e1 = P1.edge(2 * (k / h2));
+    const int4 e2 = P2.edge(2 * (k % h2));
+    if (!sat_minkowski_face(P1, e1, P2, e2, t12)) return false;
     V3 axis = v3zero();
-    pen = sat_edge_distance(e1a, e2a, tapply(t12, P1.centroid()), e1b - e1a, e2b - e2a, axis, P1.tri(),
-                            P1.tri() ? P2.centroid() : v3zero());
+    pen = sat_edge_pen(P1, P2, t12, e1, e2, axis);
     if (axis_out) *axis_out = axis;
     return true;
 }
@@ -1014,10 +1022,10 @@ struct EdgeSearch {
     int k;       // first pair of the smallest penetration among the others, INT_MAX when none
     float pen;   // its penetration (+inf when none)
     __device__ void init(float start = __builtin_huge_valf()) { sep = INT_MAX; k = INT_MAX; pen = start; }
-    __device__ void visit(int kk, bool valid, float p) {   // in increasing kk within one lane
+    __device__ void visit(int kk, bool valid, float p) {
         if (!valid) return;
         if (p <= 0.0f) { if (kk < sep) sep = kk; return; }
-        if (p < pen) { pen = p; k = kk; }
+        if (p < pen || (p == pen && k != INT_MAX && kk < k)) { pen = p; k = kk; }
     }
     __device__ void combine(const EdgeSearch& o) {
         if (o.sep < sep) sep = o.sep;
@@ -1059,11 +1067,11 @@ __device__ __forceinline__ bool sat_finish(const Poly& P1, const Poly& P2, const
 }
 
 // One search shared by the wavefront for every lane in m (wave-uniform): the lane's colliders (ca, cb)
-// and transform t are broadcast, each lane evaluates every 64th candidate kk < count(B1, B2) with
-// eval(B1, B2, tb, kk, pen) -> valid, and the combined result lands in es of the lane it belongs to.
-template <bool BOX, class Count, class Eval>
+// and transform t are broadcast, search(B1, B2, tb, w) adds the lane's share of the candidates to w, and the
+// combined result lands in es of the lane it belongs to.
+template <bool BOX, class Search>
 __device__ __forceinline__ void shared_search(const NpArgs& A, uint64_t m, int lane, const Tf& t, int ca, int cb,
-                                              float start, EdgeSearch& es, Count count, Eval eval) {
+                                              float start, EdgeSearch& es, Search search) {
     while (m) {
         const int L = __ffsll((unsigned long long)m) - 1;
         m &= m - 1;
@@ -1071,17 +1079,12 @@ __device__ __forceinline__ void shared_search(const NpArgs& A, uint64_t m, int l
         tb.p = v3(__shfl(t.p.x, L), __shfl(t.p.y, L), __shfl(t.p.z, L));
         tb.q.x = __shfl(t.q.x, L); tb.q.y = __shfl(t.q.y, L);
         tb.q.z = __shfl(t.q.z, L); tb.q.w = __shfl(t.q.w, L);
-        const int cx = __shfl(ca, L), cy = __shfl(cb, L);
+        const int cx = __builtin_amdgcn_readlane(ca, L), cy = __builtin_amdgcn_readlane(cb, L);
         const Poly B1 = BOX ? box_poly(A, cx) : make_poly(A, cx);
         const Poly B2 = BOX ? box_poly(A, cy) : make_poly(A, cy);
-        const int np = count(B1, B2);
         EdgeSearch w;
         w.init(start);
-        for (int kk = lane; kk < np; kk += kWave) {
-            float p = 0.0f;
-            const bool v = eval(B1, B2, tb, kk, p);
-            w.visit(kk, v, p);
-        }
+        search(B1, B2, tb, w);
         for (int off = kWave / 2; off > 0; off >>= 1) {
             EdgeSearch o;
             o.sep = __shfl_xor(w.sep, off);
@@ -1091,6 +1094,106 @@ __device__ __forceinline__ void shared_search(const NpArgs& A, uint64_t m, int l
         }
         if (lane == L) es = w;
     }
+}
+
+// The wavefront's own part of the workgroup's LDS, and the order of its lanes' accesses to it.
+constexpr int kSearchVecs = kNpLdsFloats / 4 / (kNpThreads / kWave);
+__device__ __forceinline__ float4* search_lds() {
+    return reinterpret_cast<float4*>(np_lds()) + kSearchVecs * (threadIdx.x / kWave);
+}
+__device__ __forceinline__ void search_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Faces of B1 as separating planes, a lane each, B2's vertices in LDS: every lane walks all of them for its
+// support point, and from memory each step of that walk was a load of its own to wait for.
+__device__ __forceinline__ void mesh_face_search(const Poly& B1, const Poly& B2, const Tf& tb, int lane, EdgeSearch& w) {
+    float4* s_v = search_lds();
+    const int nv = B2.hull >= 0 ? B2.h.nv : 0, nf = B1.nfaces();
+    const bool staged = nv > 0;   // (a mesh has at most 255 half-edges)
+    static_assert(kSearchVecs >= 255 && kSearchVecs >= 3 * kWave + 2 * kWave / 4, "search tables");
+    search_fence();
+    if (staged)
+        for (int i = lane; i < nv; i += kWave) s_v[i] = B2.hv[B2.h.vbase + i];
+    search_fence();
+    for (int f = lane; f < nf; f += kWave) {
+        float pen;
+        if (staged) {   // sat_single_face with Poly::support over the staged vertices
+            const V3 n2 = qrot(tb.q, B1.face_normal(f));
+            const V3 d = -n2;
+            float best = kDecimalSmallest;
+            V3 sp = xyz(s_v[0]);
+            for (int i = 0; i < nv; i++) {
+                const V3 v = xyz(s_v[i]);
+                const float dp = dot(d, v);
+                if (dp > best) { sp = v; best = dp; }
+            }
+            const V3 fv = tapply(tb, B1.vertex(B1.face_vertex(f, 0)));
+            pen = dot(fv - sp, n2);
+        } else {
+            pen = sat_single_face(B1, B2, tb, f);
+        }
+        w.visit(f, true, pen);
+    }
+}
+
+// The edge pairs of two polyhedra.  What the Minkowski test reads of an edge (two face normals and the edge's
+// direction) is prepared once an edge instead of once a pair: 64 edges of B2 in the lanes' registers, 64 of B1
+// at a time in LDS, read by all lanes at once.  Few pairs pass the test; they are listed and their penetrations
+// found 64 at a time, where nearly every step of a walk over all pairs waited for some lane's.  6,000 convex
+// meshes of 24 points (66 edges): 224 us for the step's pairs, 492 in a walk with each edge pair from memory.
+__device__ __forceinline__ void mesh_edge_search(const Poly& B1, const Poly& B2, const Tf& tb, int lane, EdgeSearch& w) {
+    float4* s_e = search_lds();                                  // [3 * edge]: a | b | b x a
+    int* s_pass = reinterpret_cast<int*>(s_e + 3 * kWave);       // pairs that passed
+    int h2;
+    sat_edge_pairs(B1, B2, h2);
+    const int h1 = (B1.nhalfedges() + 1) / 2;
+    int pass = 0;
+    auto measure = [&](int n) {   // the first n listed pairs, at most 64
+        search_fence();
+        if (lane < n) {
+            const int kk = s_pass[lane];
+            V3 axis;
+            w.visit(kk, true, sat_edge_pen(B1, B2, tb, B1.edge(2 * (kk / h2)), B2.edge(2 * (kk % h2)), axis));
+        }
+        search_fence();
+    };
+    for (int j0 = 0; j0 < h2; j0 += kWave) {
+        const int j = min(j0 + lane, h2 - 1);
+        const int4 e2 = B2.edge(2 * j), o2 = B2.edge(e2.y);
+        const V3 nc = -B2.face_normal(e2.z), nd = -B2.face_normal(o2.z);
+        const V3 dxc = B2.vertex(e2.x) - B2.vertex(o2.x);
+        for (int i0 = 0; i0 < h1; i0 += kWave) {
+            const int ni = min(kWave, h1 - i0);
+            search_fence();
+            if (lane < ni) {
+                const int4 e1 = B1.edge(2 * (i0 + lane)), o1 = B1.edge(e1.y);
+                s_e[3 * lane] = f4(qrot(tb.q, B1.face_normal(e1.z)), 0.f);
+                s_e[3 * lane + 1] = f4(qrot(tb.q, B1.face_normal(o1.z)), 0.f);
+                s_e[3 * lane + 2] = f4(qrot(tb.q, B1.vertex(e1.x) - B1.vertex(o1.x)), 0.f);
+            }
+            search_fence();
+            for (int i = 0; i < ni; i++) {
+                const V3 a = xyz(s_e[3 * i]), b = xyz(s_e[3 * i + 1]), bxa = xyz(s_e[3 * i + 2]);
+                const float cba = dot(nc, bxa), dba = dot(nd, bxa), adc = dot(a, dxc), bdc = dot(b, dxc);
+                const bool ok = j0 + lane < h2 && cba * dba < 0.0f && adc * bdc < 0.0f && cba * bdc > 0.0f;
+                const uint64_t m = __ballot(ok);
+                if (m == 0) continue;
+                if (ok) s_pass[pass + __popcll(m & ((1ull << lane) - 1ull))] = (i0 + i) * h2 + j;
+                pass += __popcll(m);
+                if (pass >= kWave) {
+                    measure(kWave);
+                    pass -= kWave;
+                    int rest = 0;
+                    if (lane < pass) rest = s_pass[kWave + lane];
+                    search_fence();
+                    if (lane < pass) s_pass[lane] = rest;
+                }
+            }
+        }
+    }
+    measure(pass);
 }
 
 // sat_faces (SATAlgorithm.cpp:1119-1143) as a shared search: the first face with pen <= 0, else the
@@ -1140,14 +1243,12 @@ __device__ __forceinline__ void sat_pairs(const NpArgs& A, const int* list, int 
     if constexpr (!BOX) {
         // mesh pairs share the two face searches as well (each face's support point walks every
         // vertex of the other mesh)
-        auto nfaces = [](const Poly& B1, const Poly&) { return B1.nfaces(); };
-        auto face_pen = [](const Poly& B1, const Poly& B2, const Tf& tb, int f, float& p) {
-            p = sat_single_face(B1, B2, tb, f);
-            return true;
+        auto faces = [&](const Poly& B1, const Poly& B2, const Tf& tb, EdgeSearch& w) {
+            mesh_face_search(B1, B2, tb, lane, w);
         };
         EdgeSearch fs;
         fs.init(kDecimalLargest);
-        shared_search<BOX>(A, __ballot(stage == 3), lane, t12, c.x, c.y, kDecimalLargest, fs, nfaces, face_pen);
+        shared_search<BOX>(A, __ballot(stage == 3), lane, t12, c.x, c.y, kDecimalLargest, fs, faces);
         int face1 = 0, face2 = 0;
         float pen1 = 0.0f;
         if (stage == 3) {
@@ -1158,7 +1259,7 @@ __device__ __forceinline__ void sat_pairs(const NpArgs& A, const int* list, int 
             }
         }
         fs.init(kDecimalLargest);
-        shared_search<BOX>(A, __ballot(stage == 3), lane, t21, c.y, c.x, kDecimalLargest, fs, nfaces, face_pen);
+        shared_search<BOX>(A, __ballot(stage == 3), lane, t21, c.y, c.x, kDecimalLargest, fs, faces);
         if (stage == 3) {
             const float pen2 = face_search_result(fs, face2);
             if (fs.sep != INT_MAX) {
@@ -1187,16 +1288,20 @@ __device__ __forceinline__ void sat_pairs(const NpArgs& A, const int* list, int 
             }
         }
     } else {
-        auto npairs = [](const Poly& B1, const Poly& B2) {
-            int h2;
-            return sat_edge_pairs(B1, B2, h2);
+        auto edges = [&](const Poly& B1, const Poly& B2, const Tf& tb, EdgeSearch& w) {
+            if constexpr (BOX) {
+                int h2;
+                const int np = sat_edge_pairs(B1, B2, h2);
+                for (int kk = lane; kk < np; kk += kWave) {
+                    float p = 0.0f;
+                    const bool v = sat_edge_pair(B1, B2, tb, kk, h2, p);
+                    w.visit(kk, v, p);
+                }
+            } else {
+                mesh_edge_search(B1, B2, tb, lane, w);
+            }
         };
-        auto edge_pen = [](const Poly& B1, const Poly& B2, const Tf& tb, int kk, float& p) {
-            int h2;
-            sat_edge_pairs(B1, B2, h2);
-            return sat_edge_pair(B1, B2, tb, kk, h2, p);
-        };
-        shared_search<BOX>(A, m, lane, t12, c.x, c.y, __builtin_huge_valf(), es, npairs, edge_pen);
+        shared_search<BOX>(A, m, lane, t12, c.x, c.y, __builtin_huge_valf(), es, edges);
     }
     if (act) {
         bool hit = stage == 1;
@@ -1901,7 +2006,7 @@ __device__ __forceinline__ void np_concave_mid(const NpArgs& A, int k) {
     A.P.ctn[k] = n;
 }
 
-// Every pair of the step, 128 of one test list to a workgroup; the workgroups share out the lists by their
+// Every pair of the step, each workgroup some of one test list; the workgroups share out the lists by their
 // counts, the longest tests first.  A launch a list took 6 us for each of up to eight lists, empty ones too, and
 // the lists that are there waited for each other's last wavefront: a colliding box pair is a chain of some
 // 30 us however few there are, and so are a capsule's or a mesh's.  All lists' launches before, and now: 27 boxes
@@ -1918,7 +2023,7 @@ __global__ __launch_bounds__(kNpThreads, 3) void np_pairs(NpArgs A, NpLists L) {
         int run = 0;
         for (int i = 0; i < kNpLists; i++) {
             s_first[i] = run;
-            run += (s_count[i] + kNpThreads - 1) / kNpThreads;
+            run += np_tiles(kNpOrder[i], s_count[i]);
         }
         s_first[kNpLists] = run;
     }
@@ -1928,15 +2033,16 @@ __global__ __launch_bounds__(kNpThreads, 3) void np_pairs(NpArgs A, NpLists L) {
         int i = 0;
         while (w >= s_first[i + 1]) i++;
         i = __builtin_amdgcn_readfirstlane(i);
-        const int n = s_count[i], t = (w - s_first[i]) * kNpThreads + threadIdx.x;
         const int* list = L.list[i];
-        const int bin = kNpOrder[i];
-        if (bin == ALGO_POLY_POLY) sat_pairs<false, Raw>(A, list, n, t, kWave);
-        else if (bin == ALGO_COUNT || bin == ALGO_COUNT + 1) sat_pairs<true, RawBoxView>(A, list, n, t, 32);
+        const int bin = kNpOrder[i], n = s_count[i], p = np_wave_pairs(bin, n);
+        const int first = ((w - s_first[i]) * (kNpThreads / kWave) + (int)threadIdx.x / kWave) * p;
+        const int t = lane_id() < p ? first + lane_id() : n;
+        if (bin == ALGO_POLY_POLY || bin == BIN_POLY_POLY_SEP) sat_pairs<false, Raw>(A, list, n, t, kWave);
+        else if (bin == BIN_BOX || bin == BIN_BOX_SEP) sat_pairs<true, RawBoxView>(A, list, n, t, 32);
         else if (t < n) {
             const int k = list[t];
-            if (bin == ALGO_CAPSULE_POLY) np_capsule_poly(A, k);
-            else if (bin == ALGO_SPHERE_POLY) np_sphere_poly(A, k);
+            if (bin == ALGO_CAPSULE_POLY || bin == BIN_CAPSULE_POLY_SEP) np_capsule_poly(A, k);
+            else if (bin == ALGO_SPHERE_POLY || bin == BIN_SPHERE_POLY_SEP) np_sphere_poly(A, k);
             else if (bin == ALGO_CONCAVE) np_concave_mid(A, k);
             else if (bin == ALGO_CAPSULE_CAPSULE) np_capsule_capsule(A, k);
             else if (bin == ALGO_SPHERE_CAPSULE) np_sphere_capsule(A, k);
@@ -1949,8 +2055,10 @@ __global__ __launch_bounds__(kNpThreads, 3) void np_pairs(NpArgs A, NpLists L) {
 // shape with the pair's algorithm, the triangle's LastFrameCollisionInfo (kept by the pair for the
 // triangles it tested in the last step, OverlappingPairs.h:231-294) and smoothed contacts.
 __global__ __launch_bounds__(128) void np_concave_tri(NpArgs A) {
-    const int n = min(*A.CT.count, A.CT.cap);
-    RP3DG_GRID_STRIDE(t, n) {
+    const int n = min(*A.CT.count, A.CT.cap), p = np_wave_pairs(ALGO_CONCAVE, n);
+    if (lane_id() >= p) return;
+    const int waves = gridDim.x * (blockDim.x / kWave), wave = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    for (int t = wave * p + lane_id(); t < n; t += waves * p) {
         const int k = A.CT.pair[t];
         if (k < 0) continue;
         const int id = A.CT.tri[t];
@@ -2115,8 +2223,10 @@ struct IntList {
 // smallest largest depth removed first, swapped with the last), each reduced to four points and without
 // duplicates, then the warm-start transfer over the pair's previous manifolds (initContactsWithPreviousOnes,
 // :1069-1160) and the cache write: manifold 0 in the pair's entry, the others in tail entries.
-__global__ void np_concave_reduce(NpArgs A, const int* list, const int* count) {
-    RP3DG_GRID_STRIDE(t, *count) {
+__global__ __launch_bounds__(64) void np_concave_reduce(NpArgs A, const int* list, const int* count) {
+    const int n = *count, p = np_wave_pairs(ALGO_CONCAVE, n);
+    if (lane_id() >= p) return;
+    for (int t = blockIdx.x * p + lane_id(); t < n; t += gridDim.x * p) {
         const int k = list[t];
         DevPairs P = A.P;
         const DevPairs& O = A.O;

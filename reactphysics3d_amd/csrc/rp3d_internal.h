@@ -214,10 +214,16 @@ struct Settings {
 constexpr int kColorRoundsMax = 48;   // parallel colouring rounds launched at most per step
 
 // Per-step counters, cleared by a fill kernel at the start of every step and read back after it.
+// Narrowphase bins: the algorithms, with the polyhedron tests split by shape and by whether the pair collided in
+// the last step (a separated one is mostly decided by its cached axis).  ALGO_* holds the colliding ones.
+constexpr int BIN_BOX = ALGO_COUNT, BIN_BOX_SEP = ALGO_COUNT + 1, BIN_POLY_POLY_SEP = ALGO_COUNT + 2,
+              BIN_CAPSULE_POLY_SEP = ALGO_COUNT + 3, BIN_SPHERE_POLY_SEP = ALGO_COUNT + 4;
+constexpr int kNpBins = ALGO_COUNT + 5;
+
 struct DevCounters {
     int nb_pairs;              // pairs in the current table
     int nb_overlaps;           // overlapping pairs found by the traversal (may exceed the capacity)
-    int nb_tests[ALGO_COUNT];
+    int nb_bin[kNpBins];       // tests per narrowphase bin
     int nb_manifolds;
     int nb_points;
     int nb_colors;
@@ -225,9 +231,6 @@ struct DevCounters {
     int finish_rounds;         // rounds taken by the single-workgroup colouring finisher
     int nb_new_points;         // contact points without a cached impulse
     int color_left[kColorRoundsMax];   // set: manifolds left uncoloured by each colouring launch
-    int nb_box_tests;          // box-box subset of nb_tests[ALGO_POLY_POLY] that collided last step
-    int nb_box_sep_tests;      // box-box pairs that did not (cheap temporal-coherence rejects, listed apart)
-    int nb_hull_tests;         // the rest of nb_tests[ALGO_POLY_POLY] (a convex mesh involved)
     int nb_large;              // colliders with more overlaps than their broadphase slab holds
     int nb_events;             // contact events of the step (may exceed the event buffer)
     int nb_concave_tests;      // triangle tests of the convex vs concave pairs
