@@ -143,6 +143,7 @@ struct rp3dg_batch {
 
     // launch hints from the last completed step (grids are grid-stride, any size is correct)
     int hint_pairs = 0, hint_manifolds = 0, hint_rounds = 8;
+    int hint_colors = 0;               // colours of the last step whose first rows are in hseg (fused), or 0
     rp3dg::DevCounters last{};         // counters of the last completed step
 
     // captured step graphs, one per pair-table parity
@@ -200,7 +201,7 @@ struct rp3dg_batch {
 
     rp3dg::DevCounters* counters = nullptr;
     rp3dg::DevCounters* hcounters = nullptr;
-    int* hseg = nullptr;               // per-colour layout: first row of every colour
+    int* hseg = nullptr;               // first row of every colour (per-colour layout, split solve)
 
     bool profiling = false;
     std::string profile_only;          // time only this kernel (empty: all)
@@ -216,6 +217,11 @@ struct rp3dg_batch {
     int class_block(int max_bodies) const;
     int launch_world_classes(const char* name, const rp3dg::FusedArgs& F);
     int upload_joints(rp3dg_world* const* worlds, int n);
+    static int color_tail(const int* rows, int ncol);
+    void color_warmstart(const rp3dg::SvArgs& SA, const int* rows, int tail, int ncol);
+    void color_sweep(const rp3dg::SvArgs& SA, const int* rows, int tail, int ncol, float beta_dt);
+    bool one_group() const;
+    bool split_solve() const;
     void enqueue_sleep(float dt, const rp3dg::DevPairs& N, int pair_grid);
     int enqueue_step(float dt, bool capturing);
     int finish_steps(int n);

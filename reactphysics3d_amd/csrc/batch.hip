@@ -189,6 +189,9 @@ using namespace rp3dg;
         }                                                                                        \
     } while (0)
 
+// rows of a split solve at least: in all, and a colour on average
+constexpr int kSplitRows = 1000, kSplitColorRows = 150;
+
 static int grid_for(int n, int threads = 256, int max_blocks = 4096) {
     int g = (n + threads - 1) / threads;
     if (g < 1) g = 1;
@@ -1476,8 +1479,22 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
                          nullptr, row_slot, S.pred);
             }
         }
-        r = launch_world_classes("sv_world_solve", F);
-        if (r) return r;
+        if (split_solve()) {
+            int rows[kMaxColors];   // as in the last step and a quarter more; the rest of the colours go with the tail
+            for (int c = 0; c < hint_colors; c++) {
+                const int n = hseg[c + 1] - hseg[c];
+                rows[c] = n + n / 4;
+            }
+            const int tail = color_tail(rows, hint_colors);
+            color_warmstart(SA, rows, tail, kMaxColors);
+            for (int it = 0; it < settings.vel_iters; it++) color_sweep(SA, rows, tail, kMaxColors, beta_dt);
+            LAUNCH_T("sv_store", mg, 256, sv_store, SA);
+            LAUNCH_T("sv_note_iterations", grid_for(nworlds), 256, sv_note_iterations, world_iters, world_res, nworlds,
+                     settings.vel_iters);
+        } else {
+            r = launch_world_classes("sv_world_solve", F);
+            if (r) return r;
+        }
         if (log_cap > 0) {
             LAUNCH_T("sv_log_samples", grid_for(feat_cap), 256, sv_log_samples, F, log_feats, log_targets, log_count,
                      log_cap);
@@ -1506,35 +1523,22 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     HIPCHECK(hipMemcpyAsync(hseg, seg_start, sizeof(int) * (kMaxColors + 1), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
     const int ncol = hcounters->nb_colors;
-    // The last colours, at most kTailRows rows each, go to one workgroup in one launch (one such colour would
-    // gain nothing), the others to a launch each that has a quad for every row.  65,536-body heap, 16 colours
-    // of 31,890 to 4 rows: 10 us a launch with the grid of a mean colour
-    int tail = ncol;
-    while (tail > 0 && hseg[tail] - hseg[tail - 1] <= kTailRows) tail--;
-    if (ncol - tail < 2) tail = ncol;
-    auto color_grid = [&](int c) { return grid_for(4 * (hseg[c + 1] - hseg[c]), color_block, 1 << 16); };
+    int rows[kMaxColors];
+    for (int c = 0; c < ncol; c++) rows[c] = hseg[c + 1] - hseg[c];
     const int bg = grid_for(nb);
     // inverse world inertia + velocity integration (PhysicsWorld.cpp:266-272), contact and joint rows
     if (J.bfirst) LAUNCH_T("fill_int", grid_for(nworlds), 256, fill_int, J.bfirst, nworlds, INT_MAX);
     LAUNCH_T("sv_setup", grid_for(nb + hm + J.n + 128), 256, sv_setup, SA, J, settings, dt);
     // contact solver (PhysicsWorld.cpp:321-345)
     const int jg = grid_for(std::max(J.n, 1)), jg2 = grid_for(std::max(2 * J.n, 1));
-    for (int c = 0; c < tail; c++) LAUNCH_T("sv_warmstart", color_grid(c), color_block, sv_warmstart, SA, c);
-    if (tail < ncol) LAUNCH_T("sv_warmstart", 1, 4 * kTailRows, sv_warmstart_tail, SA, tail, ncol);
+    const int tail = color_tail(rows, ncol);
+    color_warmstart(SA, rows, tail, ncol);
     // ConstraintSolverSystem::initialize: warm start of every joint kind
     for (int s = 0; s < jt_slots; s++) LAUNCH_T("jt_warmstart", jg, 256, jt_warmstart, B, J, jt_ranges, s);
     for (int it = 0; it < settings.vel_iters; it++) {
         for (int s = 0; s < jt_slots; s++)
             LAUNCH_T("jt_solve_velocity", jg2, 256, jt_solve_velocity, B, J, jt_ranges, s, jt_kind[s], dt);
-        for (int c = 0; c < tail; c++) {
-            if (settings.split_impulse)
-                LAUNCH_T("sv_solve_color", color_grid(c), color_block, sv_solve_color<true>, SA, c, beta_dt);
-            else LAUNCH_T("sv_solve_color", color_grid(c), color_block, sv_solve_color<false>, SA, c, beta_dt);
-        }
-        if (tail < ncol) {
-            if (settings.split_impulse) LAUNCH_T("sv_solve_color", 1, 4 * kTailRows, sv_solve_tail<true>, SA, tail, ncol, beta_dt);
-            else LAUNCH_T("sv_solve_color", 1, 4 * kTailRows, sv_solve_tail<false>, SA, tail, ncol, beta_dt);
-        }
+        color_sweep(SA, rows, tail, ncol, beta_dt);
     }
     LAUNCH_T("sv_store", mg, 256, sv_store, SA);
     // position integration, joint position correction, state update, refit (PhysicsWorld.cpp:275-288, :348-360)
@@ -1548,12 +1552,51 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
     return RP3DG_OK;
 }
 
+// Sweeps by colour over the whole batch.  The last colours, at most kTailRows rows each, go to one workgroup in
+// one launch (one such colour would gain nothing), the others to a launch each that has a quad for every row.
+// 65,536-body heap, 16 colours of 31,890 to 4 rows: 10 us a launch with the grid of a mean colour.
+int rp3dg_batch::color_tail(const int* rows, int ncol) {
+    int tail = ncol;
+    while (tail > 0 && rows[tail - 1] <= kTailRows) tail--;
+    return ncol - tail < 2 ? ncol : tail;
+}
+
+void rp3dg_batch::color_warmstart(const SvArgs& SA, const int* rows, int tail, int ncol) {
+    for (int c = 0; c < tail; c++)
+        LAUNCH_T("sv_warmstart", grid_for(4 * rows[c], color_block, 1 << 16), color_block, sv_warmstart, SA, c);
+    if (tail < ncol) LAUNCH_T("sv_warmstart", 1, 4 * kTailRows, sv_warmstart_tail, SA, tail);
+}
+
+void rp3dg_batch::color_sweep(const SvArgs& SA, const int* rows, int tail, int ncol, float beta_dt) {
+    for (int c = 0; c < tail; c++) {
+        const int grid = grid_for(4 * rows[c], color_block, 1 << 16);
+        if (settings.split_impulse) LAUNCH_T("sv_solve_color", grid, color_block, sv_solve_color<true>, SA, c, beta_dt);
+        else LAUNCH_T("sv_solve_color", grid, color_block, sv_solve_color<false>, SA, c, beta_dt);
+    }
+    if (tail < ncol) {
+        if (settings.split_impulse) LAUNCH_T("sv_solve_color", 1, 4 * kTailRows, sv_solve_tail<true>, SA, tail, beta_dt);
+        else LAUNCH_T("sv_solve_color", 1, 4 * kTailRows, sv_solve_tail<false>, SA, tail, beta_dt);
+    }
+}
+
 // PhysicsWorld::updateSleepingBodies (PhysicsWorld.cpp:871-926), after the colliders are refit
 void rp3dg_batch::enqueue_sleep(float dt, const DevPairs& N, int pair_grid) {
     if (!settings.sleeping_enabled) return;
     LAUNCH_T("isl_sleep", grid_for(nb), 256, isl_sleep_time, B, isl, settings, dt);
     LAUNCH_T("isl_sleep", grid_for(nb), 256, isl_sleep, B, isl, settings);
     LAUNCH_T("isl_sleep", pair_grid, 256, isl_reset_disabled_pairs, B, C, N, &counters->nb_pairs);
+}
+
+// A fused batch of one group, without joints, at a fixed number of iterations may be solved by launches over all
+// CUs instead of by the group's one workgroup: its rows are in colour order as a whole.  In one workgroup a
+// sweep takes as long as one CU needs to issue its rows and the colours' phases some 2.4 us each at least; a
+// launch a colour takes some 5 us, the tail 3 us a colour.  A step in one workgroup and split: heaps of 605
+// bodies (1,360 rows, 13 colours) 398 and 455 us, 1,005 (2,355, 11) 502 and 491, 2,005 (4,708, 14) 789 and 579,
+// 4,095 (9,541, 14) 1839 and 773; piles of 1,001 boxes (1,194, 6) 484 and 466, 3,501 (4,315, 8) 1221 and 598.
+bool rp3dg_batch::one_group() const { return fused && ngroups == 1 && J.n == 0; }
+bool rp3dg_batch::split_solve() const {
+    return one_group() && res_thr <= 0.0f && hint_colors > 0 &&
+           hint_manifolds >= std::max(kSplitRows, kSplitColorRows * hint_colors);
 }
 
 using SolveKernel = void (*)(FusedArgs);
@@ -1632,7 +1675,10 @@ int rp3dg_batch::launch_world_classes(const char* name, const FusedArgs& F0) {
 int rp3dg_batch::finish_steps(int n) {
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipMemcpyAsync(hcounters, counters, sizeof(DevCounters), hipMemcpyDeviceToHost, stream));
+    const bool colors = one_group() && hint_manifolds >= kSplitRows;
+    if (colors) HIPCHECK(hipMemcpyAsync(hseg, seg_start, sizeof(int) * (kMaxColors + 1), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
+    hint_colors = colors ? std::min(kMaxColors, hcounters->nb_colors) : 0;
     timer_flush();
     last = *hcounters;
     steps_done += n;

@@ -62,8 +62,9 @@ __global__ void sv_color_keys(const int* color, const int* nm_ptr, uint64_t* key
 __global__ void sv_warmstart(SvArgs A, int color);
 constexpr int kTailRows = 256;   // rows at most of a colour that one workgroup takes in a pass
 template <bool SPLIT>
-__global__ void sv_solve_tail(SvArgs A, int c0, int c1, float beta_dt);
-__global__ void sv_warmstart_tail(SvArgs A, int c0, int c1);
+__global__ void sv_solve_tail(SvArgs A, int c0, float beta_dt);
+__global__ void sv_warmstart_tail(SvArgs A, int c0);
+__global__ void sv_note_iterations(int* world_iters, float* world_res, int n, int iters);
 template <bool SPLIT>
 __global__ void sv_solve_color(SvArgs A, int color, float beta_dt);   // one quad of lanes per manifold
 __global__ void sv_store(SvArgs A);

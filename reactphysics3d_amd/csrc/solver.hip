@@ -46,25 +46,34 @@ __global__ __launch_bounds__(512) void sv_solve_color(SvArgs A, int color, float
 template __global__ void sv_solve_color<true>(SvArgs A, int color, float beta_dt);
 template __global__ void sv_solve_color<false>(SvArgs A, int color, float beta_dt);
 
-// The colours [c0, c1) one after another in one workgroup: the last colours of a batch have a few rows each,
+// The colours from c0 on, one after another in one workgroup: the last colours of a batch have a few rows each,
 // and a launch of their own costs twice what the rows do.
 template <bool SPLIT>
-__global__ __launch_bounds__(4 * kTailRows) void sv_solve_tail(SvArgs A, int c0, int c1, float beta_dt) {
+__global__ __launch_bounds__(4 * kTailRows) void sv_solve_tail(SvArgs A, int c0, float beta_dt) {
     const QuadSrc Q(A.S, threadIdx.x);
+    const int c1 = *A.ncolors;
     for (int c = c0; c < c1; c++) {
         const int lo = A.cstart[c], n = 4 * (A.cstart[c + 1] - lo);
         for (int t = threadIdx.x; t < n; t += 4 * kTailRows) quad_sweep_row<STATE_HBM, SPLIT>(A, Q, lo + (t >> 2), beta_dt);
         __syncthreads();
     }
 }
-template __global__ void sv_solve_tail<true>(SvArgs A, int c0, int c1, float beta_dt);
-template __global__ void sv_solve_tail<false>(SvArgs A, int c0, int c1, float beta_dt);
-__global__ __launch_bounds__(4 * kTailRows) void sv_warmstart_tail(SvArgs A, int c0, int c1) {
+template __global__ void sv_solve_tail<true>(SvArgs A, int c0, float beta_dt);
+template __global__ void sv_solve_tail<false>(SvArgs A, int c0, float beta_dt);
+__global__ __launch_bounds__(4 * kTailRows) void sv_warmstart_tail(SvArgs A, int c0) {
     const QuadSrc Q(A.S, threadIdx.x);
+    const int c1 = *A.ncolors;
     for (int c = c0; c < c1; c++) {
         const int lo = A.cstart[c], n = 4 * (A.cstart[c + 1] - lo);
         for (int t = threadIdx.x; t < n; t += 4 * kTailRows) quad_warmstart(A, Q, lo + (t >> 2));
         __syncthreads();
+    }
+}
+
+__global__ void sv_note_iterations(int* world_iters, float* world_res, int n, int iters) {
+    RP3DG_GRID_STRIDE(w, n) {
+        world_iters[w] = iters;
+        world_res[w] = 0.0f;
     }
 }
 
