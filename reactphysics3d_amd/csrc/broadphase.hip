@@ -280,13 +280,6 @@ __global__ __launch_bounds__(256) void bp_tiles(DevColliders C, const int* sorte
     }
 }
 
-__device__ __forceinline__ float4 wave_read4(float4 v, int lane) {
-    return make_float4(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.x), lane)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.y), lane)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.z), lane)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.w), lane)));
-}
-
 // Does collider c emit the pair (c, o)?  (Their boxes overlap; both are of one world.)
 __device__ __forceinline__ bool emits(const DevColliders& C, int c, int o, const NoColLists& L) {
     return o != c && (C.is_static[o] || o > c) && pair_allowed(C, c, o, L);
@@ -294,8 +287,10 @@ __device__ __forceinline__ bool emits(const DevColliders& C, int c, int o, const
 
 // One workgroup per tile of 64 querying colliders, one per lane, the same in every wavefront.  The
 // wavefronts share the tiles whose box meets the queries': a wavefront loads a tile's boxes (one per lane),
-// drops those outside the queries' union, and every lane tests its box against the others one by one from
-// scalar registers.  A tree walk is a chain of dependent loads per collider with most lanes of a wavefront
+// drops those outside the queries' union, and every lane tests its box against the others eight at a time from
+// scalar registers, collecting a bit for each (one at a time, read from the lanes that hold them, with the
+// bookkeeping of a hit after every test: 36 us for 1001 boxes, 74 for 3,006 bodies, 129 for 6,965, in index
+// order; now 30, 56 and 93).  A tree walk is a chain of dependent loads per collider with most lanes of a wavefront
 // waiting for the deepest; here every load is a full tile, and the arithmetic grows with the overlapping
 // tiles only.  Overlaps are collected in LDS, filtered (pair_allowed), sorted by rank and written to the
 // collider's slab; count[c] = its partners.  A collider with more overlaps than the slab holds is counted
@@ -305,8 +300,14 @@ __global__ __launch_bounds__(1024) void bp_pairs(DevColliders C, int n, const fl
                                                  int* count, int* slab, int* large, int* nb_large) {
     __shared__ int s_cnt[kTile], s_id[kTile];
     __shared__ int s_list[kTile][kSlab];
+    __shared__ int2 s_box[1024 / kWave][kTile];   // the collider and kind of a wavefront's current boxes
     __shared__ int s_total;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, nw = blockDim.x / kWave;
+    typedef float Vec4 __attribute__((ext_vector_type(4)));
+    using BoxTable = const __attribute__((address_space(4))) Vec4*;   // read through the scalar cache
+    const BoxTable bmin = (BoxTable)(uintptr_t)smn, bmax = (BoxTable)(uintptr_t)smx;
+    constexpr int kBoxGroup = 8;   // boxes loaded and tested at a time
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), nw = blockDim.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int nt = (n + kTile - 1) / kTile;
     const int s0 = blockIdx.x * kTile + lane;
     float4 qmn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), qmx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
@@ -355,17 +356,36 @@ __global__ __launch_bounds__(1024) void bp_pairs(DevColliders C, int n, const fl
                 bmn = smn[s];
                 bmx = smx[s];
             }
-            unsigned long long cand = __ballot(s < n && aabb_overlap(umn, umx, bmn, bmx));
-            while (cand) {
-                const int q = __ffsll(cand) - 1;
-                cand &= cand - 1;
-                const float4 amn = wave_read4(bmn, q), amx = wave_read4(bmx, q);
-                const int o = __float_as_int(amn.w), t = __float_as_int(amx.w);
-                if (aabb_overlap(qmn, qmx, amn, amx) && (t >> 1) == world && o != c && ((t & 1) || o > c)) {
+            const unsigned long long cand = __ballot(s < n && aabb_overlap(umn, umx, bmn, bmx));
+            if (!cand) continue;
+            s_box[wave][lane] = make_int2(__float_as_int(bmn.w), __float_as_int(bmx.w));
+            const int base = __builtin_amdgcn_readfirstlane((T0 + k) * kTile);
+            unsigned long long hits = 0;
+            for (int g = 0; g < kTile; g += kBoxGroup) {
+                if (!((cand >> g) & ((1u << kBoxGroup) - 1u))) continue;
+                unsigned int bits = 0;
+#pragma unroll
+                for (int j = 0; j < kBoxGroup; j++) {
+                    const int i = min(base + g + j, n - 1);   // (beyond n: no candidate)
+                    const Vec4 a = bmin[i], b = bmax[i];
+                    const bool apart = (qmx.x < a.x) | (b.x < qmn.x) | (qmx.y < a.y) | (b.y < qmn.y) | (qmx.z < a.z) |
+                                       (b.z < qmn.z);   // aabb_overlap
+                    bits |= apart ? 0u : 1u << j;
+                }
+                hits |= (unsigned long long)bits << g;
+            }
+            hits &= cand;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            while (hits) {
+                const int q = __ffsll(hits) - 1;
+                hits &= hits - 1;
+                const int o = s_box[wave][q].x, t = s_box[wave][q].y;
+                if ((t >> 1) == world && o != c && ((t & 1) || o > c)) {
                     const int pos = atomicAdd(&s_cnt[lane], 1);
                     if (pos < kSlab) s_list[lane][pos] = o;
                 }
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
     }
     __syncthreads();
