@@ -1131,6 +1131,8 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     alloc_bytes.push_back(sizeof(DevCounters));
     HIPCHECK(hipHostMalloc(&hcounters, sizeof(DevCounters), hipHostMallocDefault));
     HIPCHECK(hipHostMalloc(&hseg, sizeof(int) * (kMaxColors + 1), hipHostMallocDefault));
+    // for bodies and forces (pinning memory takes some 300 us: not in the first call that passes them)
+    if (const int rs = stage_reserve(std::min(kStageBytes, (size_t)nb * 13 * sizeof(float) + 64))) return rs;
     HIPCHECK(hipMemsetAsync(counters, 0, sizeof(DevCounters), stream));
     if (!sort_offs || !S.lam || !S.lq) { set_error("device allocation failed (pair arenas)"); return RP3DG_EHIP; }
     // collider creation: world transforms, initial fat AABBs, all colliders in the moved set
