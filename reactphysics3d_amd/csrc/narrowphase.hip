@@ -2010,8 +2010,8 @@ __device__ __forceinline__ void np_concave_mid(const NpArgs& A, int k) {
 // counts, the longest tests first.  A launch a list took 6 us for each of up to eight lists, empty ones too, and
 // the lists that are there waited for each other's last wavefront: a colliding box pair is a chain of some
 // 30 us however few there are, and so are a capsule's or a mesh's.  All lists' launches before, and now: 27 boxes
-// 99 and 52 us, 1000 boxes 165 and 81, 65,536 spheres, boxes and capsules 360 and 188, 600 bodies on a mesh
-// (middle phase included) 375 and 142.
+// 99 and 46 us, 1000 boxes 165 and 62, 65,536 spheres, boxes and capsules 360 and 200, 600 bodies on a mesh
+// (middle phase included) 375 and 128.
 // Box-box pairs: the box topology is known at compile time and the buffers are box-sized; a lane's own
 // walk over the 144 edge pairs costs about as much as 32 shared searches, hence the limit.  Pairs with a
 // convex mesh (the general buffers): their edge searches run over hundreds of pairs, so they are always shared.
@@ -2369,6 +2369,9 @@ __global__ __launch_bounds__(64) void np_concave_reduce(NpArgs A, const int* lis
                 P.pl1[4 * slot + i] = f4(l1, imp);
                 P.pl2[4 * slot + i] = f4(xyz(A.cp_l2[r]), resting);
             }
+            // tail entries go to pairs in the order the wavefronts come: nothing of a former owner stays in them
+            for (int i = n; j > 0 && i < kMaxManifoldPoints; i++)
+                P.pn[4 * slot + i] = P.pl1[4 * slot + i] = P.pl2[4 * slot + i] = make_float4(0.f, 0.f, 0.f, 0.f);
             P.fv1[slot] = fv1;
             P.fv2[slot] = fv2;
             P.fimp[slot] = fimp;
