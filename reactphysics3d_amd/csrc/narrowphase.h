@@ -95,9 +95,18 @@ struct NpLists {
     const int* list[kNpLists];
     const int* count[kNpLists];
 };
-// np_pairs runs in workgroups of exactly this many threads (the boxes' clip buffers are sliced from LDS by
-// threadIdx.x)
+// np_pairs runs in workgroups of exactly this many threads.
 constexpr int kNpThreads = 128;
+// LDS of a narrowphase wavefront: the clip buffers of its box pairs (two a lane), or the search tables of its mesh
+// pairs.  A wavefront goes on to its workgroup's next tile, of whatever list, without waiting for the other, so
+// each keeps to a part of its own, the same for both uses.
+constexpr int kBoxClip = 8;   // vertices of a box face clipped by the four side planes at most
+constexpr int kNpWaveFloats = 2 * 3 * kBoxClip * 64;
+__host__ __device__ constexpr int np_wave_lds(int thread) { return thread / 64 * kNpWaveFloats; }
+// component c of vertex i in clip buffer b of a thread (consecutive lanes, consecutive words)
+__host__ __device__ constexpr int np_clip_lds(int thread, int b, int i, int c) {
+    return np_wave_lds(thread) + (3 * (kBoxClip * b + i) + c) * 64 + thread % 64;
+}
 __host__ __device__ inline int np_tiles(int bin, int n) {   // workgroups' worth of a list
     const int p = np_wave_pairs(bin, n) * (kNpThreads / 64);
     return (n + p - 1) / p;

@@ -182,16 +182,14 @@ struct IdxList {
     __device__ void set(int i, int x) { v = (v & ~(15ull << (4 * i))) | ((uint64_t)x << (4 * i)); }
 };
 
-// LDS of a narrowphase workgroup: the clip buffers of its box pairs, or the search tables of its mesh pairs
-// (a workgroup has pairs of one kind).
-constexpr int kNpLdsFloats = 2 * 3 * 8 * kNpThreads;
+// LDS of a narrowphase workgroup, a part for each wavefront (np_wave_lds, np_clip_lds).
 __device__ __forceinline__ float* np_lds() {
-    __shared__ float4 s_np[kNpLdsFloats / 4];
+    __shared__ float4 s_np[kNpWaveFloats / 4 * (kNpThreads / kWave)];
     return reinterpret_cast<float*>(s_np);
 }
 
-// Clip buffers of one thread.  General polyhedra keep them in private arrays; the box-box kernel keeps
-// them in a strided slice of its workgroup's LDS, so that it needs no scratch memory.
+// Clip buffers of one thread.  General polyhedra keep them in private arrays; box-box tests keep them in a
+// strided slice of their wavefront's LDS, so that they need no scratch memory.
 template <int CM>
 struct PrivClip {
     V3 v[CM];
@@ -199,14 +197,14 @@ struct PrivClip {
     __device__ void put(int i, V3 x) { v[i] = x; }
 };
 struct LdsClip {
-    float* p;   // component c of vertex i at p[(3 * i + c) * kNpThreads]
+    float* p;   // component c of vertex i at p[(3 * i + c) * kWave] (np_clip_lds)
     __device__ V3 get(int i) const {
-        return v3(p[(3 * i) * kNpThreads], p[(3 * i + 1) * kNpThreads], p[(3 * i + 2) * kNpThreads]);
+        return v3(p[(3 * i) * kWave], p[(3 * i + 1) * kWave], p[(3 * i + 2) * kWave]);
     }
     __device__ void put(int i, V3 x) {
-        p[(3 * i) * kNpThreads] = x.x;
-        p[(3 * i + 1) * kNpThreads] = x.y;
-        p[(3 * i + 2) * kNpThreads] = x.z;
+        p[(3 * i) * kWave] = x.x;
+        p[(3 * i + 1) * kWave] = x.y;
+        p[(3 * i + 2) * kWave] = x.z;
     }
 };
 
@@ -256,8 +254,6 @@ struct RawBoxView {
         return refIs1 ? project_point_onto_plane(c, axisRef, refV) : tapply(refToInc, c);
     }
 };
-
-constexpr int kBoxClip = 8;     // vertices of a box face clipped by the four side planes at most
 
 // ------------------------------------------------------------------------------------------------
 // SAT, polyhedron vs polyhedron (SATAlgorithm.cpp:485-1191)
@@ -431,11 +427,9 @@ template <bool BOX, class R>
 __device__ __forceinline__ bool face_contacts(bool refIs1, const Poly& P1, const Poly& P2, const Tf& t12, const Tf& t21,
                                               int minFace, const Tf& T1, const Tf& T2, R& raw) {
     if constexpr (BOX) {
-        // one slice per thread of the np_box_box workgroup (kNpThreads threads), shared by every
-        // inlined call site of the test
-        float* s_box_clip = np_lds();
-        LdsClip bufA{s_box_clip + threadIdx.x};
-        LdsClip bufB{s_box_clip + 3 * kBoxClip * kNpThreads + threadIdx.x};
+        // the thread's two buffers, shared by every inlined call site of the test
+        LdsClip bufA{np_lds() + np_clip_lds(threadIdx.x, 0, 0, 0)};
+        LdsClip bufB{np_lds() + np_clip_lds(threadIdx.x, 1, 0, 0)};
         return sat_face_contacts_t<kBoxClip>(refIs1, P1, P2, t12, t21, minFace, T1, T2, raw, bufA, bufB);
     } else {
         return sat_face_contacts(refIs1, P1, P2, t12, t21, minFace, T1, T2, raw);
@@ -1097,9 +1091,9 @@ __device__ __forceinline__ void shared_search(const NpArgs& A, uint64_t m, int l
 }
 
 // The wavefront's own part of the workgroup's LDS, and the order of its lanes' accesses to it.
-constexpr int kSearchVecs = kNpLdsFloats / 4 / (kNpThreads / kWave);
+constexpr int kSearchVecs = kNpWaveFloats / 4;
 __device__ __forceinline__ float4* search_lds() {
-    return reinterpret_cast<float4*>(np_lds()) + kSearchVecs * (threadIdx.x / kWave);
+    return reinterpret_cast<float4*>(np_lds() + np_wave_lds(threadIdx.x));
 }
 __device__ __forceinline__ void search_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -2037,6 +2031,7 @@ __global__ __launch_bounds__(kNpThreads, 3) void np_pairs(NpArgs A, NpLists L) {
         const int bin = kNpOrder[i], n = s_count[i], p = np_wave_pairs(bin, n);
         const int first = ((w - s_first[i]) * (kNpThreads / kWave) + (int)threadIdx.x / kWave) * p;
         const int t = lane_id() < p ? first + lane_id() : n;
+        search_fence();   // the last tile's test has done with the wavefront's LDS
         if (bin == ALGO_POLY_POLY || bin == BIN_POLY_POLY_SEP) sat_pairs<false, Raw>(A, list, n, t, kWave);
         else if (bin == BIN_BOX || bin == BIN_BOX_SEP) sat_pairs<true, RawBoxView>(A, list, n, t, 32);
         else if (t < n) {

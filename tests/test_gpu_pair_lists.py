@@ -1,6 +1,6 @@
-"""One narrowphase launch takes the test lists of all pair types, 128 pairs of a list to a workgroup.  Batches
-with one, almost, exactly and more than a workgroup's pairs of several types at once give every pair the
-contacts it has alone."""
+"""One narrowphase launch takes the test lists of all pair types; a workgroup has 4 mesh pairs or 16 others of a
+list (np_tiles), more in long lists.  Batches with one, almost, exactly and more than that of several types at once,
+and with more such shares than workgroups, give every pair the contacts it has alone."""
 import numpy as np
 import pytest
 
@@ -27,10 +27,10 @@ def _pair(a, b, k):
     return sc
 
 
-def _run(scenes):
+def _run(scenes, steps=3):
     from reactphysics3d_amd.lib import Batch
     dev = Batch(scenes)
-    dev.step(1.0 / 60.0, 3)
+    dev.step(1.0 / 60.0, steps)
     ct, state = dev.contacts(), dev.bodies()
     out = []
     for w, b0 in enumerate(dev.body_base[:len(scenes)]):
@@ -41,17 +41,31 @@ def _run(scenes):
     return out
 
 
-@pytest.mark.parametrize("counts", [(1, 1, 1, 1, 1, 1, 1, 1), (127, 0, 129, 0, 1, 0, 128, 0), (0, 130, 0, 128, 0, 300, 0, 1)])
-def test_every_pair_has_the_contacts_it_has_alone(counts):
-    types = [(S.SPHERE, S.SPHERE), (S.SPHERE, S.CAPSULE), (S.CAPSULE, S.CAPSULE), (S.BOX, S.SPHERE),
-             (S.CAPSULE, S.BOX), (S.BOX, S.BOX), (S.HULL, S.BOX), (S.HULL, S.CAPSULE)]
+TYPES = [(S.SPHERE, S.SPHERE), (S.SPHERE, S.CAPSULE), (S.CAPSULE, S.CAPSULE), (S.BOX, S.SPHERE),
+         (S.CAPSULE, S.BOX), (S.BOX, S.BOX), (S.HULL, S.BOX), (S.HULL, S.CAPSULE), (S.HULL, S.HULL)]
+
+
+def _check(counts, steps):
     kinds = [(t, k % 5) for t, n in enumerate(counts) for k in range(n)]
-    alone = {tk: _run([_pair(*types[tk[0]], tk[1])])[0] for tk in set(kinds)}
+    alone = {tk: _run([_pair(*TYPES[tk[0]], tk[1])], steps)[0] for tk in set(kinds)}
     assert all(len(a[0]) for a in alone.values())
     order = np.random.default_rng(3).permutation(len(kinds))
-    for i, got in zip(order, _run([_pair(*types[kinds[i][0]], kinds[i][1]) for i in order])):
+    for i, got in zip(order, _run([_pair(*TYPES[kinds[i][0]], kinds[i][1]) for i in order], steps)):
         for a, b in zip(alone[kinds[i]], got):
             assert np.array_equal(a, b), kinds[i]
+
+
+@pytest.mark.parametrize("counts", [(1, 1, 1, 1, 1, 1, 1, 1), (127, 0, 129, 0, 1, 0, 128, 0), (0, 130, 0, 128, 0, 300, 0, 1),
+                                    (15, 16, 17, 33, 31, 15, 3, 16, 4), (1, 0, 0, 0, 0, 17, 5, 0, 8)])
+def test_every_pair_has_the_contacts_it_has_alone(counts):
+    _check(counts, 3)
+
+
+# The first step is launched for the counts of a step before it, of which there is none: 72 workgroups.  The mesh and
+# box pairs are 150 and 253 workgroups' shares, so that workgroups go from mesh pairs to box pairs.
+@pytest.mark.parametrize("counts", [(0, 0, 0, 0, 0, 800, 200, 0, 200), (100, 0, 0, 0, 100, 2000, 300, 40, 210)])
+def test_workgroups_with_pairs_of_several_types(counts):
+    _check(counts, 1)
 
 
 # points: 12 (30 edges), 24 (66 edges, two chunks of the edge tables), 44 (the most a mesh may have: 126 edges, 84
