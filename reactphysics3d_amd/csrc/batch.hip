@@ -1320,15 +1320,15 @@ int rp3dg_batch::enqueue_narrowphase(const NpArgs& A, bool capturing, int pg) {
     // workgroups for the last step's counts and a quarter more
     auto more = [&](int n) { return capturing ? pair_cap : std::min(pair_cap, n + n / 4 + 64); };
     for (int i = 0; i < kNpLists; i++) {
-        tiles += np_tiles(kNpOrder[i], more(last.nb_bin[kNpOrder[i]]));
+        tiles += np_grid(kNpOrder[i], more(last.nb_bin[kNpOrder[i]]));
     }
     LAUNCH_T("np_pairs", std::min(tiles, 4096), kNpThreads, np_pairs, A, NL);
     if (has_concave) {   // convex vs concave pairs: triangle tests, manifolds
         const int* lc = L + (size_t)np_list_slot(ALGO_CONCAVE) * pair_cap;
         const int ht = capturing ? A.CT.cap : std::min(A.CT.cap, last.nb_concave_tests + last.nb_concave_tests / 4 + 64);
-        LAUNCH_T("np_concave_tri", std::min(np_tiles(ALGO_CONCAVE, ht), 4096), kNpThreads, np_concave_tri, A);
+        LAUNCH_T("np_concave_tri", std::min(np_grid(ALGO_CONCAVE, ht), 4096), kNpThreads, np_concave_tri, A);
         const int hc = more(last.nb_bin[ALGO_CONCAVE]);
-        LAUNCH_T("np_concave_reduce", std::min(2 * np_tiles(ALGO_CONCAVE, hc), 4096), 64, np_concave_reduce, A, lc, T + ALGO_CONCAVE);
+        LAUNCH_T("np_concave_reduce", std::min(2 * np_grid(ALGO_CONCAVE, hc), 4096), 64, np_concave_reduce, A, lc, T + ALGO_CONCAVE);
     }
 
     return RP3DG_OK;

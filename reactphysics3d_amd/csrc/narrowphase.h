@@ -86,8 +86,9 @@ constexpr int kNpOrder[kNpLists] = {ALGO_POLY_POLY, ALGO_CAPSULE_POLY, ALGO_SPHE
 // of polyhedra one pair after another, and pairs that part at a branch one side after the other.  Pairs of 1000
 // boxes (3,952): 81 us with 64 a wavefront, 60 with 8; triangle tests of 600 bodies on a mesh 315 and 248.
 constexpr int kNpWaves = 2048;
+__host__ __device__ constexpr int np_least_pairs(int bin) { return bin == ALGO_POLY_POLY || bin == BIN_POLY_POLY_SEP ? 2 : 8; }
 __host__ __device__ inline int np_wave_pairs(int bin, int n) {
-    int p = bin == ALGO_POLY_POLY || bin == BIN_POLY_POLY_SEP ? 2 : 8;
+    int p = np_least_pairs(bin);
     while (p < 64 && p * kNpWaves < n) p *= 2;
     return p;
 }
@@ -110,6 +111,16 @@ __host__ __device__ constexpr int np_clip_lds(int thread, int b, int i, int c) {
 __host__ __device__ inline int np_tiles(int bin, int n) {   // workgroups' worth of a list
     const int p = np_wave_pairs(bin, n) * (kNpThreads / 64);
     return (n + p - 1) / p;
+}
+// first pair of a wavefront's share in a tile of a list of n
+__host__ __device__ inline int np_first_pair(int bin, int n, int tile, int wave) {
+    return (tile * (kNpThreads / 64) + wave) * np_wave_pairs(bin, n);
+}
+// Workgroups for a list of any length up to n: a list takes fewer tiles than a shorter one where the share of a
+// wavefront doubles (4,096 mesh pairs are 1,024 tiles, 4,097 are 513), kNpWaves wavefronts' worth before each.
+__host__ __device__ inline int np_grid(int bin, int n) {
+    const int most = kNpWaves / (kNpThreads / 64), t = np_tiles(bin, n);
+    return n > np_least_pairs(bin) * kNpWaves && t < most ? most : t;
 }
 __global__ void np_pairs(NpArgs A, NpLists L);   // convex vs concave pairs: the middle phase (lists the triangle tests)
 void upload_box_topology(const int* edges4, const int* face_edge, const int* face_verts);

@@ -2029,7 +2029,7 @@ __global__ __launch_bounds__(kNpThreads, 3) void np_pairs(NpArgs A, NpLists L) {
         i = __builtin_amdgcn_readfirstlane(i);
         const int* list = L.list[i];
         const int bin = kNpOrder[i], n = s_count[i], p = np_wave_pairs(bin, n);
-        const int first = ((w - s_first[i]) * (kNpThreads / kWave) + (int)threadIdx.x / kWave) * p;
+        const int first = np_first_pair(bin, n, w - s_first[i], threadIdx.x / kWave);
         const int t = lane_id() < p ? first + lane_id() : n;
         search_fence();   // the last tile's test has done with the wavefront's LDS
         if (bin == ALGO_POLY_POLY || bin == BIN_POLY_POLY_SEP) sat_pairs<false, Raw>(A, list, n, t, kWave);

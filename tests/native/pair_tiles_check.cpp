@@ -25,7 +25,33 @@ static int lds_violations() {
     return bad;
 }
 
+// Every pair of a list is in one wavefront's share of one tile, and the grid for n pairs has a workgroup for every
+// tile of any list up to n.
+static void list_violations(int& shares, int& grid) {
+    shares = grid = 0;
+    for (int bin : {(int)ALGO_POLY_POLY, BIN_POLY_POLY_SEP, BIN_BOX, (int)ALGO_CONCAVE, (int)ALGO_SPHERE_SPHERE}) {
+        std::vector<unsigned char> taken;
+        for (int n = 0, most = 0; n < 300000; n += n < 20000 ? 1 : 611) {
+            const int tiles = np_tiles(bin, n), p = np_wave_pairs(bin, n);
+            most = tiles > most ? tiles : most;
+            if (np_grid(bin, n) < most) grid++;
+            if (p < 1 || p > 64) shares++;
+            if (n > 1200 && n % 97) continue;
+            taken.assign(n, 0);
+            for (int t = 0; t < tiles; t++)
+                for (int w = 0; w < kNpThreads / 64; w++)
+                    for (int l = 0; l < p; l++) {
+                        const int k = np_first_pair(bin, n, t, w) + l;
+                        if (k < n) taken[k]++;
+                    }
+            for (int k = 0; k < n; k++) shares += taken[k] != 1;
+        }
+    }
+}
+
 int main() {
-    printf("lds %d\n", lds_violations());
+    int shares, grid;
+    list_violations(shares, grid);
+    printf("lds %d\nshares %d\ngrid %d\n", lds_violations(), shares, grid);
     return 0;
 }

@@ -8,6 +8,8 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 
+pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not available")
+
 
 @pytest.fixture(scope="module")
 def violations(tmp_path_factory):
@@ -19,6 +21,13 @@ def violations(tmp_path_factory):
     return {line.split()[0]: int(line.split()[1]) for line in out.splitlines()}
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not available")
 def test_a_wavefront_keeps_to_its_part_of_the_lds(violations):
     assert violations["lds"] == 0
+
+
+def test_every_pair_of_a_list_is_in_one_share(violations):
+    assert violations["shares"] == 0
+
+
+def test_the_grid_has_a_workgroup_for_every_tile_of_a_shorter_list(violations):
+    assert violations["grid"] == 0
