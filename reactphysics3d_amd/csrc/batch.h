@@ -63,12 +63,12 @@ struct rp3dg_batch {
     // solver layout: fused = one workgroup per world for the whole solver phase, (world, colour)-major
     // rows; otherwise one launch per colour over colour-major rows.
     bool fused = false;
-    int fused_block = 64;              // threads per world of the position kernel (and of the single-class solve)
+    int fused_block = 64;              // threads per group of the position kernel
     int color_block = 64;              // per-colour layout: threads per block of the colour kernels (autotuned)
     // fused layout: worlds grouped into size classes (bodies in (L/2, L], L = 64, 128, ... 4096), largest
     // first, `largest` bodies the largest); each class is one launch with its own workgroup size and LDS, the
     // classes run concurrently
-    struct WorldClass { int first, count, max_bodies, largest, block; };
+    struct WorldClass { int first, count, max_bodies, largest; };
     // LDS layout of a class's workgroups (STATE_* of solver_quad.h, bodies and manifolds held)
     struct ClassLds { int state, bodies, rows; };
     ClassLds class_lds(const WorldClass& c) const;
@@ -213,7 +213,6 @@ struct rp3dg_batch {
 
     ~rp3dg_batch();
     int upload(rp3dg_world* const* worlds, int n, const rp3dg_batch_options* opt);
-    void set_class_blocks();
     int class_block(int max_bodies) const;
     int launch_world_classes(const char* name, const rp3dg::FusedArgs& F);
     int upload_joints(rp3dg_world* const* worlds, int n);

@@ -1086,10 +1086,9 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
                 int j = i;
                 while (j < ng && gsize(order[j]) > L / 2) j++;
                 if (L == 64) j = ng;   // everything up to 64 bodies is one class
-                wclasses.push_back({i, j - i, L, sz, 64});
+                wclasses.push_back({i, j - i, L, sz});
                 i = j;
             }
-            set_class_blocks();
             std::vector<int2> cr;
             for (const WorldClass& wc : wclasses) cr.push_back(make_int2(wc.first, wc.count));
             d_class_ranges = dalloc<int2>(this, std::max<size_t>(1, cr.size()));
@@ -1608,10 +1607,6 @@ static const SolveKernel kSolveKernels[2][3] = {   // [split impulses][STATE_*]
 
 // Workgroup size of every world class: clamp(2 L / block_div, 64, 1024).  Four lanes solve a manifold and
 // a world of n bodies has about n / 6 to n / 4 manifolds a colour, so L threads fill the colour phases.
-void rp3dg_batch::set_class_blocks() {
-    for (WorldClass& c : wclasses)
-        c.block = class_block(c.max_bodies);
-}
 int rp3dg_batch::class_block(int L) const {
     // (with a CU for every group, a wavefront for every strand of joints costs nothing)
     const int least = jt_slots > 0 && ngroups <= 256 ? kWave * kJointStrands : kWave;
@@ -1633,7 +1628,7 @@ rp3dg_batch::ClassLds rp3dg_batch::class_lds(const WorldClass& c) const {
         l.bodies = 0;
     }
     const size_t base = fused_lds_bytes(l.state, l.bodies, 0);
-    int k = std::max(1, std::min(16 * kWave / c.block, (ngroups + 255) / 256));
+    int k = std::max(1, std::min(16 * kWave / class_block(c.max_bodies), (ngroups + 255) / 256));
     const size_t rows_min = (size_t)(c.largest + c.largest / 8) * kRow;   // 1.1 manifolds a body
     while (k > 1 && base + rows_min + kStatic > cu / k) k--;
     const size_t share = std::min(cu / k, block_max + kStatic) - kStatic;
@@ -1661,7 +1656,7 @@ int rp3dg_batch::launch_world_classes(const char* name, const FusedArgs& F0) {
         F.lds_rows = l.rows;
         const size_t shmem = fused_lds_bytes(l.state, l.bodies, l.rows);
         hipStream_t s = c == 0 ? stream : side_streams[c - 1];
-        kSolveKernels[settings.split_impulse ? 1 : 0][l.state]<<<wc.count, wc.block, shmem, s>>>(F);
+        kSolveKernels[settings.split_impulse ? 1 : 0][l.state]<<<wc.count, class_block(wc.max_bodies), shmem, s>>>(F);
     }
     if (nclass > 1) {
         for (int c = 1; c < nclass; c++) {
@@ -2843,7 +2838,7 @@ int rp3dg_batch_autotune(rp3dg_batch* b, float dt, int32_t steps_per_trial, int3
     int best = -1;
     double best_t = 1e300;
     for (int c : cand) {
-        if (b->fused) { b->block_div = c; b->set_class_blocks(); }
+        if (b->fused) b->block_div = c;
         else b->color_block = c;
         int r = b->step(dt);   // one untimed step with the new shape
         if (r) { b->profiling = prof; return r; }
@@ -2859,7 +2854,7 @@ int rp3dg_batch_autotune(rp3dg_batch* b, float dt, int32_t steps_per_trial, int3
         b->tune_table.push_back({c, ms});
         if (ms < best_t) { best_t = ms; best = c; }
     }
-    if (b->fused) { b->block_div = best; b->set_class_blocks(); }
+    if (b->fused) b->block_div = best;
     else b->color_block = best;
     b->profiling = prof;
     if (chosen) *chosen = best;
@@ -2897,7 +2892,6 @@ int rp3dg_batch_set_solver_shape(rp3dg_batch* b, int32_t choice) {
             return RP3DG_EINVAL;
         }
         b->block_div = choice;
-        b->set_class_blocks();
     } else {
         if (choice < 64 || choice > 512 || choice % 64) { set_error("per-colour layout: threads per block 64..512"); return RP3DG_EINVAL; }
         b->color_block = choice;

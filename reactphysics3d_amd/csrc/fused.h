@@ -53,7 +53,8 @@ constexpr int kPositionLds = 64;       // LDS bytes of a body in the position ke
 // long as its longest strand and not as the number of kinds and colours in the group.  Where that would be
 // longer (one large component, that many wavefronts share better), strand 0 has every segment of the group
 // and the workgroup takes them together, with a barrier after each (w = 1).  64 joints of 3 kinds in 24
-// components: a joint sweep is 2 phases long instead of 6, and sv_world_solve takes 78 us instead of 123.
+// components: a joint sweep is 2 phases long instead of 6, and sv_world_solve takes 65 us instead of 123 (80 on two
+// wavefronts, which take two strands each one after the other).
 constexpr int kJointStrands = 4;
 constexpr int kMaxJointSegs = 256;     // of a group with several strands
 constexpr int kGroupMaxWorlds = 64;   // worlds per group at most (one bit each in the convergence mask)
