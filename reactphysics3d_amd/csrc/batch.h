@@ -146,10 +146,13 @@ struct rp3dg_batch {
     int hint_colors = 0;               // colours of the last step whose first rows are in hseg (fused), or 0
     rp3dg::DevCounters last{};         // counters of the last completed step
 
-    // captured step graphs, one per pair-table parity
-    hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
-    hipGraph_t graph[2] = {nullptr, nullptr};
+    // captured step graphs, one per route of the solver (split solve or not) and pair-table parity
+    hipGraphExec_t graph_exec[2][2] = {};
+    hipGraph_t graph[2][2] = {};
     float graph_dt = 0.0f;
+    int graph_tail = 0;                       // first colour of the captured split solve's tail
+    int graph_rows[rp3dg::kMaxColors] = {};   // rows of a colour that it is captured for at least
+    void drop_route(int split);
 
     // hull arena
     rp3dg::HullHeader* d_hulls = nullptr;

@@ -1482,11 +1482,15 @@ int rp3dg_batch::enqueue_step(float dt, bool capturing) {
         }
         if (split_solve()) {
             int rows[kMaxColors];   // as in the last step and a quarter more; the rest of the colours go with the tail
-            for (int c = 0; c < hint_colors; c++) {
-                const int n = hseg[c + 1] - hseg[c];
+            int known = 0;
+            for (int c = 0; c < kMaxColors; c++) {
+                const int n = c < hint_colors ? hseg[c + 1] - hseg[c] : 0;
                 rows[c] = n + n / 4;
+                if (capturing) rows[c] = std::max(rows[c], graph_rows[c]);
+                if (rows[c] > 0) known = c + 1;
             }
-            const int tail = color_tail(rows, hint_colors);
+            const int tail = color_tail(rows, known);
+            if (capturing) graph_tail = tail;
             color_warmstart(SA, rows, tail, kMaxColors);
             for (int it = 0; it < settings.vel_iters; it++) color_sweep(SA, rows, tail, kMaxColors, beta_dt);
             LAUNCH_T("sv_store", mg, 256, sv_store, SA);
@@ -1675,7 +1679,9 @@ int rp3dg_batch::finish_steps(int n) {
     const bool colors = one_group() && hint_manifolds >= kSplitRows;
     if (colors) HIPCHECK(hipMemcpyAsync(hseg, seg_start, sizeof(int) * (kMaxColors + 1), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
-    hint_colors = colors ? std::min(kMaxColors, hcounters->nb_colors) : 0;
+    const bool grown = !colors && one_group() && hcounters->nb_manifolds >= kSplitRows;
+    if (grown) HIPCHECK(hipMemcpy(hseg, seg_start, sizeof(int) * (kMaxColors + 1), hipMemcpyDeviceToHost));
+    hint_colors = colors || grown ? std::min(kMaxColors, hcounters->nb_colors) : 0;
     timer_flush();
     last = *hcounters;
     steps_done += n;
@@ -1695,6 +1701,14 @@ int rp3dg_batch::finish_steps(int n) {
     int used = 0;
     while (used < kColorRoundsMax && last.color_left[used] != 0) used++;
     hint_rounds = used + 2;
+    if (graph_exec[1][0]) {   // captured again when a colour has outgrown the tail (each colour at most once)
+        bool outgrown = false;
+        for (int c = graph_tail; c < hint_colors; c++) outgrown = outgrown || hseg[c + 1] - hseg[c] > 2 * kTailRows;
+        if (outgrown) {
+            for (int c = 0; c < hint_colors; c++) graph_rows[c] = std::max(graph_rows[c], hseg[c + 1] - hseg[c]);
+            drop_route(1);
+        }
+    }
     return RP3DG_OK;
 }
 
@@ -1707,18 +1721,24 @@ int rp3dg_batch::step(float dt) {
     return finish_steps(1);
 }
 
-void rp3dg_batch::drop_graphs() {
+void rp3dg_batch::drop_route(int split) {
     for (int p = 0; p < 2; p++) {
-        if (graph_exec[p]) hipGraphExecDestroy(graph_exec[p]);
-        if (graph[p]) hipGraphDestroy(graph[p]);
-        graph_exec[p] = nullptr;
-        graph[p] = nullptr;
+        if (graph_exec[split][p]) hipGraphExecDestroy(graph_exec[split][p]);
+        if (graph[split][p]) hipGraphDestroy(graph[split][p]);
+        graph_exec[split][p] = nullptr;
+        graph[split][p] = nullptr;
     }
+}
+void rp3dg_batch::drop_graphs() {
+    drop_route(0);
+    drop_route(1);
 }
 
 // The pair tables alternate between steps, so two graphs are captured (one per parity) and replayed
-// alternately.  Capture happens once per time-step value; the colouring round count is frozen at
-// capture (the finisher completes any remainder).
+// alternately.  Each route of the solver has its own two, captured when a call first takes it after a change of the
+// time step or a setting (some 1 ms): the route follows the last step's counts, as the eager step's does, so that a
+// world captured while it falls is not solved by one workgroup for good (1160 us a step at 3,001 bodies and 2137
+// at 4,091; 741 and 798 as it is).
 int rp3dg_batch::step_graph(float dt, int n) {
     if (nb == 0 || n <= 0) return RP3DG_OK;
     if (!fused) { set_error("graph capture needs the fused solver layout"); return RP3DG_EUNSUPPORTED; }
@@ -1729,8 +1749,9 @@ int rp3dg_batch::step_graph(float dt, int n) {
         const int r0 = step(dt);
         if (r0 || --n == 0) return r0;
     }
-    if (graph_exec[0] && graph_dt != dt) drop_graphs();
-    if (!graph_exec[0]) {
+    if (graph_dt != dt) drop_graphs();
+    const int route = split_solve() ? 1 : 0;
+    if (!graph_exec[route][0]) {
         const bool start = cur_is_a;
         for (int p = 0; p < 2; p++) {
             const int parity = start == (p == 0) ? 0 : 1;   // parity 0: a -> b
@@ -1747,14 +1768,14 @@ int rp3dg_batch::step_graph(float dt, int n) {
                 if (r) return r;
                 HIPCHECK(e);
             }
-            graph[parity] = g;
-            HIPCHECK(hipGraphInstantiate(&graph_exec[parity], g, nullptr, nullptr, 0));
+            graph[route][parity] = g;
+            HIPCHECK(hipGraphInstantiate(&graph_exec[route][parity], g, nullptr, nullptr, 0));
         }
         cur_is_a = start;   // capture does not run anything; the flips above are undone
         graph_dt = dt;
     }
     for (int i = 0; i < n; i++) {
-        HIPCHECK(hipGraphLaunch(graph_exec[cur_is_a ? 0 : 1], stream));
+        HIPCHECK(hipGraphLaunch(graph_exec[route][cur_is_a ? 0 : 1], stream));
         cur_is_a = !cur_is_a;
     }
     contacts_is_a = cur_is_a;
@@ -1926,7 +1947,8 @@ struct rp3dg_snapshot {
     size_t bytes = 0;
     DevCounters last{};
     bool cur_is_a = true, contacts_is_a = true, ev_pending = false, query_points = false;
-    int contacts_np = 0, hint_pairs = 0, hint_manifolds = 0, hint_rounds = 0;
+    int contacts_np = 0, hint_pairs = 0, hint_manifolds = 0, hint_rounds = 0, hint_colors = 0;
+    int seg[kMaxColors + 1] = {};    // hseg
     int64_t steps_done = 0;
     std::vector<int> body_type, coll_kind;
 };
@@ -1992,6 +2014,8 @@ int rp3dg_batch_snapshot(rp3dg_batch* b, rp3dg_snapshot** out) {
     s->ev_pending = b->ev_pending; s->query_points = b->query_points;
     s->contacts_np = b->contacts_np;
     s->hint_pairs = b->hint_pairs; s->hint_manifolds = b->hint_manifolds; s->hint_rounds = b->hint_rounds;
+    s->hint_colors = b->hint_colors;
+    memcpy(s->seg, b->hseg, sizeof s->seg);
     s->steps_done = b->steps_done;
     s->body_type = b->body_type; s->coll_kind = b->coll_kind;
     *out = s;
@@ -2021,6 +2045,8 @@ int rp3dg_batch_restore(rp3dg_batch* b, const rp3dg_snapshot* s) {
     b->ev_pending = s->ev_pending; b->query_points = s->query_points;
     b->contacts_np = s->contacts_np;
     b->hint_pairs = s->hint_pairs; b->hint_manifolds = s->hint_manifolds; b->hint_rounds = s->hint_rounds;
+    b->hint_colors = s->hint_colors;
+    memcpy(b->hseg, s->seg, sizeof s->seg);
     b->steps_done = s->steps_done;
     b->body_type = s->body_type; b->coll_kind = s->coll_kind;
     for (rp3dg_world* w : b->worlds) w->mirror_dirty = true;
