@@ -107,7 +107,7 @@ BYTE_MODEL = {
     "np_pairs": "176 B/test + 40 B/contact point",
 }
 
-KERNELS = ["bp_bounds", "bp_cells", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
+KERNELS = ["bp_cells", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
            "bp_merge",
            "np_classify", "np_pairs", "sv_flag", "sv_compact", "sv_adj_count", "sv_adj_fill",
            "sv_color_round", "sv_color_finish", "sv_color_keys", "sv_color_sort", "sv_world_ranges", "sv_group_color",

@@ -185,7 +185,8 @@ struct rp3dg_batch {
     int *bp_vals = nullptr, *bp_vtmp = nullptr;
     int* bp_count = nullptr;
     int* bp_offs_ab[2] = {nullptr, nullptr};   // per-collider segment starts of pair table A / B
-    float4* bp_partial = nullptr;
+    int* bp_sample = nullptr;          // moving colliders that give the order its extents
+    int bp_nsample = 0;
     // narrowphase
     int *np_lists = nullptr, *np_counts = nullptr;
     // manifolds / colouring

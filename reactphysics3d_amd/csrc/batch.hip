@@ -21,15 +21,14 @@
 #include "narrowphase.h"
 #include "solver.h"
 #include "solver_quad.h"
+#include "strips.h"
 #include "world.h"
 
 namespace rp3dg {
 
 // broadphase.hip
 __global__ void bp_refit(DevBodies B, DevColliders C, const float4* hull_bounds, int init);
-__global__ void bp_bounds(DevColliders C, float4* partial);
-__global__ void bp_cells(DevColliders C, const float4* partial, int nparts, float world_colliders, uint64_t* keys,
-                         int* vals);
+__global__ void bp_cells(DevColliders C, const int* sample, int nsample, float world_colliders, uint64_t* keys, int* vals);
 template <int ITEMS>
 __global__ void rs_hist(const uint64_t* keys, int n, const int* nptr, int shift, int* hist, int nblocks);
 template <int ITEMS>
@@ -1022,7 +1021,7 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
         if (nc > kIndexOrderColliders) {
             bp_keys = dalloc<uint64_t>(this, nc); bp_vals = dalloc<int>(this, nc);
             bp_ktmp = dalloc<uint64_t>(this, nc); bp_vtmp = dalloc<int>(this, nc);
-            bp_partial = dalloc<float4>(this, 2 * 256);
+            bp_sample = dalloc<int>(this, kOrderSamples);
         }
         bp_smn = dalloc<float4>(this, nc); bp_smx = dalloc<float4>(this, nc);
         bp_tmn = dalloc<float4>(this, nt); bp_tmx = dalloc<float4>(this, nt);
@@ -1182,6 +1181,19 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     C.ss_offs = dalloc<int>(this, nc + 1);
     C.ss_list = dalloc<int>(this, std::max<size_t>(1, ss_list.size()));
     HIPCHECK(hipMemcpy(C.is_static, is_static.data(), sizeof(int) * nc, hipMemcpyHostToDevice));
+    if (bp_sample) {   // one of each 256th of the moving colliders (a floor or wall need not lie where the others are)
+        std::vector<int> moving;
+        for (int i = 0; i < nc; i++)
+            if (!is_static[i]) moving.push_back(i);
+        const size_t m = std::min(moving.size(), (size_t)kOrderSamples);
+        std::vector<int> sample(m);
+        for (size_t k = 0; k < m; k++) {   // at a spread place in it, for colliders that are numbered row by row
+            const size_t lo = k * moving.size() / m, hi = (k + 1) * moving.size() / m;
+            sample[k] = moving[lo + (size_t)((uint32_t)k * 0x9E3779B1u >> 8) % (hi - lo)];
+        }
+        bp_nsample = (int)m;
+        if (m) HIPCHECK(hipMemcpy(bp_sample, sample.data(), sizeof(int) * m, hipMemcpyHostToDevice));
+    }
     HIPCHECK(hipMemcpy(C.ss_offs, ss_offs.data(), sizeof(int) * (nc + 1), hipMemcpyHostToDevice));
     if (!ss_list.empty()) HIPCHECK(hipMemcpy(C.ss_list, ss_list.data(), sizeof(int) * ss_list.size(), hipMemcpyHostToDevice));
     if (settings.sleeping_enabled) {
@@ -1233,9 +1245,7 @@ int rp3dg_batch::enqueue_broadphase(bool capturing, const DevEvents& E, int pg) 
         // more tiles costs less than the launches of the sort
         const int* order = nullptr;
         if (nc > kIndexOrderColliders) {
-            const int nparts = std::min(256, grid_for(nc));
-            LAUNCH_T("bp_bounds", nparts, 256, bp_bounds, C, bp_partial);
-            LAUNCH_T("bp_cells", grid_for(nc), 256, bp_cells, C, bp_partial, nparts,
+            LAUNCH_T("bp_cells", grid_for(nc, kOrderSamples), kOrderSamples, bp_cells, C, bp_sample, bp_nsample,
                      (float)std::max(1, nc / nworlds), bp_keys, bp_vals);
             uint64_t* k = bp_keys;
             int* v = bp_vals;

@@ -22,6 +22,7 @@
 #include "kcommon.h"
 #include "rp3d_internal.h"
 #include "refit_dev.h"
+#include "strips.h"
 
 namespace rp3dg {
 
@@ -76,81 +77,53 @@ __device__ __forceinline__ bool pair_allowed(const DevColliders& C, int a, int b
 }
 
 // ---------------------------------------------------------------------------------------------
-// Order of the colliders: strips across the second largest extent of the moving colliders' centres, run along
-// the largest, every other strip backwards; 8 bits of strip, 16 of position, the world id above them.  A
-// strip is as wide as 64 colliders of a world of mean density are long, so a run of 64 is about square, and
-// as consecutive keys are neighbours throughout, no run has a box larger than its neighbours'.  (On a curve
-// in three dimensions, Morton or Hilbert, the runs across its larger turns meet a good part of the scene,
-// and the longest workgroup sets the time: bp_pairs took 1238 and 650 us for 65,536 bodies there, 70 on strips.)
+// Order of the colliders (strips.h).  Every workgroup finds the bounds for itself, by the ranks of the sample's
+// centres: 3 us of integer compares, where bounds from all centres took a launch of their own.
 // ---------------------------------------------------------------------------------------------
 
-__global__ void bp_bounds(DevColliders C, float4* partial) {
-    __shared__ float smn[3][256], smx[3][256];
-    V3 mn = v3(kDecimalLargest, kDecimalLargest, kDecimalLargest);
-    V3 mx = v3(kDecimalSmallest, kDecimalSmallest, kDecimalSmallest);
-    RP3DG_GRID_STRIDE(i, C.n) {
-        if (C.is_static[i]) continue;   // a floor or wall need not lie where the others are
-        const V3 a = ld3(C.amin, i), b = ld3(C.amax, i);
-        const V3 c = v3((a.x + b.x) * 0.5f, (a.y + b.y) * 0.5f, (a.z + b.z) * 0.5f);
-        mn = vmin(mn, c);
-        mx = vmax(mx, c);
-    }
-    const int t = threadIdx.x;
-    smn[0][t] = mn.x; smn[1][t] = mn.y; smn[2][t] = mn.z;
-    smx[0][t] = mx.x; smx[1][t] = mx.y; smx[2][t] = mx.z;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (t < s) {
-            for (int k = 0; k < 3; k++) {
-                smn[k][t] = fminf(smn[k][t], smn[k][t + s]);
-                smx[k][t] = fmaxf(smx[k][t], smx[k][t + s]);
-            }
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        partial[2 * blockIdx.x] = make_float4(smn[0][0], smn[1][0], smn[2][0], 0.f);
-        partial[2 * blockIdx.x + 1] = make_float4(smx[0][0], smx[1][0], smx[2][0], 0.f);
-    }
+__device__ __forceinline__ V3 box_centre(const DevColliders& C, int i) {
+    const V3 a = ld3(C.amin, i), b = ld3(C.amax, i);
+    return v3((a.x + b.x) * 0.5f, (a.y + b.y) * 0.5f, (a.z + b.z) * 0.5f);
 }
 
-// world_colliders: colliders of a mean world
-__global__ __launch_bounds__(256) void bp_cells(DevColliders C, const float4* partial, int nparts, float world_colliders,
-                                                uint64_t* keys, int* vals) {
-    __shared__ float s_lo[2], s_scale[2];   // of the strips, of the positions in a strip
-    __shared__ int s_axis[2], s_strips;
-    if (threadIdx.x < kWave) {
-        float4 mn = make_float4(INFINITY, INFINITY, INFINITY, 0.f), mx = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
-        for (int p = threadIdx.x; p < nparts; p += kWave) box_union(mn, mx, partial[2 * p], partial[2 * p + 1]);
-        wave_box_union(mn, mx);
-        if (threadIdx.x == 0) {
-            const float lo[3] = {mn.x, mn.y, mn.z};
-            float e[3] = {mx.x - mn.x, mx.y - mn.y, mx.z - mn.z};
-            for (float& x : e) x = x > 0.f && x < INFINITY ? x : 0.f;   // (no moving collider: all 0)
-            int a = 0;
-            for (int k = 1; k < 3; k++) a = e[k] > e[a] ? k : a;
-            int b = a == 0 ? 1 : 0;
-            for (int k = 0; k < 3; k++) b = k != a && e[k] > e[b] ? k : b;
-            const float width = 8.0f * sqrtf(e[a] * e[b] / world_colliders);
-            const float strips = width > 0.f ? fminf(fmaxf(ceilf(e[b] / width), 1.f), (float)(1 << kStripBits)) : 1.f;
-            s_axis[0] = b;
-            s_axis[1] = a;
-            s_strips = (int)strips;
-            s_lo[0] = lo[b];
-            s_lo[1] = lo[a];
-            s_scale[0] = e[b] > 0.f ? strips / e[b] : 0.f;
-            s_scale[1] = e[a] > 0.f ? 65535.0f / e[a] : 0.f;
-        }
+// sample: up to kOrderSamples moving colliders; world_colliders: colliders of a mean world
+__global__ __launch_bounds__(kOrderSamples) void bp_cells(DevColliders C, const int* sample, int nsample, float world_colliders,
+                                                          uint64_t* keys, int* vals) {
+    __shared__ uint4 s_rank[kOrderSamples];
+    __shared__ float s_bound[2][3];
+    __shared__ StripOrder s_order;
+    static_assert(kOrderSamples == 256, "eight bits of thread in a rank key");
+    const int t = threadIdx.x;
+    V3 c = v3(INFINITY, INFINITY, INFINITY);
+    if (t < nsample) c = box_centre(C, sample[t]);
+    const bool ok = fabsf(c.x) < INFINITY && fabsf(c.y) < INFINITY && fabsf(c.z) < INFINITY;
+    // the float's leading 24 bits in an order of integers, and the thread, so that no two are equal
+    auto key = [&](float x) -> uint32_t {
+        const uint32_t u = __float_as_uint(x);
+        return ok ? ((u ^ (u >> 31 ? 0xffffffffu : 0x80000000u)) & ~255u) | (uint32_t)t : 0xffffffffu;
+    };
+    const uint4 mine = make_uint4(key(c.x), key(c.y), key(c.z), 0u);
+    s_rank[t] = mine;
+    if (t < 3) s_bound[0][t] = s_bound[1][t] = 0.f;
+    const int m = __syncthreads_count(ok);
+    int rank[3] = {0, 0, 0};
+#pragma unroll 8
+    for (int j = 0; j < kOrderSamples; j++) {
+        const uint4 o = s_rank[j];
+        rank[0] += o.x < mine.x ? 1 : 0;
+        rank[1] += o.y < mine.y ? 1 : 0;
+        rank[2] += o.z < mine.z ? 1 : 0;
+    }
+    for (int k = 0; k < 3; k++) {
+        if (ok && rank[k] == m / kOrderCut) s_bound[0][k] = comp(c, k);
+        if (ok && rank[k] == m - 1 - m / kOrderCut) s_bound[1][k] = comp(c, k);
     }
     __syncthreads();
+    if (t == 0) s_order = strip_order(s_bound[0], s_bound[1], world_colliders);
+    __syncthreads();
     RP3DG_GRID_STRIDE(i, C.n) {
-        const V3 a = ld3(C.amin, i), b = ld3(C.amax, i);
-        const V3 c = v3((a.x + b.x) * 0.5f, (a.y + b.y) * 0.5f, (a.z + b.z) * 0.5f);
-        const float u = (comp(c, s_axis[0]) - s_lo[0]) * s_scale[0], v = (comp(c, s_axis[1]) - s_lo[1]) * s_scale[1];
-        const uint32_t strip = (uint32_t)fminf(fmaxf(u, 0.f), (float)(s_strips - 1));
-        uint32_t pos = (uint32_t)fminf(fmaxf(v, 0.f), 65535.f);
-        if (strip & 1u) pos = 65535u - pos;
-        keys[i] = ((uint64_t)(uint32_t)C.world[i] << kCellBits) | (strip << 16) | pos;
+        const V3 p = box_centre(C, i);
+        keys[i] = ((uint64_t)(uint32_t)C.world[i] << kCellBits) | strip_key(s_order, comp(p, s_order.axis[0]), comp(p, s_order.axis[1]));
         vals[i] = i;
     }
 }

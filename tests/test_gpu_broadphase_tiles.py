@@ -1,6 +1,7 @@
 """The tile broadphase (index order up to 8,192 colliders, strips beyond) lists the same oriented pairs as
 the per-world box scan, step after step: sizes around a tile, several worlds per tile, more colliders
-than the index order takes, and moving bodies that overlap more colliders than a slab holds."""
+than the index order takes, moving bodies that overlap more colliders than a slab holds, and bodies far from the
+others."""
 import numpy as np
 import pytest
 
@@ -12,6 +13,20 @@ pytestmark = pytest.mark.gpu
 def _heap(n, seed):
     side = max(6.0, float(np.sqrt(n * 0.6)))
     return S.mixed_container(n, extent=(side, side, 12.0), seed=seed)
+
+
+def _spread(n, seed):
+    """A heap of n bodies, a twentieth of them far away in all directions, two beyond what a float resolves."""
+    sc = _heap(n, seed)
+    rng = np.random.default_rng(seed)
+    for i in range(5, len(sc.bodies), 20):   # (a floor and four walls first)
+        b = list(sc.bodies[i])
+        b[1] = tuple(float(x) for x in rng.normal(size=3) * 10.0 ** rng.uniform(2.0, 6.0))
+        sc.bodies[i] = tuple(b)
+    for i, x in ((6, 3e18), (7, -3e18)):
+        if i < len(sc.bodies):
+            sc.bodies[i] = (sc.bodies[i][0], (x, x, x)) + tuple(sc.bodies[i][2:])
+    return sc
 
 
 def _plate(n, seed):
@@ -32,6 +47,7 @@ def _plate(n, seed):
     ("plate over a slab", lambda: [_plate(150, 7), _plate(64, 8)]),
     ("plates, many", lambda: [_plate(400, 9 + k) for k in range(4)]),
     ("strips", lambda: [_heap(380, 20 + k) for k in range(22)] + [_plate(300, 50)]),
+    ("strips, far bodies", lambda: [_spread(380, 20 + k) for k in range(23)]),
 ], ids=lambda x: x if isinstance(x, str) else "")
 def test_tiles_list_the_scans_pairs(name, worlds):
     from reactphysics3d_amd.lib import Batch
