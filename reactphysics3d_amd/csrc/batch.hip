@@ -1255,7 +1255,7 @@ int rp3dg_batch::enqueue_broadphase(bool capturing, const DevEvents& E, int pg) 
             if (r) { set_error("radix sort overflow"); return r; }
             order = v;
         }
-        const int ntiles = (nc + 63) / 64;
+        const int ntiles = std::max(1, (nc + 63) / 64);   // (a launch without workgroups is an error)
         LAUNCH_T("bp_tiles", grid_for(nc), 256, bp_tiles, C, order, nc, bp_smn, bp_smx, bp_tmn, bp_tmx);
         LAUNCH_T("bp_pairs", ntiles, ntiles > 512 ? 256 : 1024, bp_pairs, C, nc, bp_smn, bp_smx, bp_tmn, bp_tmx, d_wcoll,
                  nocol_lists, bp_count, bp_slab, bp_large, &counters->nb_large);

@@ -61,3 +61,16 @@ def test_tiles_list_the_scans_pairs(name, worlds):
             assert np.array_equal(x, y), f"step {k}: pairs differ"
     for x, y in zip(a.bodies(), b.bodies()):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("kw", [dict(solver="per_color"), dict(solver="fused", broadphase="tree"), dict(solver="fused")])
+def test_worlds_without_colliders_step(kw):
+    from reactphysics3d_amd.lib import Batch
+    sc = S.Scene("points", S.make_settings(gravity=(0.0, 0.0, -10.0)))
+    for i in range(5):   # (no collider, no mass: gravity leaves them alone)
+        sc.add_body(S.DYNAMIC, (3.0 * i, 0.0, 0.0), lin=(0.0, 0.5, 0.25))
+    dev = Batch([sc, sc], **kw)
+    dev.step(1.0 / 64.0, 8)
+    p = dev.bodies()[0]
+    want = np.array([(3.0 * (i % 5), 0.5 * 8 / 64, 0.25 * 8 / 64) for i in range(10)], np.float32)
+    assert np.array_equal(p, want) and len(dev.pairs()[0]) == 0   # (exact in FP32)
