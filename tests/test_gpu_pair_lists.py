@@ -110,3 +110,43 @@ def test_mesh_search_finds_the_smallest_penetration(points):
     assert (depth[touch] <= 1.005 * want[touch] + 0.0015).all()
     hit = touch & (depth > 0.0)
     assert np.median(depth[hit] / want[hit]) > 0.9
+
+
+class _Copies:
+    """A batch of worlds that repeat a few built ones."""
+
+    def __init__(self, scenes, which):
+        import ctypes
+        from reactphysics3d_amd import lib
+        self.batch = lib.Batch.__new__(lib.Batch)
+        worlds = [lib.world_from_scene(sc) for sc in scenes]
+        handles = (ctypes.c_void_p * len(which))(*[worlds[w] for w in which])
+        b = self.batch
+        b.worlds, b.scenes, b.nb = worlds, [scenes[w] for w in which], 2 * len(which)
+        b.body_base = b.collider_base = 2 * np.arange(len(which) + 1)
+        b.joint_base = np.zeros(len(which) + 1, np.int64)
+        b.h = lib.load().rp3dg_batch_create(handles, len(which))
+        assert b.h, lib.last_error()
+
+
+# 4,096 mesh pairs are the last with 2 a wavefront, 16,384 box pairs the last with 8 (np_wave_pairs)
+@pytest.mark.parametrize("counts", [(4096, 16385), (4097, 16384), (8195, 17)])
+def test_wider_shares_in_long_lists(counts):
+    types = [(S.HULL, S.HULL), (S.HULL, S.BOX), (S.BOX, S.BOX)]
+    kinds = [(t, k) for t in range(3) for k in range(5)]
+    which = np.array([i % 10 for i in range(counts[0])] + [10 + i % 5 for i in range(counts[1])])
+    which = which[np.random.default_rng(3).permutation(len(which))]
+    scenes = [_pair(*types[t], k) for t, k in kinds]
+    dev = _Copies(scenes, which).batch
+    dev.step(1.0 / 60.0, 1)
+    ct, state = dev.contacts(), dev.bodies()
+    order = np.argsort(ct["colliders"][:, 0] // 2, kind="stable")
+    assert np.array_equal(ct["colliders"][order, 0] // 2, np.arange(len(which)))   # one manifold a world
+    for k, sc in enumerate(scenes):
+        n, *want = _run([sc], 1)[0]
+        at = order[which == k]
+        assert (ct["nb_points"][at] == n[0]).all()
+        for key, w in zip(("normal_depth", "local1", "local2", "impulse"), want):
+            assert (ct[key][at][:, :n[0]] == w).all(), (kinds[k], key)
+        for a, w in zip(state, want[4:]):
+            assert (a.reshape(len(which), 2, -1)[which == k] == w).all(), kinds[k]
