@@ -19,6 +19,10 @@ REF_LIB_F64 = os.path.join(HERE, "_ref", "librp3d_ref_harness_f64.so")
 _libs = {}
 
 
+class HarnessMissing(RuntimeError):
+    """The reference harness is not built (its sources are not here)."""
+
+
 def available(f64=False) -> bool:
     return os.path.exists(REF_LIB_F64 if f64 else REF_LIB)
 
@@ -28,7 +32,7 @@ def load(f64=False):
     if path in _libs:
         return _libs[path]
     if not os.path.exists(path):
-        raise RuntimeError(f"reference harness not built: {path} (make -C oracle)")
+        raise HarnessMissing(f"reference harness not built: {path} (make -C oracle)")
     L = C.CDLL(path)
     vp, i32, f = C.c_void_p, C.c_int32, C.c_float
     fptr, iptr = C.POINTER(C.c_float), C.POINTER(C.c_int32)
