@@ -42,11 +42,10 @@ def log(*a):
 
 
 # Algorithmic (compulsory) HBM bytes per launch: every datum a launch must read or write, once.
-# c = counts of a step, nj = joints, ndyn = dynamic bodies.
-def bytes_per_launch(name, c, ndyn, nj):
+# c = counts of a step, nj = joints, ndyn = dynamic bodies, sweep_launches = launches that share a sweep's rows.
+def bytes_per_launch(name, c, ndyn, nj, sweep_launches=1.0):
     nt = c["nb_tests"]
     m, p = c["nb_manifolds"], c["nb_contact_points"]
-    ncol = max(1, c["nb_colors"])
     nb, ncl, npairs = c["nb_bodies"], c["nb_colliders"], c["nb_pairs"]
     if name == "np_pairs":
         # the pair records and contact points; with convex meshes (their data is L2 resident) the kernel is
@@ -60,7 +59,8 @@ def bytes_per_launch(name, c, ndyn, nj):
         # position integration + commit (192 B / dynamic body), world_position also refits (48 B / collider)
         return 192 * ndyn + (48 * ncl if name == "world_position" else 0)
     if name in ("sv_solve_color", "sv_warmstart"):
-        return (48 * p + 88 * m + 140 * 2 * m) / ncol
+        # a launch a colour, the last colours together in one
+        return (48 * p + 88 * m + 140 * 2 * m) / sweep_launches
     if name == "sv_setup":   # velocity integration and contact rows
         return nb * (16 * 9 + 16 * 5) + 420 * m + 256 * p
     if name == "bp_pairs":   # boxes in, partner lists out
@@ -105,6 +105,7 @@ BYTE_MODEL = {
     "sv_world_solve": "48 B/contact point + 88 B/manifold + 140 B/dynamic body + 200 B/joint per launch (one step)",
     "world_position": "192 B/dynamic body + 48 B/collider per launch (one step)",
     "np_pairs": "176 B/test + 40 B/contact point",
+    "sv_solve_color": "a sweep's 48 B/contact point + 368 B/manifold (two bodies with it) over its launches",
 }
 
 KERNELS = ["bp_cells", "bp_sort", "bp_tiles", "bp_pairs", "bp_emit", "bp_emit_large", "bp_world_scan",
@@ -469,8 +470,12 @@ def main():
         cp = main_dev.counts()
         main_dev.profile(False)
         kernels = {}
+
+        def sweep_launches(k, per_step):   # launches of k that share the rows of one sweep
+            return per_step / max(1, main_dev.scenes[0].settings["vel_iters"]) if k == "sv_solve_color" else max(1.0, per_step)
+
         for k, (ms, n) in items.items():
-            b = bytes_per_launch(k, cp, ndyn, nj)
+            b = bytes_per_launch(k, cp, ndyn, nj, sweep_launches(k, n / nprof))
             e = {"mean_us": round(ms * 1e3, 2), "launches_per_step": round(n / nprof, 2)}
             if b is not None:
                 e["gb_s"] = round(b / (ms * 1e-3) / 1e9, 2)
@@ -479,6 +484,7 @@ def main():
                 fl = poly_flops_per_launch(cp, hs)
                 e["tflop_s"] = round(fl / (ms * 1e-3) / 1e12, 3)
                 e["valu_frac"] = round(fl / (ms * 1e-3) / VALU_FP32_PEAK, 5)
+                e["flop_model"] = "mesh pairs only, over the time of the launch that takes all pairs"
             if k == "mlp_infer":
                 fl = MLP_INFER_FLOP * cp["nb_new_points"]
                 e["tflop_s"] = round(fl / (ms * 1e-3) / 1e12, 3)
@@ -512,9 +518,10 @@ def main():
                             "peak": VALU_FP32_PEAK / 1e12, "unit": "TFLOP/s",
                             "frac": round(achieved * 1e12 / VALU_FP32_PEAK, 5), "traffic": traffic,
                             "flop_model": "6 (F1 V2 + F2 V1) + 30 E1 E2 per mesh test, mean mesh "
-                                          f"F {hs[0]:.1f} V {hs[1]:.1f} E {hs[2]:.1f}"}
+                                          f"F {hs[0]:.1f} V {hs[1]:.1f} E {hs[2]:.1f}; mesh pairs only, over the "
+                                          "time of the launch that takes all pairs"}
             else:
-                b = bytes_per_launch(dominant, cd, ndyn, nj)
+                b = bytes_per_launch(dominant, cd, ndyn, nj, sweep_launches(dominant, n / args.steps))
                 achieved = b / (ms * 1e-3) / 1e9
                 roofline = {"kernel": dominant, "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
@@ -522,7 +529,7 @@ def main():
             roofline.update({"traffic_source": traffic_src, "mean_launch_us": round(ms * 1e3, 2), "launches": n,
                              "timing": "HIP events around the kernel on the batch's stream, eager pass of the same "
                                        "number of steps directly after the timed regions",
-                             "share_of_step": round(ms / (wall * 1e3 / args.steps), 3)})
+                             "share_of_step": round(ms * n / (wall * 1e3), 3)})
             if dominant == "sv_world_solve" and learned and learned.get("mean_velocity_iterations"):
                 # every sweep re-reads the rows: 80 B / point (normal, r1, r2, impulse r/w) + 124 B / manifold
                 sweep = 80 * cd["nb_contact_points"] + 124 * cd["nb_manifolds"]

@@ -91,7 +91,7 @@ struct rp3dg_batch {
     int2* d_class_ranges = nullptr;      // (first, count) of every world class in that order
     bool order_by_sweeps = true;
     std::vector<int> world_group;        // [nworlds]
-    int *d_gworld = nullptr, *d_world_group = nullptr;
+    int* d_gworld = nullptr;
     int* d_wmstart = nullptr;            // [nworlds + 1] first manifold of each world (fused colouring)
     int max_group_bodies = 0;
     bool world_scan = false;             // broadphase by per-world box scans in LDS instead of tiles
@@ -188,7 +188,7 @@ struct rp3dg_batch {
     int* bp_sample = nullptr;          // moving colliders that give the order its extents
     int bp_nsample = 0;
     // narrowphase
-    int *np_lists = nullptr, *np_counts = nullptr;
+    int* np_lists = nullptr;
     // manifolds / colouring
     int *m_flag = nullptr, *m_offs = nullptr, *m_list = nullptr;
     int *adj_cnt = nullptr, *adj_offs = nullptr, *adj_cursor = nullptr, *adj = nullptr;

@@ -1036,7 +1036,6 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     }
     bp_out = dalloc<uint64_t>(this, pair_cap);
     np_lists = dalloc<int>(this, (size_t)kNpListSlots * pair_cap);
-    np_counts = dalloc<int>(this, ALGO_COUNT);
     m_flag = dalloc<int>(this, pair_cap); m_offs = dalloc<int>(this, pair_cap + 1);
     m_list = dalloc<int>(this, man_cap);
     adj_cnt = dalloc<int>(this, nb + 1); adj_offs = dalloc<int>(this, nb + 1); adj_cursor = dalloc<int>(this, nb);
@@ -1053,7 +1052,6 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     d_wcoll = dalloc<int>(this, nw + 1);
     d_block_world = dalloc<int>(this, ngroups);
     d_gworld = dalloc<int>(this, ngroups + 1);
-    d_world_group = dalloc<int>(this, nw);
     d_wmstart = dalloc<int>(this, nw + 1);
     res_pv = dalloc<float4>(this, nb);
     res_pw = dalloc<float4>(this, nb);
@@ -1074,7 +1072,6 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
         if (!d_block_static) { set_error("device allocation failed (group order)"); return RP3DG_EHIP; }
         HIPCHECK(hipMemcpy(d_block_static, order.data(), sizeof(int) * ng, hipMemcpyHostToDevice));
         HIPCHECK(hipMemcpy(d_gworld, group_world.data(), sizeof(int) * (ng + 1), hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(d_world_group, world_group.data(), sizeof(int) * nw, hipMemcpyHostToDevice));
         // size classes over the size-sorted group order (largest class first)
         wclasses.clear();
         if (fused) {
@@ -1139,7 +1136,7 @@ int rp3dg_batch::upload(rp3dg_world* const* ws, int nw, const rp3dg_batch_option
     HIPCHECK(hipStreamSynchronize(stream));
 
     // Static colliders never move, so their mutual overlaps are fixed at creation: list them once
-    // (same closed AABB test and pair filter as the device traversal).
+    // (the closed AABB test and the pair filter of the device).
     std::vector<int> is_static(nc, 0), ss_offs(nc + 1, 0), ss_list;
     for (int i = 0; i < nc; i++) is_static[i] = (flags[cbody[i]] & (BF_DYNAMIC | BF_KINEMATIC)) == 0;
     {
@@ -1699,7 +1696,6 @@ int rp3dg_batch::finish_steps(int n) {
         std::string what;
         if (last.status & STATUS_PAIR_OVERFLOW) what += " pair table overflow (raise pairs_per_collider);";
         if (last.status & STATUS_COLOR_OVERFLOW) what += " more than 64 solver colours;";
-        if (last.status & STATUS_STACK_OVERFLOW) what += " broadphase traversal stack overflow;";
         if (last.status & STATUS_COLOR_STALL) what += " colouring did not finish;";
         if (last.status & STATUS_CLIP_OVERFLOW) what += " face clipping exceeded its buffer;";
         set_error("device status " + std::to_string(last.status) + ":" + what);
@@ -1841,7 +1837,6 @@ int rp3dg_batch::query(int mode, int report, int body1, int body2) {
     if (c.status) {
         std::string what;
         if (c.status & STATUS_PAIR_OVERFLOW) what += " pair table overflow (raise pairs_per_collider);";
-        if (c.status & STATUS_STACK_OVERFLOW) what += " broadphase traversal stack overflow;";
         if (c.status & STATUS_CLIP_OVERFLOW) what += " face clipping exceeded its buffer;";
         set_error("world query: device status " + std::to_string(c.status) + ":" + what);
         return RP3DG_EOVERFLOW;

@@ -194,7 +194,6 @@ __global__ __launch_bounds__(kSortThreads) void rs_scatter(const uint64_t* kin, 
                 wcnt[w][t] = run;
                 run += c;
             }
-            wcnt[0][t] += 0;
             __syncthreads();
             if (valid) {
                 const int pos = base[d] + wcnt[wid][d] + rank;
@@ -541,7 +540,7 @@ __device__ __forceinline__ int select_algo(int t1, int t2) {
     return ALGO_POLY_POLY;
 }
 
-// nkeys_ptr: overlapping pairs found (clamped to the capacity; an overflow is flagged by the traversal).
+// nkeys_ptr: overlapping pairs found (clamped to the capacity; bp_emit and bp_world_scan flag an overflow).
 // nold_ptr: size of the previous table O.  nnew_ptr / nb_pairs_ptr receive the size of the new table N.
 // old_offs: first entry of every emitter's segment in the previous table (its keys are sorted and
 // grouped by emitter, key >> 32), so a key is searched only within its emitter's few old entries.

@@ -222,7 +222,6 @@ constexpr int kNpBins = ALGO_COUNT + 5;
 
 struct DevCounters {
     int nb_pairs;              // pairs in the current table
-    int nb_overlaps;           // overlapping pairs found by the traversal (may exceed the capacity)
     int nb_bin[kNpBins];       // tests per narrowphase bin
     int nb_manifolds;
     int nb_points;
@@ -240,7 +239,6 @@ struct DevCounters {
 
 constexpr int STATUS_PAIR_OVERFLOW = 1;
 constexpr int STATUS_COLOR_OVERFLOW = 2;
-constexpr int STATUS_STACK_OVERFLOW = 4;
 constexpr int STATUS_COLOR_STALL = 8;
 constexpr int STATUS_CLIP_OVERFLOW = 16;   // a face clip produced more vertices than its buffer holds
 constexpr int STATUS_CONCAVE_OVERFLOW = 32;   // concave pairs: triangle tests, their points or manifolds over capacity

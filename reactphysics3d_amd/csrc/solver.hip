@@ -3,9 +3,10 @@
 // Colouring is Jones-Plassmann with hashed priorities: a manifold takes the
 // smallest colour unused by its higher-priority neighbours once they are all
 // coloured, which equals sequential greedy colouring in priority order and is
-// therefore deterministic.  A fixed number of parallel rounds is launched (each
-// returns at once when nothing is left) and a single-workgroup finisher
-// completes whatever remains, so the step needs no host round trip.
+// therefore deterministic.  A launch colours as far as bounded waiting goes,
+// nearly always everything; another finds nothing left and returns at once, or
+// goes on, and a single-workgroup finisher completes whatever remains, so the
+// step needs no host round trip.
 #include <hip/hip_runtime.h>
 
 #include "kcommon.h"
@@ -522,9 +523,8 @@ __global__ __launch_bounds__(1024) void sv_group_color(ColorArgs A) {
     }
 }
 
-// Segment key of every manifold: its colour, or (world group, colour) when the solver runs one workgroup
-// per group of consecutive worlds (world_group != null).  Counts per segment and the number of colours
-// are accumulated for the segment table.
+// Segment key of every manifold: its colour.  Counts per segment and the number of colours are accumulated for
+// the segment table.
 __global__ __launch_bounds__(256) void sv_color_keys(const int* color, const int* nm_ptr, uint64_t* keys, int* vals,
                                                      int* seg_cnt, int* ncolors) {
     __shared__ int hist[kMaxColors];

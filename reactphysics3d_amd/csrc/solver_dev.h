@@ -238,19 +238,6 @@ __device__ __forceinline__ void sv_prepare_one(const SvArgs& A, int i) {
     }
 }
 
-// ------------------------------------------------------------------------------------------------
-// Per-colour sweeps
-// ------------------------------------------------------------------------------------------------
-
-struct BodyVel {
-    V3 v, w;
-};
-
-__device__ __forceinline__ void load_body(const DevBodies& B, int b, const float4* lin, const float4* ang, V3& v, V3& w) {
-    v = ld3(lin, b);
-    w = ld3(ang, b);
-}
-
 // Learned warm start: the 24 features of contact point p of solver row i (after sv_prepare_one and
 // the velocity integration): normal, r1, r2, relative velocity in the (t1, t2, n) frame, inverse
 // masses, world inverse inertia (xx of each body), the manifold's cached normal impulses (sum over
