@@ -531,8 +531,9 @@ def main():
                                        "number of steps directly after the timed regions",
                              "share_of_step": round(ms * n / (wall * 1e3), 3)})
             if dominant == "sv_world_solve" and learned and learned.get("mean_velocity_iterations"):
-                # every sweep re-reads the rows: 80 B / point (normal, r1, r2, impulse r/w) + 124 B / manifold
-                sweep = 80 * cd["nb_contact_points"] + 124 * cd["nb_manifolds"]
+                # every sweep re-reads the constant rows: 80 B / point (normal, lever arms and inverse inertia x (arm x
+                # normal) of both bodies) + 96 B / manifold (friction arms, tangents, normal, masses)
+                sweep = 80 * cd["nb_contact_points"] + 96 * cd["nb_manifolds"]
                 its = learned["mean_velocity_iterations"]
                 roofline["row_bytes_per_sweep"] = int(sweep)
                 roofline["row_traffic_gbs"] = round(sweep * its / (ms * 1e-3) / 1e9, 2)

@@ -173,7 +173,7 @@ __device__ __forceinline__ int header_points(unsigned int h) { return (int)(h >>
 // Warm start, velocity iterations and impulse store of one group of worlds.  The body state is in LDS or
 // HBM as STATE says (solver_quad.h).  When the group has at most F.lds_rows manifolds and only unit lock
 // factors (`fast`), the accumulated impulses and the headers of its rows are in LDS too: the sweeps then
-// read the constant part of a row (up to 352 B) from HBM and write nothing there, and the next row is
+// read the constant part of a row (up to 416 B) from HBM and write nothing there, and the next row is
 // loaded while the current one is solved.  (The two cases are separate code: a pointer that may be either
 // becomes a flat access, which waits for every load in flight.)
 template <bool SPLIT, int STATE>
