@@ -19,6 +19,8 @@
            --bytes-read / --bytes-write (repeatable) is also turned into bytes by the value it reads on
            the copy kernel, which moves copy-bytes each way.
 --kernels K1,K2 : restrict the --pmc tables to these kernels (and the copy kernel).
+--classes KERNEL : count the dispatches of KERNEL by workgroup size, as KERNEL/size (repeatable; the solver's
+           size classes are launches side by side, and a step's is their sum, which --traffic-json writes).
 --top-dispatches KERNEL=N : count only the N dispatches of KERNEL with the largest value of each
            counter (repeatable; for counter runs whose records carry no usable dispatch times).
 """
@@ -32,19 +34,27 @@ from collections import defaultdict
 
 
 def short_name(name: str) -> str:
-    """`rp3dg::np_poly_poly(rp3dg::NpArgs, ...)` -> `np_poly_poly`; torch kernels keep a short tag."""
+    """`rp3dg::np_pairs(rp3dg::NpArgs, ...)` -> `np_pairs`; torch kernels keep a short tag."""
     base = name.split("(")[0]
     base = re.sub(r"<.*", "", base)
     return base.split("::")[-1][:60]
 
 
+CLASSES = set()   # kernels counted by workgroup size (--classes)
+
+
+def class_name(name, workgroup):
+    k = short_name(name)
+    return f"{k}/{workgroup}" if k in CLASSES else k
+
+
 def kernel_trace(db: str, min_us=None):
     """Per kernel: list of dispatch durations in microseconds (from start/end timestamps in ns)."""
     c = sqlite3.connect(db)
-    rows = c.execute("select name, start, end from kernels").fetchall()
+    rows = c.execute("select name, start, end, workgroup_x from kernels").fetchall()
     agg = defaultdict(list)
-    for name, t0, t1 in rows:
-        k, us = short_name(name), (t1 - t0) / 1e3
+    for name, t0, t1, wg in rows:
+        k, us = class_name(name, wg), (t1 - t0) / 1e3
         if min_us and us < min_us.get(k, 0.0):
             continue
         agg[k].append(us)
@@ -55,17 +65,17 @@ TOP = {}   # kernel -> number of largest dispatches kept (--top-dispatches)
 
 
 def _keep(k, vals):
-    n = TOP.get(k)
+    n = TOP.get(k.split("/")[0])
     return sorted(vals)[-n:] if n else vals
 
 
 def counter_means(db: str, counter: str, min_us=None):
     c = sqlite3.connect(db)
-    rows = c.execute("select kernel_name, value, start, end from counters_collection where counter_name = ?",
+    rows = c.execute("select kernel_name, value, start, end, workgroup_size_x from counters_collection where counter_name = ?",
                      (counter,)).fetchall()
     agg = defaultdict(list)
-    for name, v, t0, t1 in rows:
-        k = short_name(name)
+    for name, v, t0, t1, wg in rows:
+        k = class_name(name, wg)
         if min_us and (t1 - t0) / 1e3 < min_us.get(k, 0.0):
             continue
         agg[k].append(float(v))
@@ -76,10 +86,10 @@ def counter_means(db: str, counter: str, min_us=None):
 def all_counters(db: str, min_us=None):
     """{counter: {kernel: (mean per dispatch, dispatches)}} of every counter in a --pmc database."""
     c = sqlite3.connect(db)
-    rows = c.execute("select counter_name, kernel_name, value, start, end from counters_collection").fetchall()
+    rows = c.execute("select counter_name, kernel_name, value, start, end, workgroup_size_x from counters_collection").fetchall()
     agg = defaultdict(lambda: defaultdict(list))
-    for cn, name, v, t0, t1 in rows:
-        k = short_name(name)
+    for cn, name, v, t0, t1, wg in rows:
+        k = class_name(name, wg)
         if min_us and (t1 - t0) / 1e3 < min_us.get(k, 0.0):
             continue
         agg[cn][k].append(float(v))
@@ -112,10 +122,12 @@ def main(argv=None):
     ap.add_argument("--bytes-read", action="append", default=[], metavar="COUNTER")
     ap.add_argument("--bytes-write", action="append", default=[], metavar="COUNTER")
     ap.add_argument("--kernels", default="")
+    ap.add_argument("--classes", action="append", default=[], metavar="KERNEL")
     ap.add_argument("--top-dispatches", action="append", default=[], metavar="KERNEL=N")
     a = ap.parse_args(argv)
     min_us = {kv.split("=")[0]: float(kv.split("=")[1]) for kv in a.min_us}
     TOP.update({kv.split("=")[0]: int(kv.split("=")[1]) for kv in a.top_dispatches})
+    CLASSES.update(a.classes)
     if min_us:
         out_filter = ", ".join(f"{k} >= {v:g} us" for k, v in min_us.items())
     out = []
@@ -165,6 +177,10 @@ def main(argv=None):
         if a.traffic_json and scale_f and scale_w:
             import json
             tj = {k: int(f[k][0] * 1024 * scale_f + w[k][0] * 1024 * scale_w) for k in set(f) & set(w)}
+            for k in CLASSES:
+                parts = [v for n, v in tj.items() if n.startswith(k + "/")]
+                if parts:
+                    tj[k] = sum(parts)
             tj["_measured"] = {"commit": a.commit, "command": a.command,
                                "fetch": a.fetch, "write": a.write, "copy_bytes": a.copy_bytes}
             with open(a.traffic_json, "w") as fh:
