@@ -265,7 +265,8 @@ rp3dg_batch* rp3dg_batch_create(rp3dg_world* const* worlds, int32_t nb_worlds);
 typedef struct rp3dg_batch_options {
     int32_t solver;           /* RP3DG_SOLVER_* */
     int32_t fused_block;      /* threads per world group in the fused solver (64, 128, 192 or 256; 0 = per size
-                                 class: its bodies bound, clamped to [64, 1024], autotunable) */
+                                 class: its bodies bound, clamped to [64, 1024], 256 at least in up to
+                                 256 groups with joints; autotunable) */
     int32_t pairs_per_collider; /* pair-table capacity per collider (0 = 16) */
     int32_t group_bodies;     /* fused solver: consecutive worlds are packed into one workgroup up to this many
                                  bodies together (at most 64 worlds, 512 bodies; 0 = 256, 1 = one world per
