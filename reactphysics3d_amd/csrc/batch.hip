@@ -40,8 +40,9 @@ __global__ void bp_pairs(DevColliders C, int n, const float4* smn, const float4*
                          int* nb_large);
 __global__ void bp_emit(DevColliders C, int n, const int* count, const int* offset, const int* slab, uint64_t* out_keys,
                         int capacity, int* status);
-__global__ void bp_emit_large(DevColliders C, const int* wcoll, NoColLists L, const int* offset, uint64_t* out_keys,
-                              int capacity, const int* large, const int* nb_large, int* status);
+__global__ void bp_emit_large(DevColliders C, int n, const float4* smn, const float4* smx, const float4* tmn,
+                              const float4* tmx, const int* wcoll, NoColLists L, const int* count, const int* offset,
+                              const int* slab, uint64_t* out_keys, int capacity, const int* large, const int* nb_large, int* status);
 __global__ void bp_world_scan(DevColliders C, const int* gworld, const int* wcoll, const int* block_group, NoColLists L,
                               int* count, const int* offset, uint64_t* out_keys, int capacity, int pass, int* status);
 __global__ void bp_merge(DevColliders C, const uint64_t* keys, const int* nkeys_ptr, int capacity, DevPairs O,
@@ -1266,8 +1267,8 @@ int rp3dg_batch::enqueue_broadphase(bool capturing, const DevEvents& E, int pg) 
         LAUNCH_T("bp_emit", grid_for(nc * 8, 256, 1 << 20), 256, bp_emit, C, nc, bp_count, bp_offs, bp_slab, bp_out,
                  pair_cap, dstatus);
         const int hl = capturing ? 256 : std::min(nc, last.nb_large + last.nb_large / 4 + 16);
-        LAUNCH_T("bp_emit_large", std::max(1, std::min(hl, 1024)), 1024, bp_emit_large, C, d_wcoll, nocol_lists, bp_offs,
-                 bp_out, pair_cap, bp_large, &counters->nb_large, dstatus);
+        LAUNCH_T("bp_emit_large", std::max(1, std::min(hl, 1024)), 1024, bp_emit_large, C, nc, bp_smn, bp_smx, bp_tmn,
+                 bp_tmx, d_wcoll, nocol_lists, bp_count, bp_offs, bp_slab, bp_out, pair_cap, bp_large, &counters->nb_large, dstatus);
     }
     if (events_on) fill_int_n<<<pg, 256, 0, stream>>>(O.kept, pair_cap, old_count, 0);
     LAUNCH_T("bp_merge", pg, 256, bp_merge, C, bp_out, bp_offs + nc, pair_cap, O, old_count, old_offs, N, new_count,

@@ -40,6 +40,20 @@ def _plate(n, seed):
     return sc
 
 
+def _crowd(n, seed):
+    """n bodies that each overlap some 100 others, among them a compound of 80 overlapping parts."""
+    rng = np.random.default_rng(seed)
+    sc = S.Scene("crowd", S.make_settings(gravity=(0.0, 0.0, 0.0)))
+    side = 1.2 * (n / 100.0 * 4.2) ** (1.0 / 3.0)
+    parts = sc.add_body(S.DYNAMIC, (side / 2, side / 2, side / 2))
+    for p in rng.uniform(-0.3, 0.3, (80, 3)):
+        sc.add_collider(parts, S.SPHERE, (0.4,), lpos=tuple(p), trigger=True)
+    for p, v in zip(rng.uniform(0.0, side, (n, 3)), rng.normal(size=(n, 3))):
+        b = sc.add_body(S.KINEMATIC, tuple(p), lin=tuple(v))
+        sc.add_collider(b, S.SPHERE, (0.5,))
+    return sc
+
+
 @pytest.mark.parametrize("name,worlds", [
     ("one", lambda: [_heap(1, 3)]),
     ("tile edge", lambda: [_heap(59, 3), _heap(58, 4), _heap(1, 5)]),
@@ -47,13 +61,15 @@ def _plate(n, seed):
     ("plate over a slab", lambda: [_plate(150, 7), _plate(64, 8)]),
     ("plates, many", lambda: [_plate(400, 9 + k) for k in range(4)]),
     ("strips", lambda: [_heap(380, 20 + k) for k in range(22)] + [_plate(300, 50)]),
+    ("crowd", lambda: [_crowd(700, 60)]),
+    ("crowds, strips", lambda: [_crowd(600, 61 + k) for k in range(13)]),
     ("strips, far bodies", lambda: [_spread(380, 20 + k) for k in range(23)]),
 ], ids=lambda x: x if isinstance(x, str) else "")
 def test_tiles_list_the_scans_pairs(name, worlds):
     from reactphysics3d_amd.lib import Batch
     scenes = worlds()
-    a = Batch(scenes, solver="fused", broadphase="tree", pairs_per_collider=64)
-    b = Batch(scenes, solver="fused", broadphase="world_scan", pairs_per_collider=64)
+    a = Batch(scenes, solver="fused", broadphase="tree", pairs_per_collider=96)
+    b = Batch(scenes, solver="fused", broadphase="world_scan", pairs_per_collider=96)
     for k in range(12):
         a.step(1.0 / 60.0)
         b.step(1.0 / 60.0)
@@ -61,6 +77,27 @@ def test_tiles_list_the_scans_pairs(name, worlds):
             assert np.array_equal(x, y), f"step {k}: pairs differ"
     for x, y in zip(a.bodies(), b.bodies()):
         assert np.array_equal(x, y)
+
+
+# 64 partners fill a slab, 1,024 the list that is sorted in LDS; beyond 8,192 colliders the order is by strips and that
+# list is collected by tiles
+@pytest.mark.parametrize("inside,outside", [(63, 200), (64, 200), (65, 200), (1023, 200), (1024, 200), (1025, 200),
+                                            (64, 8300), (65, 8300), (300, 8300), (1024, 8300), (1025, 8300), (9000, 200)])
+def test_a_body_lists_everything_inside_it(inside, outside):
+    from reactphysics3d_amd.lib import Batch
+    sc = S.Scene("inside", S.make_settings(gravity=(0.0, 0.0, 0.0)))
+    plate = sc.add_body(S.KINEMATIC, (0.0, 0.0, 0.0))
+    sc.add_collider(plate, S.BOX, (80.0, 80.0, 1.0))
+    for i in np.random.default_rng(inside).permutation(inside + outside):
+        b = sc.add_body(S.DYNAMIC, (1.5 * (i % 100) - 75.0, 1.5 * (i // 100) - 70.0, 0.0 if i < inside else 9.0))
+        sc.add_collider(b, S.SPHERE, (0.5,), trigger=True)
+    dev = Batch(sc, solver="per_color")
+    for _ in range(2):
+        dev.step(1.0 / 60.0)
+        a, b = dev.pairs()
+        partners = np.where(a == 0, b, a)[(a == 0) | (b == 0)]
+        low = np.array([c for c in range(1, inside + outside + 1) if sc.bodies[c][1][2] == 0.0])
+        assert np.array_equal(partners, low)
 
 
 @pytest.mark.parametrize("kw", [dict(solver="per_color"), dict(solver="fused", broadphase="tree"), dict(solver="fused")])
