@@ -159,8 +159,8 @@ def cpu_baseline(scenes, args, ndyn_total):
     if not ref.available():
         log("[bench] reference harness not built; no CPU baseline")
         return None
-    # one world per host thread; 16 threads = the host CPU share of one GPU on the GPU box (the box
-    # reports more CPUs than a single-GPU job may use)
+    # one world per host thread; at most 16 threads: one GPU's share of its host's CPUs (os.cpu_count()
+    # gives those of all the GPUs)
     threads = args.cpu_threads or min(16, os.cpu_count() or 1)
     stride = max(1, len(scenes) // args.cpu_worlds) if len(scenes) > 1 else 1
     sample = scenes[::stride][: args.cpu_worlds] if len(scenes) > 1 else scenes
